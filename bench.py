@@ -501,7 +501,7 @@ def main():
     if c_cnt:
         from phd_amd.flops import chem_flops
         c_avg_s = c_ms / c_cnt / 1e3
-        c_flop = chem_flops(chem_stats) / c_cnt
+        c_flop = chem_flops(chem_stats, closed_form=tuned[3] == 2) / c_cnt
         c_ach = c_flop / c_avg_s / 1e12
         chem_roof = {"kernel": "k_reaction_queue", "bound": "fp64-valu", "achieved": c_ach,
                      "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",

@@ -280,10 +280,11 @@ int izem_chem_setup(izem_ctx *ctx, const double *mech, long nmech, double rtol, 
  * autotuner (phd_amd/autotune.py): register budget as waves per SIMD the
  * kernel variant is compiled for (1, 2 or 4), resident 64-lane blocks per
  * CU, Jacobian reuse age in BDF steps, kinetics form (0 table-driven,
- * 1 straight-line code generated for the bundled mechanism -- IZEM_E_ARG if
- * the loaded mechanism is another one or waves is not 1 --, 2 the same with
- * the closed-form mass-fraction columns of the Jacobian (same conditions),
- * -1 straight-line when it matches and waves is 1, table-driven otherwise).  No counterpart
+ * 1 straight-line code generated for the bundled mechanism with a
+ * finite-difference Jacobian -- IZEM_E_ARG if the loaded mechanism is
+ * another one or waves is not 1 --, 2 the same with the Jacobian in closed
+ * form (same conditions), -1 form 2 when it matches and waves is 1,
+ * table-driven otherwise; the setup's default is -1 at one wave).  No counterpart
  * in the reference (DVODE runs on the CPU). */
 int izem_chem_tune(izem_ctx *ctx, int waves, int blocks_per_cu, int jac_age, int kinetics);
 /* work counters of the chemistry integrations since the previous call:

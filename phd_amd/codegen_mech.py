@@ -7,22 +7,40 @@ CKWYR / FUN arithmetic (devel-izem/src/chemkin/vode.f:935-1314, 1797-1904;
 reaction_v.f:69-114) as straight-line code with every index and constant
 folded, split into
 
-  gen_kT(T, kt)              the temperature-only part: forward rate
-                             constants, equilibrium constants, falloff
-                             low-pressure limits and centring, species
-                             enthalpies / heat capacities;
-  gen_rhs(rho, z, kt, zp)    the concentration part and the reactor RHS,
+  gen_kT(T, kt)              the temperature-only part: forward and reverse
+                             rate constants, falloff limits, species
+                             internal energies / heat capacities;
+  gen_rhs(rho, z, kt, zp)    the concentration part and the reactor RHS;
+  gen_jac(rho, z, kt, f0T, J), gen_jac_T(rho, z, kt, f0, J)
+                             the mass-fraction columns and the temperature
+                             column of the reactor Jacobian in closed form.
 
-so that a finite-difference Jacobian column that perturbs a mass fraction
-reuses kt.  Both functions are compiled without FMA contraction: the
-Jacobian subtracts two inlined evaluations that share most of their terms,
-and contraction decided separately in each copy would round the shared
-terms differently and put noise of order f * eps / r into the columns.  Run:  python -m phd_amd.codegen_mech  (writes
+The integrator is bound by the instructions of these three, so the
+generator spends none that the mechanism does not need:
+
+  * Species' Gibbs energies are taken relative to a basis of species (for
+    H2/air: H2, O2, N2), which leaves every reaction's sum unchanged because
+    reactions conserve elements.  Equilibrium constants are then products of
+    one exponential per remaining species and their reciprocals, instead of
+    an exponential and a division per reaction.
+  * Rate constants without a temperature dependence, with an integer or half
+    power of T, or with a common activation energy share what they can; a
+    falloff limit enters as the ratio k0/kinf; a constant centring factor is
+    folded.
+  * Reactions with the same species on both sides (DUPLICATE) are one rate.
+  * The Jacobian's columns hold nine accumulators at a time.
+
+FMA contraction is on at the level of the source expression, which the
+compiler applies to every inlined copy alike: a finite-difference Jacobian
+column that subtracts two copies sees the same rounding in both.  (Left to
+the optimiser, contraction was decided per copy and put noise of order
+f * eps / r into the columns.)  Run:  python -m phd_amd.codegen_mech  (writes
 phd_amd/csrc/mech_gen.h, committed).
 """
 from __future__ import annotations
 
 import hashlib
+import math
 import os
 
 import numpy as np
@@ -30,6 +48,10 @@ import numpy as np
 from . import chemdata as cd
 
 OUT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc", "mech_gen.h")
+
+# |ln| bound of a species' relative equilibrium factor, so that it and its
+# reciprocal stay finite (reached below 43 K for H2/air)
+GIBBS_CLAMP = 700.0
 
 
 def _lit(x: float) -> str:
@@ -45,6 +67,49 @@ def mechanism_hash(mech: cd.Mechanism) -> str:
     return h.hexdigest()[:16]
 
 
+def _basis(mech: cd.Mechanism):
+    """Basis species of the element space, those nearest to zero enthalpy at
+    298 K first, and B[k][j]: species k has the elements of sum_j B_kj
+    basis_j."""
+    ncf = np.asarray(mech.ncf, dtype=np.float64)
+    T = 298.15
+
+    def h298(k):
+        a = mech.a[k][0]
+        return abs(sum(a[q] / (q + 1) * T ** q for q in range(5)) + a[5] / T)
+
+    basis = []
+    for k in sorted(range(mech.kk), key=h298):
+        if np.linalg.matrix_rank(ncf[basis + [k]]) > len(basis):
+            basis.append(k)
+    B, *_ = np.linalg.lstsq(ncf[basis].T, ncf.T, rcond=None)
+    B = np.round(B.T * 12) / 12.0
+    assert np.allclose(B @ ncf[basis], ncf)
+    return basis, B
+
+
+def _net(r):
+    nu = {}
+    for k, n in r["reac"]:
+        nu[k] = nu.get(k, 0) - n
+    for k, n in r["prod"]:
+        nu[k] = nu.get(k, 0) + n
+    return nu
+
+
+def _sum(terms):
+    return " + ".join(terms).replace("+ -", "- ") if terms else "0.0"
+
+
+def _scaled(coef, name):
+    """coef * name as an expression (coef a nonzero number)."""
+    if coef == 1:
+        return name
+    if coef == -1:
+        return f"-{name}"
+    return f"{_lit(coef)} * {name}"
+
+
 def generate(mech: cd.Mechanism) -> str:
     kk, ii = mech.kk, mech.ii
     L = []
@@ -54,348 +119,489 @@ def generate(mech: cd.Mechanism) -> str:
     w("// Straight-line form of CKWYR + FUN (devel-izem/src/chemkin/vode.f:935-1314,")
     w("// 1797-1904; chemkin/reaction_v.f:69-114).")
     w("#pragma once")
+    w('#include "iz_math.h"')
     w(f"#define GEN_KK {kk}")
     w(f"#define GEN_II {ii}")
     w(f'#define GEN_MECH_HASH "{mechanism_hash(mech)}"')
-    nkt = 0
+    basis, B = _basis(mech)
+    R = mech.reactions
+    # species up to the last one that any reaction changes
+    live = [k for k in range(kk) if any(_net(r).get(k) for r in R)]
+    w(f"#define GEN_NLIVE {max(live) + 1}")
+
+    # reactions that are one rate: the same sides, no falloff, the same third
+    # bodies, reverse from the equilibrium constant
+    groups = []
+    at = {}
+    for i, r in enumerate(R):
+        key = None
+        if not r["fal"] and r["rev"] and not r.get("rpar"):
+            key = (tuple(sorted(r["reac"])), tuple(sorted(r["prod"])),
+                   tuple(r["eff"]) if r["tb"] else None)
+        if key is not None and key in at:
+            groups[at[key]].append(i)
+        else:
+            if key is not None:
+                at[key] = len(groups)
+            groups.append([i])
+    # a rate constant without any dependence on T is a literal
+    const_kf = {g[0]: R[g[0]]["A"] for g in groups
+                if len(g) == 1 and R[g[0]]["b"] == 0 and R[g[0]]["EoR"] == 0}
+
+    def troe_const(r):
+        """log10 of a Troe centring factor whose temperatures make it
+        constant (exp(-T / 1e-30) = 0, exp(-T / 1e30) = 1), else None."""
+        if r["fal"] == 3 and r["fpar"][4] <= 1e-20 and r["fpar"][5] >= 1e20:
+            return math.log10(max(r["fpar"][3], 1e-300))
+        return None
+
     slots = {}
 
     def slot(name):
-        nonlocal nkt
-        slots[name] = nkt
-        nkt += 1
-        return slots[name]
+        slots[name] = len(slots)
 
-    for i in range(ii):
-        slot(f"kf{i}")
-        slot(f"kr{i}")
-        if mech.reactions[i]["fal"] == 2:
-            slot(f"klow{i}")
-            slot(f"srib{i}")
-            slot(f"srid{i}")
-        elif mech.reactions[i]["fal"]:
-            slot(f"klow{i}")
-            slot(f"fclog{i}")
+    for g in groups:
+        i, r = g[0], R[g[0]]
+        if i not in const_kf:
+            slot(f"kf{i}")
+        if r["rev"]:
+            slot(f"kr{i}")
+        if len(g) > 1:
+            slot(f"dkf{i}")  # d kf / dT of a sum of Arrhenius terms
+        if r["fal"]:
+            slot(f"rk{i}")
+            if r["fal"] == 2:
+                slot(f"srib{i}")
+                slot(f"srid{i}")
+            elif r["fal"] >= 3 and troe_const(r) is None:
+                slot(f"fclog{i}")
     for k in range(kk):
         slot(f"cvk{k}")
-        slot(f"hk{k}")
-    w(f"#define GEN_NKT {nkt}")
+        slot(f"uk{k}")
+    w(f"#define GEN_NKT {len(slots)}")
     w("")
 
-    def thermo_lines():
-        """log T, powers, and per species S/R - H/RT, cp/R, H/RT (NASA-7)."""
-        parts = ("smh", "cpR", "hRT")
-        o = ["  const double lt = log(T), it = 1.0 / T;",
-             "  const double T2 = T * T, T3 = T2 * T, T4 = T3 * T;",
-             "  const double pfac = 1.01325e6 / (8.314510e7 * T);"]
-        for k in range(kk):
-            o.append("  double " + ", ".join(f"{n}{k}" for n in parts) + ";")
-        for k in range(kk):
-            a_hi, a_lo = mech.a[k][1], mech.a[k][0]
+    def load(name):
+        if name.startswith("kf") and int(name[2:]) in const_kf:
+            return _lit(const_kf[int(name[2:])])
+        return f"kt[{slots[name]}]"
 
-            def smh(a):
-                return (f"{_lit(a[0])} * (lt - 1.0) + {_lit(a[1] / 2)} * T + "
-                        f"{_lit(a[2] / 6)} * T2 + {_lit(a[3] / 12)} * T3 + "
-                        f"{_lit(a[4] / 20)} * T4 + {_lit(a[6])} - {_lit(a[5])} * it")
+    def store(name, expr):
+        return f"  kt[{slots[name]}] = {expr};"
 
-            def cpR(a):
-                return (f"{_lit(a[0])} + {_lit(a[1])} * T + {_lit(a[2])} * T2 + "
-                        f"{_lit(a[3])} * T3 + {_lit(a[4])} * T4")
+    # ---- temperature-only part
+    exps = {}  # common exp(-E it) factors: E -> name
 
-            def hRT(a):
-                return (f"{_lit(a[0])} + {_lit(a[1] / 2)} * T + {_lit(a[2] / 3)} * T2 + "
-                        f"{_lit(a[3] / 4)} * T3 + {_lit(a[4] / 5)} * T4 + {_lit(a[5])} * it")
+    def arrhenius(A, b, E, o):
+        """A T^b exp(-E / T) as an expression; lines for shared exponentials
+        go to o."""
+        pw = {0.0: None, 1.0: "T", 2.0: "T2", 3.0: "T3", -1.0: "it", -2.0: "it * it",
+              0.5: "sT", -0.5: "sT * it"}
+        if b in pw:
+            fac = [_lit(A)] + ([pw[b]] if pw[b] else [])
+            if E != 0:
+                if E not in exps:
+                    exps[E] = f"ex{len(exps)}"
+                    o.append(f"  const double {exps[E]} = d_exp({_lit(-E)} * it);")
+                fac.append(exps[E])
+            return " * ".join(fac)
+        arg = f"{_lit(b)} * lt" + (f" + {_lit(-E)} * it" if E != 0 else "")
+        return f"{_lit(A)} * d_exp({arg})"
 
-            fn = {"smh": smh, "cpR": cpR, "hRT": hRT}
-            o.append(f"  if (T > {_lit(mech.tmid[k])}) {{")
-            for n in parts:
-                o.append(f"    {n}{k} = {fn[n](a_hi)};")
-            o.append("  } else {")
-            for n in parts:
-                o.append(f"    {n}{k} = {fn[n](a_lo)};")
-            o.append("  }")
-        return o
+    def kT_lines():
+        o = ["  const double ru = 8.314510e7;",
+             "  const double lt = d_log(T), it = 1.0 / T, sT = sqrt(T);",
+             "  const double T2 = T * T, T3 = T2 * T, T4 = T3 * T, ruT = ru * T;",
+             # R T / p_atm and its inverse: concentration units of Kc
+             "  const double rtp = ruT * (1.0 / 1.01325e6), pfac = 1.01325e6 / ru * it;"]
+        used = sorted({k for g in groups if R[g[0]]["rev"] and not R[g[0]].get("rpar")
+                       for k, n in _net(R[g[0]]).items() if n and k not in basis})
+        for k in used:
+            o.append(f"  double w{k};")
 
-    def kt_lines(i, put):
-        """Temperature-only values of reaction i: forward rate constant,
-        reverse from the equilibrium constant, falloff limit and centring.
-        put(slot, expr) gives the line that stores one value."""
-        r = mech.reactions[i]
-        A, b, E = r["A"], r["b"], r["EoR"]
-        o = [f"  const double kf{i} = {_lit(A)} * exp({_lit(b)} * lt - {_lit(E)} * it);",
-             put(f"kf{i}", f"kf{i}")]
-        nu = {}
-        for k, n in r["reac"]:
-            nu[k] = nu.get(k, 0) - n
-        for k, n in r["prod"]:
-            nu[k] = nu.get(k, 0) + n
-        sm = " + ".join(f"{_lit(n)} * smh{k}" for k, n in nu.items() if n != 0) or "0.0"
-        dn = sum(nu.values())
-        pf = "1.0" if dn == 0 else ("pfac" if dn == 1 else ("1.0 / pfac" if dn == -1 else
-                                                               f"pow(pfac, {dn}.0)"))
-        if r["rev"] and r.get("rpar"):
-            # explicit reverse parameters (REV, CKRATT vode.f:1028-1032)
-            Ar, br, Er = r["rpar"]
-            o.append(put(f"kr{i}", f"{_lit(Ar)} * exp({_lit(br)} * lt - {_lit(Er)} * it)"))
-        elif r["rev"]:
-            o.append(f"  const double eqk{i} = exp(fmin({sm}, 690.77552789821368)) * {pf};")
-            o.append(put(f"kr{i}", f"kf{i} / fmax(eqk{i}, 1e-300)"))
-        else:
-            o.append(put(f"kr{i}", "0.0"))
-        if r["fal"]:
-            fp = r["fpar"]
-            o.append(put(f"klow{i}", f"{_lit(fp[0])} * exp({_lit(fp[1])} * lt - "
-                                     f"{_lit(fp[2])} * it)"))
-            if r["fal"] == 2:
-                # SRI: the T-only factors of F = d (a e^(-b/T) + e^(-T/c))^X T^e
-                a_, b_, c_, d_, e_ = fp[3:8]
-                o.append(put(f"srib{i}", f"{_lit(a_)} * exp(-{_lit(b_)} / T) + "
-                                         f"exp(-T / {_lit(c_)})"))
-                o.append(put(f"srid{i}", f"{_lit(d_)} * pow(T, {_lit(e_)})"))
-            elif r["fal"] >= 3:
-                al, t3, t1 = fp[3], fp[4], fp[5]
-                fc = (f"(1.0 - {_lit(al)}) * exp(-T / {_lit(t3)}) + {_lit(al)} * "
-                      f"exp(-T / {_lit(t1)})")
-                if r["fal"] == 4:
-                    fc += f" + exp(-{_lit(fp[6])} * it)"
-                o.append(put(f"fclog{i}", f"log10(fmax({fc}, 1e-300))"))
+        def g100(k):
+            """w_k at 100 K"""
+            c = np.asarray(mech.a[k][0]) - sum(B[k][j] * np.asarray(mech.a[b][0])
+                                               for j, b in enumerate(basis))
+            return float(c[0] * (math.log(100.0) - 1.0) + c[1] / 2 * 1e2 + c[2] / 6 * 1e4 +
+                         c[3] / 12 * 1e6 + c[4] / 20 * 1e8 + c[6] - c[5] / 100.0)
+
+        def poly(c, names=("", " * T", " * T2", " * T3", " * T4")):
+            return " + ".join(f"{_lit(x)}{n}" for x, n in zip(c, names)).replace("+ -", "- ")
+
+        def thermo(rng):
+            q = []
+            # S/R - H/RT of the species relative to the basis
+            for k in used:
+                a = [np.asarray(mech.a[k][rng])] + [np.asarray(mech.a[b][rng]) for b in basis]
+                c = a[0] - sum(B[k][j] * a[1 + j] for j in range(len(basis)))
+                q.append(f"    w{k} = {_lit(c[0])} * (lt - 1.0) + {_lit(c[1] / 2)} * T + "
+                         f"{_lit(c[2] / 6)} * T2 + {_lit(c[3] / 12)} * T3 + {_lit(c[4] / 20)} * T4"
+                         f" + {_lit(c[6])} - {_lit(c[5])} * it;".replace("+ -", "- "))
+            for k in range(kk):
+                a, wt = mech.a[k][rng], mech.wt[k]
+                cv = [a[0] - 1.0] + list(a[1:5])
+                q.append("  " + store(f"cvk{k}", f"{_lit(8.314510e7 / wt)} * ({poly(cv)})"))
+                u = [a[0] - 1.0, a[1] / 2, a[2] / 3, a[3] / 4, a[4] / 5]
+                q.append("  " + store(f"uk{k}", f"ruT * ({poly(u)} + {_lit(a[5])} * it)"
+                                      .replace("+ -", "- ")))
+            return q
+
+        tm = sorted(set(float(t) for t in mech.tmid))
+        assert len(tm) == 1, "one common mid temperature expected"
+        o.append(f"  if (T > {_lit(tm[0])}) {{")
+        o += thermo(1)
+        o.append("  } else {")
+        o += thermo(0)
+        o.append("  }")
+        need_inv = {k for g in groups if R[g[0]]["rev"] and not R[g[0]].get("rpar")
+                    for k, n in _net(R[g[0]]).items() if n > 0}
+        for k in used:
+            o.append(f"  const double e{k} = d_exp(fmin(fmax(w{k}, {_lit(-GIBBS_CLAMP)}), "
+                     f"{_lit(GIBBS_CLAMP)}));")
+            if k in need_inv:
+                o.append(f"  const double r{k} = d_rcp(e{k});")
+        for g in groups:
+            i, r = g[0], R[g[0]]
+            o.append(f"  // {r['eq']}")
+            if len(g) == 1:
+                if i in const_kf:
+                    kf = _lit(const_kf[i])
+                else:
+                    e = arrhenius(r["A"], r["b"], r["EoR"], o)
+                    o.append(f"  const double kf{i} = {e};")
+                    kf = f"kf{i}"
+                    o.append(store(f"kf{i}", kf))
             else:
-                o.append(put(f"fclog{i}", "0.0"))
+                for m in g:
+                    e = arrhenius(R[m]["A"], R[m]["b"], R[m]["EoR"], o)
+                    o.append(f"  const double kp{m} = {e};")
+                kf = f"kf{i}"
+                o.append(f"  const double kf{i} = " + " + ".join(f"kp{m}" for m in g) + ";")
+                o.append(store(f"kf{i}", kf))
+                o.append(store(f"dkf{i}", "(" + " + ".join(
+                    f"kp{m} * ({_lit(R[m]['b'])} + {_lit(R[m]['EoR'])} * it)" for m in g) +
+                    ") * it"))
+            nu = _net(r)
+            dn = sum(nu.values())
+            if r["rev"] and r.get("rpar"):
+                # explicit reverse parameters (REV, CKRATT vode.f:1028-1032)
+                o.append(store(f"kr{i}", arrhenius(*r["rpar"], o)))
+            elif r["rev"]:
+                # kf / Kc: factors e_k of the reactants and 1 / e_k of the
+                # products, the next one always that which keeps the partial
+                # product nearest to 1 at 100 K, so that none
+                # leaves the range of a double where the product does not
+                left = [(f"r{k}", -g100(k)) if n > 0 else (f"e{k}", g100(k))
+                        for k, n in nu.items() if k not in basis for _ in range(abs(n))]
+                fac, at100 = [kf], -max(R[m]["EoR"] for m in g) / 100.0
+                while left:
+                    nxt = min(left, key=lambda f: abs(at100 + f[1]))
+                    left.remove(nxt)
+                    fac.append(nxt[0])
+                    at100 += nxt[1]
+                fac += ["rtp"] * dn if dn > 0 else ["pfac"] * (-dn)
+                o.append(store(f"kr{i}", " * ".join(fac)))
+            if r["fal"]:
+                # k0 / kinf of the falloff
+                fp = r["fpar"]
+                o.append(store(f"rk{i}", arrhenius(fp[0] / r["A"], fp[1] - r["b"],
+                                                   fp[2] - r["EoR"], o)))
+                if r["fal"] == 2:
+                    # SRI: the T-only factors of F = d (a e^(-b/T) + e^(-T/c))^X T^e
+                    a_, b_, c_, d_, e_ = fp[3:8]
+                    o.append(store(f"srib{i}", f"{_lit(a_)} * d_exp({_lit(-b_)} * it) + "
+                                               f"d_exp(-T / {_lit(c_)})"))
+                    o.append(store(f"srid{i}", f"{_lit(d_)} * pow(T, {_lit(e_)})"))
+                elif r["fal"] >= 3 and troe_const(r) is None:
+                    al, t3, t1 = fp[3], fp[4], fp[5]
+                    fc = (f"(1.0 - {_lit(al)}) * d_exp(-T / {_lit(t3)}) + {_lit(al)} * "
+                          f"d_exp(-T / {_lit(t1)})")
+                    if r["fal"] == 4:
+                        fc += f" + d_exp(-{_lit(fp[6])} * it)"
+                    o.append(store(f"fclog{i}", f"log10(fmax({fc}, 1e-300))"))
         return o
 
-    def species_kt_lines(put):
-        o = []
-        for k in range(kk):
-            wt = mech.wt[k]
-            o.append(put(f"cvk{k}", f"ru * (cpR{k} - 1.0) / {_lit(wt)}"))
-            o.append(put(f"hk{k}", f"ru * T * hRT{k} / {_lit(wt)}"))
-        return o
+    # ---- concentration part
+    # third-body sums of equal efficiencies are formed once
+    mset = {}
+
+    def third(r):
+        eff = tuple(sorted(r["eff"]))
+        if eff not in mset:
+            mset[eff] = f"M{len(mset)}"
+        return mset[eff]
+
+    for g in groups:
+        if R[g[0]]["tb"]:
+            third(R[g[0]])
 
     def conc_lines():
         o = []
         for k in range(kk):
             o.append(f"  const double c{k} = rho * z[{1 + k}] * {_lit(1.0 / mech.wt[k])};")
         o.append("  const double ctot = " + " + ".join(f"c{k}" for k in range(kk)) + ";")
-        for k in range(kk):
-            o.append(f"  double wd{k} = 0.0;")
+        for eff, name in mset.items():
+            o.append(f"  const double {name} = ctot" +
+                     "".join(f" + {_lit(e - 1.0)} * c{k}" for k, e in eff).replace("+ -", "- ") +
+                     ";")
         return o
 
-    def reaction_block(i, ref):
-        """Rate of progress of reaction i and its species production terms;
-        ref(slot) is the expression that reads a temperature-only value."""
-        r = mech.reactions[i]
-        o = [f"  {{ // {r['eq']}"]
-        if r["tb"]:
-            expr = "ctot" + "".join(f" + {_lit(e - 1.0)} * c{k}" for k, e in r["eff"])
-            o.append(f"    double ctb = {expr};")
+    def prod(side):
+        return " * ".join(f"c{k}" for k, n in side for _ in range(n)) or "1.0"
+
+    def falloff_lines(i, deriv):
+        """pcor of falloff reaction i ([M]: the third-body sum, or the named
+        collider); with deriv also dpcor = d pcor / d pr."""
+        r = R[i]
+        cm = f"c{r['kfal'] - 1}" if r.get("kfal") else third(r)
+        o = [f"    const double pr = {load(f'rk{i}')} * {cm};",
+             "    const double lin1 = d_rcp(1.0 + pr);"]
+        if r["fal"] == 1:
+            o.append("    const double pcor = pr * lin1;")
+            if deriv:
+                o.append("    const double dpcor = lin1 * lin1;")
+            return o
+        o.append("    const double prlog = 0.43429448190325182 * d_log(fmax(pr, 1e-300));")
+        if r["fal"] == 2:
+            o.append("    const double xp = 1.0 / (1.0 + prlog * prlog);")
+            o.append(f"    const double fcent = pow({load(f'srib{i}')}, xp) * {load(f'srid{i}')};")
+            if deriv:
+                o.append("    const double dfdpr = (pr > 1e-300) ? fcent * "
+                         f"d_log({load(f'srib{i}')}) * (-2.0 * prlog * xp * xp) / "
+                         "(pr * 2.302585092994046) : 0.0;")
         else:
-            o.append("    double ctb = 1.0;")
-        o.append(f"    double kf = {ref(f'kf{i}')}, kr = {ref(f'kr{i}')};")
-        if r["fal"]:
-            # [M]: the third-body sum, or the named collider's concentration
-            cm = f"c{r['kfal'] - 1}" if r.get("kfal") else "ctb"
-            o.append(f"    double pr = {ref(f'klow{i}')} * {cm} / kf;")
-            o.append("    double pcor = pr / (1.0 + pr);")
-            if r["fal"] == 2:
-                o.append("    double prlog = log10(fmax(pr, 1e-300));")
-                o.append("    double xp = 1.0 / (1.0 + prlog * prlog);")
-                o.append(f"    pcor *= pow({ref(f'srib{i}')}, xp) * {ref(f'srid{i}')};")
-            elif r["fal"] >= 3:
-                o.append(f"    double fclog = {ref(f'fclog{i}')};")
-                o.append("    double prlog = log10(fmax(pr, 1e-300));")
-                o.append("    double xn = 0.75 - 1.27 * fclog;")
-                o.append("    double cprlog = prlog - (0.4 + 0.67 * fclog);")
-                o.append("    double qq = cprlog / (xn - 0.14 * cprlog);")
-                o.append("    pcor *= exp((fclog / (1.0 + qq * qq)) * 2.302585092994046);")
-            o.append("    kf *= pcor; kr *= pcor; ctb = 1.0;")
-        o.append("    kf *= ctb; kr *= ctb;")
-
-        def prod(side):
-            out = []
-            for k, n in side:
-                out += [f"c{k}"] * n
-            return " * ".join(out)
-
-        o.append(f"    double q = kf * {prod(r['reac'])} - kr * {prod(r['prod'])};")
-        nu = {}
-        for k, n in r["reac"]:
-            nu[k] = nu.get(k, 0) - n
-        for k, n in r["prod"]:
-            nu[k] = nu.get(k, 0) + n
-        for k, n in nu.items():
-            if n == 1:
-                o.append(f"    wd{k} += q;")
-            elif n == -1:
-                o.append(f"    wd{k} -= q;")
-            elif n != 0:
-                o.append(f"    wd{k} += {_lit(n)} * q;")
-        o.append("  }")
-        return o
-
-    def energy_lines(ref):
-        o = ["  double cvb = " + " + ".join(f"z[{1 + k}] * {ref(f'cvk{k}')}"
-                                           for k in range(kk)) + ";",
-             "  const double rho_i = 1.0 / rho;",
-             "  double sum = 0.0;"]
-        for k in range(kk):
-            wt = _lit(mech.wt[k])
-            o.append(f"  zp[{1 + k}] = wd{k} * {wt} * rho_i;")
-            o.append(f"  sum += {ref(f'hk{k}')} * wd{k} * {wt} - ru * T * wd{k};")
-        o.append("  zp[0] = -sum / (rho * cvb);")
-        return o
-
-    def jac_block(i, ref):
-        """d(wdot)/d(c_m) of reaction i accumulated into jy{k}_{m}: the
-        mass-action products, the third-body sum and the falloff factor
-        (Lindemann, Troe, SRI) differentiated term by term."""
-        r = mech.reactions[i]
-        o = [f"  {{ // {r['eq']}"]
-        effs = {k: e for k, e in r["eff"]} if r["tb"] else {}
-        if r["tb"]:
-            expr = "ctot" + "".join(f" + {_lit(e - 1.0)} * c{k}" for k, e in r["eff"])
-            o.append(f"    double ctb = {expr};")
-        else:
-            o.append("    double ctb = 1.0;")
-        o.append(f"    double kf = {ref(f'kf{i}')}, kr = {ref(f'kr{i}')};")
-        dM = {}  # d[M]/dc_m of the falloff collider
-        if r["fal"]:
-            if r.get("kfal"):
-                o.append(f"    const double cm = c{r['kfal'] - 1};")
-                dM = {r["kfal"] - 1: "1.0"}
+            fl = troe_const(r)
+            if fl is not None:
+                o.append(f"    const double cpr = prlog - {_lit(0.4 + 0.67 * fl)};")
+                o.append(f"    const double xn = {_lit(0.75 - 1.27 * fl)};")
+                ln10fl = _lit(fl * math.log(10.0))
             else:
-                o.append("    const double cm = ctb;")
-                dM = {m: _lit(effs.get(m, 1.0)) for m in range(kk)}
-            o.append(f"    const double klo = {ref(f'klow{i}')};")
-            o.append("    const double pr = klo * cm / kf;")
-            o.append("    const double lin = pr / (1.0 + pr);")
-            o.append("    double fcent = 1.0, dfdpr = 0.0;")
-            if r["fal"] == 2:
-                o.append("    const double prlog = log10(fmax(pr, 1e-300));")
-                o.append("    const double xp = 1.0 / (1.0 + prlog * prlog);")
-                o.append(f"    const double sb = {ref(f'srib{i}')};")
-                o.append(f"    fcent = pow(sb, xp) * {ref(f'srid{i}')};")
-                o.append("    if (pr > 1e-300) dfdpr = fcent * log(sb) * (-2.0 * prlog * xp * xp) / "
-                         "(pr * 2.302585092994046);")
-            elif r["fal"] >= 3:
-                o.append(f"    const double fclog = {ref(f'fclog{i}')};")
-                o.append("    const double prlog = log10(fmax(pr, 1e-300));")
+                o.append(f"    const double fclog = {load(f'fclog{i}')};")
+                o.append("    const double cpr = prlog - (0.4 + 0.67 * fclog);")
                 o.append("    const double xn = 0.75 - 1.27 * fclog;")
-                o.append("    const double cprlog = prlog - (0.4 + 0.67 * fclog);")
-                o.append("    const double den = xn - 0.14 * cprlog;")
-                o.append("    const double qq = cprlog / den;")
-                o.append("    const double g = 1.0 / (1.0 + qq * qq);")
-                o.append("    fcent = exp((fclog * g) * 2.302585092994046);")
-                o.append("    if (pr > 1e-300) dfdpr = -2.0 * fcent * fclog * qq * xn * g * g / "
-                         "(den * den * pr);")
-            o.append("    const double dpcor = fcent / ((1.0 + pr) * (1.0 + pr)) + lin * dfdpr;")
-            o.append("    const double kinf = kf, krinf = kr;")
-            o.append("    kf *= lin * fcent; kr *= lin * fcent;")
-        elif r["tb"]:
-            o.append("    const double kf0 = kf, kr0 = kr;")
-            o.append("    kf *= ctb; kr *= ctb;")
-
-        def prod_terms(side):
-            mult = {}
-            for k, n in side:
-                mult[k] = mult.get(k, 0) + n
-            full = " * ".join(f"c{k}" for k, n in side for _ in range(n)) or "1.0"
-            ders = {}
-            for m, n in mult.items():
-                rest = [f"c{k}" for k, nn in mult.items() if k != m for _ in range(nn)]
-                rest += [f"c{m}"] * (n - 1)
-                coef = "" if n == 1 else f"{_lit(float(n))} * "
-                ders[m] = coef + (" * ".join(rest) if rest else "1.0")
-            return full, ders
-
-        pf, dpf = prod_terms(r["reac"])
-        pp, dpp = prod_terms(r["prod"])
-        dq = {}
-        for m, e in dpf.items():
-            dq[m] = [f"kf * ({e})"]
-        for m, e in dpp.items():
-            dq.setdefault(m, []).append(f"-kr * ({e})")
-        if r["fal"]:
-            o.append(f"    const double qinf = kinf * {pf} - krinf * {pp};")
-            o.append("    const double dqdm = qinf * dpcor * klo / kinf;")
-            for m, d in dM.items():
-                dq.setdefault(m, []).append(f"dqdm * {d}")
-        elif r["tb"]:
-            o.append(f"    const double q0 = kf0 * {pf} - kr0 * {pp};")
-            for m in range(kk):
-                dq.setdefault(m, []).append(f"q0 * {_lit(effs.get(m, 1.0))}")
-        for m in sorted(dq):
-            terms = " + ".join(dq[m]).replace("+ -", "- ")
-            o.append(f"    const double dq{m} = {terms};")
-        nu = {}
-        for k, n in r["reac"]:
-            nu[k] = nu.get(k, 0) - n
-        for k, n in r["prod"]:
-            nu[k] = nu.get(k, 0) + n
-        for k, n in nu.items():
-            for m in sorted(dq):
-                if n == 1:
-                    o.append(f"    jy{k}_{m} += dq{m};")
-                elif n == -1:
-                    o.append(f"    jy{k}_{m} -= dq{m};")
-                elif n != 0:
-                    o.append(f"    jy{k}_{m} += {_lit(n)} * dq{m};")
-        o.append("  }")
+                ln10fl = "(fclog * 2.302585092994046)"
+            # 1 / (1 + (cpr / den)^2) with one division
+            o.append("    const double den = xn - 0.14 * cpr, den2 = den * den;")
+            o.append("    const double g = den2 * d_rcp(den2 + cpr * cpr);")
+            o.append(f"    const double fcent = d_exp({ln10fl} * g);")
+            if deriv:
+                o.append(f"    const double dfdpr = (pr > 1e-300) ? -2.0 * fcent * {ln10fl} * "
+                         "0.43429448190325182 * cpr * xn * g * g / (den2 * den * pr) : 0.0;")
+        o.append("    const double pcor = pr * lin1 * fcent;")
+        if deriv:
+            o.append("    const double dpcor = fcent * lin1 * lin1 + pr * lin1 * dfdpr;")
         return o
 
-    store = lambda name, expr: f"  kt[{slots[name]}] = {expr};"
-    load = lambda name: f"kt[{slots[name]}]"
-    # FMA contraction decided per inlined copy would round the terms that a
-    # finite-difference Jacobian column shares with the base evaluation
-    # differently, and turn rounding into O(1) noise
+    def rhs_lines():
+        o = [f"  double wd{k} = 0.0;" for k in range(kk)]
+        for g in groups:
+            i, r = g[0], R[g[0]]
+            o.append(f"  {{ // {r['eq']}")
+            q = f"{load(f'kf{i}')} * {prod(r['reac'])}"
+            if r["rev"]:
+                q += f" - {load(f'kr{i}')} * {prod(r['prod'])}"
+            if r["fal"]:
+                o += falloff_lines(i, False)
+                q = f"pcor * ({q})"
+            elif r["tb"]:
+                q = f"{third(r)} * ({q})"
+            o.append(f"    const double q = {q};")
+            for k, n in _net(r).items():
+                if n:
+                    o.append(f"    wd{k} {'+' if n > 0 else '-'}= "
+                             f"{_scaled(abs(n), 'q')};")
+            o.append("  }")
+        o.append("  const double cvb = " + " + ".join(f"z[{1 + k}] * {load(f'cvk{k}')}"
+                                                       for k in range(kk)) + ";")
+        o.append("  const double rho_i = d_rcp(rho);")
+        for k in range(kk):
+            o.append(f"  zp[{1 + k}] = wd{k} * ({_lit(mech.wt[k])} * rho_i);")
+        o.append("  const double sum = " + " + ".join(f"{load(f'uk{k}')} * wd{k}" for k in live) +
+                 ";")
+        o.append("  zp[0] = -sum * d_rcp(rho * cvb);")
+        return o
+
+    def falloff_scale(i):
+        """sc{i} = pcor and dp{i} = d pcor / d[M] of falloff reaction i."""
+        o = [f"  double sc{i}, dp{i};", "  {"]
+        o += falloff_lines(i, True)
+        return o + [f"    sc{i} = pcor;", f"    dp{i} = dpcor * {load(f'rk{i}')};", "  }"]
+
+    def sides(i):
+        r = R[i]
+        return (f"{load(f'kf{i}')} * {prod(r['reac'])}",
+                f"{load(f'kr{i}')} * {prod(r['prod'])}" if r["rev"] else None)
+
+    def mixture_cv():
+        return ["  const double cvb = " + " + ".join(f"z[{1 + k}] * {load(f'cvk{k}')}"
+                                                      for k in range(kk)) + ";",
+                "  const double cvi = d_rcp(cvb);"]
+
+    def jac_lines():
+        """Mass-fraction columns: per reaction the partial derivatives of its
+        rate, then column by column the production terms they make."""
+        o = []
+        dq = {}      # (group, m): terms of d q_g / d c_m by mass action
+        effsum = {}  # third-body set: (group, the rate that its sum scales)
+        for n_, g in enumerate(groups):
+            i, r = g[0], R[g[0]]
+            o.append(f"  // {r['eq']}")
+            scale = None
+            if r["fal"]:
+                o += falloff_scale(i)
+                scale = f"sc{i}"
+            elif r["tb"]:
+                scale = third(r)
+
+            def partials(side, coef, sign):
+                mult = {}
+                for k, n in side:
+                    mult[k] = mult.get(k, 0) + n
+                for m, n in mult.items():
+                    rest = [f"c{k}" for k, nn in mult.items() if k != m for _ in range(nn)]
+                    rest += [f"c{m}"] * (n - 1)
+                    if n != 1:
+                        rest = [_lit(float(n))] + rest
+                    e = " * ".join([coef if scale is None else f"({coef} * {scale})"] + rest)
+                    dq.setdefault((n_, m), []).append(("-" if sign < 0 else "") + e)
+
+            partials(r["reac"], load(f"kf{i}"), 1)
+            if r["rev"]:
+                partials(r["prod"], load(f"kr{i}"), -1)
+            if r["fal"] or r["tb"]:
+                q0 = " - ".join(x for x in sides(i) if x)
+                if r["fal"]:
+                    q0 = f"({q0}) * dp{i}"
+                o.append(f"  const double qm{i} = {q0};")
+                if r.get("kfal"):
+                    dq.setdefault((n_, r["kfal"] - 1), []).append(f"qm{i}")
+                else:
+                    effsum.setdefault(third(r), []).append((n_, f"qm{i}"))
+        has = set()
+        for name, lst in effsum.items():
+            for k in live:
+                t = [_scaled(_net(R[groups[n_][0]])[k], q) for n_, q in lst
+                     if _net(R[groups[n_][0]]).get(k)]
+                if t:
+                    has.add((name, k))
+                    o.append(f"  const double {name}_{k} = {_sum(t)};")
+        effs = {name: dict(eff) for eff, name in mset.items()}
+        o += mixture_cv()
+        for m in range(kk):
+            o.append(f"  {{ // column d / d Y_{m}")
+            names = {}
+            for n_, g in enumerate(groups):
+                if (n_, m) in dq:
+                    names[n_] = f"d{g[0]}"
+                    o.append(f"    const double d{g[0]} = {_sum(dq[(n_, m)])};")
+            for k in live:
+                t = [_scaled(_net(R[groups[n_][0]])[k], nm) for n_, nm in names.items()
+                     if _net(R[groups[n_][0]]).get(k)]
+                for name in effsum:
+                    e = effs[name].get(m, 1.0)
+                    if (name, k) in has and e != 0.0:
+                        t.append(_scaled(e, f"{name}_{k}"))
+                o.append(f"    const double y{k} = {_sum(t)};")
+            for k in range(kk):
+                v = f"y{k} * {_lit(mech.wt[k] / mech.wt[m])}" if k in live else "0.0"
+                o.append(f"    J[{1 + k}][{1 + m}] = {v};")
+            ds = " + ".join(f"{load(f'uk{k}')} * y{k}" for k in live)
+            o.append(f"    J[0][{1 + m}] = -(({ds}) * {_lit(1.0 / mech.wt[m])} + f0T * "
+                     f"{load(f'cvk{m}')}) * cvi;")
+            o.append("  }")
+        return o
+
+    def jacT_lines():
+        """Temperature column: kf' = kf (b + E/T) / T, kr' = kr (kf'/kf -
+        d ln Kc / dT) with d ln Kc / dT = sum nu u / (ru T^2), the falloff's
+        dependence through k0/kinf."""
+        o = []
+        for g in groups:
+            i, r = g[0], R[g[0]]
+            o.append(f"  // {r['eq']}")
+            if r["fal"]:
+                o += falloff_scale(i)
+            nu = _net(r)
+            slope = lambda b_, E_: f"({_lit(b_)} + {_lit(E_)} * it) * it"
+            if len(g) > 1:
+                o.append(f"  const double af{i} = {load(f'dkf{i}')} / {load(f'kf{i}')};")
+            else:
+                o.append(f"  const double af{i} = {slope(r['b'], r['EoR'])};")
+            f, b = sides(i)
+            dT = f"af{i} * ({f})"
+            if r["rev"] and r.get("rpar"):
+                dT += f" - {slope(r['rpar'][1], r['rpar'][2])} * ({b})"
+            elif r["rev"]:
+                du = _sum([_scaled(n, load(f"uk{k}")) for k, n in nu.items() if n])
+                dT += f" - (af{i} - ({du}) * rut2) * ({b})"
+            if r["fal"]:
+                al = slope(r["fpar"][1] - r["b"], r["fpar"][2] - r["EoR"])
+                cm = f"c{r['kfal'] - 1}" if r.get("kfal") else third(r)
+                q0 = " - ".join(x for x in (f, b) if x)
+                dT = f"sc{i} * ({dT}) + ({q0}) * dp{i} * {cm} * {al}"
+            elif r["tb"]:
+                dT = f"{third(r)} * ({dT})"
+            o.append(f"  const double qT{i} = {dT};")
+        o += mixture_cv()
+        o.append("  const double rho_i = d_rcp(rho);")
+        for k in live:
+            t = [_scaled(_net(R[g[0]])[k], f"qT{g[0]}") for g in groups if _net(R[g[0]]).get(k)]
+            o.append(f"  const double y{k} = {_sum(t)};")
+        for k in range(kk):
+            v = f"y{k} * ({_lit(mech.wt[k])} * rho_i)" if k in live else "0.0"
+            o.append(f"  J[{1 + k}][0] = {v};")
+        o.append("  const double ut = (" + " + ".join(f"{load(f'uk{k}')} * y{k}" for k in live) +
+                 ") * rho_i;")
+        o.append("  const double cf = " + " + ".join(f"{load(f'cvk{k}')} * f0[{1 + k}]"
+                                                      for k in live) + ";")
+        # d cvb / dT from the mixture's polynomial
+        o.append("  double p1, p2, p3, p4;")
+        for cond, rng in ((f"if (T > {_lit(mech.tmid[0])})", 1), ("else", 0)):
+            o.append(f"  {cond} {{")
+            for q in range(1, 5):
+                o.append(f"    p{q} = " + _sum([f"{_lit(mech.a[k][rng][q] * q)} * c{k}"
+                                                for k in range(kk)]) + ";")
+            o.append("  }")
+        o.append("  const double dcv = (p1 + T * (p2 + T * (p3 + T * p4))) * (ru * rho_i);")
+        o.append("  J[0][0] = -(ut + cf + f0[0] * dcv) * cvi;")
+        return o
+
     # ---- gen_kT
     w("IZ_HD inline void gen_kT(double T, double *kt) {")
-    w("#pragma clang fp contract(off)")
-    w("  const double ru = 8.314510e7;")
-    L.extend(thermo_lines())
-    for i in range(ii):
-        L.extend(kt_lines(i, store))
-    w("  (void)(" + " + ".join(f"smh{k}" for k in range(kk)) + ");")
-    L.extend(species_kt_lines(store))
+    w("#pragma clang fp contract(on)")
+    L.extend(kT_lines())
     w("}")
     w("")
     # ---- gen_rhs
     w("IZ_HD inline void gen_rhs(double rho, const double *z, const double *kt, double *zp) {")
-    w("#pragma clang fp contract(off)")
-    w("  const double T = z[0], ru = 8.314510e7;")
+    w("#pragma clang fp contract(on)")
     L.extend(conc_lines())
-    for i in range(ii):
-        L.extend(reaction_block(i, load))
-    L.extend(energy_lines(load))
+    L.extend(rhs_lines())
     w("}")
     w("")
-    # ---- gen_jac: the mass-fraction columns of the reactor Jacobian
-    w("// d zp / d z[1 + j] for j = 0 .. GEN_KK - 1 (columns 1 .. GEN_KK of J;")
-    w("// column 0, d/dT, is left to the caller) at the state z whose")
-    w("// temperature part is kt and whose dT/dt is f0T: the analytic form of")
-    w("// the mass-fraction columns of a finite-difference Jacobian.")
+    # ---- gen_jac, gen_jac_T
+    w("// The reactor Jacobian d zp / d z in closed form (mass action, third-body")
+    w("// sums, falloff factors, Arrhenius and equilibrium slopes) at the state z")
+    w("// whose temperature part is kt: both functions together cost about as")
+    w("// much as one right-hand side, where finite differences take GEN_KK + 1 of")
+    w("// them and the temperature part again.  gen_jac: columns 1 .. GEN_KK,")
+    w("// given f0T = dT/dt; column 0 is left alone.")
     w("IZ_HD inline void gen_jac(double rho, const double *z, const double *kt, double f0T,")
     w("                          double (*J)[GEN_KK + 1]) {")
-    w("#pragma clang fp contract(off)")
-    w("  const double T = z[0], ru = 8.314510e7;")
-    L.extend(conc_lines()[:-kk])  # concentrations and their sum
-    for k in range(kk):
-        w("  double " + ", ".join(f"jy{k}_{m} = 0.0" for m in range(kk)) + ";")
-    for i in range(ii):
-        L.extend(jac_block(i, load))
-    w("  double cvb = " + " + ".join(f"z[{1 + k}] * {load(f'cvk{k}')}" for k in range(kk)) + ";")
-    w("  const double rcv = 1.0 / (rho * cvb);")
-    for k in range(kk):
-        w(f"  const double um{k} = {load(f'hk{k}')} * {_lit(mech.wt[k])} - ru * T;")
-    for j in range(kk):
-        wj = mech.wt[j]
-        w(f"  {{ // column d / d Y_{j}")
-        w(f"    const double s = rho * {_lit(1.0 / wj)};")
-        for k in range(kk):
-            w(f"    J[{1 + k}][{1 + j}] = jy{k}_{j} * s * ({_lit(mech.wt[k])} / rho);")
-        w("    const double dsum = " + " + ".join(f"um{k} * jy{k}_{j}" for k in range(kk))
-          + ";")
-        w(f"    J[0][{1 + j}] = -(dsum * s) * rcv - f0T * {load(f'cvk{j}')} / cvb;")
-        w("  }")
+    w("#pragma clang fp contract(on)")
+    L.extend(conc_lines())
+    L.extend(jac_lines())
+    w("}")
+    w("")
+    w("// column 0, d / d T, given f0 = dz/dt; a Troe or SRI centring factor's own")
+    w("// temperature dependence is left out (the column serves an iteration matrix)")
+    w("IZ_HD inline void gen_jac_T(double rho, const double *z, const double *kt, const double *f0,")
+    w("                            double (*J)[GEN_KK + 1]) {")
+    w("#pragma clang fp contract(on)")
+    w("  const double T = z[0], ru = 8.314510e7, it = 1.0 / T, rut2 = it * it * (1.0 / ru);")
+    L.extend(conc_lines())
+    L.extend(jacT_lines())
     w("}")
     w("")
     return "\n".join(L) + "\n"

@@ -14,6 +14,7 @@
 #endif
 
 #include "chem_tables.h"
+#include "iz_math.h"
 
 // --------------------------------------------------------------- kinetics
 // CKSMH (vode.f:1474-1535): S/R - H/RT per species
@@ -156,24 +157,29 @@ IZ_HD inline double d_wrms(const double *v, const double *w) {
 
 // x^e for x >= 0: the step-ratio powers of the step and order selection
 // (DVSTEP's (BIAS*DSM)**(1/L), vode.f:6516, 6693-6708)
-IZ_HD inline double d_powpos(double x, double e) { return exp(e * log(x)); }
+IZ_HD inline double d_powpos(double x, double e) {
+  return x > 1e-300 ? d_exp(e * d_log(x)) : 0.0;
+}
 
 // LU with partial pivoting in LINPACK's form (dgefa / dgesl, vode.f:7033,
-// 7630): step k swaps rows k and p over columns k..N-1 only, so the
-// multipliers of the earlier steps stay in the rows where the solve
-// applies them, interleaved with the same swaps.  Every index is a
-// compile-time constant, so that the factors can stay in registers: the
-// row swap is a run of selects, skipped when no lane of the wave pivots.
-// The diagonal keeps the reciprocal of each pivot (0 for a missing one), so
-// the back substitution multiplies where dgesl divides.
+// 7630) on the leading M x M block: step k swaps rows k and p over columns
+// k..M-1 only, so the multipliers of the earlier steps stay in the rows
+// where the solve applies them, interleaved with the same swaps.  Every
+// index is a compile-time constant, so that the factors can stay in
+// registers: a row swap is a run of selects, skipped for the rows that no
+// lane of the wave pivots to.  The diagonal keeps the reciprocal of each
+// pivot (0 for a missing one), so the back substitution multiplies where
+// dgesl divides.
+template <int M = N_>
 IZ_HD inline bool d_lu(double (&A)[N_][N_], int (&piv)[N_]) {
+#pragma clang fp contract(on)
   bool ok = true;
 #pragma unroll
-  for (int k = 0; k < N_; k++) {
+  for (int k = 0; k < M; k++) {
     int p = k;
     double amax = fabs(A[k][k]);
 #pragma unroll
-    for (int i = k + 1; i < N_; i++) {
+    for (int i = k + 1; i < M; i++) {
       const double a = fabs(A[i][k]);
       p = (a > amax) ? i : p;
       amax = (a > amax) ? a : amax;
@@ -181,39 +187,41 @@ IZ_HD inline bool d_lu(double (&A)[N_][N_], int (&piv)[N_]) {
     piv[k] = p;
     if (IZ_ANY(p != k)) {
 #pragma unroll
-      for (int j = k; j < N_; j++) {
-        const double akj = A[k][j];
-        double apj = akj;
+      for (int i = k + 1; i < M; i++) {
+        if (IZ_ANY(p == i)) {
 #pragma unroll
-        for (int i = k + 1; i < N_; i++) {
-          apj = (p == i) ? A[i][j] : apj;
-          A[i][j] = (p == i) ? akj : A[i][j];
+          for (int j = k; j < M; j++) {
+            const double akj = A[k][j], aij = A[i][j];
+            A[k][j] = (p == i) ? aij : akj;
+            A[i][j] = (p == i) ? akj : aij;
+          }
         }
-        A[k][j] = apj;
       }
     }
     if (amax == 0.0) ok = false;  // dgefa's INFO = k: column k has no pivot
     const double inv = (amax == 0.0) ? 0.0 : 1.0 / A[k][k];
     A[k][k] = inv;
 #pragma unroll
-    for (int i = k + 1; i < N_; i++) {
+    for (int i = k + 1; i < M; i++) {
       const double m = A[i][k] * inv;
       A[i][k] = m;
 #pragma unroll
-      for (int j = k + 1; j < N_; j++) A[i][j] -= m * A[k][j];
+      for (int j = k + 1; j < M; j++) A[i][j] -= m * A[k][j];
     }
   }
   return ok;
 }
+template <int M = N_>
 IZ_HD inline void d_lusolve(const double (&A)[N_][N_], const int (&piv)[N_], double (&x)[N_]) {
+#pragma clang fp contract(on)
 #pragma unroll
-  for (int k = 0; k < N_; k++) {
+  for (int k = 0; k < M; k++) {
     const int p = piv[k];
     if (IZ_ANY(p != k)) {
       const double xk = x[k];
       double xp = xk;
 #pragma unroll
-      for (int i = k + 1; i < N_; i++) {
+      for (int i = k + 1; i < M; i++) {
         xp = (p == i) ? x[i] : xp;
         x[i] = (p == i) ? xk : x[i];
       }
@@ -221,24 +229,29 @@ IZ_HD inline void d_lusolve(const double (&A)[N_][N_], const int (&piv)[N_], dou
     }
     const double t = x[k];
 #pragma unroll
-    for (int i = k + 1; i < N_; i++) x[i] -= A[i][k] * t;
+    for (int i = k + 1; i < M; i++) x[i] -= A[i][k] * t;
   }
 #pragma unroll
-  for (int k = N_ - 1; k >= 0; k--) {
+  for (int k = M - 1; k >= 0; k--) {
     double s = x[k];
 #pragma unroll
-    for (int j = k + 1; j < N_; j++) s -= A[k][j] * x[j];
+    for (int j = k + 1; j < M; j++) s -= A[k][j] * x[j];
     x[k] = s * A[k][k];
   }
 }
 
 // Nordsieck history of one cell, z(j, n) for column j = 0..5 and component
-// n.  ZArr holds it in the lane's own (private) memory; ZLds holds it in
-// LDS with one 64-lane wave's worth of stride between elements, so that
-// element (j, n) of lane l sits at base[(j * N_ + n) * 64 + l] and a wave
-// reads a column component as one contiguous 512-byte row.
+// n, and in column IZ_ZSAVE the correction kept for the order-up estimate.
+// Columns above the current order are zero, so that the sums below run over
+// fixed columns.  ZArr holds the history in the lane's own (private)
+// memory; ZLds holds it in LDS with one 64-lane wave's worth of stride
+// between elements, so that element (j, n) of lane l sits at
+// base[(j * N_ + n) * 64 + l] and a wave reads a column component as one
+// contiguous 512-byte row.
+#define IZ_ZSAVE 6
+#define IZ_ZCOLS 7
 struct ZArr {
-  double a[6][N_];
+  double a[IZ_ZCOLS][N_];
   IZ_MHD inline double &operator()(int j, int n) { return a[j][n]; }
 };
 struct ZLds {
@@ -248,21 +261,49 @@ struct ZLds {
 
 template <class Z>
 IZ_HD inline double d_wrms_col(Z &z, int j, const double *w) {
+#pragma clang fp contract(on)
   double s = 0.0;
 #pragma unroll
   for (int i = 0; i < N_; i++) { double x = z(j, i) * w[i]; s += x * x; }
   return sqrt(s / N_);
 }
 
-// Pascal-triangle update of the Nordsieck history (sign +1: predict to t+h,
-// sign -1: retract); sweeps jb = 1..q over columns q-jb..q-1 in ascending
-// order, which makes the -1 sweep the exact inverse of the +1 sweep.
-template <class Z>
-IZ_HD inline void d_nordsieck_shift(Z &z, int q, double sign) {
-  for (int jb = 1; jb <= q; jb++)
-    for (int i = q - jb; i <= q - 1; i++)
+// predicted state sum_j z_j and its scaled derivative sum_j j z_j of orders
+// up to QM (the first two rows of the Pascal triangle's product)
+template <int QM, class Z>
+IZ_HD inline void d_predict(Z &z, double *y, double *zp1) {
+#pragma clang fp contract(on)
 #pragma unroll
-      for (int n = 0; n < N_; n++) z(i, n) += sign * z(i + 1, n);
+  for (int n = 0; n < N_; n++) {
+    double a = z(QM, n), b = QM * a;
+#pragma unroll
+    for (int j = QM - 1; j >= 1; j--) {
+      const double zj = z(j, n);
+      a += zj;
+      b += j * zj;
+    }
+    y[n] = z(0, n) + a;
+    zp1[n] = b;
+  }
+}
+
+// the accepted step: the history times the Pascal triangle plus the
+// corrector's l_j acor
+template <int QM, class Z>
+IZ_HD inline void d_advance(Z &z, const double *el, const double *acor) {
+#pragma clang fp contract(on)
+#pragma unroll
+  for (int n = 0; n < N_; n++) {
+    double a[QM + 1];
+#pragma unroll
+    for (int j = 0; j <= QM; j++) a[j] = z(j, n);
+#pragma unroll
+    for (int k = 0; k < QM; k++)
+#pragma unroll
+      for (int j = QM - 1; j >= k; j--) a[j] += a[j + 1];
+#pragma unroll
+    for (int j = 0; j <= QM; j++) z(j, n) = a[j] + el[j] * acor[n];
+  }
 }
 
 // rescale the Nordsieck history for a step change h -> rh*h
@@ -305,7 +346,10 @@ IZ_HD inline double d_fd_increment(int j, double yj, double wj, double r0) {
 // same y can reuse; jac_c(rho, y, f0, c, hl0, w, r0, P), given f0 = f(y) and
 // the c of that evaluation, writes P = -hl0 * J with a finite-difference
 // Jacobian (DVJAC with MF = 22, vode.f:3728-3770).  None of them writes y.
+// NACT: the leading equations that react; the ones after them are zero
+// rates (an inert last species), whose corrections stay exactly zero.
 struct KinTables {
+  static constexpr int NACT = N_;
   struct Cache {};
   IZ_MHD inline void rhs(double rho, const double *y, double *f) const {
     d_reactor_rhs(rho, y, f);
@@ -331,298 +375,397 @@ struct KinTables {
 };
 
 // Jacobian and iteration-matrix reuse follow DVODE (DVNLSD / DVJAC,
-// vode.f:4032-4259, 3596-3780): the finite-difference Jacobian J is kept,
-// and the iteration matrix P = I - h l0 J is refactored from it whenever
-// h l0 has changed by more than CCMAX = 0.3 or MSBP = 20 steps have
-// passed; J itself is re-evaluated only at the first step, after jac_age
-// (DVODE's MSBJ, default 50) steps, or after a corrector failure that a
-// new h l0 cannot explain (DRC < CCMXJ = 0.2) or that a current J did not
-// prevent.
+// vode.f:4032-4259, 3596-3780): the Jacobian J is kept, and the iteration
+// matrix P = I - h l0 J is refactored from it whenever h l0 has changed by
+// more than CCMAX = 0.3 or MSBP = 20 steps have passed; J itself is
+// re-evaluated only at the first step, after jac_age (DVODE's MSBJ,
+// default 50) steps, or after a corrector failure that a new h l0 cannot
+// explain (DRC < CCMXJ = 0.2) or that a current J did not prevent.
+//
+// Integrates cell after cell: io.next(rho, y) gives the next cell's density
+// and state (false: none left), io.done(y, res) takes its end state.  On the
+// GPU each lane runs its own sequence of cells, and a lane whose cell is
+// finished takes the next one while the others go on: the wave's time is
+// the lanes' mean number of steps, not the largest of 64 cells.  One turn of
+// the loop is one step of the cell (or one evaluation of a new cell's
+// initial-step search, made by the same code as the step's predictor
+// evaluation, so the right-hand side is compiled in twice only: at this
+// place and in the corrector).
 // J is the caller's storage for the saved Jacobian.  The first step of
 // every integration evaluates a new one before any read, so the caller
-// initialises J once (the kernels once per lane, not once per cell) and
-// may pass the storage of a previous integration.
-template <class Kin, class Z>
-IZ_HD IZ_FORCEINLINE BdfResult d_bdf_integrate(const Kin &kin, Z &z, double (&J)[N_][N_],
-                                               double rho, double *y, double tout, double rtol,
-                                               double atol, int jac_age) {
+// initialises J once (the kernels once per lane, not once per cell).
+template <class Kin, class Z, class IO>
+IZ_HD IZ_FORCEINLINE void d_bdf_run(const Kin &kin, Z &z, double (&J)[N_][N_], IO &io,
+                                    double tout, double rtol, double atol, int jac_age) {
+#pragma clang fp contract(on)
+  constexpr int M = Kin::NACT;
   const double uround = 2.220446049250313e-16;
   const int maxstep = 10000, maxcor = 3, msbp = 20;
   const double ccmax = 0.3, ccmxj = 0.2;
+  const double hlb = 100.0 * uround * tout;
+  // evaluation the next turn makes: a step's predictor, f of a new cell's
+  // state, one of its initial-step search (1..4), or f of the current state
+  // to restart from after error-test failures
+  enum { STEP = -1, FIRST = 0, RESTART = 5 };
   BdfResult res{0, 0, 0, 1, 0};
-  // a first call with tout = t returns at once, y untouched (vode.f:5475)
-  if (!(tout > 0.0)) return res;
-  double acor[N_], ewt[N_], savf[N_], yy[N_];  // ewt: reciprocal weights
-  double P[N_][N_];
-  int piv[N_];
-#pragma unroll
-  for (int i = 0; i < N_; i++) { z(0, i) = y[i]; ewt[i] = 1.0 / (rtol * fabs(y[i]) + atol); }
-  kin.rhs(rho, y, savf);
-  res.nfe++;
-  // initial step by DVHIN's rule (vode.f:3338-3460): between 100 uround tout
-  // and a tenth of tout, and no component moving by more than a tenth of
-  // itself plus atol in one step; within that, h ~ sqrt(2 / ||y''||) with
-  // y'' from a difference of derivatives, refined at most four times, then
-  // halved
-  double h;
-  {
-    const double hlb = 100.0 * uround * tout;
-    double hub = 0.1 * tout;
-#pragma unroll
-    for (int i = 0; i < N_; i++) {
-      const double dely = 0.1 * fabs(y[i]) + atol, af = fabs(savf[i]);
-      if (af * hub > dely) hub = dely / af;
-    }
-    double hg = sqrt(hlb * hub);
-    if (hub < hlb) {
-      h = hg;
-    } else {
-      double hnew = hg;
-      for (int it = 1; it <= 4; it++) {
-        double fy[N_];
-#pragma unroll
-        for (int i = 0; i < N_; i++) yy[i] = y[i] + hg * savf[i];
-        kin.rhs(rho, yy, fy);
-        res.nfe++;
-        const double rhg = 1.0 / hg;
-#pragma unroll
-        for (int i = 0; i < N_; i++) fy[i] = (fy[i] - savf[i]) * rhg;
-        const double ydd = d_wrms(fy, ewt);
-        hnew = (ydd * hub * hub > 2.0) ? sqrt(2.0 / ydd) : sqrt(hg * hub);
-        if (it == 4) break;
-        const double hrat = hnew / hg;
-        if (hrat > 0.5 && hrat < 2.0) break;
-        if (it >= 2 && hnew > 2.0 * hg) { hnew = hg; break; }
-        hg = hnew;
-      }
-      h = fmin(fmax(0.5 * hnew, hlb), hub);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < N_; i++) z(1, i) = h * savf[i];
+  bool alive = false, more = true;
+  int ev = FIRST;
+  double rho = 1.0, h = 0.0, t = 0.0, hub = 0.0, hg = 0.0;
   int q = 1, nqwait = 2, ncf = 0, kflag = 0;
   // etamax: largest step growth (DVSTEP's ETAMX1 = 1e4 after the first step,
   // then 10; 1 right after a failure)
-  double t = 0.0, rc = 0.0, crate = 1.0, hl0 = 0.0, etamax = 1.0e4, hsave = 1.0;
+  double rc = 0.0, crate = 1.0, etamax = 1.0e4, hsave = 1.0;
   bool need_p = true;   // DVODE's IPUP
-  bool p_ok = true;     // the last factorisation found a pivot in every column
   int nslp = 0, nslj = 0;
   int icf = 0;          // 1: corrector failed with a saved J, 2: with a current J
-  while (t < tout) {
-    if (res.nst >= maxstep) { res.ok = 0; break; }
-    // error weights at the start of the step
+  for (;;) {
+    if (!alive && more) {
+      double y[N_];
+      more = io.next(rho, y);
+      if (more) {
+        res = BdfResult{0, 0, 0, 1, 0};
+        // a first call with tout = t returns at once, y untouched
+        // (vode.f:5475)
+        if (!(tout > 0.0)) {
+          io.done(y, res);
+        } else {
 #pragma unroll
-    for (int i = 0; i < N_; i++) ewt[i] = 1.0 / (rtol * fabs(z(0, i)) + atol);
-    // predictor: multiply the Nordsieck array by the Pascal triangle
-    d_nordsieck_shift(z, q, 1.0);
-    const double l0 = IZ_CBDF.el[q][0];
-    hl0 = h * l0;
-    const double drc = (rc != 0.0) ? fabs(hl0 / rc - 1.0) : 0.0;
-    if (drc > ccmax || res.nst >= nslp + msbp) need_p = true;
-    // corrector (chord Newton on G(e) = h f(z0 + l0 e) - z1 - e)
-#pragma unroll
-    for (int n = 0; n < N_; n++) { yy[n] = z(0, n); acor[n] = 0.0; }
-    typename Kin::Cache kc;
-    kin.rhs_c(rho, yy, savf, kc);
-    res.nfe++;
-    bool jcur = false;
-    // The iteration matrix is factored at every step: a lane that asked
-    // for a new one builds it from h l0 (after a new J where one is due),
-    // every other lane rebuilds its current one from the same J and the
-    // h l0 it was built with (rc), which reproduces it bit for bit.  So the
-    // factors are never live across the step's kinetics (the predictor
-    // right-hand side, the Jacobian, the error test and order selection):
-    // the register budget goes to the kinetics instead of spills, which
-    // costs less than the extra factorisations (8.7 % less time on the
-    // 256^3 reacting half step, 4 % on the ignition ensemble).
-    {
-      const bool new_j = need_p && (res.nst == 0 || res.nst > nslj + jac_age ||
-                                    (icf == 1 && drc < ccmxj) || icf == 2);
-      if (new_j) {
-        double fac = d_wrms(savf, ewt);
-        double r0 = 1000.0 * fabs(h) * uround * N_ * fac;
-        if (r0 == 0.0) r0 = 1.0;
-        kin.jac_c(rho, yy, savf, kc, -1.0, ewt, r0, J);  // J = (f(y + r e_j) - f(y)) / r
-        res.nfe += N_;
-        res.nje++;
-        nslj = res.nst;
-        jcur = true;
-      }
-      const double con = need_p ? -hl0 : -rc;
-#pragma unroll
-      for (int i = 0; i < N_; i++)
-#pragma unroll
-        for (int j = 0; j < N_; j++) P[i][j] = con * J[i][j];
-#pragma unroll
-      for (int i = 0; i < N_; i++) P[i][i] += 1.0;
-      p_ok = d_lu(P, piv);
-      if (need_p) {
-        rc = hl0;
-        nslp = res.nst;
-        need_p = false;
-        crate = 1.0;
+          for (int n = 0; n < N_; n++) z(0, n) = y[n];
+          alive = true;
+          ev = FIRST;
+        }
       }
     }
-    bool conv = false;
-    double del = 0.0, delp = 0.0;
-    // a singular iteration matrix counts as a corrector failure (DVNLSD,
-    // IERPJ != 0)
-    for (int m = 0; m < maxcor && p_ok; m++) {
-      double d[N_];
+    if (!IZ_ANY(alive || more)) break;
+    if (alive) {
+      double ewt[N_], yy[N_], zp1[N_], f[N_];  // ewt: reciprocal error weights
+      bool fin = false;
 #pragma unroll
-      for (int n = 0; n < N_; n++) d[n] = h * savf[n] - z(1, n) - acor[n];
-      d_lusolve(P, piv, d);
-      res.nsol++;
-      if (rc != hl0) {  // chord correction for a stale h*l0
-        double cs = 2.0 / (1.0 + hl0 / rc);
-#pragma unroll
-        for (int n = 0; n < N_; n++) d[n] *= cs;
-      }
-      del = d_wrms(d, ewt);
-#pragma unroll
-      for (int n = 0; n < N_; n++) { acor[n] += d[n]; yy[n] = z(0, n) + l0 * acor[n]; }
-      // DVNLSD's convergence test: the rate estimate decays by CRDOWN = 0.3,
-      // and the correction must be below CORTES = 0.1 of the error-test
-      // tolerance
-      if (m > 0) crate = fmax(0.3 * crate, del / delp);
-      double dcon = del * fmin(1.0, crate) / (0.1 * IZ_CBDF.tesco[q][1]);
-      if (dcon <= 1.0) { conv = true; break; }
-      if (m >= 1 && del > 2.0 * delp) break;
-      delp = del;
-      kin.rhs(rho, yy, savf);
-      res.nfe++;
-    }
-    if (!conv) {
-      // undo the prediction; retry with a new iteration matrix, and with a
-      // quarter of the step (DVSTEP's ETACF) when the Jacobian was already
-      // current; the step after a failure keeps its size (ETAMAX = 1)
-      d_nordsieck_shift(z, q, -1.0);
-      ncf++;
-      need_p = true;
-      etamax = 1.0;
-      const bool hard = jcur || !p_ok;
-      icf = hard ? 2 : 1;
-      if (hard || ncf > 10) {
-        if (ncf > 10) { res.ok = 0; break; }
-        d_nordsieck_rescale(z, q, 0.25);
-        h *= 0.25;
-      }
-      continue;
-    }
-    icf = 0;
-    // local error test
-    double dsm = d_wrms(acor, ewt) / IZ_CBDF.tesco[q][1];
-#ifdef IZ_BDF_TRACE
-    printf("t %.4e h %.3e q %d dsm %.3e conv %d jcur %d T %.6f\n", t, h, q, dsm, (int)conv,
-           (int)jcur, z(0, 0));
-#endif
-    if (dsm > 1.0) {
-      // DVSTEP's policy after an error-test failure: eta = 1 / ((6 dsm)^(1/L)
-      // + 1e-6), at least 0.1 and at most 0.2 after the second failure in a
-      // row; after the third, one order lower at a tenth of the step, or at
-      // order 1 a restart from a fresh derivative; the seventh gives up
-      d_nordsieck_shift(z, q, -1.0);
-      kflag--;
-      etamax = 1.0;
-      if (kflag <= -7) { res.ok = 0; break; }
-      if (kflag > -3) {
-        double eta = fmax(1.0 / (d_powpos(6.0 * dsm, IZ_CBDF.rexp[q + 1]) + 1.0e-6), 0.1);
-        if (kflag <= -2) eta = fmin(eta, 0.2);
-        d_nordsieck_rescale(z, q, eta);
-        h *= eta;
-        continue;
-      }
-      if (q > 1) {
-        q--;
-        d_nordsieck_rescale(z, q, 0.1);
-        h *= 0.1;
-        nqwait = q + 1;
-        continue;
-      }
-      h *= 0.1;
-#pragma unroll
-      for (int n = 0; n < N_; n++) yy[n] = z(0, n);
-      kin.rhs(rho, yy, savf);
-      res.nfe++;
-#pragma unroll
-      for (int n = 0; n < N_; n++) z(1, n) = h * savf[n];
-      nqwait = 10;
-      need_p = true;
-      continue;
-    }
-    // accept
-    kflag = 0;
-    ncf = 0;
-    t += h;
-    res.nst++;
-    for (int j = 0; j <= q; j++) {
-      double e = IZ_CBDF.el[q][j];
-#pragma unroll
-      for (int n = 0; n < N_; n++) z(j, n) += e * acor[n];
-    }
-    nqwait--;
-    if (nqwait == 1 && q < 5) {
-#pragma unroll
-      for (int n = 0; n < N_; n++) z(5, n) = acor[n];  // kept for the order-up estimate
-      hsave = h;
-    }
-    if (etamax == 1.0) {
-      // the step after a failure keeps h and q
-      if (nqwait < 2) nqwait = 2;
-      etamax = 10.0;
-      continue;
-    }
-    // step size every step, order every q+1 steps (DVSTEP: ETAQ, and
-    // ETAQM1 / ETAQP1 when NQWAIT reaches 0; biases 6, 6 and 10)
-    double eta = 1.0 / (d_powpos(6.0 * dsm, IZ_CBDF.rexp[q + 1]) + 1.0e-6);
-    int newq = q;
-    if (nqwait == 0) {
-      nqwait = 2;
-      double etam = 0.0, etap = 0.0;
-      if (q > 1) {
-        double ddn = d_wrms_col(z, q, ewt) / IZ_CBDF.tesco[q][0];
-        etam = 1.0 / (d_powpos(6.0 * ddn, IZ_CBDF.rexp[q]) + 1.0e-6);
-      }
-      if (q < 5) {
-        // the saved correction, scaled to the current step (acor ~ h^(q+1))
-        const double cq = d_powpos(h / hsave, (double)(q + 1));
-        double dd[N_];
-#pragma unroll
-        for (int n = 0; n < N_; n++) dd[n] = acor[n] - cq * z(5, n);
-        double dup = d_wrms(dd, ewt) / IZ_CBDF.tesco[q][2];
-        etap = 1.0 / (d_powpos(10.0 * dup, IZ_CBDF.rexp[q + 2]) + 1.0e-6);
-      }
-      if (eta >= etap) {
-        if (eta < etam) { eta = etam; newq = q - 1; }
-      } else if (etap > etam) {
-        eta = etap; newq = q + 1;
+      for (int n = 0; n < N_; n++) ewt[n] = d_rcp(rtol * fabs(z(0, n)) + atol);
+      if (ev == STEP) {
+        // predictor
+        if (IZ_ANY(q > 3)) d_predict<5>(z, yy, zp1);
+        else if (IZ_ANY(q > 2)) d_predict<3>(z, yy, zp1);
+        else d_predict<2>(z, yy, zp1);
       } else {
-        eta = etam; newq = q - 1;
+        const double a = (ev == FIRST || ev == RESTART) ? 0.0 : hg;
+#pragma unroll
+        for (int n = 0; n < N_; n++) {
+          yy[n] = z(0, n);
+          zp1[n] = 0.0;
+          if (a != 0.0) yy[n] += a * z(1, n);
+        }
+      }
+      typename Kin::Cache kc;
+      kin.rhs_c(rho, yy, f, kc);
+      res.nfe++;
+      if (ev != STEP) {
+        // initial step by DVHIN's rule (vode.f:3338-3460): between 100
+        // uround tout and a tenth of tout, and no component moving by more
+        // than a tenth of itself plus atol in one step; within that, h ~
+        // sqrt(2 / ||y''||) with y'' from a difference of derivatives,
+        // refined at most four times, then halved
+        bool start = false;
+        if (ev == FIRST || ev == RESTART) {
+#pragma unroll
+          for (int n = 0; n < N_; n++) z(1, n) = f[n];
+          if (ev == RESTART) {
+            nqwait = 10;
+            need_p = true;
+          } else {
+            hub = 0.1 * tout;
+#pragma unroll
+            for (int n = 0; n < N_; n++) {
+              const double dely = 0.1 * fabs(yy[n]) + atol, af = fabs(f[n]);
+              if (af * hub > dely) hub = dely / af;
+            }
+            hg = sqrt(hlb * hub);
+            if (hub < hlb) {
+              h = hg;
+              start = true;
+            } else {
+              ev = 1;
+            }
+          }
+        } else {
+          const double rhg = 1.0 / hg;
+#pragma unroll
+          for (int n = 0; n < N_; n++) f[n] = (f[n] - z(1, n)) * rhg;
+          const double ydd = d_wrms(f, ewt);
+          double hnew = (ydd * hub * hub > 2.0) ? sqrt(2.0 / ydd) : sqrt(hg * hub);
+          const double hrat = hnew / hg;
+          if (ev == 4 || (hrat > 0.5 && hrat < 2.0)) {
+            start = true;
+          } else if (ev >= 2 && hnew > 2.0 * hg) {
+            hnew = hg;
+            start = true;
+          }
+          if (start) {
+            h = fmin(fmax(0.5 * hnew, hlb), hub);
+          } else {
+            hg = hnew;
+            ev++;
+          }
+        }
+        if (start) {
+          q = 1; nqwait = 2; ncf = 0; kflag = 0;
+          t = 0.0; rc = 0.0; crate = 1.0; etamax = 1.0e4; hsave = 1.0;
+          need_p = true;
+          nslp = 0; nslj = 0; icf = 0;
+        }
+        if (start || ev == RESTART) {
+#pragma unroll
+          for (int n = 0; n < N_; n++) {
+            z(1, n) *= h;
+            z(2, n) = 0.0; z(3, n) = 0.0; z(4, n) = 0.0; z(5, n) = 0.0;
+          }
+          ev = STEP;
+        }
+      } else {
+        // ------------------------------------------------------- one step
+        const double l0 = IZ_CBDF.el[q][0];
+        const double hl0 = h * l0;
+        const double drc = (rc != 0.0) ? fabs(hl0 / rc - 1.0) : 0.0;
+        if (drc > ccmax || res.nst >= nslp + msbp) need_p = true;
+        // corrector (chord Newton on G(e) = h f(z0 + l0 e) - z1 - e)
+        bool jcur = false;
+        // The iteration matrix is factored at every step: a lane that asked
+        // for a new one builds it from h l0 (after a new J where one is
+        // due), every other lane rebuilds its current one from the same J
+        // and the h l0 it was built with (rc), which reproduces it bit for
+        // bit.  So the factors are never live across the predictor's
+        // kinetics, the Jacobian and the error test: the register budget
+        // goes to the kinetics instead of spills.
+        const bool new_j = need_p && (res.nst == 0 || res.nst > nslj + jac_age ||
+                                      (icf == 1 && drc < ccmxj) || icf == 2);
+        if (new_j) {
+          const double fac = d_wrms(f, ewt);
+          double r0 = 1000.0 * fabs(h) * uround * N_ * fac;
+          if (r0 == 0.0) r0 = 1.0;
+          kin.jac_c(rho, yy, f, kc, -1.0, ewt, r0, J);  // J = (f(y + r e_j) - f(y)) / r
+          res.nfe += N_;
+          res.nje++;
+          nslj = res.nst;
+          jcur = true;
+        }
+        double P[N_][N_];
+        int piv[N_];
+        const double con = need_p ? -hl0 : -rc;
+#pragma unroll
+        for (int i = 0; i < M; i++)
+#pragma unroll
+          for (int j = 0; j < M; j++) P[i][j] = con * J[i][j] + (i == j ? 1.0 : 0.0);
+        // a singular iteration matrix counts as a corrector failure (DVNLSD,
+        // IERPJ != 0)
+        const bool p_ok = d_lu<M>(P, piv);
+        if (need_p) {
+          rc = hl0;
+          nslp = res.nst;
+          need_p = false;
+          crate = 1.0;
+        }
+        // chord correction for a stale h*l0
+        const double cs = (rc != hl0) ? 2.0 / (1.0 + hl0 / rc) : 1.0;
+        const double rtes = 1.0 / (0.1 * IZ_CBDF.tesco[q][1]);
+        double acor[N_];
+#pragma unroll
+        for (int n = 0; n < N_; n++) acor[n] = 0.0;
+        bool conv = false;
+        double delp = 1.0;
+        for (int m = 0; m < maxcor && p_ok; m++) {
+          if (m > 0) {
+            kin.rhs(rho, yy, f);
+            res.nfe++;
+          }
+          double d[N_];
+#pragma unroll
+          for (int n = 0; n < N_; n++) d[n] = h * f[n] - zp1[n] - acor[n];
+          d_lusolve<M>(P, piv, d);
+          res.nsol++;
+          double s2 = 0.0;
+#pragma unroll
+          for (int n = 0; n < N_; n++) {
+            d[n] *= cs;
+            acor[n] += d[n];
+            yy[n] += l0 * d[n];
+            const double x = d[n] * ewt[n];
+            s2 += x * x;
+          }
+          const double del = sqrt(s2 / N_);
+          // DVNLSD's convergence test: the rate estimate decays by CRDOWN =
+          // 0.3, and the correction must be below CORTES = 0.1 of the
+          // error-test tolerance
+          if (m > 0) crate = fmax(0.3 * crate, del / delp);
+          const double dcon = del * fmin(1.0, crate) * rtes;
+          if (dcon <= 1.0) { conv = true; break; }
+          if (m >= 1 && del > 2.0 * delp) break;
+          delp = del;
+        }
+        // local error test
+        const double dsm = d_wrms(acor, ewt) / IZ_CBDF.tesco[q][1];
+        if (!conv) {
+          // retry with a new iteration matrix, and with a quarter of the
+          // step (DVSTEP's ETACF) when the Jacobian was already current;
+          // the step after a failure keeps its size (ETAMAX = 1)
+          ncf++;
+          need_p = true;
+          etamax = 1.0;
+          const bool hard = jcur || !p_ok;
+          icf = hard ? 2 : 1;
+          if (ncf > 10) {
+            res.ok = 0;
+            fin = true;
+          } else if (hard) {
+            d_nordsieck_rescale(z, q, 0.25);
+            h *= 0.25;
+          }
+        } else if (dsm > 1.0) {
+          // DVSTEP's policy after an error-test failure: eta = 1 / ((6
+          // dsm)^(1/L) + 1e-6), at least 0.1 and at most 0.2 after the
+          // second failure in a row; after the third, one order lower at a
+          // tenth of the step, or at order 1 a restart from a fresh
+          // derivative; the seventh gives up
+          icf = 0;
+          kflag--;
+          etamax = 1.0;
+          if (kflag <= -7) {
+            res.ok = 0;
+            fin = true;
+          } else if (kflag > -3) {
+            double eta = fmax(1.0 / (d_powpos(6.0 * dsm, IZ_CBDF.rexp[q + 1]) + 1.0e-6), 0.1);
+            if (kflag <= -2) eta = fmin(eta, 0.2);
+            d_nordsieck_rescale(z, q, eta);
+            h *= eta;
+          } else if (q > 1) {
+#pragma unroll
+            for (int n = 0; n < N_; n++) z(q, n) = 0.0;
+            q--;
+            d_nordsieck_rescale(z, q, 0.1);
+            h *= 0.1;
+            nqwait = q + 1;
+          } else {
+            h *= 0.1;
+            ev = RESTART;
+          }
+        } else {
+          // accept
+          icf = 0;
+          kflag = 0;
+          ncf = 0;
+          t += h;
+          res.nst++;
+          double el[6];
+#pragma unroll
+          for (int j = 0; j < 6; j++) el[j] = (j <= q) ? IZ_CBDF.el[q][j] : 0.0;
+          if (IZ_ANY(q > 3)) d_advance<5>(z, el, acor);
+          else if (IZ_ANY(q > 2)) d_advance<3>(z, el, acor);
+          else d_advance<2>(z, el, acor);
+          nqwait--;
+          if (nqwait == 1 && q < 5) {
+#pragma unroll
+            for (int n = 0; n < N_; n++) z(IZ_ZSAVE, n) = acor[n];  // for the order-up estimate
+            hsave = h;
+          }
+          if (t >= tout) {
+            fin = true;  // interpolated below with this step's h and history
+          } else if (etamax == 1.0) {
+            // the step after a failure keeps h and q
+            if (nqwait < 2) nqwait = 2;
+            etamax = 10.0;
+          } else {
+            // step size every step, order every q+1 steps (DVSTEP: ETAQ, and
+            // ETAQM1 / ETAQP1 when NQWAIT reaches 0; biases 6, 6 and 10)
+            double eta = 1.0 / (d_powpos(6.0 * dsm, IZ_CBDF.rexp[q + 1]) + 1.0e-6);
+            int newq = q;
+            if (nqwait == 0) {
+              nqwait = 2;
+              double etam = 0.0, etap = 0.0;
+              if (q > 1) {
+                double ddn = d_wrms_col(z, q, ewt) / IZ_CBDF.tesco[q][0];
+                etam = 1.0 / (d_powpos(6.0 * ddn, IZ_CBDF.rexp[q]) + 1.0e-6);
+              }
+              if (q < 5) {
+                // the saved correction, scaled to the current step (acor ~ h^(q+1))
+                const double cq = d_powpos(h / hsave, (double)(q + 1));
+                double dd[N_];
+#pragma unroll
+                for (int n = 0; n < N_; n++) dd[n] = acor[n] - cq * z(IZ_ZSAVE, n);
+                double dup = d_wrms(dd, ewt) / IZ_CBDF.tesco[q][2];
+                etap = 1.0 / (d_powpos(10.0 * dup, IZ_CBDF.rexp[q + 2]) + 1.0e-6);
+              }
+              if (eta >= etap) {
+                if (eta < etam) { eta = etam; newq = q - 1; }
+              } else if (etap > etam) {
+                eta = etap; newq = q + 1;
+              } else {
+                eta = etam; newq = q - 1;
+              }
+            }
+            if (eta >= 1.5) {  // below THRESH: keep h and q
+              eta = fmin(eta, etamax);
+              if (newq > q) {
+                // new highest-order column from the last correction
+                double e = IZ_CBDF.el[q][q] / (q + 1);
+#pragma unroll
+                for (int n = 0; n < N_; n++) z(newq, n) = acor[n] * e;
+              } else if (newq < q) {
+#pragma unroll
+                for (int n = 0; n < N_; n++) z(q, n) = 0.0;
+              }
+              if (newq != q) nqwait = newq + 1;
+              q = newq;
+              d_nordsieck_rescale(z, q, eta);
+              h *= eta;
+            }
+            etamax = 10.0;
+          }
+        }
+        if (!fin && ev == STEP && res.nst >= maxstep) {
+          res.ok = 0;
+          fin = true;
+        }
+        if (fin) {
+          // interpolate back to tout: y = sum_j z(j) s^j
+          const double s = (tout - t) / h;
+#pragma unroll
+          for (int n = 0; n < N_; n++) {
+            double acc = z(5, n);
+#pragma unroll
+            for (int j = 4; j >= 0; j--) acc = acc * s + z(j, n);
+            yy[n] = acc;
+          }
+          io.done(yy, res);
+          alive = false;
+        }
       }
     }
-    if (eta < 1.5) { etamax = 10.0; continue; }  // THRESH: keep h and q
-    eta = fmin(eta, etamax);
-    etamax = 10.0;
-    if (newq > q) {
-      // new highest-order column from the last correction
-      double e = IZ_CBDF.el[q][q] / (q + 1);
-#pragma unroll
-      for (int n = 0; n < N_; n++) z(newq, n) = acor[n] * e;
-    }
-    if (newq != q) nqwait = newq + 1;
-    q = newq;
-    d_nordsieck_rescale(z, q, eta);
-    h *= eta;
   }
-  // interpolate back to tout: y = sum_j z(j) s^j
-  double s = (tout - t) / h;
-#pragma unroll
-  for (int n = 0; n < N_; n++) {
-    double acc = z(q, n);
-    for (int j = q - 1; j >= 0; j--) acc = acc * s + z(j, n);
-    y[n] = acc;
+}
+
+// one cell from 0 to tout (ITASK = 1: step past tout and interpolate back)
+struct BdfOneCell {
+  double rho, *y;
+  bool taken;
+  BdfResult res;
+  IZ_MHD inline bool next(double &r, double *yc) {
+    if (taken) return false;
+    taken = true;
+    r = rho;
+    for (int n = 0; n < N_; n++) yc[n] = y[n];
+    return true;
   }
-  return res;
+  IZ_MHD inline void done(const double *yc, const BdfResult &r) {
+    for (int n = 0; n < N_; n++) y[n] = yc[n];
+    res = r;
+  }
+};
+template <class Kin, class Z>
+IZ_HD inline BdfResult d_bdf_integrate(const Kin &kin, Z &z, double (&J)[N_][N_], double rho,
+                                       double *y, double tout, double rtol, double atol,
+                                       int jac_age) {
+  BdfOneCell io{rho, y, false, {0, 0, 0, 1, 0}};
+  d_bdf_run(kin, z, J, io, tout, rtol, atol, jac_age);
+  return io.res;
 }
 
 
@@ -630,6 +773,7 @@ IZ_HD IZ_FORCEINLINE BdfResult d_bdf_integrate(const Kin &kin, Z &z, double (&J)
 // straight-line kinetics of the compiled-in mechanism; the T-only part kt is
 // shared by the Jacobian columns that perturb mass fractions
 struct KinGen {
+  static constexpr int NACT = 1 + GEN_NLIVE;
   struct Cache { double kt[GEN_NKT]; };  // rate constants at the evaluated T
   IZ_MHD inline void rhs(double rho, const double *y, double *f) const {
     double kt[GEN_NKT];
@@ -675,33 +819,23 @@ struct KinGen {
   }
 };
 
-// The straight-line kinetics with the mass-fraction columns of the
-// Jacobian in closed form (gen_jac, generated with the rates: mass action,
-// third-body sums, falloff factors differentiated) and the temperature
-// column by a finite difference as above: one evaluation of the kinetics
-// per Jacobian instead of GEN_KK + 1.  DVODE's user-Jacobian form (MF = 21,
-// vode.f:3596-3727) in place of the reference's MF = 22; the integration
-// keeps the same error control, so results stay within its tolerance.
+// The straight-line kinetics with the Jacobian in closed form (gen_jac and
+// gen_jac_T, generated with the rates): about one evaluation of the
+// concentration part per Jacobian instead of GEN_KK + 1 and another
+// temperature part.  DVODE's user-Jacobian form (MF = 21, vode.f:3596-3727)
+// in place of the reference's MF = 22; the integration keeps the same error
+// control, so results stay within its tolerance.
 struct KinGenAJ : KinGen {
   IZ_MHD inline void jac_c(double rho, const double *y, const double *f0, const Cache &c,
                            double hl0, const double *w, double r0, double (*P)[N_]) const {
     gen_jac(rho, y, c.kt, f0[0], P);
+    gen_jac_T(rho, y, c.kt, f0, P);
     if (hl0 != -1.0) {
 #pragma unroll
       for (int i = 0; i < N_; i++)
 #pragma unroll
-        for (int j = 1; j < N_; j++) P[i][j] = -hl0 * P[i][j];
+        for (int j = 0; j < N_; j++) P[i][j] = -hl0 * P[i][j];
     }
-    double yl[N_], ftmp[N_], kt0[GEN_NKT];
-#pragma unroll
-    for (int n = 0; n < N_; n++) yl[n] = y[n];
-    const double r = d_fd_increment(0, yl[0], w[0], r0);
-    yl[0] = yl[0] + r;
-    gen_kT(yl[0], kt0);
-    gen_rhs(rho, yl, kt0, ftmp);
-    const double ri = 1.0 / r;
-#pragma unroll
-    for (int i = 0; i < N_; i++) P[i][0] = -hl0 * (ftmp[i] - f0[i]) * ri;
   }
 };
 #endif

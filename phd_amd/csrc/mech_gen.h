@@ -3,219 +3,184 @@
 // Straight-line form of CKWYR + FUN (devel-izem/src/chemkin/vode.f:935-1314,
 // 1797-1904; chemkin/reaction_v.f:69-114).
 #pragma once
+#include "iz_math.h"
 #define GEN_KK 9
 #define GEN_II 21
 #define GEN_MECH_HASH "0f6fcba421d460f4"
-#define GEN_NKT 64
+#define GEN_NLIVE 8
+#define GEN_NKT 59
 
 IZ_HD inline void gen_kT(double T, double *kt) {
-#pragma clang fp contract(off)
+#pragma clang fp contract(on)
   const double ru = 8.314510e7;
-  const double lt = log(T), it = 1.0 / T;
-  const double T2 = T * T, T3 = T2 * T, T4 = T3 * T;
-  const double pfac = 1.01325e6 / (8.314510e7 * T);
-  double smh0, cpR0, hRT0;
-  double smh1, cpR1, hRT1;
-  double smh2, cpR2, hRT2;
-  double smh3, cpR3, hRT3;
-  double smh4, cpR4, hRT4;
-  double smh5, cpR5, hRT5;
-  double smh6, cpR6, hRT6;
-  double smh7, cpR7, hRT7;
-  double smh8, cpR8, hRT8;
+  const double lt = d_log(T), it = 1.0 / T, sT = sqrt(T);
+  const double T2 = T * T, T3 = T2 * T, T4 = T3 * T, ruT = ru * T;
+  const double rtp = ruT * (1.0 / 1.01325e6), pfac = 1.01325e6 / ru * it;
+  double w0;
+  double w2;
+  double w4;
+  double w5;
+  double w6;
+  double w7;
   if (T > 1000.0) {
-    smh0 = 2.50000001 * (lt - 1.0) + -1.154214865e-11 * T + 2.6926991333333336e-15 * T2 + -3.945960291666667e-19 * T3 + 2.490986785e-23 * T4 + -0.446682914 - 25473.6599 * it;
-    cpR0 = 2.50000001 + -2.30842973e-11 * T + 1.61561948e-14 * T2 + -4.73515235e-18 * T3 + 4.98197357e-22 * T4;
-    hRT0 = 2.50000001 + -1.154214865e-11 * T + 5.385398266666667e-15 * T2 + -1.1837880875e-18 * T3 + 9.96394714e-23 * T4 + 25473.6599 * it;
+    w0 = 0.83136041 * (lt - 1.0) + 1.2350606732851349e-05 * T - 4.162139547396753e-08 * T2 + 7.481932688737305e-12 * T3 - 5.006384150901322e-16 * T4 + 1.155828741 - 25948.739361 * it;
+    w2 = 0.9281518600000003 * (lt - 1.0) - 0.00041375894185 * T + 7.01552989e-08 * T2 - 9.562754783333333e-12 * T3 + 6.032113304999999e-16 * T4 + 2.0577229949999998 - 29761.80796 * it;
+    w4 = -0.2170208499999995 * (lt - 1.0) - 8.4206408725e-05 * T + 4.2626695583333334e-08 * T2 - 8.574853008333332e-12 * T3 + 6.28217925e-16 * T4 + 3.35259211 - 4877.965321 * it;
+    w5 = -1.944555629999999 * (lt - 1.0) + 0.00074238837155 * T - 4.742432691666666e-08 * T2 - 1.850905874999999e-12 * T3 + 3.8152256499999997e-16 * T4 + 5.445177765 - -28509.909317999998 * it;
+    w6 = -0.9339665399999992 * (lt - 1.0) + 0.00039071691327500005 * T - 2.0903311666666663e-08 * T2 - 4.5341566666666543e-13 * T3 + 4.340785499999996e-17 * T4 - 0.06561748499999975 - 1675.393894 * it;
+    w7 = -2.4548141899999996 * (lt - 1.0) + 0.00173731593655 * T - 2.738137265e-07 * T2 + 2.8440152083333333e-11 * T3 - 1.357229435e-15 * T4 + 0.6679486400000005 - -15823.171058 * it;
+    kt[41] = 82487675.25154442 * (1.50000001 - 2.30842973e-11 * T + 1.61561948e-14 * T2 - 4.73515235e-18 * T3 + 4.98197357e-22 * T4);
+    kt[42] = ruT * (1.50000001 - 1.154214865e-11 * T + 5.385398266666667e-15 * T2 - 1.1837880875e-18 * T3 + 9.96394714e-23 * T4 + 25473.6599 * it);
+    kt[43] = 41243837.62577221 * (2.3372792 - 4.94024731e-05 * T + 4.99456778e-07 * T2 - 1.79566394e-10 * T3 + 2.00255376e-14 * T4);
+    kt[44] = ruT * (2.3372792 - 2.470123655e-05 * T + 1.6648559266666665e-07 * T2 - 4.48915985e-11 * T3 + 4.00510752e-15 * T4 - 950.158922 * it);
+    kt[45] = 5196763.583534601 * (1.5694207800000002 - 8.59741137e-05 * T + 4.19484589e-08 * T2 - 1.00177799e-11 * T3 + 1.22833691e-15 * T4);
+    kt[46] = ruT * (1.5694207800000002 - 4.298705685e-05 * T + 1.3982819633333334e-08 * T2 - 2.504444975e-12 * T3 + 2.4566738199999997e-16 * T4 + 29217.5791 * it);
+    kt[47] = 2598381.7917673006 * (2.28253784 + 0.00148308754 * T - 7.57966669e-07 * T2 + 2.09470555e-10 * T3 - 2.16717794e-14 * T4);
+    kt[48] = ruT * (2.28253784 + 0.00074154377 * T - 2.526555563333333e-07 * T2 + 5.236763875e-11 * T3 - 4.33435588e-15 * T4 - 1088.45772 * it);
+    kt[49] = 4888768.777364419 * (2.09288767 + 0.000548429716 * T + 1.26505228e-07 * T2 - 8.79461556e-11 * T3 + 1.17412376e-14 * T4);
+    kt[50] = ruT * (2.09288767 + 0.000274214858 * T + 4.216840933333333e-08 * T2 - 2.19865389e-11 * T3 + 2.34824752e-15 * T4 + 3858.657 * it);
+    kt[51] = 4615238.989969709 * (2.03399249 + 0.00217691804 * T - 1.64072518e-07 * T2 - 9.7041987e-11 * T3 + 1.68200992e-14 * T4);
+    kt[52] = ruT * (2.03399249 + 0.00108845902 * T - 5.469083933333333e-08 * T2 - 2.426049675e-11 * T3 + 3.36401984e-15 * T4 - 30004.2971 * it);
+    kt[53] = 2519031.682355707 * (3.0172109000000003 + 0.00223982013 * T - 6.3365815e-07 * T2 + 1.1424637e-10 * T3 - 1.07908535e-14 * T4);
+    kt[54] = ruT * (3.0172109000000003 + 0.001119910065 * T - 2.1121938333333332e-07 * T2 + 2.85615925e-11 * T3 - 2.1581707e-15 * T4 + 111.856713 * it);
+    kt[55] = 2444384.3886822094 * (3.1650028499999996 + 0.00490831694 * T - 1.90139225e-06 * T2 + 3.71185986e-10 * T3 - 2.87908305e-14 * T4);
+    kt[56] = ruT * (3.1650028499999996 + 0.00245415847 * T - 6.337974166666666e-07 * T2 + 9.27964965e-11 * T3 - 5.7581661e-15 * T4 - 17861.7877 * it);
+    kt[57] = 2968047.527239741 * (1.92664 + 0.0014879768 * T - 5.68476e-07 * T2 + 1.0097038e-10 * T3 - 6.753351e-15 * T4);
+    kt[58] = ruT * (1.92664 + 0.0007439884 * T - 1.8949200000000001e-07 * T2 + 2.5242595e-11 * T3 - 1.3506701999999999e-15 * T4 - 922.7977 * it);
   } else {
-    smh0 = 2.5 * (lt - 1.0) + 3.526664095e-13 * T + -3.3265327333333333e-16 * T2 + 1.9173469333333331e-19 * T3 + -4.63866166e-23 * T4 + -0.446682853 - 25473.6599 * it;
-    cpR0 = 2.5 + 7.05332819e-13 * T + -1.99591964e-15 * T2 + 2.30081632e-18 * T3 + -9.27732332e-22 * T4;
-    hRT0 = 2.5 + 3.526664095e-13 * T + -6.653065466666667e-16 * T2 + 5.7520408e-19 * T3 + -1.855464664e-22 * T4 + 25473.6599 * it;
+    w0 = 1.32783444 * (lt - 1.0) - 0.0019951301871473336 * T + 1.6231792496673465e-06 * T2 - 8.398837248082654e-10 * T3 + 1.844029402036134e-13 * T4 - 0.788187972 - 25932.627486499998 * it;
+    w2 = 1.27703892 * (lt - 1.0) - 0.00089047588 * T + 2.865688258333333e-07 * T2 - 1.0728489124999998e-10 * T3 + 2.4539776249999996e-14 * T4 + 0.22309559499999998 - 29654.23098 * it;
+    w4 = 0.9286216899999999 * (lt - 1.0) - 0.0024466054075 * T + 1.5722271508333332e-06 * T2 - 7.599242070833334e-10 * T3 + 1.7151546600000003e-13 * T4 - 2.274268442 - 4606.0199265 * it;
+    w5 = -0.03691873999999995 * (lt - 1.0) - 0.004259293884999999 * T + 3.5124836841666664e-06 * T2 - 1.7337110395833333e-09 * T3 + 3.763115797500001e-13 * T4 - 3.3608803110000003 - -28843.819746999998 * it;
+    w6 = -0.6528239100000004 * (lt - 1.0) - 0.0028713233625 * T + 3.5083437649999998e-06 * T2 - 2.0561415841666666e-09 * T3 + 4.868290837500001e-13 * T4 - 0.2825183990000002 - 1817.7191865 * it;
+    w7 = -1.8506747900000002 * (lt - 1.0) - 0.0027633045034999994 * T + 4.394069848333334e-06 * T2 - 2.6710829675e-09 * T3 + 6.378466435e-13 * T4 - 0.905635228 - -15720.703367 * it;
+    kt[41] = 82487675.25154442 * (1.5 + 7.05332819e-13 * T - 1.99591964e-15 * T2 + 2.30081632e-18 * T3 - 9.27732332e-22 * T4);
+    kt[42] = ruT * (1.5 + 3.526664095e-13 * T - 6.653065466666667e-16 * T2 + 5.7520408e-19 * T3 - 1.855464664e-22 * T4 + 25473.6599 * it);
+    kt[43] = 41243837.62577221 * (1.34433112 + 0.00798052075 * T - 1.9478151e-05 * T2 + 2.01572094e-08 * T3 - 7.37611761e-12 * T4);
+    kt[44] = ruT * (1.34433112 + 0.003990260375 * T - 6.4927169999999995e-06 * T2 + 5.03930235e-09 * T3 - 1.4752235220000002e-12 * T4 - 917.935173 * it);
+    kt[45] = 5196763.583534601 * (2.1682671 - 0.00327931884 * T + 6.64306396e-06 * T2 - 6.12806624e-09 * T3 + 2.11265971e-12 * T4);
+    kt[46] = ruT * (2.1682671 - 0.00163965942 * T + 2.2143546533333334e-06 * T2 - 1.53201656e-09 * T3 + 4.22531942e-13 * T4 + 29122.2592 * it);
+    kt[47] = 2598381.7917673006 * (2.78245636 - 0.00299673416 * T + 9.84730201e-06 * T2 - 9.68129509e-09 * T3 + 3.24372837e-12 * T4);
+    kt[48] = ruT * (2.78245636 - 0.00149836708 * T + 3.282434003333333e-06 * T2 - 2.4203237725e-09 * T3 + 6.48745674e-13 * T4 - 1063.94356 * it);
+    kt[49] = 4888768.777364419 * (2.99201543 - 0.00240131752 * T + 4.61793841e-06 * T2 - 3.88113333e-09 * T3 + 1.3641147e-12 * T4);
+    kt[50] = ruT * (2.99201543 - 0.00120065876 * T + 1.5393128033333333e-06 * T2 - 9.702833325e-10 * T3 + 2.7282294e-13 * T4 + 3615.08056 * it);
+    kt[51] = 4615238.989969709 * (3.1986405600000003 - 0.0020364341 * T + 6.52040211e-06 * T2 - 5.48797062e-09 * T3 + 1.77197817e-12 * T4);
+    kt[52] = ruT * (3.1986405600000003 - 0.00101821705 * T + 2.17346737e-06 * T2 - 1.371992655e-09 * T3 + 3.54395634e-13 * T4 - 30293.7267 * it);
+    kt[53] = 2519031.682355707 * (3.3017980099999997 - 0.00474912051 * T + 2.11582891e-05 * T2 - 2.42763894e-08 * T3 + 9.29225124e-12 * T4);
+    kt[54] = ruT * (3.3017980099999997 - 0.002374560255 * T + 7.0527630333333326e-06 * T2 - 6.06909735e-09 * T3 + 1.8584502480000002e-12 * T4 + 294.80804 * it);
+    kt[55] = 2444384.3886822094 * (3.2761126899999997 - 0.000542822417 * T + 1.67335701e-05 * T2 - 2.15770813e-08 * T3 + 8.62454363e-12 * T4);
+    kt[56] = ruT * (3.2761126899999997 - 0.0002714112085 * T + 5.5778567000000005e-06 * T2 - 5.394270325e-09 * T3 + 1.724908726e-12 * T4 - 17702.5821 * it);
+    kt[57] = 2968047.527239741 * (2.298677 + 0.0014082404 * T - 3.963222e-06 * T2 + 5.641515e-09 * T3 - 2.444854e-12 * T4);
+    kt[58] = ruT * (2.298677 + 0.0007041202 * T - 1.3210739999999999e-06 * T2 + 1.41037875e-09 * T3 - 4.889707999999999e-13 * T4 - 1020.8999 * it);
   }
-  if (T > 1000.0) {
-    smh1 = 3.3372792 * (lt - 1.0) + -2.470123655e-05 * T + 8.324279633333333e-08 * T2 + -1.4963866166666668e-11 * T3 + 1.00127688e-15 * T4 + -3.20502331 - -950.158922 * it;
-    cpR1 = 3.3372792 + -4.94024731e-05 * T + 4.99456778e-07 * T2 + -1.79566394e-10 * T3 + 2.00255376e-14 * T4;
-    hRT1 = 3.3372792 + -2.470123655e-05 * T + 1.6648559266666665e-07 * T2 + -4.48915985e-11 * T3 + 4.00510752e-15 * T4 + -950.158922 * it;
-  } else {
-    smh1 = 2.34433112 * (lt - 1.0) + 0.003990260375 * T + -3.2463584999999998e-06 * T2 + 1.67976745e-09 * T3 + -3.6880588050000004e-13 * T4 + 0.683010238 - -917.935173 * it;
-    cpR1 = 2.34433112 + 0.00798052075 * T + -1.9478151e-05 * T2 + 2.01572094e-08 * T3 + -7.37611761e-12 * T4;
-    hRT1 = 2.34433112 + 0.003990260375 * T + -6.4927169999999995e-06 * T2 + 5.03930235e-09 * T3 + -1.4752235220000002e-12 * T4 + -917.935173 * it;
-  }
-  if (T > 1000.0) {
-    smh2 = 2.56942078 * (lt - 1.0) + -4.298705685e-05 * T + 6.991409816666667e-09 * T2 + -8.348149916666666e-13 * T3 + 6.141684549999999e-17 * T4 + 4.78433864 - 29217.5791 * it;
-    cpR2 = 2.56942078 + -8.59741137e-05 * T + 4.19484589e-08 * T2 + -1.00177799e-11 * T3 + 1.22833691e-15 * T4;
-    hRT2 = 2.56942078 + -4.298705685e-05 * T + 1.3982819633333334e-08 * T2 + -2.504444975e-12 * T3 + 2.4566738199999997e-16 * T4 + 29217.5791 * it;
-  } else {
-    smh2 = 3.1682671 * (lt - 1.0) + -0.00163965942 * T + 1.1071773266666667e-06 * T2 + -5.106721866666666e-10 * T3 + 1.056329855e-13 * T4 + 2.05193346 - 29122.2592 * it;
-    cpR2 = 3.1682671 + -0.00327931884 * T + 6.64306396e-06 * T2 + -6.12806624e-09 * T3 + 2.11265971e-12 * T4;
-    hRT2 = 3.1682671 + -0.00163965942 * T + 2.2143546533333334e-06 * T2 + -1.53201656e-09 * T3 + 4.22531942e-13 * T4 + 29122.2592 * it;
-  }
-  if (T > 1000.0) {
-    smh3 = 3.28253784 * (lt - 1.0) + 0.00074154377 * T + -1.2632777816666666e-07 * T2 + 1.745587958333333e-11 * T3 + -1.08358897e-15 * T4 + 5.45323129 - -1088.45772 * it;
-    cpR3 = 3.28253784 + 0.00148308754 * T + -7.57966669e-07 * T2 + 2.09470555e-10 * T3 + -2.16717794e-14 * T4;
-    hRT3 = 3.28253784 + 0.00074154377 * T + -2.526555563333333e-07 * T2 + 5.236763875e-11 * T3 + -4.33435588e-15 * T4 + -1088.45772 * it;
-  } else {
-    smh3 = 3.78245636 * (lt - 1.0) + -0.00149836708 * T + 1.6412170016666666e-06 * T2 + -8.067745908333334e-10 * T3 + 1.621864185e-13 * T4 + 3.65767573 - -1063.94356 * it;
-    cpR3 = 3.78245636 + -0.00299673416 * T + 9.84730201e-06 * T2 + -9.68129509e-09 * T3 + 3.24372837e-12 * T4;
-    hRT3 = 3.78245636 + -0.00149836708 * T + 3.282434003333333e-06 * T2 + -2.4203237725e-09 * T3 + 6.48745674e-13 * T4 + -1063.94356 * it;
-  }
-  if (T > 1000.0) {
-    smh4 = 3.09288767 * (lt - 1.0) + 0.000274214858 * T + 2.1084204666666666e-08 * T2 + -7.3288463e-12 * T3 + 5.8706188e-16 * T4 + 4.4766961 - 3858.657 * it;
-    cpR4 = 3.09288767 + 0.000548429716 * T + 1.26505228e-07 * T2 + -8.79461556e-11 * T3 + 1.17412376e-14 * T4;
-    hRT4 = 3.09288767 + 0.000274214858 * T + 4.216840933333333e-08 * T2 + -2.19865389e-11 * T3 + 2.34824752e-15 * T4 + 3858.657 * it;
-  } else {
-    smh4 = 3.99201543 * (lt - 1.0) + -0.00120065876 * T + 7.696564016666666e-07 * T2 + -3.234277775e-10 * T3 + 6.8205735e-14 * T4 + -0.103925458 - 3615.08056 * it;
-    cpR4 = 3.99201543 + -0.00240131752 * T + 4.61793841e-06 * T2 + -3.88113333e-09 * T3 + 1.3641147e-12 * T4;
-    hRT4 = 3.99201543 + -0.00120065876 * T + 1.5393128033333333e-06 * T2 + -9.702833325e-10 * T3 + 2.7282294e-13 * T4 + 3615.08056 * it;
-  }
-  if (T > 1000.0) {
-    smh5 = 3.03399249 * (lt - 1.0) + 0.00108845902 * T + -2.7345419666666664e-08 * T2 + -8.08683225e-12 * T3 + 8.4100496e-16 * T4 + 4.9667701 - -30004.2971 * it;
-    cpR5 = 3.03399249 + 0.00217691804 * T + -1.64072518e-07 * T2 + -9.7041987e-11 * T3 + 1.68200992e-14 * T4;
-    hRT5 = 3.03399249 + 0.00108845902 * T + -5.469083933333333e-08 * T2 + -2.426049675e-11 * T3 + 3.36401984e-15 * T4 + -30004.2971 * it;
-  } else {
-    smh5 = 4.19864056 * (lt - 1.0) + -0.00101821705 * T + 1.086733685e-06 * T2 + -4.57330885e-10 * T3 + 8.85989085e-14 * T4 + -0.849032208 - -30293.7267 * it;
-    cpR5 = 4.19864056 + -0.0020364341 * T + 6.52040211e-06 * T2 + -5.48797062e-09 * T3 + 1.77197817e-12 * T4;
-    hRT5 = 4.19864056 + -0.00101821705 * T + 2.17346737e-06 * T2 + -1.371992655e-09 * T3 + 3.54395634e-13 * T4 + -30293.7267 * it;
-  }
-  if (T > 1000.0) {
-    smh6 = 4.0172109 * (lt - 1.0) + 0.001119910065 * T + -1.0560969166666666e-07 * T2 + 9.520530833333334e-12 * T3 + -5.39542675e-16 * T4 + 3.78510215 - 111.856713 * it;
-    cpR6 = 4.0172109 + 0.00223982013 * T + -6.3365815e-07 * T2 + 1.1424637e-10 * T3 + -1.07908535e-14 * T4;
-    hRT6 = 4.0172109 + 0.001119910065 * T + -2.1121938333333332e-07 * T2 + 2.85615925e-11 * T3 + -2.1581707e-15 * T4 + 111.856713 * it;
-  } else {
-    smh6 = 4.30179801 * (lt - 1.0) + -0.002374560255 * T + 3.5263815166666663e-06 * T2 + -2.02303245e-09 * T3 + 4.646125620000001e-13 * T4 + 3.71666245 - 294.80804 * it;
-    cpR6 = 4.30179801 + -0.00474912051 * T + 2.11582891e-05 * T2 + -2.42763894e-08 * T3 + 9.29225124e-12 * T4;
-    hRT6 = 4.30179801 + -0.002374560255 * T + 7.0527630333333326e-06 * T2 + -6.06909735e-09 * T3 + 1.8584502480000002e-12 * T4 + 294.80804 * it;
-  }
-  if (T > 1000.0) {
-    smh7 = 4.16500285 * (lt - 1.0) + 0.00245415847 * T + -3.168987083333333e-07 * T2 + 3.0932165499999996e-11 * T3 + -1.439541525e-15 * T4 + 2.91615662 - -17861.7877 * it;
-    cpR7 = 4.16500285 + 0.00490831694 * T + -1.90139225e-06 * T2 + 3.71185986e-10 * T3 + -2.87908305e-14 * T4;
-    hRT7 = 4.16500285 + 0.00245415847 * T + -6.337974166666666e-07 * T2 + 9.27964965e-11 * T3 + -5.7581661e-15 * T4 + -17861.7877 * it;
-  } else {
-    smh7 = 4.27611269 * (lt - 1.0) + -0.0002714112085 * T + 2.7889283500000002e-06 * T2 + -1.7980901083333332e-09 * T3 + 4.312271815e-13 * T4 + 3.43505074 - -17702.5821 * it;
-    cpR7 = 4.27611269 + -0.000542822417 * T + 1.67335701e-05 * T2 + -2.15770813e-08 * T3 + 8.62454363e-12 * T4;
-    hRT7 = 4.27611269 + -0.0002714112085 * T + 5.5778567000000005e-06 * T2 + -5.394270325e-09 * T3 + 1.724908726e-12 * T4 + -17702.5821 * it;
-  }
-  if (T > 1000.0) {
-    smh8 = 2.92664 * (lt - 1.0) + 0.0007439884 * T + -9.474600000000001e-08 * T2 + 8.414198333333333e-12 * T3 + -3.3766754999999997e-16 * T4 + 5.980528 - -922.7977 * it;
-    cpR8 = 2.92664 + 0.0014879768 * T + -5.68476e-07 * T2 + 1.0097038e-10 * T3 + -6.753351e-15 * T4;
-    hRT8 = 2.92664 + 0.0007439884 * T + -1.8949200000000001e-07 * T2 + 2.5242595e-11 * T3 + -1.3506701999999999e-15 * T4 + -922.7977 * it;
-  } else {
-    smh8 = 3.298677 * (lt - 1.0) + 0.0007041202 * T + -6.605369999999999e-07 * T2 + 4.701262500000001e-10 * T3 + -1.2224269999999999e-13 * T4 + 3.950372 - -1020.8999 * it;
-    cpR8 = 3.298677 + 0.0014082404 * T + -3.963222e-06 * T2 + 5.641515e-09 * T3 + -2.444854e-12 * T4;
-    hRT8 = 3.298677 + 0.0007041202 * T + -1.3210739999999999e-06 * T2 + 1.41037875e-09 * T3 + -4.889707999999999e-13 * T4 + -1020.8999 * it;
-  }
-  const double kf0 = 3547000000000000.0 * exp(-0.406 * lt - 8352.893466155027 * it);
+  const double e0 = d_exp(fmin(fmax(w0, -700.0), 700.0));
+  const double r0 = d_rcp(e0);
+  const double e2 = d_exp(fmin(fmax(w2, -700.0), 700.0));
+  const double r2 = d_rcp(e2);
+  const double e4 = d_exp(fmin(fmax(w4, -700.0), 700.0));
+  const double r4 = d_rcp(e4);
+  const double e5 = d_exp(fmin(fmax(w5, -700.0), 700.0));
+  const double r5 = d_rcp(e5);
+  const double e6 = d_exp(fmin(fmax(w6, -700.0), 700.0));
+  const double r6 = d_rcp(e6);
+  const double e7 = d_exp(fmin(fmax(w7, -700.0), 700.0));
+  const double r7 = d_rcp(e7);
+  // H+O2=O+OH
+  const double kf0 = 3547000000000000.0 * d_exp(-0.406 * lt + -8352.893466155027 * it);
   kt[0] = kf0;
-  const double eqk0 = exp(fmin(-1.0 * smh0 + -1.0 * smh3 + 1.0 * smh2 + 1.0 * smh4, 690.77552789821368)) * 1.0;
-  kt[1] = kf0 / fmax(eqk0, 1e-300);
-  const double kf1 = 50800.0 * exp(2.67 * lt - 3165.2328394550946 * it);
+  kt[1] = kf0 * r4 * r2 * e0;
+  // O+H2=H+OH
+  const double kf1 = 50800.0 * d_exp(2.67 * lt + -3165.2328394550946 * it);
   kt[2] = kf1;
-  const double eqk1 = exp(fmin(-1.0 * smh2 + -1.0 * smh1 + 1.0 * smh0 + 1.0 * smh4, 690.77552789821368)) * 1.0;
-  kt[3] = kf1 / fmax(eqk1, 1e-300);
-  const double kf2 = 216000000.0 * exp(1.51 * lt - 1726.0331700049244 * it);
+  kt[3] = kf1 * r4 * r0 * e2;
+  // H2+OH=H2O+H
+  const double kf2 = 216000000.0 * d_exp(1.51 * lt + -1726.0331700049244 * it);
   kt[4] = kf2;
-  const double eqk2 = exp(fmin(-1.0 * smh1 + -1.0 * smh4 + 1.0 * smh5 + 1.0 * smh0, 690.77552789821368)) * 1.0;
-  kt[5] = kf2 / fmax(eqk2, 1e-300);
-  const double kf3 = 2970000.0 * exp(2.02 * lt - 6743.103346374924 * it);
+  kt[5] = kf2 * e4 * r0 * r5;
+  // O+H2O=OH+OH
+  const double kf3 = 2970000.0 * d_exp(2.02 * lt + -6743.103346374924 * it);
   kt[6] = kf3;
-  const double eqk3 = exp(fmin(-1.0 * smh2 + -1.0 * smh5 + 2.0 * smh4, 690.77552789821368)) * 1.0;
-  kt[7] = kf3 / fmax(eqk3, 1e-300);
-  const double kf4 = 4.577e+19 * exp(-1.4 * lt - 52525.755768254814 * it);
+  kt[7] = kf3 * r4 * r4 * e2 * e5;
+  // H2+M=H+H+M
+  const double kf4 = 4.577e+19 * d_exp(-1.4 * lt + -52525.755768254814 * it);
   kt[8] = kf4;
-  const double eqk4 = exp(fmin(-1.0 * smh1 + 2.0 * smh0, 690.77552789821368)) * pfac;
-  kt[9] = kf4 / fmax(eqk4, 1e-300);
-  const double kf5 = 6165000000000000.0 * exp(-0.5 * lt - 0.0 * it);
+  kt[9] = kf4 * r0 * r0 * rtp;
+  // O+O+M=O2+M
+  const double kf5 = 6165000000000000.0 * sT * it;
   kt[10] = kf5;
-  const double eqk5 = exp(fmin(-2.0 * smh2 + 1.0 * smh3, 690.77552789821368)) * 1.0 / pfac;
-  kt[11] = kf5 / fmax(eqk5, 1e-300);
-  const double kf6 = 4.714e+18 * exp(-1.0 * lt - 0.0 * it);
+  kt[11] = kf5 * e2 * e2 * pfac;
+  // O+H+M=OH+M
+  const double kf6 = 4.714e+18 * it;
   kt[12] = kf6;
-  const double eqk6 = exp(fmin(-1.0 * smh2 + -1.0 * smh0 + 1.0 * smh4, 690.77552789821368)) * 1.0 / pfac;
-  kt[13] = kf6 / fmax(eqk6, 1e-300);
-  const double kf7 = 3.8e+22 * exp(-2.0 * lt - 0.0 * it);
+  kt[13] = kf6 * r4 * e0 * e2 * pfac;
+  // H+OH+M=H2O+M
+  const double kf7 = 3.8e+22 * it * it;
   kt[14] = kf7;
-  const double eqk7 = exp(fmin(-1.0 * smh0 + -1.0 * smh4 + 1.0 * smh5, 690.77552789821368)) * 1.0 / pfac;
-  kt[15] = kf7 / fmax(eqk7, 1e-300);
-  const double kf8 = 1475000000000.0 * exp(0.6 * lt - 0.0 * it);
+  kt[15] = kf7 * e4 * e0 * r5 * pfac;
+  // H+O2(+M)=HO2(+M)
+  const double kf8 = 1475000000000.0 * d_exp(0.6 * lt);
   kt[16] = kf8;
-  const double eqk8 = exp(fmin(-1.0 * smh0 + -1.0 * smh3 + 1.0 * smh6, 690.77552789821368)) * 1.0 / pfac;
-  kt[17] = kf8 / fmax(eqk8, 1e-300);
-  kt[18] = 6.366e+20 * exp(-1.72 * lt - 264.08810717742983 * it);
-  kt[19] = log10(fmax((1.0 - 0.8) * exp(-T / 1e-30) + 0.8 * exp(-T / 1e+30), 1e-300));
-  const double kf9 = 16600000000000.0 * exp(0.0 * lt - 414.1473174676539 * it);
-  kt[20] = kf9;
-  const double eqk9 = exp(fmin(-1.0 * smh6 + -1.0 * smh0 + 1.0 * smh1 + 1.0 * smh3, 690.77552789821368)) * 1.0;
-  kt[21] = kf9 / fmax(eqk9, 1e-300);
-  const double kf10 = 70790000000000.0 * exp(0.0 * lt - 148.44891695377632 * it);
-  kt[22] = kf10;
-  const double eqk10 = exp(fmin(-1.0 * smh6 + -1.0 * smh0 + 2.0 * smh4, 690.77552789821368)) * 1.0;
-  kt[23] = kf10 / fmax(eqk10, 1e-300);
-  const double kf11 = 32500000000000.0 * exp(0.0 * lt - 0.0 * it);
-  kt[24] = kf11;
-  const double eqk11 = exp(fmin(-1.0 * smh6 + -1.0 * smh2 + 1.0 * smh3 + 1.0 * smh4, 690.77552789821368)) * 1.0;
-  kt[25] = kf11 / fmax(eqk11, 1e-300);
-  const double kf12 = 28900000000000.0 * exp(0.0 * lt - -250.09868381704007 * it);
-  kt[26] = kf12;
-  const double eqk12 = exp(fmin(-1.0 * smh6 + -1.0 * smh4 + 1.0 * smh5 + 1.0 * smh3, 690.77552789821368)) * 1.0;
-  kt[27] = kf12 / fmax(eqk12, 1e-300);
-  const double kf13 = 420000000000000.0 * exp(0.0 * lt - 6029.542111661518 * it);
-  kt[28] = kf13;
-  const double eqk13 = exp(fmin(-2.0 * smh6 + 1.0 * smh7 + 1.0 * smh3, 690.77552789821368)) * 1.0;
-  kt[29] = kf13 / fmax(eqk13, 1e-300);
-  const double kf14 = 130000000000.0 * exp(0.0 * lt - -819.8909165857211 * it);
-  kt[30] = kf14;
-  const double eqk14 = exp(fmin(-2.0 * smh6 + 1.0 * smh7 + 1.0 * smh3, 690.77552789821368)) * 1.0;
-  kt[31] = kf14 / fmax(eqk14, 1e-300);
-  const double kf15 = 295100000000000.0 * exp(0.0 * lt - 24370.78321380131 * it);
-  kt[32] = kf15;
-  const double eqk15 = exp(fmin(-1.0 * smh7 + 2.0 * smh4, 690.77552789821368)) * pfac;
-  kt[33] = kf15 / fmax(eqk15, 1e-300);
-  kt[34] = 1.202e+17 * exp(0.0 * lt - 22896.358377616347 * it);
-  kt[35] = log10(fmax((1.0 - 0.5) * exp(-T / 1e-30) + 0.5 * exp(-T / 1e+30), 1e-300));
-  const double kf16 = 24100000000000.0 * exp(0.0 * lt - 1997.7701705304812 * it);
-  kt[36] = kf16;
-  const double eqk16 = exp(fmin(-1.0 * smh7 + -1.0 * smh0 + 1.0 * smh5 + 1.0 * smh4, 690.77552789821368)) * 1.0;
-  kt[37] = kf16 / fmax(eqk16, 1e-300);
-  const double kf17 = 48200000000000.0 * exp(0.0 * lt - 4000.5725077373613 * it);
-  kt[38] = kf17;
-  const double eqk17 = exp(fmin(-1.0 * smh7 + -1.0 * smh0 + 1.0 * smh6 + 1.0 * smh1, 690.77552789821368)) * 1.0;
-  kt[39] = kf17 / fmax(eqk17, 1e-300);
-  const double kf18 = 9550000.0 * exp(2.0 * lt - 1997.7701705304812 * it);
-  kt[40] = kf18;
-  const double eqk18 = exp(fmin(-1.0 * smh7 + -1.0 * smh2 + 1.0 * smh4 + 1.0 * smh6, 690.77552789821368)) * 1.0;
-  kt[41] = kf18 / fmax(eqk18, 1e-300);
-  const double kf19 = 1000000000000.0 * exp(0.0 * lt - 0.0 * it);
-  kt[42] = kf19;
-  const double eqk19 = exp(fmin(-1.0 * smh7 + -1.0 * smh4 + 1.0 * smh6 + 1.0 * smh5, 690.77552789821368)) * 1.0;
-  kt[43] = kf19 / fmax(eqk19, 1e-300);
-  const double kf20 = 580000000000000.0 * exp(0.0 * lt - 4809.241692634712 * it);
-  kt[44] = kf20;
-  const double eqk20 = exp(fmin(-1.0 * smh7 + -1.0 * smh4 + 1.0 * smh6 + 1.0 * smh5, 690.77552789821368)) * 1.0;
-  kt[45] = kf20 / fmax(eqk20, 1e-300);
-  (void)(smh0 + smh1 + smh2 + smh3 + smh4 + smh5 + smh6 + smh7 + smh8);
-  kt[46] = ru * (cpR0 - 1.0) / 1.0079699754714966;
-  kt[47] = ru * T * hRT0 / 1.0079699754714966;
-  kt[48] = ru * (cpR1 - 1.0) / 2.015939950942993;
-  kt[49] = ru * T * hRT1 / 2.015939950942993;
-  kt[50] = ru * (cpR2 - 1.0) / 15.99940013885498;
-  kt[51] = ru * T * hRT2 / 15.99940013885498;
-  kt[52] = ru * (cpR3 - 1.0) / 31.99880027770996;
-  kt[53] = ru * T * hRT3 / 31.99880027770996;
-  kt[54] = ru * (cpR4 - 1.0) / 17.007370114326477;
-  kt[55] = ru * T * hRT4 / 17.007370114326477;
-  kt[56] = ru * (cpR5 - 1.0) / 18.015340089797974;
-  kt[57] = ru * T * hRT5 / 18.015340089797974;
-  kt[58] = ru * (cpR6 - 1.0) / 33.00677025318146;
-  kt[59] = ru * T * hRT6 / 33.00677025318146;
-  kt[60] = ru * (cpR7 - 1.0) / 34.014740228652954;
-  kt[61] = ru * T * hRT7 / 34.014740228652954;
-  kt[62] = ru * (cpR8 - 1.0) / 28.013399124145508;
-  kt[63] = ru * T * hRT8 / 28.013399124145508;
+  kt[17] = kf8 * r6 * e0 * pfac;
+  kt[18] = 431593220.33898306 * d_exp(-2.32 * lt + -264.08810717742983 * it);
+  // HO2+H=H2+O2
+  const double ex0 = d_exp(-414.1473174676539 * it);
+  const double kf9 = 16600000000000.0 * ex0;
+  kt[19] = kf9;
+  kt[20] = kf9 * e6 * e0;
+  // HO2+H=OH+OH
+  const double ex1 = d_exp(-148.44891695377632 * it);
+  const double kf10 = 70790000000000.0 * ex1;
+  kt[21] = kf10;
+  kt[22] = kf10 * e6 * r4 * r4 * e0;
+  // HO2+O=O2+OH
+  kt[23] = 32500000000000.0 * e6 * r4 * e2;
+  // HO2+OH=H2O+O2
+  const double ex2 = d_exp(250.09868381704007 * it);
+  const double kf12 = 28900000000000.0 * ex2;
+  kt[24] = kf12;
+  kt[25] = kf12 * e6 * e4 * r5;
+  // HO2+HO2=H2O2+O2
+  const double ex3 = d_exp(-6029.542111661518 * it);
+  const double kp13 = 420000000000000.0 * ex3;
+  const double ex4 = d_exp(819.8909165857211 * it);
+  const double kp14 = 130000000000.0 * ex4;
+  const double kf13 = kp13 + kp14;
+  kt[26] = kf13;
+  kt[28] = (kp13 * (0.0 + 6029.542111661518 * it) + kp14 * (0.0 + -819.8909165857211 * it)) * it;
+  kt[27] = kf13 * e6 * e6 * r7;
+  // H2O2(+M)=OH+OH(+M)
+  const double ex5 = d_exp(-24370.78321380131 * it);
+  const double kf15 = 295100000000000.0 * ex5;
+  kt[29] = kf15;
+  kt[30] = kf15 * e7 * r4 * r4 * rtp;
+  const double ex6 = d_exp(1474.424836184964 * it);
+  kt[31] = 407.319552694002 * ex6;
+  // H2O2+H=H2O+OH
+  const double ex7 = d_exp(-1997.7701705304812 * it);
+  const double kf16 = 24100000000000.0 * ex7;
+  kt[32] = kf16;
+  kt[33] = kf16 * r4 * e7 * e0 * r5;
+  // H2O2+H=HO2+H2
+  const double ex8 = d_exp(-4000.5725077373613 * it);
+  const double kf17 = 48200000000000.0 * ex8;
+  kt[34] = kf17;
+  kt[35] = kf17 * r6 * e7 * e0;
+  // H2O2+O=OH+HO2
+  const double kf18 = 9550000.0 * T2 * ex7;
+  kt[36] = kf18;
+  kt[37] = kf18 * r6 * r4 * e7 * e2;
+  // H2O2+OH=HO2+H2O
+  const double kp19 = 1000000000000.0;
+  const double ex9 = d_exp(-4809.241692634712 * it);
+  const double kp20 = 580000000000000.0 * ex9;
+  const double kf19 = kp19 + kp20;
+  kt[38] = kf19;
+  kt[40] = (kp19 * (0.0 + 0.0 * it) + kp20 * (0.0 + 4809.241692634712 * it)) * it;
+  kt[39] = kf19 * r6 * e4 * e7 * r5;
 }
 
 IZ_HD inline void gen_rhs(double rho, const double *z, const double *kt, double *zp) {
-#pragma clang fp contract(off)
-  const double T = z[0], ru = 8.314510e7;
+#pragma clang fp contract(on)
   const double c0 = rho * z[1] * 0.9920930427835725;
   const double c1 = rho * z[2] * 0.49604652139178623;
   const double c2 = rho * z[3] * 0.06250234329545097;
@@ -226,6 +191,8 @@ IZ_HD inline void gen_rhs(double rho, const double *z, const double *kt, double 
   const double c7 = rho * z[8] * 0.029399019168684735;
   const double c8 = rho * z[9] * 0.035697203169395925;
   const double ctot = c0 + c1 + c2 + c3 + c4 + c5 + c6 + c7 + c8;
+  const double M0 = ctot + 1.5 * c1 + 11.0 * c5;
+  const double M1 = ctot + 1.0 * c1 - 0.21999999999999997 * c3 + 10.0 * c5;
   double wd0 = 0.0;
   double wd1 = 0.0;
   double wd2 = 0.0;
@@ -236,252 +203,168 @@ IZ_HD inline void gen_rhs(double rho, const double *z, const double *kt, double 
   double wd7 = 0.0;
   double wd8 = 0.0;
   { // H+O2=O+OH
-    double ctb = 1.0;
-    double kf = kt[0], kr = kt[1];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c0 * c3 - kr * c2 * c4;
+    const double q = kt[0] * c0 * c3 - kt[1] * c2 * c4;
     wd0 -= q;
     wd3 -= q;
     wd2 += q;
     wd4 += q;
   }
   { // O+H2=H+OH
-    double ctb = 1.0;
-    double kf = kt[2], kr = kt[3];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c2 * c1 - kr * c0 * c4;
+    const double q = kt[2] * c2 * c1 - kt[3] * c0 * c4;
     wd2 -= q;
     wd1 -= q;
     wd0 += q;
     wd4 += q;
   }
   { // H2+OH=H2O+H
-    double ctb = 1.0;
-    double kf = kt[4], kr = kt[5];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c1 * c4 - kr * c5 * c0;
+    const double q = kt[4] * c1 * c4 - kt[5] * c5 * c0;
     wd1 -= q;
     wd4 -= q;
     wd5 += q;
     wd0 += q;
   }
   { // O+H2O=OH+OH
-    double ctb = 1.0;
-    double kf = kt[6], kr = kt[7];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c2 * c5 - kr * c4 * c4;
+    const double q = kt[6] * c2 * c5 - kt[7] * c4 * c4;
     wd2 -= q;
     wd5 -= q;
     wd4 += 2.0 * q;
   }
   { // H2+M=H+H+M
-    double ctb = ctot + 1.5 * c1 + 11.0 * c5;
-    double kf = kt[8], kr = kt[9];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c1 - kr * c0 * c0;
+    const double q = M0 * (kt[8] * c1 - kt[9] * c0 * c0);
     wd1 -= q;
     wd0 += 2.0 * q;
   }
   { // O+O+M=O2+M
-    double ctb = ctot + 1.5 * c1 + 11.0 * c5;
-    double kf = kt[10], kr = kt[11];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c2 * c2 - kr * c3;
-    wd2 += -2.0 * q;
+    const double q = M0 * (kt[10] * c2 * c2 - kt[11] * c3);
+    wd2 -= 2.0 * q;
     wd3 += q;
   }
   { // O+H+M=OH+M
-    double ctb = ctot + 1.5 * c1 + 11.0 * c5;
-    double kf = kt[12], kr = kt[13];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c2 * c0 - kr * c4;
+    const double q = M0 * (kt[12] * c2 * c0 - kt[13] * c4);
     wd2 -= q;
     wd0 -= q;
     wd4 += q;
   }
   { // H+OH+M=H2O+M
-    double ctb = ctot + 1.5 * c1 + 11.0 * c5;
-    double kf = kt[14], kr = kt[15];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c0 * c4 - kr * c5;
+    const double q = M0 * (kt[14] * c0 * c4 - kt[15] * c5);
     wd0 -= q;
     wd4 -= q;
     wd5 += q;
   }
   { // H+O2(+M)=HO2(+M)
-    double ctb = ctot + 1.0 * c1 + 10.0 * c5 + -0.21999999999999997 * c3;
-    double kf = kt[16], kr = kt[17];
-    double pr = kt[18] * ctb / kf;
-    double pcor = pr / (1.0 + pr);
-    double fclog = kt[19];
-    double prlog = log10(fmax(pr, 1e-300));
-    double xn = 0.75 - 1.27 * fclog;
-    double cprlog = prlog - (0.4 + 0.67 * fclog);
-    double qq = cprlog / (xn - 0.14 * cprlog);
-    pcor *= exp((fclog / (1.0 + qq * qq)) * 2.302585092994046);
-    kf *= pcor; kr *= pcor; ctb = 1.0;
-    kf *= ctb; kr *= ctb;
-    double q = kf * c0 * c3 - kr * c6;
+    const double pr = kt[18] * M1;
+    const double lin1 = d_rcp(1.0 + pr);
+    const double prlog = 0.43429448190325182 * d_log(fmax(pr, 1e-300));
+    const double cpr = prlog - 0.33507029128460225;
+    const double xn = 0.8730757165202316;
+    const double den = xn - 0.14 * cpr, den2 = den * den;
+    const double g = den2 * d_rcp(den2 + cpr * cpr);
+    const double fcent = d_exp(-0.22314355131420974 * g);
+    const double pcor = pr * lin1 * fcent;
+    const double q = pcor * (kt[16] * c0 * c3 - kt[17] * c6);
     wd0 -= q;
     wd3 -= q;
     wd6 += q;
   }
   { // HO2+H=H2+O2
-    double ctb = 1.0;
-    double kf = kt[20], kr = kt[21];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c6 * c0 - kr * c1 * c3;
+    const double q = kt[19] * c6 * c0 - kt[20] * c1 * c3;
     wd6 -= q;
     wd0 -= q;
     wd1 += q;
     wd3 += q;
   }
   { // HO2+H=OH+OH
-    double ctb = 1.0;
-    double kf = kt[22], kr = kt[23];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c6 * c0 - kr * c4 * c4;
+    const double q = kt[21] * c6 * c0 - kt[22] * c4 * c4;
     wd6 -= q;
     wd0 -= q;
     wd4 += 2.0 * q;
   }
   { // HO2+O=O2+OH
-    double ctb = 1.0;
-    double kf = kt[24], kr = kt[25];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c6 * c2 - kr * c3 * c4;
+    const double q = 32500000000000.0 * c6 * c2 - kt[23] * c3 * c4;
     wd6 -= q;
     wd2 -= q;
     wd3 += q;
     wd4 += q;
   }
   { // HO2+OH=H2O+O2
-    double ctb = 1.0;
-    double kf = kt[26], kr = kt[27];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c6 * c4 - kr * c5 * c3;
+    const double q = kt[24] * c6 * c4 - kt[25] * c5 * c3;
     wd6 -= q;
     wd4 -= q;
     wd5 += q;
     wd3 += q;
   }
   { // HO2+HO2=H2O2+O2
-    double ctb = 1.0;
-    double kf = kt[28], kr = kt[29];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c6 * c6 - kr * c7 * c3;
-    wd6 += -2.0 * q;
-    wd7 += q;
-    wd3 += q;
-  }
-  { // HO2+HO2=H2O2+O2
-    double ctb = 1.0;
-    double kf = kt[30], kr = kt[31];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c6 * c6 - kr * c7 * c3;
-    wd6 += -2.0 * q;
+    const double q = kt[26] * c6 * c6 - kt[27] * c7 * c3;
+    wd6 -= 2.0 * q;
     wd7 += q;
     wd3 += q;
   }
   { // H2O2(+M)=OH+OH(+M)
-    double ctb = ctot + 1.5 * c1 + 11.0 * c5;
-    double kf = kt[32], kr = kt[33];
-    double pr = kt[34] * ctb / kf;
-    double pcor = pr / (1.0 + pr);
-    double fclog = kt[35];
-    double prlog = log10(fmax(pr, 1e-300));
-    double xn = 0.75 - 1.27 * fclog;
-    double cprlog = prlog - (0.4 + 0.67 * fclog);
-    double qq = cprlog / (xn - 0.14 * cprlog);
-    pcor *= exp((fclog / (1.0 + qq * qq)) * 2.302585092994046);
-    kf *= pcor; kr *= pcor; ctb = 1.0;
-    kf *= ctb; kr *= ctb;
-    double q = kf * c7 - kr * c4 * c4;
+    const double pr = kt[31] * M0;
+    const double lin1 = d_rcp(1.0 + pr);
+    const double prlog = 0.43429448190325182 * d_log(fmax(pr, 1e-300));
+    const double cpr = prlog - 0.19830990290513262;
+    const double xn = 1.1323080944932562;
+    const double den = xn - 0.14 * cpr, den2 = den * den;
+    const double g = den2 * d_rcp(den2 + cpr * cpr);
+    const double fcent = d_exp(-0.6931471805599454 * g);
+    const double pcor = pr * lin1 * fcent;
+    const double q = pcor * (kt[29] * c7 - kt[30] * c4 * c4);
     wd7 -= q;
     wd4 += 2.0 * q;
   }
   { // H2O2+H=H2O+OH
-    double ctb = 1.0;
-    double kf = kt[36], kr = kt[37];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c7 * c0 - kr * c5 * c4;
+    const double q = kt[32] * c7 * c0 - kt[33] * c5 * c4;
     wd7 -= q;
     wd0 -= q;
     wd5 += q;
     wd4 += q;
   }
   { // H2O2+H=HO2+H2
-    double ctb = 1.0;
-    double kf = kt[38], kr = kt[39];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c7 * c0 - kr * c6 * c1;
+    const double q = kt[34] * c7 * c0 - kt[35] * c6 * c1;
     wd7 -= q;
     wd0 -= q;
     wd6 += q;
     wd1 += q;
   }
   { // H2O2+O=OH+HO2
-    double ctb = 1.0;
-    double kf = kt[40], kr = kt[41];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c7 * c2 - kr * c4 * c6;
+    const double q = kt[36] * c7 * c2 - kt[37] * c4 * c6;
     wd7 -= q;
     wd2 -= q;
     wd4 += q;
     wd6 += q;
   }
   { // H2O2+OH=HO2+H2O
-    double ctb = 1.0;
-    double kf = kt[42], kr = kt[43];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c7 * c4 - kr * c6 * c5;
+    const double q = kt[38] * c7 * c4 - kt[39] * c6 * c5;
     wd7 -= q;
     wd4 -= q;
     wd6 += q;
     wd5 += q;
   }
-  { // H2O2+OH=HO2+H2O
-    double ctb = 1.0;
-    double kf = kt[44], kr = kt[45];
-    kf *= ctb; kr *= ctb;
-    double q = kf * c7 * c4 - kr * c6 * c5;
-    wd7 -= q;
-    wd4 -= q;
-    wd6 += q;
-    wd5 += q;
-  }
-  double cvb = z[1] * kt[46] + z[2] * kt[48] + z[3] * kt[50] + z[4] * kt[52] + z[5] * kt[54] + z[6] * kt[56] + z[7] * kt[58] + z[8] * kt[60] + z[9] * kt[62];
-  const double rho_i = 1.0 / rho;
-  double sum = 0.0;
-  zp[1] = wd0 * 1.0079699754714966 * rho_i;
-  sum += kt[47] * wd0 * 1.0079699754714966 - ru * T * wd0;
-  zp[2] = wd1 * 2.015939950942993 * rho_i;
-  sum += kt[49] * wd1 * 2.015939950942993 - ru * T * wd1;
-  zp[3] = wd2 * 15.99940013885498 * rho_i;
-  sum += kt[51] * wd2 * 15.99940013885498 - ru * T * wd2;
-  zp[4] = wd3 * 31.99880027770996 * rho_i;
-  sum += kt[53] * wd3 * 31.99880027770996 - ru * T * wd3;
-  zp[5] = wd4 * 17.007370114326477 * rho_i;
-  sum += kt[55] * wd4 * 17.007370114326477 - ru * T * wd4;
-  zp[6] = wd5 * 18.015340089797974 * rho_i;
-  sum += kt[57] * wd5 * 18.015340089797974 - ru * T * wd5;
-  zp[7] = wd6 * 33.00677025318146 * rho_i;
-  sum += kt[59] * wd6 * 33.00677025318146 - ru * T * wd6;
-  zp[8] = wd7 * 34.014740228652954 * rho_i;
-  sum += kt[61] * wd7 * 34.014740228652954 - ru * T * wd7;
-  zp[9] = wd8 * 28.013399124145508 * rho_i;
-  sum += kt[63] * wd8 * 28.013399124145508 - ru * T * wd8;
-  zp[0] = -sum / (rho * cvb);
+  const double cvb = z[1] * kt[41] + z[2] * kt[43] + z[3] * kt[45] + z[4] * kt[47] + z[5] * kt[49] + z[6] * kt[51] + z[7] * kt[53] + z[8] * kt[55] + z[9] * kt[57];
+  const double rho_i = d_rcp(rho);
+  zp[1] = wd0 * (1.0079699754714966 * rho_i);
+  zp[2] = wd1 * (2.015939950942993 * rho_i);
+  zp[3] = wd2 * (15.99940013885498 * rho_i);
+  zp[4] = wd3 * (31.99880027770996 * rho_i);
+  zp[5] = wd4 * (17.007370114326477 * rho_i);
+  zp[6] = wd5 * (18.015340089797974 * rho_i);
+  zp[7] = wd6 * (33.00677025318146 * rho_i);
+  zp[8] = wd7 * (34.014740228652954 * rho_i);
+  zp[9] = wd8 * (28.013399124145508 * rho_i);
+  const double sum = kt[42] * wd0 + kt[44] * wd1 + kt[46] * wd2 + kt[48] * wd3 + kt[50] * wd4 + kt[52] * wd5 + kt[54] * wd6 + kt[56] * wd7;
+  zp[0] = -sum * d_rcp(rho * cvb);
 }
 
-// d zp / d z[1 + j] for j = 0 .. GEN_KK - 1 (columns 1 .. GEN_KK of J;
-// column 0, d/dT, is left to the caller) at the state z whose
-// temperature part is kt and whose dT/dt is f0T: the analytic form of
-// the mass-fraction columns of a finite-difference Jacobian.
+// The reactor Jacobian d zp / d z in closed form (mass action, third-body
+// sums, falloff factors, Arrhenius and equilibrium slopes) at the state z
+// whose temperature part is kt: both functions together cost about as
+// much as one right-hand side, where finite differences take GEN_KK + 1 of
+// them and the temperature part again.  gen_jac: columns 1 .. GEN_KK,
+// given f0T = dT/dt; column 0 is left alone.
 IZ_HD inline void gen_jac(double rho, const double *z, const double *kt, double f0T,
                           double (*J)[GEN_KK + 1]) {
-#pragma clang fp contract(off)
-  const double T = z[0], ru = 8.314510e7;
+#pragma clang fp contract(on)
   const double c0 = rho * z[1] * 0.9920930427835725;
   const double c1 = rho * z[2] * 0.49604652139178623;
   const double c2 = rho * z[3] * 0.06250234329545097;
@@ -492,742 +375,466 @@ IZ_HD inline void gen_jac(double rho, const double *z, const double *kt, double 
   const double c7 = rho * z[8] * 0.029399019168684735;
   const double c8 = rho * z[9] * 0.035697203169395925;
   const double ctot = c0 + c1 + c2 + c3 + c4 + c5 + c6 + c7 + c8;
-  double jy0_0 = 0.0, jy0_1 = 0.0, jy0_2 = 0.0, jy0_3 = 0.0, jy0_4 = 0.0, jy0_5 = 0.0, jy0_6 = 0.0, jy0_7 = 0.0, jy0_8 = 0.0;
-  double jy1_0 = 0.0, jy1_1 = 0.0, jy1_2 = 0.0, jy1_3 = 0.0, jy1_4 = 0.0, jy1_5 = 0.0, jy1_6 = 0.0, jy1_7 = 0.0, jy1_8 = 0.0;
-  double jy2_0 = 0.0, jy2_1 = 0.0, jy2_2 = 0.0, jy2_3 = 0.0, jy2_4 = 0.0, jy2_5 = 0.0, jy2_6 = 0.0, jy2_7 = 0.0, jy2_8 = 0.0;
-  double jy3_0 = 0.0, jy3_1 = 0.0, jy3_2 = 0.0, jy3_3 = 0.0, jy3_4 = 0.0, jy3_5 = 0.0, jy3_6 = 0.0, jy3_7 = 0.0, jy3_8 = 0.0;
-  double jy4_0 = 0.0, jy4_1 = 0.0, jy4_2 = 0.0, jy4_3 = 0.0, jy4_4 = 0.0, jy4_5 = 0.0, jy4_6 = 0.0, jy4_7 = 0.0, jy4_8 = 0.0;
-  double jy5_0 = 0.0, jy5_1 = 0.0, jy5_2 = 0.0, jy5_3 = 0.0, jy5_4 = 0.0, jy5_5 = 0.0, jy5_6 = 0.0, jy5_7 = 0.0, jy5_8 = 0.0;
-  double jy6_0 = 0.0, jy6_1 = 0.0, jy6_2 = 0.0, jy6_3 = 0.0, jy6_4 = 0.0, jy6_5 = 0.0, jy6_6 = 0.0, jy6_7 = 0.0, jy6_8 = 0.0;
-  double jy7_0 = 0.0, jy7_1 = 0.0, jy7_2 = 0.0, jy7_3 = 0.0, jy7_4 = 0.0, jy7_5 = 0.0, jy7_6 = 0.0, jy7_7 = 0.0, jy7_8 = 0.0;
-  double jy8_0 = 0.0, jy8_1 = 0.0, jy8_2 = 0.0, jy8_3 = 0.0, jy8_4 = 0.0, jy8_5 = 0.0, jy8_6 = 0.0, jy8_7 = 0.0, jy8_8 = 0.0;
-  { // H+O2=O+OH
-    double ctb = 1.0;
-    double kf = kt[0], kr = kt[1];
-    const double dq0 = kf * (c3);
-    const double dq2 = -kr * (c4);
-    const double dq3 = kf * (c0);
-    const double dq4 = -kr * (c2);
-    jy0_0 -= dq0;
-    jy0_2 -= dq2;
-    jy0_3 -= dq3;
-    jy0_4 -= dq4;
-    jy3_0 -= dq0;
-    jy3_2 -= dq2;
-    jy3_3 -= dq3;
-    jy3_4 -= dq4;
-    jy2_0 += dq0;
-    jy2_2 += dq2;
-    jy2_3 += dq3;
-    jy2_4 += dq4;
-    jy4_0 += dq0;
-    jy4_2 += dq2;
-    jy4_3 += dq3;
-    jy4_4 += dq4;
+  const double M0 = ctot + 1.5 * c1 + 11.0 * c5;
+  const double M1 = ctot + 1.0 * c1 - 0.21999999999999997 * c3 + 10.0 * c5;
+  // H+O2=O+OH
+  // O+H2=H+OH
+  // H2+OH=H2O+H
+  // O+H2O=OH+OH
+  // H2+M=H+H+M
+  const double qm4 = kt[8] * c1 - kt[9] * c0 * c0;
+  // O+O+M=O2+M
+  const double qm5 = kt[10] * c2 * c2 - kt[11] * c3;
+  // O+H+M=OH+M
+  const double qm6 = kt[12] * c2 * c0 - kt[13] * c4;
+  // H+OH+M=H2O+M
+  const double qm7 = kt[14] * c0 * c4 - kt[15] * c5;
+  // H+O2(+M)=HO2(+M)
+  double sc8, dp8;
+  {
+    const double pr = kt[18] * M1;
+    const double lin1 = d_rcp(1.0 + pr);
+    const double prlog = 0.43429448190325182 * d_log(fmax(pr, 1e-300));
+    const double cpr = prlog - 0.33507029128460225;
+    const double xn = 0.8730757165202316;
+    const double den = xn - 0.14 * cpr, den2 = den * den;
+    const double g = den2 * d_rcp(den2 + cpr * cpr);
+    const double fcent = d_exp(-0.22314355131420974 * g);
+    const double dfdpr = (pr > 1e-300) ? -2.0 * fcent * -0.22314355131420974 * 0.43429448190325182 * cpr * xn * g * g / (den2 * den * pr) : 0.0;
+    const double pcor = pr * lin1 * fcent;
+    const double dpcor = fcent * lin1 * lin1 + pr * lin1 * dfdpr;
+    sc8 = pcor;
+    dp8 = dpcor * kt[18];
   }
-  { // O+H2=H+OH
-    double ctb = 1.0;
-    double kf = kt[2], kr = kt[3];
-    const double dq0 = -kr * (c4);
-    const double dq1 = kf * (c2);
-    const double dq2 = kf * (c1);
-    const double dq4 = -kr * (c0);
-    jy2_0 -= dq0;
-    jy2_1 -= dq1;
-    jy2_2 -= dq2;
-    jy2_4 -= dq4;
-    jy1_0 -= dq0;
-    jy1_1 -= dq1;
-    jy1_2 -= dq2;
-    jy1_4 -= dq4;
-    jy0_0 += dq0;
-    jy0_1 += dq1;
-    jy0_2 += dq2;
-    jy0_4 += dq4;
-    jy4_0 += dq0;
-    jy4_1 += dq1;
-    jy4_2 += dq2;
-    jy4_4 += dq4;
+  const double qm8 = (kt[16] * c0 * c3 - kt[17] * c6) * dp8;
+  // HO2+H=H2+O2
+  // HO2+H=OH+OH
+  // HO2+O=O2+OH
+  // HO2+OH=H2O+O2
+  // HO2+HO2=H2O2+O2
+  // H2O2(+M)=OH+OH(+M)
+  double sc15, dp15;
+  {
+    const double pr = kt[31] * M0;
+    const double lin1 = d_rcp(1.0 + pr);
+    const double prlog = 0.43429448190325182 * d_log(fmax(pr, 1e-300));
+    const double cpr = prlog - 0.19830990290513262;
+    const double xn = 1.1323080944932562;
+    const double den = xn - 0.14 * cpr, den2 = den * den;
+    const double g = den2 * d_rcp(den2 + cpr * cpr);
+    const double fcent = d_exp(-0.6931471805599454 * g);
+    const double dfdpr = (pr > 1e-300) ? -2.0 * fcent * -0.6931471805599454 * 0.43429448190325182 * cpr * xn * g * g / (den2 * den * pr) : 0.0;
+    const double pcor = pr * lin1 * fcent;
+    const double dpcor = fcent * lin1 * lin1 + pr * lin1 * dfdpr;
+    sc15 = pcor;
+    dp15 = dpcor * kt[31];
   }
-  { // H2+OH=H2O+H
-    double ctb = 1.0;
-    double kf = kt[4], kr = kt[5];
-    const double dq0 = -kr * (c5);
-    const double dq1 = kf * (c4);
-    const double dq4 = kf * (c1);
-    const double dq5 = -kr * (c0);
-    jy1_0 -= dq0;
-    jy1_1 -= dq1;
-    jy1_4 -= dq4;
-    jy1_5 -= dq5;
-    jy4_0 -= dq0;
-    jy4_1 -= dq1;
-    jy4_4 -= dq4;
-    jy4_5 -= dq5;
-    jy5_0 += dq0;
-    jy5_1 += dq1;
-    jy5_4 += dq4;
-    jy5_5 += dq5;
-    jy0_0 += dq0;
-    jy0_1 += dq1;
-    jy0_4 += dq4;
-    jy0_5 += dq5;
-  }
-  { // O+H2O=OH+OH
-    double ctb = 1.0;
-    double kf = kt[6], kr = kt[7];
-    const double dq2 = kf * (c5);
-    const double dq4 = -kr * (2.0 * c4);
-    const double dq5 = kf * (c2);
-    jy2_2 -= dq2;
-    jy2_4 -= dq4;
-    jy2_5 -= dq5;
-    jy5_2 -= dq2;
-    jy5_4 -= dq4;
-    jy5_5 -= dq5;
-    jy4_2 += 2.0 * dq2;
-    jy4_4 += 2.0 * dq4;
-    jy4_5 += 2.0 * dq5;
-  }
-  { // H2+M=H+H+M
-    double ctb = ctot + 1.5 * c1 + 11.0 * c5;
-    double kf = kt[8], kr = kt[9];
-    const double kf0 = kf, kr0 = kr;
-    kf *= ctb; kr *= ctb;
-    const double q0 = kf0 * c1 - kr0 * c0 * c0;
-    const double dq0 = -kr * (2.0 * c0) + q0 * 1.0;
-    const double dq1 = kf * (1.0) + q0 * 2.5;
-    const double dq2 = q0 * 1.0;
-    const double dq3 = q0 * 1.0;
-    const double dq4 = q0 * 1.0;
-    const double dq5 = q0 * 12.0;
-    const double dq6 = q0 * 1.0;
-    const double dq7 = q0 * 1.0;
-    const double dq8 = q0 * 1.0;
-    jy1_0 -= dq0;
-    jy1_1 -= dq1;
-    jy1_2 -= dq2;
-    jy1_3 -= dq3;
-    jy1_4 -= dq4;
-    jy1_5 -= dq5;
-    jy1_6 -= dq6;
-    jy1_7 -= dq7;
-    jy1_8 -= dq8;
-    jy0_0 += 2.0 * dq0;
-    jy0_1 += 2.0 * dq1;
-    jy0_2 += 2.0 * dq2;
-    jy0_3 += 2.0 * dq3;
-    jy0_4 += 2.0 * dq4;
-    jy0_5 += 2.0 * dq5;
-    jy0_6 += 2.0 * dq6;
-    jy0_7 += 2.0 * dq7;
-    jy0_8 += 2.0 * dq8;
-  }
-  { // O+O+M=O2+M
-    double ctb = ctot + 1.5 * c1 + 11.0 * c5;
-    double kf = kt[10], kr = kt[11];
-    const double kf0 = kf, kr0 = kr;
-    kf *= ctb; kr *= ctb;
-    const double q0 = kf0 * c2 * c2 - kr0 * c3;
-    const double dq0 = q0 * 1.0;
-    const double dq1 = q0 * 2.5;
-    const double dq2 = kf * (2.0 * c2) + q0 * 1.0;
-    const double dq3 = -kr * (1.0) + q0 * 1.0;
-    const double dq4 = q0 * 1.0;
-    const double dq5 = q0 * 12.0;
-    const double dq6 = q0 * 1.0;
-    const double dq7 = q0 * 1.0;
-    const double dq8 = q0 * 1.0;
-    jy2_0 += -2.0 * dq0;
-    jy2_1 += -2.0 * dq1;
-    jy2_2 += -2.0 * dq2;
-    jy2_3 += -2.0 * dq3;
-    jy2_4 += -2.0 * dq4;
-    jy2_5 += -2.0 * dq5;
-    jy2_6 += -2.0 * dq6;
-    jy2_7 += -2.0 * dq7;
-    jy2_8 += -2.0 * dq8;
-    jy3_0 += dq0;
-    jy3_1 += dq1;
-    jy3_2 += dq2;
-    jy3_3 += dq3;
-    jy3_4 += dq4;
-    jy3_5 += dq5;
-    jy3_6 += dq6;
-    jy3_7 += dq7;
-    jy3_8 += dq8;
-  }
-  { // O+H+M=OH+M
-    double ctb = ctot + 1.5 * c1 + 11.0 * c5;
-    double kf = kt[12], kr = kt[13];
-    const double kf0 = kf, kr0 = kr;
-    kf *= ctb; kr *= ctb;
-    const double q0 = kf0 * c2 * c0 - kr0 * c4;
-    const double dq0 = kf * (c2) + q0 * 1.0;
-    const double dq1 = q0 * 2.5;
-    const double dq2 = kf * (c0) + q0 * 1.0;
-    const double dq3 = q0 * 1.0;
-    const double dq4 = -kr * (1.0) + q0 * 1.0;
-    const double dq5 = q0 * 12.0;
-    const double dq6 = q0 * 1.0;
-    const double dq7 = q0 * 1.0;
-    const double dq8 = q0 * 1.0;
-    jy2_0 -= dq0;
-    jy2_1 -= dq1;
-    jy2_2 -= dq2;
-    jy2_3 -= dq3;
-    jy2_4 -= dq4;
-    jy2_5 -= dq5;
-    jy2_6 -= dq6;
-    jy2_7 -= dq7;
-    jy2_8 -= dq8;
-    jy0_0 -= dq0;
-    jy0_1 -= dq1;
-    jy0_2 -= dq2;
-    jy0_3 -= dq3;
-    jy0_4 -= dq4;
-    jy0_5 -= dq5;
-    jy0_6 -= dq6;
-    jy0_7 -= dq7;
-    jy0_8 -= dq8;
-    jy4_0 += dq0;
-    jy4_1 += dq1;
-    jy4_2 += dq2;
-    jy4_3 += dq3;
-    jy4_4 += dq4;
-    jy4_5 += dq5;
-    jy4_6 += dq6;
-    jy4_7 += dq7;
-    jy4_8 += dq8;
-  }
-  { // H+OH+M=H2O+M
-    double ctb = ctot + 1.5 * c1 + 11.0 * c5;
-    double kf = kt[14], kr = kt[15];
-    const double kf0 = kf, kr0 = kr;
-    kf *= ctb; kr *= ctb;
-    const double q0 = kf0 * c0 * c4 - kr0 * c5;
-    const double dq0 = kf * (c4) + q0 * 1.0;
-    const double dq1 = q0 * 2.5;
-    const double dq2 = q0 * 1.0;
-    const double dq3 = q0 * 1.0;
-    const double dq4 = kf * (c0) + q0 * 1.0;
-    const double dq5 = -kr * (1.0) + q0 * 12.0;
-    const double dq6 = q0 * 1.0;
-    const double dq7 = q0 * 1.0;
-    const double dq8 = q0 * 1.0;
-    jy0_0 -= dq0;
-    jy0_1 -= dq1;
-    jy0_2 -= dq2;
-    jy0_3 -= dq3;
-    jy0_4 -= dq4;
-    jy0_5 -= dq5;
-    jy0_6 -= dq6;
-    jy0_7 -= dq7;
-    jy0_8 -= dq8;
-    jy4_0 -= dq0;
-    jy4_1 -= dq1;
-    jy4_2 -= dq2;
-    jy4_3 -= dq3;
-    jy4_4 -= dq4;
-    jy4_5 -= dq5;
-    jy4_6 -= dq6;
-    jy4_7 -= dq7;
-    jy4_8 -= dq8;
-    jy5_0 += dq0;
-    jy5_1 += dq1;
-    jy5_2 += dq2;
-    jy5_3 += dq3;
-    jy5_4 += dq4;
-    jy5_5 += dq5;
-    jy5_6 += dq6;
-    jy5_7 += dq7;
-    jy5_8 += dq8;
-  }
-  { // H+O2(+M)=HO2(+M)
-    double ctb = ctot + 1.0 * c1 + 10.0 * c5 + -0.21999999999999997 * c3;
-    double kf = kt[16], kr = kt[17];
-    const double cm = ctb;
-    const double klo = kt[18];
-    const double pr = klo * cm / kf;
-    const double lin = pr / (1.0 + pr);
-    double fcent = 1.0, dfdpr = 0.0;
-    const double fclog = kt[19];
-    const double prlog = log10(fmax(pr, 1e-300));
-    const double xn = 0.75 - 1.27 * fclog;
-    const double cprlog = prlog - (0.4 + 0.67 * fclog);
-    const double den = xn - 0.14 * cprlog;
-    const double qq = cprlog / den;
-    const double g = 1.0 / (1.0 + qq * qq);
-    fcent = exp((fclog * g) * 2.302585092994046);
-    if (pr > 1e-300) dfdpr = -2.0 * fcent * fclog * qq * xn * g * g / (den * den * pr);
-    const double dpcor = fcent / ((1.0 + pr) * (1.0 + pr)) + lin * dfdpr;
-    const double kinf = kf, krinf = kr;
-    kf *= lin * fcent; kr *= lin * fcent;
-    const double qinf = kinf * c0 * c3 - krinf * c6;
-    const double dqdm = qinf * dpcor * klo / kinf;
-    const double dq0 = kf * (c3) + dqdm * 1.0;
-    const double dq1 = dqdm * 2.0;
-    const double dq2 = dqdm * 1.0;
-    const double dq3 = kf * (c0) + dqdm * 0.78;
-    const double dq4 = dqdm * 1.0;
-    const double dq5 = dqdm * 11.0;
-    const double dq6 = -kr * (1.0) + dqdm * 1.0;
-    const double dq7 = dqdm * 1.0;
-    const double dq8 = dqdm * 1.0;
-    jy0_0 -= dq0;
-    jy0_1 -= dq1;
-    jy0_2 -= dq2;
-    jy0_3 -= dq3;
-    jy0_4 -= dq4;
-    jy0_5 -= dq5;
-    jy0_6 -= dq6;
-    jy0_7 -= dq7;
-    jy0_8 -= dq8;
-    jy3_0 -= dq0;
-    jy3_1 -= dq1;
-    jy3_2 -= dq2;
-    jy3_3 -= dq3;
-    jy3_4 -= dq4;
-    jy3_5 -= dq5;
-    jy3_6 -= dq6;
-    jy3_7 -= dq7;
-    jy3_8 -= dq8;
-    jy6_0 += dq0;
-    jy6_1 += dq1;
-    jy6_2 += dq2;
-    jy6_3 += dq3;
-    jy6_4 += dq4;
-    jy6_5 += dq5;
-    jy6_6 += dq6;
-    jy6_7 += dq7;
-    jy6_8 += dq8;
-  }
-  { // HO2+H=H2+O2
-    double ctb = 1.0;
-    double kf = kt[20], kr = kt[21];
-    const double dq0 = kf * (c6);
-    const double dq1 = -kr * (c3);
-    const double dq3 = -kr * (c1);
-    const double dq6 = kf * (c0);
-    jy6_0 -= dq0;
-    jy6_1 -= dq1;
-    jy6_3 -= dq3;
-    jy6_6 -= dq6;
-    jy0_0 -= dq0;
-    jy0_1 -= dq1;
-    jy0_3 -= dq3;
-    jy0_6 -= dq6;
-    jy1_0 += dq0;
-    jy1_1 += dq1;
-    jy1_3 += dq3;
-    jy1_6 += dq6;
-    jy3_0 += dq0;
-    jy3_1 += dq1;
-    jy3_3 += dq3;
-    jy3_6 += dq6;
-  }
-  { // HO2+H=OH+OH
-    double ctb = 1.0;
-    double kf = kt[22], kr = kt[23];
-    const double dq0 = kf * (c6);
-    const double dq4 = -kr * (2.0 * c4);
-    const double dq6 = kf * (c0);
-    jy6_0 -= dq0;
-    jy6_4 -= dq4;
-    jy6_6 -= dq6;
-    jy0_0 -= dq0;
-    jy0_4 -= dq4;
-    jy0_6 -= dq6;
-    jy4_0 += 2.0 * dq0;
-    jy4_4 += 2.0 * dq4;
-    jy4_6 += 2.0 * dq6;
-  }
-  { // HO2+O=O2+OH
-    double ctb = 1.0;
-    double kf = kt[24], kr = kt[25];
-    const double dq2 = kf * (c6);
-    const double dq3 = -kr * (c4);
-    const double dq4 = -kr * (c3);
-    const double dq6 = kf * (c2);
-    jy6_2 -= dq2;
-    jy6_3 -= dq3;
-    jy6_4 -= dq4;
-    jy6_6 -= dq6;
-    jy2_2 -= dq2;
-    jy2_3 -= dq3;
-    jy2_4 -= dq4;
-    jy2_6 -= dq6;
-    jy3_2 += dq2;
-    jy3_3 += dq3;
-    jy3_4 += dq4;
-    jy3_6 += dq6;
-    jy4_2 += dq2;
-    jy4_3 += dq3;
-    jy4_4 += dq4;
-    jy4_6 += dq6;
-  }
-  { // HO2+OH=H2O+O2
-    double ctb = 1.0;
-    double kf = kt[26], kr = kt[27];
-    const double dq3 = -kr * (c5);
-    const double dq4 = kf * (c6);
-    const double dq5 = -kr * (c3);
-    const double dq6 = kf * (c4);
-    jy6_3 -= dq3;
-    jy6_4 -= dq4;
-    jy6_5 -= dq5;
-    jy6_6 -= dq6;
-    jy4_3 -= dq3;
-    jy4_4 -= dq4;
-    jy4_5 -= dq5;
-    jy4_6 -= dq6;
-    jy5_3 += dq3;
-    jy5_4 += dq4;
-    jy5_5 += dq5;
-    jy5_6 += dq6;
-    jy3_3 += dq3;
-    jy3_4 += dq4;
-    jy3_5 += dq5;
-    jy3_6 += dq6;
-  }
-  { // HO2+HO2=H2O2+O2
-    double ctb = 1.0;
-    double kf = kt[28], kr = kt[29];
-    const double dq3 = -kr * (c7);
-    const double dq6 = kf * (2.0 * c6);
-    const double dq7 = -kr * (c3);
-    jy6_3 += -2.0 * dq3;
-    jy6_6 += -2.0 * dq6;
-    jy6_7 += -2.0 * dq7;
-    jy7_3 += dq3;
-    jy7_6 += dq6;
-    jy7_7 += dq7;
-    jy3_3 += dq3;
-    jy3_6 += dq6;
-    jy3_7 += dq7;
-  }
-  { // HO2+HO2=H2O2+O2
-    double ctb = 1.0;
-    double kf = kt[30], kr = kt[31];
-    const double dq3 = -kr * (c7);
-    const double dq6 = kf * (2.0 * c6);
-    const double dq7 = -kr * (c3);
-    jy6_3 += -2.0 * dq3;
-    jy6_6 += -2.0 * dq6;
-    jy6_7 += -2.0 * dq7;
-    jy7_3 += dq3;
-    jy7_6 += dq6;
-    jy7_7 += dq7;
-    jy3_3 += dq3;
-    jy3_6 += dq6;
-    jy3_7 += dq7;
-  }
-  { // H2O2(+M)=OH+OH(+M)
-    double ctb = ctot + 1.5 * c1 + 11.0 * c5;
-    double kf = kt[32], kr = kt[33];
-    const double cm = ctb;
-    const double klo = kt[34];
-    const double pr = klo * cm / kf;
-    const double lin = pr / (1.0 + pr);
-    double fcent = 1.0, dfdpr = 0.0;
-    const double fclog = kt[35];
-    const double prlog = log10(fmax(pr, 1e-300));
-    const double xn = 0.75 - 1.27 * fclog;
-    const double cprlog = prlog - (0.4 + 0.67 * fclog);
-    const double den = xn - 0.14 * cprlog;
-    const double qq = cprlog / den;
-    const double g = 1.0 / (1.0 + qq * qq);
-    fcent = exp((fclog * g) * 2.302585092994046);
-    if (pr > 1e-300) dfdpr = -2.0 * fcent * fclog * qq * xn * g * g / (den * den * pr);
-    const double dpcor = fcent / ((1.0 + pr) * (1.0 + pr)) + lin * dfdpr;
-    const double kinf = kf, krinf = kr;
-    kf *= lin * fcent; kr *= lin * fcent;
-    const double qinf = kinf * c7 - krinf * c4 * c4;
-    const double dqdm = qinf * dpcor * klo / kinf;
-    const double dq0 = dqdm * 1.0;
-    const double dq1 = dqdm * 2.5;
-    const double dq2 = dqdm * 1.0;
-    const double dq3 = dqdm * 1.0;
-    const double dq4 = -kr * (2.0 * c4) + dqdm * 1.0;
-    const double dq5 = dqdm * 12.0;
-    const double dq6 = dqdm * 1.0;
-    const double dq7 = kf * (1.0) + dqdm * 1.0;
-    const double dq8 = dqdm * 1.0;
-    jy7_0 -= dq0;
-    jy7_1 -= dq1;
-    jy7_2 -= dq2;
-    jy7_3 -= dq3;
-    jy7_4 -= dq4;
-    jy7_5 -= dq5;
-    jy7_6 -= dq6;
-    jy7_7 -= dq7;
-    jy7_8 -= dq8;
-    jy4_0 += 2.0 * dq0;
-    jy4_1 += 2.0 * dq1;
-    jy4_2 += 2.0 * dq2;
-    jy4_3 += 2.0 * dq3;
-    jy4_4 += 2.0 * dq4;
-    jy4_5 += 2.0 * dq5;
-    jy4_6 += 2.0 * dq6;
-    jy4_7 += 2.0 * dq7;
-    jy4_8 += 2.0 * dq8;
-  }
-  { // H2O2+H=H2O+OH
-    double ctb = 1.0;
-    double kf = kt[36], kr = kt[37];
-    const double dq0 = kf * (c7);
-    const double dq4 = -kr * (c5);
-    const double dq5 = -kr * (c4);
-    const double dq7 = kf * (c0);
-    jy7_0 -= dq0;
-    jy7_4 -= dq4;
-    jy7_5 -= dq5;
-    jy7_7 -= dq7;
-    jy0_0 -= dq0;
-    jy0_4 -= dq4;
-    jy0_5 -= dq5;
-    jy0_7 -= dq7;
-    jy5_0 += dq0;
-    jy5_4 += dq4;
-    jy5_5 += dq5;
-    jy5_7 += dq7;
-    jy4_0 += dq0;
-    jy4_4 += dq4;
-    jy4_5 += dq5;
-    jy4_7 += dq7;
-  }
-  { // H2O2+H=HO2+H2
-    double ctb = 1.0;
-    double kf = kt[38], kr = kt[39];
-    const double dq0 = kf * (c7);
-    const double dq1 = -kr * (c6);
-    const double dq6 = -kr * (c1);
-    const double dq7 = kf * (c0);
-    jy7_0 -= dq0;
-    jy7_1 -= dq1;
-    jy7_6 -= dq6;
-    jy7_7 -= dq7;
-    jy0_0 -= dq0;
-    jy0_1 -= dq1;
-    jy0_6 -= dq6;
-    jy0_7 -= dq7;
-    jy6_0 += dq0;
-    jy6_1 += dq1;
-    jy6_6 += dq6;
-    jy6_7 += dq7;
-    jy1_0 += dq0;
-    jy1_1 += dq1;
-    jy1_6 += dq6;
-    jy1_7 += dq7;
-  }
-  { // H2O2+O=OH+HO2
-    double ctb = 1.0;
-    double kf = kt[40], kr = kt[41];
-    const double dq2 = kf * (c7);
-    const double dq4 = -kr * (c6);
-    const double dq6 = -kr * (c4);
-    const double dq7 = kf * (c2);
-    jy7_2 -= dq2;
-    jy7_4 -= dq4;
-    jy7_6 -= dq6;
-    jy7_7 -= dq7;
-    jy2_2 -= dq2;
-    jy2_4 -= dq4;
-    jy2_6 -= dq6;
-    jy2_7 -= dq7;
-    jy4_2 += dq2;
-    jy4_4 += dq4;
-    jy4_6 += dq6;
-    jy4_7 += dq7;
-    jy6_2 += dq2;
-    jy6_4 += dq4;
-    jy6_6 += dq6;
-    jy6_7 += dq7;
-  }
-  { // H2O2+OH=HO2+H2O
-    double ctb = 1.0;
-    double kf = kt[42], kr = kt[43];
-    const double dq4 = kf * (c7);
-    const double dq5 = -kr * (c6);
-    const double dq6 = -kr * (c5);
-    const double dq7 = kf * (c4);
-    jy7_4 -= dq4;
-    jy7_5 -= dq5;
-    jy7_6 -= dq6;
-    jy7_7 -= dq7;
-    jy4_4 -= dq4;
-    jy4_5 -= dq5;
-    jy4_6 -= dq6;
-    jy4_7 -= dq7;
-    jy6_4 += dq4;
-    jy6_5 += dq5;
-    jy6_6 += dq6;
-    jy6_7 += dq7;
-    jy5_4 += dq4;
-    jy5_5 += dq5;
-    jy5_6 += dq6;
-    jy5_7 += dq7;
-  }
-  { // H2O2+OH=HO2+H2O
-    double ctb = 1.0;
-    double kf = kt[44], kr = kt[45];
-    const double dq4 = kf * (c7);
-    const double dq5 = -kr * (c6);
-    const double dq6 = -kr * (c5);
-    const double dq7 = kf * (c4);
-    jy7_4 -= dq4;
-    jy7_5 -= dq5;
-    jy7_6 -= dq6;
-    jy7_7 -= dq7;
-    jy4_4 -= dq4;
-    jy4_5 -= dq5;
-    jy4_6 -= dq6;
-    jy4_7 -= dq7;
-    jy6_4 += dq4;
-    jy6_5 += dq5;
-    jy6_6 += dq6;
-    jy6_7 += dq7;
-    jy5_4 += dq4;
-    jy5_5 += dq5;
-    jy5_6 += dq6;
-    jy5_7 += dq7;
-  }
-  double cvb = z[1] * kt[46] + z[2] * kt[48] + z[3] * kt[50] + z[4] * kt[52] + z[5] * kt[54] + z[6] * kt[56] + z[7] * kt[58] + z[8] * kt[60] + z[9] * kt[62];
-  const double rcv = 1.0 / (rho * cvb);
-  const double um0 = kt[47] * 1.0079699754714966 - ru * T;
-  const double um1 = kt[49] * 2.015939950942993 - ru * T;
-  const double um2 = kt[51] * 15.99940013885498 - ru * T;
-  const double um3 = kt[53] * 31.99880027770996 - ru * T;
-  const double um4 = kt[55] * 17.007370114326477 - ru * T;
-  const double um5 = kt[57] * 18.015340089797974 - ru * T;
-  const double um6 = kt[59] * 33.00677025318146 - ru * T;
-  const double um7 = kt[61] * 34.014740228652954 - ru * T;
-  const double um8 = kt[63] * 28.013399124145508 - ru * T;
+  const double qm15 = (kt[29] * c7 - kt[30] * c4 * c4) * dp15;
+  // H2O2+H=H2O+OH
+  // H2O2+H=HO2+H2
+  // H2O2+O=OH+HO2
+  // H2O2+OH=HO2+H2O
+  const double M0_0 = 2.0 * qm4 - qm6 - qm7;
+  const double M0_1 = -qm4;
+  const double M0_2 = -2.0 * qm5 - qm6;
+  const double M0_3 = qm5;
+  const double M0_4 = qm6 - qm7 + 2.0 * qm15;
+  const double M0_5 = qm7;
+  const double M0_7 = -qm15;
+  const double M1_0 = -qm8;
+  const double M1_3 = -qm8;
+  const double M1_6 = qm8;
+  const double cvb = z[1] * kt[41] + z[2] * kt[43] + z[3] * kt[45] + z[4] * kt[47] + z[5] * kt[49] + z[6] * kt[51] + z[7] * kt[53] + z[8] * kt[55] + z[9] * kt[57];
+  const double cvi = d_rcp(cvb);
   { // column d / d Y_0
-    const double s = rho * 0.9920930427835725;
-    J[1][1] = jy0_0 * s * (1.0079699754714966 / rho);
-    J[2][1] = jy1_0 * s * (2.015939950942993 / rho);
-    J[3][1] = jy2_0 * s * (15.99940013885498 / rho);
-    J[4][1] = jy3_0 * s * (31.99880027770996 / rho);
-    J[5][1] = jy4_0 * s * (17.007370114326477 / rho);
-    J[6][1] = jy5_0 * s * (18.015340089797974 / rho);
-    J[7][1] = jy6_0 * s * (33.00677025318146 / rho);
-    J[8][1] = jy7_0 * s * (34.014740228652954 / rho);
-    J[9][1] = jy8_0 * s * (28.013399124145508 / rho);
-    const double dsum = um0 * jy0_0 + um1 * jy1_0 + um2 * jy2_0 + um3 * jy3_0 + um4 * jy4_0 + um5 * jy5_0 + um6 * jy6_0 + um7 * jy7_0 + um8 * jy8_0;
-    J[0][1] = -(dsum * s) * rcv - f0T * kt[46] / cvb;
+    const double d0 = kt[0] * c3;
+    const double d1 = -kt[3] * c4;
+    const double d2 = -kt[5] * c5;
+    const double d4 = -(kt[9] * M0) * 2.0 * c0;
+    const double d6 = (kt[12] * M0) * c2;
+    const double d7 = (kt[14] * M0) * c4;
+    const double d8 = (kt[16] * sc8) * c3;
+    const double d9 = kt[19] * c6;
+    const double d10 = kt[21] * c6;
+    const double d16 = kt[32] * c7;
+    const double d17 = kt[34] * c7;
+    const double y0 = -d0 + d1 + d2 + 2.0 * d4 - d6 - d7 - d8 - d9 - d10 - d16 - d17 + M0_0 + M1_0;
+    const double y1 = -d1 - d2 - d4 + d9 + d17 + M0_1;
+    const double y2 = d0 - d1 - d6 + M0_2;
+    const double y3 = -d0 - d8 + d9 + M0_3 + M1_3;
+    const double y4 = d0 + d1 - d2 + d6 - d7 + 2.0 * d10 + d16 + M0_4;
+    const double y5 = d2 + d7 + d16 + M0_5;
+    const double y6 = d8 - d9 - d10 + d17 + M1_6;
+    const double y7 = -d16 - d17 + M0_7;
+    J[1][1] = y0 * 1.0;
+    J[2][1] = y1 * 2.0;
+    J[3][1] = y2 * 15.87289356646855;
+    J[4][1] = y3 * 31.7457871329371;
+    J[5][1] = y4 * 16.87289356646855;
+    J[6][1] = y5 * 17.87289356646855;
+    J[7][1] = y6 * 32.7457871329371;
+    J[8][1] = y7 * 33.7457871329371;
+    J[9][1] = 0.0;
+    J[0][1] = -((kt[42] * y0 + kt[44] * y1 + kt[46] * y2 + kt[48] * y3 + kt[50] * y4 + kt[52] * y5 + kt[54] * y6 + kt[56] * y7) * 0.9920930427835725 + f0T * kt[41]) * cvi;
   }
   { // column d / d Y_1
-    const double s = rho * 0.49604652139178623;
-    J[1][2] = jy0_1 * s * (1.0079699754714966 / rho);
-    J[2][2] = jy1_1 * s * (2.015939950942993 / rho);
-    J[3][2] = jy2_1 * s * (15.99940013885498 / rho);
-    J[4][2] = jy3_1 * s * (31.99880027770996 / rho);
-    J[5][2] = jy4_1 * s * (17.007370114326477 / rho);
-    J[6][2] = jy5_1 * s * (18.015340089797974 / rho);
-    J[7][2] = jy6_1 * s * (33.00677025318146 / rho);
-    J[8][2] = jy7_1 * s * (34.014740228652954 / rho);
-    J[9][2] = jy8_1 * s * (28.013399124145508 / rho);
-    const double dsum = um0 * jy0_1 + um1 * jy1_1 + um2 * jy2_1 + um3 * jy3_1 + um4 * jy4_1 + um5 * jy5_1 + um6 * jy6_1 + um7 * jy7_1 + um8 * jy8_1;
-    J[0][2] = -(dsum * s) * rcv - f0T * kt[48] / cvb;
+    const double d1 = kt[2] * c2;
+    const double d2 = kt[4] * c4;
+    const double d4 = (kt[8] * M0);
+    const double d9 = -kt[20] * c3;
+    const double d17 = -kt[35] * c6;
+    const double y0 = d1 + d2 + 2.0 * d4 - d9 - d17 + 2.5 * M0_0 + 2.0 * M1_0;
+    const double y1 = -d1 - d2 - d4 + d9 + d17 + 2.5 * M0_1;
+    const double y2 = -d1 + 2.5 * M0_2;
+    const double y3 = d9 + 2.5 * M0_3 + 2.0 * M1_3;
+    const double y4 = d1 - d2 + 2.5 * M0_4;
+    const double y5 = d2 + 2.5 * M0_5;
+    const double y6 = -d9 + d17 + 2.0 * M1_6;
+    const double y7 = -d17 + 2.5 * M0_7;
+    J[1][2] = y0 * 0.5;
+    J[2][2] = y1 * 1.0;
+    J[3][2] = y2 * 7.936446783234275;
+    J[4][2] = y3 * 15.87289356646855;
+    J[5][2] = y4 * 8.436446783234276;
+    J[6][2] = y5 * 8.936446783234276;
+    J[7][2] = y6 * 16.37289356646855;
+    J[8][2] = y7 * 16.87289356646855;
+    J[9][2] = 0.0;
+    J[0][2] = -((kt[42] * y0 + kt[44] * y1 + kt[46] * y2 + kt[48] * y3 + kt[50] * y4 + kt[52] * y5 + kt[54] * y6 + kt[56] * y7) * 0.49604652139178623 + f0T * kt[43]) * cvi;
   }
   { // column d / d Y_2
-    const double s = rho * 0.06250234329545097;
-    J[1][3] = jy0_2 * s * (1.0079699754714966 / rho);
-    J[2][3] = jy1_2 * s * (2.015939950942993 / rho);
-    J[3][3] = jy2_2 * s * (15.99940013885498 / rho);
-    J[4][3] = jy3_2 * s * (31.99880027770996 / rho);
-    J[5][3] = jy4_2 * s * (17.007370114326477 / rho);
-    J[6][3] = jy5_2 * s * (18.015340089797974 / rho);
-    J[7][3] = jy6_2 * s * (33.00677025318146 / rho);
-    J[8][3] = jy7_2 * s * (34.014740228652954 / rho);
-    J[9][3] = jy8_2 * s * (28.013399124145508 / rho);
-    const double dsum = um0 * jy0_2 + um1 * jy1_2 + um2 * jy2_2 + um3 * jy3_2 + um4 * jy4_2 + um5 * jy5_2 + um6 * jy6_2 + um7 * jy7_2 + um8 * jy8_2;
-    J[0][3] = -(dsum * s) * rcv - f0T * kt[50] / cvb;
+    const double d0 = -kt[1] * c4;
+    const double d1 = kt[2] * c1;
+    const double d3 = kt[6] * c5;
+    const double d5 = (kt[10] * M0) * 2.0 * c2;
+    const double d6 = (kt[12] * M0) * c0;
+    const double d11 = 32500000000000.0 * c6;
+    const double d18 = kt[36] * c7;
+    const double y0 = -d0 + d1 - d6 + M0_0 + M1_0;
+    const double y1 = -d1 + M0_1;
+    const double y2 = d0 - d1 - d3 - 2.0 * d5 - d6 - d11 - d18 + M0_2;
+    const double y3 = -d0 + d5 + d11 + M0_3 + M1_3;
+    const double y4 = d0 + d1 + 2.0 * d3 + d6 + d11 + d18 + M0_4;
+    const double y5 = -d3 + M0_5;
+    const double y6 = -d11 + d18 + M1_6;
+    const double y7 = -d18 + M0_7;
+    J[1][3] = y0 * 0.06300048543842678;
+    J[2][3] = y1 * 0.12600097087685355;
+    J[3][3] = y2 * 1.0;
+    J[4][3] = y3 * 2.0;
+    J[5][3] = y4 * 1.0630004854384267;
+    J[6][3] = y5 * 1.1260009708768535;
+    J[7][3] = y6 * 2.063000485438427;
+    J[8][3] = y7 * 2.1260009708768535;
+    J[9][3] = 0.0;
+    J[0][3] = -((kt[42] * y0 + kt[44] * y1 + kt[46] * y2 + kt[48] * y3 + kt[50] * y4 + kt[52] * y5 + kt[54] * y6 + kt[56] * y7) * 0.06250234329545097 + f0T * kt[45]) * cvi;
   }
   { // column d / d Y_3
-    const double s = rho * 0.031251171647725486;
-    J[1][4] = jy0_3 * s * (1.0079699754714966 / rho);
-    J[2][4] = jy1_3 * s * (2.015939950942993 / rho);
-    J[3][4] = jy2_3 * s * (15.99940013885498 / rho);
-    J[4][4] = jy3_3 * s * (31.99880027770996 / rho);
-    J[5][4] = jy4_3 * s * (17.007370114326477 / rho);
-    J[6][4] = jy5_3 * s * (18.015340089797974 / rho);
-    J[7][4] = jy6_3 * s * (33.00677025318146 / rho);
-    J[8][4] = jy7_3 * s * (34.014740228652954 / rho);
-    J[9][4] = jy8_3 * s * (28.013399124145508 / rho);
-    const double dsum = um0 * jy0_3 + um1 * jy1_3 + um2 * jy2_3 + um3 * jy3_3 + um4 * jy4_3 + um5 * jy5_3 + um6 * jy6_3 + um7 * jy7_3 + um8 * jy8_3;
-    J[0][4] = -(dsum * s) * rcv - f0T * kt[52] / cvb;
+    const double d0 = kt[0] * c0;
+    const double d5 = -(kt[11] * M0);
+    const double d8 = (kt[16] * sc8) * c0;
+    const double d9 = -kt[20] * c1;
+    const double d11 = -kt[23] * c4;
+    const double d12 = -kt[25] * c5;
+    const double d13 = -kt[27] * c7;
+    const double y0 = -d0 - d8 - d9 + M0_0 + 0.78 * M1_0;
+    const double y1 = d9 + M0_1;
+    const double y2 = d0 - 2.0 * d5 - d11 + M0_2;
+    const double y3 = -d0 + d5 - d8 + d9 + d11 + d12 + d13 + M0_3 + 0.78 * M1_3;
+    const double y4 = d0 + d11 - d12 + M0_4;
+    const double y5 = d12 + M0_5;
+    const double y6 = d8 - d9 - d11 - d12 - 2.0 * d13 + 0.78 * M1_6;
+    const double y7 = d13 + M0_7;
+    J[1][4] = y0 * 0.03150024271921339;
+    J[2][4] = y1 * 0.06300048543842678;
+    J[3][4] = y2 * 0.5;
+    J[4][4] = y3 * 1.0;
+    J[5][4] = y4 * 0.5315002427192134;
+    J[6][4] = y5 * 0.5630004854384267;
+    J[7][4] = y6 * 1.0315002427192135;
+    J[8][4] = y7 * 1.0630004854384267;
+    J[9][4] = 0.0;
+    J[0][4] = -((kt[42] * y0 + kt[44] * y1 + kt[46] * y2 + kt[48] * y3 + kt[50] * y4 + kt[52] * y5 + kt[54] * y6 + kt[56] * y7) * 0.031251171647725486 + f0T * kt[47]) * cvi;
   }
   { // column d / d Y_4
-    const double s = rho * 0.05879803833736947;
-    J[1][5] = jy0_4 * s * (1.0079699754714966 / rho);
-    J[2][5] = jy1_4 * s * (2.015939950942993 / rho);
-    J[3][5] = jy2_4 * s * (15.99940013885498 / rho);
-    J[4][5] = jy3_4 * s * (31.99880027770996 / rho);
-    J[5][5] = jy4_4 * s * (17.007370114326477 / rho);
-    J[6][5] = jy5_4 * s * (18.015340089797974 / rho);
-    J[7][5] = jy6_4 * s * (33.00677025318146 / rho);
-    J[8][5] = jy7_4 * s * (34.014740228652954 / rho);
-    J[9][5] = jy8_4 * s * (28.013399124145508 / rho);
-    const double dsum = um0 * jy0_4 + um1 * jy1_4 + um2 * jy2_4 + um3 * jy3_4 + um4 * jy4_4 + um5 * jy5_4 + um6 * jy6_4 + um7 * jy7_4 + um8 * jy8_4;
-    J[0][5] = -(dsum * s) * rcv - f0T * kt[54] / cvb;
+    const double d0 = -kt[1] * c2;
+    const double d1 = -kt[3] * c0;
+    const double d2 = kt[4] * c1;
+    const double d3 = -kt[7] * 2.0 * c4;
+    const double d6 = -(kt[13] * M0);
+    const double d7 = (kt[14] * M0) * c0;
+    const double d10 = -kt[22] * 2.0 * c4;
+    const double d11 = -kt[23] * c3;
+    const double d12 = kt[24] * c6;
+    const double d15 = -(kt[30] * sc15) * 2.0 * c4;
+    const double d16 = -kt[33] * c5;
+    const double d18 = -kt[37] * c6;
+    const double d19 = kt[38] * c7;
+    const double y0 = -d0 + d1 + d2 - d6 - d7 - d10 - d16 + M0_0 + M1_0;
+    const double y1 = -d1 - d2 + M0_1;
+    const double y2 = d0 - d1 - d3 - d6 - d11 - d18 + M0_2;
+    const double y3 = -d0 + d11 + d12 + M0_3 + M1_3;
+    const double y4 = d0 + d1 - d2 + 2.0 * d3 + d6 - d7 + 2.0 * d10 + d11 - d12 + 2.0 * d15 + d16 + d18 - d19 + M0_4;
+    const double y5 = d2 - d3 + d7 + d12 + d16 + d19 + M0_5;
+    const double y6 = -d10 - d11 - d12 + d18 + d19 + M1_6;
+    const double y7 = -d15 - d16 - d18 - d19 + M0_7;
+    J[1][5] = y0 * 0.05926665726069042;
+    J[2][5] = y1 * 0.11853331452138084;
+    J[3][5] = y2 * 0.9407333427393095;
+    J[4][5] = y3 * 1.881466685478619;
+    J[5][5] = y4 * 1.0;
+    J[6][5] = y5 * 1.0592666572606904;
+    J[7][5] = y6 * 1.9407333427393096;
+    J[8][5] = y7 * 2.0;
+    J[9][5] = 0.0;
+    J[0][5] = -((kt[42] * y0 + kt[44] * y1 + kt[46] * y2 + kt[48] * y3 + kt[50] * y4 + kt[52] * y5 + kt[54] * y6 + kt[56] * y7) * 0.05879803833736947 + f0T * kt[49]) * cvi;
   }
   { // column d / d Y_5
-    const double s = rho * 0.05550824991454347;
-    J[1][6] = jy0_5 * s * (1.0079699754714966 / rho);
-    J[2][6] = jy1_5 * s * (2.015939950942993 / rho);
-    J[3][6] = jy2_5 * s * (15.99940013885498 / rho);
-    J[4][6] = jy3_5 * s * (31.99880027770996 / rho);
-    J[5][6] = jy4_5 * s * (17.007370114326477 / rho);
-    J[6][6] = jy5_5 * s * (18.015340089797974 / rho);
-    J[7][6] = jy6_5 * s * (33.00677025318146 / rho);
-    J[8][6] = jy7_5 * s * (34.014740228652954 / rho);
-    J[9][6] = jy8_5 * s * (28.013399124145508 / rho);
-    const double dsum = um0 * jy0_5 + um1 * jy1_5 + um2 * jy2_5 + um3 * jy3_5 + um4 * jy4_5 + um5 * jy5_5 + um6 * jy6_5 + um7 * jy7_5 + um8 * jy8_5;
-    J[0][6] = -(dsum * s) * rcv - f0T * kt[56] / cvb;
+    const double d2 = -kt[5] * c0;
+    const double d3 = kt[6] * c2;
+    const double d7 = -(kt[15] * M0);
+    const double d12 = -kt[25] * c3;
+    const double d16 = -kt[33] * c4;
+    const double d19 = -kt[39] * c6;
+    const double y0 = d2 - d7 - d16 + 12.0 * M0_0 + 11.0 * M1_0;
+    const double y1 = -d2 + 12.0 * M0_1;
+    const double y2 = -d3 + 12.0 * M0_2;
+    const double y3 = d12 + 12.0 * M0_3 + 11.0 * M1_3;
+    const double y4 = -d2 + 2.0 * d3 - d7 - d12 + d16 - d19 + 12.0 * M0_4;
+    const double y5 = d2 - d3 + d7 + d12 + d16 + d19 + 12.0 * M0_5;
+    const double y6 = -d12 + d19 + 11.0 * M1_6;
+    const double y7 = -d16 - d19 + 12.0 * M0_7;
+    J[1][6] = y0 * 0.05595064930482809;
+    J[2][6] = y1 * 0.11190129860965618;
+    J[3][6] = y2 * 0.8880987013903439;
+    J[4][6] = y3 * 1.7761974027806877;
+    J[5][6] = y4 * 0.9440493506951719;
+    J[6][6] = y5 * 1.0;
+    J[7][6] = y6 * 1.8321480520855158;
+    J[8][6] = y7 * 1.8880987013903439;
+    J[9][6] = 0.0;
+    J[0][6] = -((kt[42] * y0 + kt[44] * y1 + kt[46] * y2 + kt[48] * y3 + kt[50] * y4 + kt[52] * y5 + kt[54] * y6 + kt[56] * y7) * 0.05550824991454347 + f0T * kt[51]) * cvi;
   }
   { // column d / d Y_6
-    const double s = rho * 0.030296814633161872;
-    J[1][7] = jy0_6 * s * (1.0079699754714966 / rho);
-    J[2][7] = jy1_6 * s * (2.015939950942993 / rho);
-    J[3][7] = jy2_6 * s * (15.99940013885498 / rho);
-    J[4][7] = jy3_6 * s * (31.99880027770996 / rho);
-    J[5][7] = jy4_6 * s * (17.007370114326477 / rho);
-    J[6][7] = jy5_6 * s * (18.015340089797974 / rho);
-    J[7][7] = jy6_6 * s * (33.00677025318146 / rho);
-    J[8][7] = jy7_6 * s * (34.014740228652954 / rho);
-    J[9][7] = jy8_6 * s * (28.013399124145508 / rho);
-    const double dsum = um0 * jy0_6 + um1 * jy1_6 + um2 * jy2_6 + um3 * jy3_6 + um4 * jy4_6 + um5 * jy5_6 + um6 * jy6_6 + um7 * jy7_6 + um8 * jy8_6;
-    J[0][7] = -(dsum * s) * rcv - f0T * kt[58] / cvb;
+    const double d8 = -(kt[17] * sc8);
+    const double d9 = kt[19] * c0;
+    const double d10 = kt[21] * c0;
+    const double d11 = 32500000000000.0 * c2;
+    const double d12 = kt[24] * c4;
+    const double d13 = kt[26] * 2.0 * c6;
+    const double d17 = -kt[35] * c1;
+    const double d18 = -kt[37] * c4;
+    const double d19 = -kt[39] * c5;
+    const double y0 = -d8 - d9 - d10 - d17 + M0_0 + M1_0;
+    const double y1 = d9 + d17 + M0_1;
+    const double y2 = -d11 - d18 + M0_2;
+    const double y3 = -d8 + d9 + d11 + d12 + d13 + M0_3 + M1_3;
+    const double y4 = 2.0 * d10 + d11 - d12 + d18 - d19 + M0_4;
+    const double y5 = d12 + d19 + M0_5;
+    const double y6 = d8 - d9 - d10 - d11 - d12 - 2.0 * d13 + d17 + d18 + d19 + M1_6;
+    const double y7 = d13 - d17 - d18 - d19 + M0_7;
+    J[1][7] = y0 * 0.03053827950265265;
+    J[2][7] = y1 * 0.0610765590053053;
+    J[3][7] = y2 * 0.4847308602486737;
+    J[4][7] = y3 * 0.9694617204973474;
+    J[5][7] = y4 * 0.5152691397513264;
+    J[6][7] = y5 * 0.545807419253979;
+    J[7][7] = y6 * 1.0;
+    J[8][7] = y7 * 1.0305382795026528;
+    J[9][7] = 0.0;
+    J[0][7] = -((kt[42] * y0 + kt[44] * y1 + kt[46] * y2 + kt[48] * y3 + kt[50] * y4 + kt[52] * y5 + kt[54] * y6 + kt[56] * y7) * 0.030296814633161872 + f0T * kt[53]) * cvi;
   }
   { // column d / d Y_7
-    const double s = rho * 0.029399019168684735;
-    J[1][8] = jy0_7 * s * (1.0079699754714966 / rho);
-    J[2][8] = jy1_7 * s * (2.015939950942993 / rho);
-    J[3][8] = jy2_7 * s * (15.99940013885498 / rho);
-    J[4][8] = jy3_7 * s * (31.99880027770996 / rho);
-    J[5][8] = jy4_7 * s * (17.007370114326477 / rho);
-    J[6][8] = jy5_7 * s * (18.015340089797974 / rho);
-    J[7][8] = jy6_7 * s * (33.00677025318146 / rho);
-    J[8][8] = jy7_7 * s * (34.014740228652954 / rho);
-    J[9][8] = jy8_7 * s * (28.013399124145508 / rho);
-    const double dsum = um0 * jy0_7 + um1 * jy1_7 + um2 * jy2_7 + um3 * jy3_7 + um4 * jy4_7 + um5 * jy5_7 + um6 * jy6_7 + um7 * jy7_7 + um8 * jy8_7;
-    J[0][8] = -(dsum * s) * rcv - f0T * kt[60] / cvb;
+    const double d13 = -kt[27] * c3;
+    const double d15 = (kt[29] * sc15);
+    const double d16 = kt[32] * c0;
+    const double d17 = kt[34] * c0;
+    const double d18 = kt[36] * c2;
+    const double d19 = kt[38] * c4;
+    const double y0 = -d16 - d17 + M0_0 + M1_0;
+    const double y1 = d17 + M0_1;
+    const double y2 = -d18 + M0_2;
+    const double y3 = d13 + M0_3 + M1_3;
+    const double y4 = 2.0 * d15 + d16 + d18 - d19 + M0_4;
+    const double y5 = d16 + d19 + M0_5;
+    const double y6 = -2.0 * d13 + d17 + d18 + d19 + M1_6;
+    const double y7 = d13 - d15 - d16 - d17 - d18 - d19 + M0_7;
+    J[1][8] = y0 * 0.02963332863034521;
+    J[2][8] = y1 * 0.05926665726069042;
+    J[3][8] = y2 * 0.47036667136965477;
+    J[4][8] = y3 * 0.9407333427393095;
+    J[5][8] = y4 * 0.5;
+    J[6][8] = y5 * 0.5296333286303452;
+    J[7][8] = y6 * 0.9703666713696548;
+    J[8][8] = y7 * 1.0;
+    J[9][8] = 0.0;
+    J[0][8] = -((kt[42] * y0 + kt[44] * y1 + kt[46] * y2 + kt[48] * y3 + kt[50] * y4 + kt[52] * y5 + kt[54] * y6 + kt[56] * y7) * 0.029399019168684735 + f0T * kt[55]) * cvi;
   }
   { // column d / d Y_8
-    const double s = rho * 0.035697203169395925;
-    J[1][9] = jy0_8 * s * (1.0079699754714966 / rho);
-    J[2][9] = jy1_8 * s * (2.015939950942993 / rho);
-    J[3][9] = jy2_8 * s * (15.99940013885498 / rho);
-    J[4][9] = jy3_8 * s * (31.99880027770996 / rho);
-    J[5][9] = jy4_8 * s * (17.007370114326477 / rho);
-    J[6][9] = jy5_8 * s * (18.015340089797974 / rho);
-    J[7][9] = jy6_8 * s * (33.00677025318146 / rho);
-    J[8][9] = jy7_8 * s * (34.014740228652954 / rho);
-    J[9][9] = jy8_8 * s * (28.013399124145508 / rho);
-    const double dsum = um0 * jy0_8 + um1 * jy1_8 + um2 * jy2_8 + um3 * jy3_8 + um4 * jy4_8 + um5 * jy5_8 + um6 * jy6_8 + um7 * jy7_8 + um8 * jy8_8;
-    J[0][9] = -(dsum * s) * rcv - f0T * kt[62] / cvb;
+    const double y0 = M0_0 + M1_0;
+    const double y1 = M0_1;
+    const double y2 = M0_2;
+    const double y3 = M0_3 + M1_3;
+    const double y4 = M0_4;
+    const double y5 = M0_5;
+    const double y6 = M1_6;
+    const double y7 = M0_7;
+    J[1][9] = y0 * 0.03598170900305704;
+    J[2][9] = y1 * 0.07196341800611408;
+    J[3][9] = y2 * 0.5711338373451675;
+    J[4][9] = y3 * 1.142267674690335;
+    J[5][9] = y4 * 0.6071155463482246;
+    J[6][9] = y5 * 0.6430972553512817;
+    J[7][9] = y6 * 1.1782493836933923;
+    J[8][9] = y7 * 1.2142310926964492;
+    J[9][9] = 0.0;
+    J[0][9] = -((kt[42] * y0 + kt[44] * y1 + kt[46] * y2 + kt[48] * y3 + kt[50] * y4 + kt[52] * y5 + kt[54] * y6 + kt[56] * y7) * 0.035697203169395925 + f0T * kt[57]) * cvi;
   }
+}
+
+// column 0, d / d T, given f0 = dz/dt; a Troe or SRI centring factor's own
+// temperature dependence is left out (the column serves an iteration matrix)
+IZ_HD inline void gen_jac_T(double rho, const double *z, const double *kt, const double *f0,
+                            double (*J)[GEN_KK + 1]) {
+#pragma clang fp contract(on)
+  const double T = z[0], ru = 8.314510e7, it = 1.0 / T, rut2 = it * it * (1.0 / ru);
+  const double c0 = rho * z[1] * 0.9920930427835725;
+  const double c1 = rho * z[2] * 0.49604652139178623;
+  const double c2 = rho * z[3] * 0.06250234329545097;
+  const double c3 = rho * z[4] * 0.031251171647725486;
+  const double c4 = rho * z[5] * 0.05879803833736947;
+  const double c5 = rho * z[6] * 0.05550824991454347;
+  const double c6 = rho * z[7] * 0.030296814633161872;
+  const double c7 = rho * z[8] * 0.029399019168684735;
+  const double c8 = rho * z[9] * 0.035697203169395925;
+  const double ctot = c0 + c1 + c2 + c3 + c4 + c5 + c6 + c7 + c8;
+  const double M0 = ctot + 1.5 * c1 + 11.0 * c5;
+  const double M1 = ctot + 1.0 * c1 - 0.21999999999999997 * c3 + 10.0 * c5;
+  // H+O2=O+OH
+  const double af0 = (-0.406 + 8352.893466155027 * it) * it;
+  const double qT0 = af0 * (kt[0] * c0 * c3) - (af0 - (-kt[42] - kt[48] + kt[46] + kt[50]) * rut2) * (kt[1] * c2 * c4);
+  // O+H2=H+OH
+  const double af1 = (2.67 + 3165.2328394550946 * it) * it;
+  const double qT1 = af1 * (kt[2] * c2 * c1) - (af1 - (-kt[46] - kt[44] + kt[42] + kt[50]) * rut2) * (kt[3] * c0 * c4);
+  // H2+OH=H2O+H
+  const double af2 = (1.51 + 1726.0331700049244 * it) * it;
+  const double qT2 = af2 * (kt[4] * c1 * c4) - (af2 - (-kt[44] - kt[50] + kt[52] + kt[42]) * rut2) * (kt[5] * c5 * c0);
+  // O+H2O=OH+OH
+  const double af3 = (2.02 + 6743.103346374924 * it) * it;
+  const double qT3 = af3 * (kt[6] * c2 * c5) - (af3 - (-kt[46] - kt[52] + 2.0 * kt[50]) * rut2) * (kt[7] * c4 * c4);
+  // H2+M=H+H+M
+  const double af4 = (-1.4 + 52525.755768254814 * it) * it;
+  const double qT4 = M0 * (af4 * (kt[8] * c1) - (af4 - (-kt[44] + 2.0 * kt[42]) * rut2) * (kt[9] * c0 * c0));
+  // O+O+M=O2+M
+  const double af5 = (-0.5 + 0.0 * it) * it;
+  const double qT5 = M0 * (af5 * (kt[10] * c2 * c2) - (af5 - (-2.0 * kt[46] + kt[48]) * rut2) * (kt[11] * c3));
+  // O+H+M=OH+M
+  const double af6 = (-1.0 + 0.0 * it) * it;
+  const double qT6 = M0 * (af6 * (kt[12] * c2 * c0) - (af6 - (-kt[46] - kt[42] + kt[50]) * rut2) * (kt[13] * c4));
+  // H+OH+M=H2O+M
+  const double af7 = (-2.0 + 0.0 * it) * it;
+  const double qT7 = M0 * (af7 * (kt[14] * c0 * c4) - (af7 - (-kt[42] - kt[50] + kt[52]) * rut2) * (kt[15] * c5));
+  // H+O2(+M)=HO2(+M)
+  double sc8, dp8;
+  {
+    const double pr = kt[18] * M1;
+    const double lin1 = d_rcp(1.0 + pr);
+    const double prlog = 0.43429448190325182 * d_log(fmax(pr, 1e-300));
+    const double cpr = prlog - 0.33507029128460225;
+    const double xn = 0.8730757165202316;
+    const double den = xn - 0.14 * cpr, den2 = den * den;
+    const double g = den2 * d_rcp(den2 + cpr * cpr);
+    const double fcent = d_exp(-0.22314355131420974 * g);
+    const double dfdpr = (pr > 1e-300) ? -2.0 * fcent * -0.22314355131420974 * 0.43429448190325182 * cpr * xn * g * g / (den2 * den * pr) : 0.0;
+    const double pcor = pr * lin1 * fcent;
+    const double dpcor = fcent * lin1 * lin1 + pr * lin1 * dfdpr;
+    sc8 = pcor;
+    dp8 = dpcor * kt[18];
+  }
+  const double af8 = (0.6 + 0.0 * it) * it;
+  const double qT8 = sc8 * (af8 * (kt[16] * c0 * c3) - (af8 - (-kt[42] - kt[48] + kt[54]) * rut2) * (kt[17] * c6)) + (kt[16] * c0 * c3 - kt[17] * c6) * dp8 * M1 * (-2.32 + 264.08810717742983 * it) * it;
+  // HO2+H=H2+O2
+  const double af9 = (0.0 + 414.1473174676539 * it) * it;
+  const double qT9 = af9 * (kt[19] * c6 * c0) - (af9 - (-kt[54] - kt[42] + kt[44] + kt[48]) * rut2) * (kt[20] * c1 * c3);
+  // HO2+H=OH+OH
+  const double af10 = (0.0 + 148.44891695377632 * it) * it;
+  const double qT10 = af10 * (kt[21] * c6 * c0) - (af10 - (-kt[54] - kt[42] + 2.0 * kt[50]) * rut2) * (kt[22] * c4 * c4);
+  // HO2+O=O2+OH
+  const double af11 = (0.0 + 0.0 * it) * it;
+  const double qT11 = af11 * (32500000000000.0 * c6 * c2) - (af11 - (-kt[54] - kt[46] + kt[48] + kt[50]) * rut2) * (kt[23] * c3 * c4);
+  // HO2+OH=H2O+O2
+  const double af12 = (0.0 + -250.09868381704007 * it) * it;
+  const double qT12 = af12 * (kt[24] * c6 * c4) - (af12 - (-kt[54] - kt[50] + kt[52] + kt[48]) * rut2) * (kt[25] * c5 * c3);
+  // HO2+HO2=H2O2+O2
+  const double af13 = kt[28] / kt[26];
+  const double qT13 = af13 * (kt[26] * c6 * c6) - (af13 - (-2.0 * kt[54] + kt[56] + kt[48]) * rut2) * (kt[27] * c7 * c3);
+  // H2O2(+M)=OH+OH(+M)
+  double sc15, dp15;
+  {
+    const double pr = kt[31] * M0;
+    const double lin1 = d_rcp(1.0 + pr);
+    const double prlog = 0.43429448190325182 * d_log(fmax(pr, 1e-300));
+    const double cpr = prlog - 0.19830990290513262;
+    const double xn = 1.1323080944932562;
+    const double den = xn - 0.14 * cpr, den2 = den * den;
+    const double g = den2 * d_rcp(den2 + cpr * cpr);
+    const double fcent = d_exp(-0.6931471805599454 * g);
+    const double dfdpr = (pr > 1e-300) ? -2.0 * fcent * -0.6931471805599454 * 0.43429448190325182 * cpr * xn * g * g / (den2 * den * pr) : 0.0;
+    const double pcor = pr * lin1 * fcent;
+    const double dpcor = fcent * lin1 * lin1 + pr * lin1 * dfdpr;
+    sc15 = pcor;
+    dp15 = dpcor * kt[31];
+  }
+  const double af15 = (0.0 + 24370.78321380131 * it) * it;
+  const double qT15 = sc15 * (af15 * (kt[29] * c7) - (af15 - (-kt[56] + 2.0 * kt[50]) * rut2) * (kt[30] * c4 * c4)) + (kt[29] * c7 - kt[30] * c4 * c4) * dp15 * M0 * (0.0 + -1474.424836184964 * it) * it;
+  // H2O2+H=H2O+OH
+  const double af16 = (0.0 + 1997.7701705304812 * it) * it;
+  const double qT16 = af16 * (kt[32] * c7 * c0) - (af16 - (-kt[56] - kt[42] + kt[52] + kt[50]) * rut2) * (kt[33] * c5 * c4);
+  // H2O2+H=HO2+H2
+  const double af17 = (0.0 + 4000.5725077373613 * it) * it;
+  const double qT17 = af17 * (kt[34] * c7 * c0) - (af17 - (-kt[56] - kt[42] + kt[54] + kt[44]) * rut2) * (kt[35] * c6 * c1);
+  // H2O2+O=OH+HO2
+  const double af18 = (2.0 + 1997.7701705304812 * it) * it;
+  const double qT18 = af18 * (kt[36] * c7 * c2) - (af18 - (-kt[56] - kt[46] + kt[50] + kt[54]) * rut2) * (kt[37] * c4 * c6);
+  // H2O2+OH=HO2+H2O
+  const double af19 = kt[40] / kt[38];
+  const double qT19 = af19 * (kt[38] * c7 * c4) - (af19 - (-kt[56] - kt[50] + kt[54] + kt[52]) * rut2) * (kt[39] * c6 * c5);
+  const double cvb = z[1] * kt[41] + z[2] * kt[43] + z[3] * kt[45] + z[4] * kt[47] + z[5] * kt[49] + z[6] * kt[51] + z[7] * kt[53] + z[8] * kt[55] + z[9] * kt[57];
+  const double cvi = d_rcp(cvb);
+  const double rho_i = d_rcp(rho);
+  const double y0 = -qT0 + qT1 + qT2 + 2.0 * qT4 - qT6 - qT7 - qT8 - qT9 - qT10 - qT16 - qT17;
+  const double y1 = -qT1 - qT2 - qT4 + qT9 + qT17;
+  const double y2 = qT0 - qT1 - qT3 - 2.0 * qT5 - qT6 - qT11 - qT18;
+  const double y3 = -qT0 + qT5 - qT8 + qT9 + qT11 + qT12 + qT13;
+  const double y4 = qT0 + qT1 - qT2 + 2.0 * qT3 + qT6 - qT7 + 2.0 * qT10 + qT11 - qT12 + 2.0 * qT15 + qT16 + qT18 - qT19;
+  const double y5 = qT2 - qT3 + qT7 + qT12 + qT16 + qT19;
+  const double y6 = qT8 - qT9 - qT10 - qT11 - qT12 - 2.0 * qT13 + qT17 + qT18 + qT19;
+  const double y7 = qT13 - qT15 - qT16 - qT17 - qT18 - qT19;
+  J[1][0] = y0 * (1.0079699754714966 * rho_i);
+  J[2][0] = y1 * (2.015939950942993 * rho_i);
+  J[3][0] = y2 * (15.99940013885498 * rho_i);
+  J[4][0] = y3 * (31.99880027770996 * rho_i);
+  J[5][0] = y4 * (17.007370114326477 * rho_i);
+  J[6][0] = y5 * (18.015340089797974 * rho_i);
+  J[7][0] = y6 * (33.00677025318146 * rho_i);
+  J[8][0] = y7 * (34.014740228652954 * rho_i);
+  J[9][0] = 0.0;
+  const double ut = (kt[42] * y0 + kt[44] * y1 + kt[46] * y2 + kt[48] * y3 + kt[50] * y4 + kt[52] * y5 + kt[54] * y6 + kt[56] * y7) * rho_i;
+  const double cf = kt[41] * f0[1] + kt[43] * f0[2] + kt[45] * f0[3] + kt[47] * f0[4] + kt[49] * f0[5] + kt[51] * f0[6] + kt[53] * f0[7] + kt[55] * f0[8];
+  double p1, p2, p3, p4;
+  if (T > 1000.0) {
+    p1 = -2.30842973e-11 * c0 - 4.94024731e-05 * c1 - 8.59741137e-05 * c2 + 0.00148308754 * c3 + 0.000548429716 * c4 + 0.00217691804 * c5 + 0.00223982013 * c6 + 0.00490831694 * c7 + 0.0014879768 * c8;
+    p2 = 3.23123896e-14 * c0 + 9.98913556e-07 * c1 + 8.38969178e-08 * c2 - 1.515933338e-06 * c3 + 2.53010456e-07 * c4 - 3.28145036e-07 * c5 - 1.2673163e-06 * c6 - 3.8027845e-06 * c7 - 1.136952e-06 * c8;
+    p3 = -1.4205457050000002e-17 * c0 - 5.38699182e-10 * c1 - 3.00533397e-11 * c2 + 6.28411665e-10 * c3 - 2.638384668e-10 * c4 - 2.91125961e-10 * c5 + 3.4273911e-10 * c6 + 1.113557958e-09 * c7 + 3.0291114e-10 * c8;
+    p4 = 1.992789428e-21 * c0 + 8.01021504e-14 * c1 + 4.91334764e-15 * c2 - 8.66871176e-14 * c3 + 4.69649504e-14 * c4 + 6.72803968e-14 * c5 - 4.3163414e-14 * c6 - 1.15163322e-13 * c7 - 2.7013404e-14 * c8;
+  }
+  else {
+    p1 = 7.05332819e-13 * c0 + 0.00798052075 * c1 - 0.00327931884 * c2 - 0.00299673416 * c3 - 0.00240131752 * c4 - 0.0020364341 * c5 - 0.00474912051 * c6 - 0.000542822417 * c7 + 0.0014082404 * c8;
+    p2 = -3.99183928e-15 * c0 - 3.8956302e-05 * c1 + 1.328612792e-05 * c2 + 1.969460402e-05 * c3 + 9.23587682e-06 * c4 + 1.304080422e-05 * c5 + 4.23165782e-05 * c6 + 3.34671402e-05 * c7 - 7.926444e-06 * c8;
+    p3 = 6.902448959999999e-18 * c0 + 6.04716282e-08 * c1 - 1.838419872e-08 * c2 - 2.9043885270000002e-08 * c3 - 1.164339999e-08 * c4 - 1.6463911860000002e-08 * c5 - 7.28291682e-08 * c6 - 6.47312439e-08 * c7 + 1.6924545e-08 * c8;
+    p4 = -3.710929328e-21 * c0 - 2.950447044e-11 * c1 + 8.45063884e-12 * c2 + 1.297491348e-11 * c3 + 5.4564588e-12 * c4 + 7.08791268e-12 * c5 + 3.716900496e-11 * c6 + 3.449817452e-11 * c7 - 9.779416e-12 * c8;
+  }
+  const double dcv = (p1 + T * (p2 + T * (p3 + T * p4))) * (ru * rho_i);
+  J[0][0] = -(ut + cf + f0[0] * dcv) * cvi;
 }
 

@@ -22,7 +22,7 @@ NEQ = 10  # T + 9 species
 
 _TOKEN = re.compile(r"\d+\.\d*(?:[eE][+-]?\d+)?|\d+(?:[eE][+-]?\d+)|\d+|[A-Za-z_]\w*|"
                     r"\+=|-=|\*=|/=|[-+*/()\[\],;=?:<>!&|{}]")
-_TRANS = {"exp", "log", "log10", "pow", "sqrt"}
+_TRANS = {"exp", "log", "log10", "pow", "sqrt", "d_exp", "d_log"}
 
 
 def count_ops(src: str) -> tuple[int, int]:
@@ -65,8 +65,9 @@ def kinetics_counts(path: str | None = None) -> dict:
     src = open(path).read()
     kt = count_ops(_function_body(src, "gen_kT"))
     rhs = count_ops(_function_body(src, "gen_rhs"))
+    jac = sum(sum(count_ops(_function_body(src, f))) for f in ("void gen_jac", "void gen_jac_T"))
     return {"kT": kt[0] + kt[1], "conc": rhs[0] + rhs[1], "kT_trans": kt[1],
-            "conc_trans": rhs[1]}
+            "conc_trans": rhs[1], "jac": jac}
 
 
 # Operations of one Euler face flux (euler_LLF_x/_y/_z, module_weno.f90:
@@ -141,19 +142,20 @@ def solve_ops(n: int = NEQ) -> int:
     return n * (n - 1) + n * (n - 1) + n
 
 
-def chem_flops(stats, counts: dict | None = None) -> float:
+def chem_flops(stats, counts: dict | None = None, closed_form: bool = False) -> float:
     """Operations of a batch of integrations from its counters
     (steps, RHS evaluations, Jacobians, LU solves).  A Jacobian is one
     concentration part per perturbed column and the temperature part of the
     temperature column, plus the difference quotients (3 per entry, 6 per
     column for the increment) and the diagonal: the species columns reuse
     the temperature part of the evaluation of f(y) that precedes every
-    Jacobian (counted among the plain evaluations).  One factorisation is
+    Jacobian (counted among the plain evaluations).  closed_form: the
+    operations of the generated Jacobian instead.  One factorisation is
     counted per Jacobian, DVODE's minimum."""
     nst, nfe, nje, nsol = [float(x) for x in stats]
     c = counts or kinetics_counts()
     rhs = c["kT"] + c["conc"]
-    jac = c["kT"] + NEQ * c["conc"] + NEQ * (3 * NEQ + 6) + NEQ
+    jac = c["jac"] if closed_form else c["kT"] + NEQ * c["conc"] + NEQ * (3 * NEQ + 6) + NEQ
     plain_rhs = nfe - NEQ * nje  # evaluations outside the Jacobians
     return plain_rhs * rhs + nje * (jac + lu_ops()) + nsol * solve_ops()
 

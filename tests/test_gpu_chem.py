@@ -538,3 +538,30 @@ def test_stiffness_order_flow_state(adi, thd, mech, kinetics):
     assert np.array_equal(s1, s0)
     assert np.array_equal(v1.view(np.uint64), v0.view(np.uint64))
     assert np.array_equal(T1.view(np.uint64), T0.view(np.uint64))
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 16384, 16385])
+def test_psr_batch_spread(mech, thd, n):
+    """Batches of up to one full wave per CU are spread over all CUs: each
+    cell's end state and step count are bit for bit those it has in a batch
+    of full waves (one cell's arithmetic does not depend on its neighbours)."""
+    import torch
+    from phd_amd import ics
+    s = _solver(mech)
+    big = 20000
+    T, p, Y = ics.config3_cells(thd, big, seed=17)
+    Wmix = 1.0 / (Y / (np.array(thd.W) * 1000.0)).sum(axis=1)
+    rho = (p * 10.0) * Wmix / (8.314510e7 * T)
+    out = {}
+    for m in (big, n):
+        d = [torch.tensor(np.ascontiguousarray(a[:m]), device="cuda:0") for a in (T, rho, Y)]
+        nst = torch.zeros(m, dtype=torch.int32, device="cuda:0")
+        assert s.lib.izem_psr_batch(s.ctx, m, C.c_void_p(d[0].data_ptr()),
+                                    C.c_void_p(d[1].data_ptr()), C.c_void_p(d[2].data_ptr()),
+                                    2.0e-7, C.c_void_p(nst.data_ptr())) == 0
+        s.sync()
+        assert s.status() == 0
+        out[m] = [a.cpu().numpy()[:n] for a in (d[0], d[2], nst)]
+    for a, b in zip(out[big], out[n]):
+        assert np.array_equal(a, b)
+    assert np.all(out[n][2] > 0)
