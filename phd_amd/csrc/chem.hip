@@ -879,9 +879,7 @@ static int reaction_tail(izem_ctx *ctx, const double *dt, double scale, double *
                          double *cp, double *ha, double *v) {
   int r = iz_upd_prim_woT(ctx, 0, v, T, W_i, cp, ha);
   if (r) return r;
-  r = iz_comm_cons(ctx, v, IZ_NV, 1, T, W_i, cp, dt, scale);
-  if (r) return r;
-  return iz_ghost_newton(ctx, T, W_i, cp, ha, v);
+  return iz_fill_ghost_newton(ctx, T, W_i, cp, ha, v, dt, scale);
 }
 
 extern "C" int izem_reaction_dvode(izem_ctx *ctx, const double *dt, double scale, double *T,

@@ -602,6 +602,47 @@ __device__ inline bool domset_cell(const IzDomSet &s, long tid, int &dom, int &i
   return box_cell(b, tid - f0, i, j, k);
 }
 
+// The domains of one Newton pass (the interior, a Dirichlet row, or all ghost
+// slabs together) in one launch, with blocks of their own per domain, so
+// that a block's reduction goes to one domain's mask: blocks [first[q],
+// first[q + 1]) walk the cells of box[q].  A slab alone is a few tens of
+// blocks; the six of a 3-D box one by one took 18 launches a pass.
+struct IzNewtonSet {
+  IzBox box[6];
+  int dom[6], slot[6];
+  unsigned first[7];
+  int n;
+};
+__device__ inline int nset_domain(const IzNewtonSet &s, IzBox &b, unsigned &blk, unsigned &nblk) {
+  b = s.box[0];
+  int q = 0;
+  unsigned f0 = 0, f1 = s.first[1];
+  // compile-time indices only, so the set stays in scalar registers
+#pragma unroll
+  for (int p = 1; p < 6; p++)
+    if (p < s.n && blockIdx.x >= s.first[p]) {
+      b = s.box[p];
+      q = p;
+      f0 = s.first[p];
+      f1 = s.first[p + 1];
+    }
+  blk = blockIdx.x - f0;
+  nblk = f1 - f0;
+  return q;
+}
+__device__ inline int nset_slot(const IzNewtonSet &s, int q) {
+  int v = s.slot[0];
+#pragma unroll
+  for (int p = 1; p < 6; p++) v = (p == q) ? s.slot[p] : v;
+  return v;
+}
+__device__ inline int nset_dom(const IzNewtonSet &s, int q) {
+  int v = s.dom[0];
+#pragma unroll
+  for (int p = 1; p < 6; p++) v = (p == q) ? s.dom[p] : v;
+  return v;
+}
+
 // force_sumY (npv = 0): module_thermodynamics.f90:1709-1760
 __device__ inline void d_force_sumY(double *vc) {
   double rho = vc[0], rho_i = 1.0 / rho, sum = 0.0, Y;
@@ -713,26 +754,47 @@ __device__ inline void block_extreme_pos(double *x, double *dst) {
   }
 }
 
+// force_sumY and the Newton probe on the domains of a set.  fill: the cells
+// are ghost cells of a periodic or extrapolated face and first take their
+// source cell's conserved variables (k_ghost_fill's copy), so that the ghost
+// layers are read and written once.
 __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2)))
-k_force_probe(IzDims d, IzBox b, int forcesum, double *__restrict__ v,
-                              const double *__restrict__ T, double eps,
-                              unsigned long long *__restrict__ mask) {
+k_force_probe(IzDims d, IzNewtonSet s, int fill, int forcesum, double *__restrict__ v,
+              const double *__restrict__ T, double eps, unsigned long long *__restrict__ masks) {
+  IzBox b;
+  unsigned blk, nblk;
+  const int q = nset_domain(s, b, blk, nblk), dom = nset_dom(s, q);
   int i, j, k;
   unsigned long long m = 0ull, neg = 0ull;
-  for (long tid = (long)blockIdx.x * blockDim.x + threadIdx.x; box_cell(b, tid, i, j, k);
-       tid += (long)gridDim.x * blockDim.x) {
-    long c = iz_cidx(d, i, j, k);
+  for (long tid = (long)blk * 256 + threadIdx.x; box_cell(b, tid, i, j, k);
+       tid += (long)nblk * 256) {
+    const long c = iz_cidx(d, i, j, k);
+    long cs = c;
+    if (fill) {
+      int si = i, sj = j, sk = k;
+      if (dom == -1) si = (d.phys & 1) ? 0 : i + d.nx;
+      else if (dom == 1) si = (d.phys & 2) ? d.nx - 1 : i - d.nx;
+      else if (dom == -2) sj = (d.phys & 4) ? 0 : j + d.ny;
+      else if (dom == 2) sj = (d.phys & 8) ? d.ny - 1 : j - d.ny;
+      else if (dom == -3) sk = (d.phys & 16) ? 0 : k + d.nz;
+      else sk = (d.phys & 32) ? d.nz - 1 : k - d.nz;
+      cs = iz_cidx(d, si, sj, sk);
+    }
     double vc[IZ_NV];
 #pragma unroll
-    for (int l = 0; l < IZ_NV; l++) vc[l] = v[l * d.nc + c];
-    if (forcesum) {
-      d_force_sumY(vc);
+    for (int l = 0; l < IZ_NV; l++) vc[l] = v[l * d.nc + cs];
+    if (forcesum) d_force_sumY(vc);
+    if (fill) {
+#pragma unroll
+      for (int l = 0; l < IZ_NIV; l++) v[l * d.nc + c] = vc[l];
+    }
+    if (fill || forcesum) {
 #pragma unroll
       for (int l = IZ_NIV; l < IZ_NV; l++) v[l * d.nc + c] = vc[l];
     }
     if (eps > 0.0) m |= d_newton_probe(vc, T[c], eps, neg);
   }
-  block_or_probe(m, neg, mask);
+  block_or_probe(m, neg, masks + nset_slot(s, q));
 }
 
 // number of global iterations from the OR of all probes: the first
@@ -754,17 +816,21 @@ __device__ inline bool d_newton_repairs(unsigned long long mask, unsigned long l
 // When a cell turns negative before the exit, nothing is written here and
 // k_newton_repair runs the domain's iterations instead.
 __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2)))
-k_newton_apply(IzDims d, IzBox b, const double *__restrict__ v,
+k_newton_apply(IzDims d, IzNewtonSet s, const double *__restrict__ v,
                                double *__restrict__ T, double *__restrict__ W_i,
                                double *__restrict__ cp, double *__restrict__ ha,
-                               const unsigned long long *__restrict__ mask, int itmax,
+                               const unsigned long long *__restrict__ masks, int itmax,
                                int repair, int *__restrict__ status, int *__restrict__ iters) {
-  long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  IzBox b;
+  unsigned blk, nblk;
+  const int slot = nset_slot(s, nset_domain(s, b, blk, nblk));
+  const unsigned long long *mask = masks + slot;
+  const long tid = (long)blk * 256 + threadIdx.x;
   int i, j, k;
   if (!box_cell(b, tid, i, j, k)) return;
   if (repair && d_newton_repairs(*mask, mask[IZ_NEG_MASKS], itmax)) return;
   const int N = d_newton_count(*mask, itmax);
-  if (tid == 0 && iters) *iters = N;
+  if (tid == 0) iters[slot] = N;
   long c = iz_cidx(d, i, j, k);
   double vc[IZ_NV];
 #pragma unroll
@@ -806,15 +872,31 @@ k_newton_apply(IzDims d, IzBox b, const double *__restrict__ v,
 // marks it; IZ_ST_NEG_T_ABORT marks a repair the reference aborts on (more
 // than IZ_NEGT_MAX cells, :131), one that would read outside the array (a
 // cell at its x edge) or more than IZ_NEGT_SWEEP negative cells in one
-// iteration.
+// iteration.  One block per domain of the set (a domain's repair reads no
+// cell that another's writes: slabs meet at edges, and x neighbours of a y
+// or z slab's cells are its own).  As the last kernel of a Newton pass it
+// also clears the domain's masks for the next one.
 #define IZ_NEGT_MAX 40000
 #define IZ_NEGT_SWEEP 1024
 __global__ void __launch_bounds__(1024)
-k_newton_repair(IzDims d, IzBox b, double *__restrict__ v, double *__restrict__ T,
-                double *__restrict__ W_i, double *__restrict__ cp, double *__restrict__ ha,
-                const unsigned long long *__restrict__ mask, int itmax, double eps,
-                int *__restrict__ rec, int *__restrict__ status, int *__restrict__ iters) {
-  if (!d_newton_repairs(*mask, mask[IZ_NEG_MASKS], itmax)) return;
+k_newton_repair(IzDims d, IzNewtonSet set, int repair, double *__restrict__ v,
+                double *__restrict__ T, double *__restrict__ W_i, double *__restrict__ cp,
+                double *__restrict__ ha, unsigned long long *__restrict__ masks, int itmax,
+                double eps, int *__restrict__ recs, int *__restrict__ status,
+                int *__restrict__ iters) {
+  const int slot = nset_slot(set, blockIdx.x);
+  IzBox b = set.box[0];
+#pragma unroll
+  for (int p = 1; p < 6; p++)
+    if (p == (int)blockIdx.x) b = set.box[p];
+  const unsigned long long m0 = masks[slot], n0 = masks[slot + IZ_NEG_MASKS];
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    masks[slot] = 0ull;
+    masks[slot + IZ_NEG_MASKS] = 0ull;
+  }
+  if (!repair || !d_newton_repairs(m0, n0, itmax)) return;
+  int *rec = recs + (long)slot * IZ_NEGT_MAX;
   __shared__ int s_neg[IZ_NEGT_SWEEP];
   __shared__ int s_nneg, s_it, s_ipt, s_correct, s_stop, s_bad;
   __shared__ double s_max[16], s_err;
@@ -934,7 +1016,7 @@ k_newton_repair(IzDims d, IzBox b, double *__restrict__ v, double *__restrict__ 
     if (s_err != s_err) st |= IZ_ST_NAN;
     if (s_it > itmax) st |= IZ_ST_NEWTON_ITMAX;
     atomicOr(status, st);
-    if (iters) *iters = s_it;
+    iters[slot] = s_it;
   }
 }
 
@@ -1521,7 +1603,8 @@ __global__ void k_visc_apply(IzDims d, const double *__restrict__ sf,
 
 // ===================================================================
 // Fused right-hand side + SSP-RK3 stage update + force_sumY + Newton probe
-// (rk3, module_solver.f90:769-847).  mode 0: write f only; mode 1: update.
+// (rk3, module_solver.f90:769-847).  mode 0: write f only; mode 1: update;
+// mode 2: update from the step's first state, which is kept in v0.
 // ===================================================================
 #ifndef IZ_RHS_WAVES
 #define IZ_RHS_WAVES 2
@@ -1536,7 +1619,7 @@ k_rhs_update(IzDims d, int mode, const double *__restrict__ Fx, const double *__
              const double *__restrict__ fd, const double *__restrict__ dx_i,
              const double *__restrict__ dy_i, const double *__restrict__ dz_i,
              const double *__restrict__ dtp, double bk, double ck,
-             const double *__restrict__ v0, double *__restrict__ v, double *__restrict__ fout,
+             double *__restrict__ v0, double *__restrict__ v, double *__restrict__ fout,
              int forcesum, const double *__restrict__ T, double eps,
              unsigned long long *__restrict__ mask) {
   // one cell per thread (a grid-stride loop here was 2.7x slower: the
@@ -1606,8 +1689,13 @@ k_rhs_update(IzDims d, int mode, const double *__restrict__ Fx, const double *__
       const double dt = *dtp;
       double vc[IZ_NV];
 #pragma unroll
-      for (int m = 0; m < IZ_NV; m++)
-        vc[m] = v0[m * d.nc + c] * bk + ck * (v[m * d.nc + c] - dt * f[m]);
+      for (int m = 0; m < IZ_NV; m++) {
+        const double vs = v[m * d.nc + c];
+        double vb = vs;
+        if (mode == 2) v0[m * d.nc + c] = vs;
+        else vb = v0[m * d.nc + c];
+        vc[m] = vb * bk + ck * (vs - dt * f[m]);
+      }
       if (forcesum) d_force_sumY(vc);
 #pragma unroll
       for (int m = 0; m < IZ_NV; m++) v[m * d.nc + c] = vc[m];
@@ -1620,6 +1708,18 @@ k_rhs_update(IzDims d, int mode, const double *__restrict__ Fx, const double *__
 // ===================================================================
 // Time step: timestep (module_solver.f90:202-408)
 // ===================================================================
+// the convective limit's rate of one cell
+__device__ inline double d_dt_conv(const IzDims &d, const double *__restrict__ v, double T, double Wi,
+                                   double cp, long c, double dxi, double dyi, double dzi) {
+  const double rho_i = 1.0 / v[c];
+  const double ux = v[d.nc + c] * rho_i, vy = v[2 * d.nc + c] * rho_i,
+               wz = v[3 * d.nc + c] * rho_i;
+  double gamma = c_thd.gam2 * Wi / cp;
+  gamma = 1.0 / (1.0 - gamma);
+  const double P = v[c] * T * Wi;
+  const double cs = sqrt(gamma * P * rho_i);
+  return fmax(fmax((fabs(ux) + cs) * dxi, (fabs(vy) + cs) * dyi), (fabs(wz) + cs) * dzi);
+}
 __global__ void k_dt_conv(IzDims d, const double *__restrict__ v, const double *__restrict__ T,
                           const double *__restrict__ W_i, const double *__restrict__ cp,
                           const double *__restrict__ dx_i, const double *__restrict__ dy_i,
@@ -1632,16 +1732,8 @@ __global__ void k_dt_conv(IzDims d, const double *__restrict__ v, const double *
     long r = tid / d.nx;
     int j = (int)(r % d.ny), k = (int)(r / d.ny);
     long c = iz_cidx(d, i, j, k);
-    double rho_i = 1.0 / v[c];
-    double ux = v[d.nc + c] * rho_i, vy = v[2 * d.nc + c] * rho_i, wz = v[3 * d.nc + c] * rho_i;
-    double gamma = c_thd.gam2 * W_i[c] / cp[c];
-    gamma = 1.0 / (1.0 - gamma);
-    double P = v[c] * T[c] * W_i[c];
-    double cs = sqrt(gamma * P * rho_i);
-    double a = (fabs(ux) + cs) * dx_i[i + d.ng];
-    double b = (fabs(vy) + cs) * dy_i[j + d.ng];
-    double e = (fabs(wz) + cs) * dz_i[k + d.ng];
-    dtc = fmax(dtc, fmax(fmax(a, b), e));
+    dtc = fmax(dtc, d_dt_conv(d, v, T[c], W_i[c], cp[c], c, dx_i[i + d.ng], dy_i[j + d.ng],
+                              dz_i[k + d.ng]));
   }
   block_extreme_pos<1, true>(&dtc, red);
 }
@@ -1658,7 +1750,7 @@ __device__ inline double d_filter_delta2(const IzDims &d, const double *dx_i, co
   return delta * delta;
 }
 
-// one pass over the transport properties: per species the maximum of the
+// the convective limit and one pass over the transport properties: per species the maximum of the
 // mixture diffusivity and the minimum of Delta^2 / D_l, and the minimum of
 // Delta^2 rho / (lambda / cp).  The species whose diffusivity maximum is
 // the largest is only known after the whole grid is reduced; keeping the
@@ -1670,7 +1762,7 @@ k_dt_visc(IzDims d, const double *__restrict__ v, const double *__restrict__ T,
                           const double *__restrict__ dx_i, const double *__restrict__ dy_i,
                           const double *__restrict__ dz_i, double *__restrict__ red) {
   const long ncin = (long)d.nx * d.ny * d.nz;
-  double dmax[IZ_NRV], mins[IZ_NRV + 1];
+  double dmax[IZ_NRV], mins[IZ_NRV + 1], dtc = 0.0;
 #pragma unroll
   for (int l = 0; l < IZ_NRV; l++) dmax[l] = 0.0;
 #pragma unroll
@@ -1693,7 +1785,10 @@ k_dt_visc(IzDims d, const double *__restrict__ v, const double *__restrict__ T,
       mins[l] = fmin(mins[l], d2 / (dm[l] + 0.0));
     }
     mins[IZ_NRV] = fmin(mins[IZ_NRV], d2 * v[c] / (ct / cp[c] + 0.0));
+    dtc = fmax(dtc, d_dt_conv(d, v, T[c], W_i[c], cp[c], c, dx_i[i + d.ng], dy_i[j + d.ng],
+                              dz_i[k + d.ng]));
   }
+  block_extreme_pos<1, true>(&dtc, red);
   block_extreme_pos<IZ_NRV, true>(dmax, red + 1);
   block_extreme_pos<IZ_NRV + 1, false>(mins, red + 12);
 }
@@ -1701,47 +1796,44 @@ k_dt_visc(IzDims d, const double *__restrict__ v, const double *__restrict__ T,
 // red layout: [0] dtc, [1..9] dm max, [12..20] min d2/D_l per species,
 // [21] min d2 rho cp/lambda
 // ts: [0..3] dt_4, [4] dtmin (in: previous), [5] DTmax (K)
-__global__ void k_dt_init(double *red) {
-  int t = threadIdx.x;
+__device__ inline void d_dt_init(double *red, int t) {
   if (t == 0) red[0] = 1.0;
   if (t >= 1 && t <= 9) red[t] = 0.0;
   if (t >= 12 && t <= 21) red[t] = __longlong_as_double(0x7ff0000000000000LL);
 }
+__global__ void k_dt_init(double *red) { d_dt_init(red, threadIdx.x); }
 
-__global__ void k_dt_final(const double *__restrict__ red, double CFL, double CFLmin, double Fo,
+// the limits from the reductions, which are reset for the next call (64
+// threads)
+__global__ void k_dt_final(double *__restrict__ red, double CFL, double CFLmin, double Fo,
                            double CPR, int visdt, int reaction, double rvd0_i, double rlamcp0_i,
                            double *__restrict__ ts) {
-  double dt4[4] = {1.0, 1.0, 1.0, 1.0};
-  dt4[0] = CFL / red[0];
-  if (visdt) {
-    // species of the global diffusivity maximum: the first in species order
-    double gmax = red[1];
-    int ldmax = 0;
-    for (int l = 1; l < IZ_NRV; l++)
-      if (gmax < red[1 + l]) { gmax = red[1 + l]; ldmax = l; }
-    dt4[1] = rvd0_i * Fo * red[12 + ldmax];
-    dt4[2] = rlamcp0_i * Fo * red[12 + IZ_NRV];
+  if (threadIdx.x == 0) {
+    double dt4[4] = {1.0, 1.0, 1.0, 1.0};
+    dt4[0] = CFL / red[0];
+    if (visdt) {
+      // species of the global diffusivity maximum: the first in species order
+      double gmax = red[1];
+      int ldmax = 0;
+      for (int l = 1; l < IZ_NRV; l++)
+        if (gmax < red[1 + l]) { gmax = red[1 + l]; ldmax = l; }
+      dt4[1] = rvd0_i * Fo * red[12 + ldmax];
+      dt4[2] = rlamcp0_i * Fo * red[12 + IZ_NRV];
+    }
+    if (reaction) {
+      dt4[3] = ts[4] * CPR / ts[5];
+      dt4[3] = fmin(dt4[3], 1.0);
+      dt4[3] = fmax(dt4[3], dt4[0] * CFLmin / CFL);
+    }
+    double mn = dt4[0];
+    for (int q = 1; q < 4; q++) mn = fmin(mn, dt4[q]);
+    for (int q = 0; q < 4; q++) ts[q] = dt4[q];
+    ts[4] = mn;
   }
-  if (reaction) {
-    dt4[3] = ts[4] * CPR / ts[5];
-    dt4[3] = fmin(dt4[3], 1.0);
-    dt4[3] = fmax(dt4[3], dt4[0] * CFLmin / CFL);
-  }
-  double mn = dt4[0];
-  for (int q = 1; q < 4; q++) mn = fmin(mn, dt4[q]);
-  for (int q = 0; q < 4; q++) ts[q] = dt4[q];
-  ts[4] = mn;
+  __syncthreads();
+  d_dt_init(red, threadIdx.x);
 }
 
-// small utility kernels (no hipMemsetAsync so that callers may capture them)
-__global__ void k_zero_u64(unsigned long long *p, int n) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = 0ull;
-}
-__global__ void k_copy(const double *__restrict__ a, double *__restrict__ b, long n) {
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) b[t] = a[t];
-}
 
 // batched wenorec for unit tests of the reconstruction itself
 __global__ void k_wenorec_batch(int n, int js, const double *__restrict__ vp,
@@ -1815,6 +1907,26 @@ static IzDomSet domain_set(const IzDims &d) {
   return s;
 }
 
+// the set of nd domains; capped: at most 16 blocks per CU and domain (kernels
+// that reduce walk their cells), else one thread per cell
+static IzNewtonSet newton_set(const izem_ctx *c, const int *doms, int nd, int capped) {
+  IzNewtonSet s{};
+  s.n = nd;
+  s.first[0] = 0;
+  for (int q = 0; q < 6; q++) {
+    if (q < nd) {
+      s.box[q] = domain_box(c->d, doms[q]);
+      s.dom[q] = doms[q];
+      s.slot[q] = mask_slot(doms[q]);
+      const long n = box_count(s.box[q]);
+      s.first[q + 1] = s.first[q] + (capped ? iz_blocks_capped(c, n, 256, 16) : iz_blocks(n, 256));
+    } else {
+      s.first[q + 1] = s.first[q];
+    }
+  }
+  return s;
+}
+
 extern "C" int izem_create(izem_ctx **out, const izem_grid *g, const double *thd, long nthd,
                            const izem_opts *opts) {
   if (!out || !g || !thd || !opts) return IZEM_E_ARG;
@@ -1859,7 +1971,7 @@ extern "C" int izem_create(izem_ctx **out, const izem_grid *g, const double *thd
   ok = ok && hipMalloc(&c->sf, sizeof(double) * c->nsf * d.nc) == hipSuccess;
   ok = ok && hipMalloc(&c->v0, sizeof(double) * IZ_NV * d.nc) == hipSuccess;
   ok = ok && hipMalloc(&c->masks, sizeof(unsigned long long) * 2 * IZ_NEG_MASKS) == hipSuccess;
-  ok = ok && hipMalloc(&c->negT_rec, sizeof(int) * IZ_NEGT_MAX) == hipSuccess;
+  ok = ok && hipMalloc(&c->negT_rec, sizeof(int) * IZ_NEG_MASKS * IZ_NEGT_MAX) == hipSuccess;
   ok = ok && hipMalloc(&c->status, sizeof(int) * 2) == hipSuccess;
   ok = ok && hipMalloc(&c->iters, sizeof(int) * 8) == hipSuccess;
   ok = ok && hipMalloc(&c->red, sizeof(double) * 24) == hipSuccess;
@@ -1870,6 +1982,10 @@ extern "C" int izem_create(izem_ctx **out, const izem_grid *g, const double *thd
   ok = ok && hipMemsetAsync(c->fd, 0, sizeof(double) * c->nderiv * d.nc, c->stream) == hipSuccess;
   ok = ok && hipMemsetAsync(c->sf, 0, sizeof(double) * c->nsf * d.nc, c->stream) == hipSuccess;
   ok = ok && hipMemsetAsync(c->status, 0, sizeof(int) * 2, c->stream) == hipSuccess;
+  // zero between Newton passes: k_newton_repair clears what a pass has set
+  ok = ok && hipMemsetAsync(c->masks, 0, sizeof(unsigned long long) * 2 * IZ_NEG_MASKS,
+                            c->stream) == hipSuccess;
+  if (ok) hipLaunchKernelGGL(k_dt_init, dim3(1), dim3(64), 0, c->stream, c->red);
   double ts0[6] = {1.0, 1.0, 1.0, 1.0, 1.0, 0.0};
   ok = ok && hipMemcpyAsync(c->ts, ts0, sizeof(ts0), hipMemcpyHostToDevice, c->stream) ==
                  hipSuccess;
@@ -2097,7 +2213,7 @@ extern "C" int izem_wenorec(izem_ctx *c, int n, int js, const double *vp, const 
 // k_rhs_update for the context's faces and decomposition
 typedef void (*IzRhsKernel)(IzDims, int, const double *, const double *, const double *, IzSeams,
                             int, const double *, const double *, const double *, const double *,
-                            const double *, const double *, double, double, const double *,
+                            const double *, const double *, double, double, double *,
                             double *, double *, int, const double *, double,
                             unsigned long long *);
 static IzRhsKernel rhs_update_kernel(const IzDims &d) {
@@ -2308,40 +2424,41 @@ static int dom_ok(const IzDims &d, int dom) {
 
 extern "C" int izem_force_sumY(izem_ctx *c, int dom, double *v) {
   if (!c || !v || !dom_ok(c->d, dom)) return IZEM_E_ARG;
-  IzBox b = domain_box(c->d, dom);
-  // probe output is discarded (mask slot 7)
-  hipLaunchKernelGGL(k_force_probe, dim3(iz_blocks_capped(c, box_count(b), 256, 16)), dim3(256), 0, c->stream,
-                     c->d, b, 1, v, (const double *)nullptr, -1.0, c->masks + 7);
+  // no probe: nothing reaches the masks
+  const IzNewtonSet s = newton_set(c, &dom, 1, 1);
+  hipLaunchKernelGGL(k_force_probe, dim3(s.first[1]), dim3(256), 0, c->stream, c->d, s, 0, 1, v,
+                     (const double *)nullptr, -1.0, c->masks);
   IZ_CHECK(hipGetLastError());
   return IZEM_OK;
 }
 
-// force_sumY (optional) + probe + apply on a list of domains; prim_inv_var
-// (eps 1e-5, 200 iterations, negative-temperature repair) or, with mach,
-// prim_inv_var_err_mach (module_thermodynamics.f90:201-260: eps 1e-10, 100
-// iterations, a negative temperature only warned about)
-static int newton_domains(izem_ctx *c, const int *doms, int nd, int forcesum, double *v,
-                          double *W_i, double *T, double *cp, double *ha, int mach = 0) {
+// the iterations of a probed set: apply, then the rare repair, which also
+// clears the masks
+static void newton_finish(izem_ctx *c, const int *doms, int nd, double *v, double *W_i, double *T,
+                          double *cp, double *ha, int mach) {
   const double eps = mach ? 1.0e-10 : 1.0e-5;
   const int itmax = mach ? 100 : 200;
-  const IzDims &d = c->d;
+  const IzNewtonSet s = newton_set(c, doms, nd, 0);
+  hipLaunchKernelGGL(k_newton_apply, dim3(s.first[nd]), dim3(256), 0, c->stream, c->d, s, v, T,
+                     W_i, cp, ha, c->masks, itmax, !mach, c->status, c->iters);
+  hipLaunchKernelGGL(k_newton_repair, dim3(nd), dim3(1024), 0, c->stream, c->d, s, !mach, v, T,
+                     W_i, cp, ha, c->masks, itmax, eps, c->negT_rec, c->status, c->iters);
+}
+
+// force_sumY (optional) + probe + apply on a list of at most six domains;
+// prim_inv_var (eps 1e-5, 200 iterations, negative-temperature repair) or,
+// with mach, prim_inv_var_err_mach (module_thermodynamics.f90:201-260: eps
+// 1e-10, 100 iterations, a negative temperature only warned about).  fill:
+// the domains are ghost slabs that take their source cells' conserved
+// variables first
+static int newton_domains(izem_ctx *c, const int *doms, int nd, int forcesum, double *v,
+                          double *W_i, double *T, double *cp, double *ha, int mach = 0,
+                          int fill = 0) {
+  const IzNewtonSet s = newton_set(c, doms, nd, 1);
   int pk = iz_prof_begin(c, IZP_NEWTON);
-  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, c->masks, 2 * IZ_NEG_MASKS);
-  for (int q = 0; q < nd; q++) {
-    IzBox b = domain_box(d, doms[q]);
-    hipLaunchKernelGGL(k_force_probe, dim3(iz_blocks_capped(c, box_count(b), 256, 16)), dim3(256), 0,
-                       c->stream, d, b, forcesum, v, T, eps, c->masks + mask_slot(doms[q]));
-  }
-  for (int q = 0; q < nd; q++) {
-    IzBox b = domain_box(d, doms[q]);
-    hipLaunchKernelGGL(k_newton_apply, dim3(iz_blocks(box_count(b), 256)), dim3(256), 0,
-                       c->stream, d, b, v, T, W_i, cp, ha, c->masks + mask_slot(doms[q]), itmax,
-                       !mach, c->status, c->iters + mask_slot(doms[q]));
-    if (!mach)
-      hipLaunchKernelGGL(k_newton_repair, dim3(1), dim3(1024), 0, c->stream, d, b, v, T, W_i,
-                         cp, ha, c->masks + mask_slot(doms[q]), itmax, eps, c->negT_rec,
-                         c->status, c->iters + mask_slot(doms[q]));
-  }
+  hipLaunchKernelGGL(k_force_probe, dim3(s.first[nd]), dim3(256), 0, c->stream, c->d, s, fill,
+                     forcesum, v, T, mach ? 1.0e-10 : 1.0e-5, c->masks);
+  newton_finish(c, doms, nd, v, W_i, T, cp, ha, mach);
   iz_prof_end(c, pk);
   IZ_CHECK(hipGetLastError());
   return IZEM_OK;
@@ -2393,8 +2510,8 @@ int iz_upd_prim_woT(izem_ctx *c, int dom, const double *v, const double *T, doub
 // upd_prim_var_dirichlet of a post-shock slip wall (its condition wrote the
 // first interior row: force_sumY and prim_inv_var there, module_BCs.f90:
 // 93-96, 131, 297-314), then upd_prim_var_ghost on the ghost slabs
+static const int ghost_faces[6] = {-1, 1, -2, 2, -3, 3};
 int iz_ghost_newton(izem_ctx *c, double *T, double *W_i, double *cp, double *ha, double *v) {
-  static const int faces[6] = {-1, 1, -2, 2, -3, 3};
   // the Dirichlet rows in face order (their force_sumY came with the fill)
   if (c->d.nscbc) {
     static const int row = 10;
@@ -2406,7 +2523,22 @@ int iz_ghost_newton(izem_ctx *c, double *T, double *W_i, double *cp, double *ha,
     int r = newton_domains(c, &row, 1, 0, v, W_i, T, cp, ha);
     if (r) return r;
   }
-  return newton_domains(c, faces, 2 * c->d.ndim, c->o.forcesum, v, W_i, T, cp, ha);
+  return newton_domains(c, ghost_faces, 2 * c->d.ndim, c->o.forcesum, v, W_i, T, cp, ha);
+}
+
+// comm_cons + upd_boundaries + the ghost cells' primitives, as a stage or a
+// reaction ends.  Without a Dirichlet face the conditions of all faces read
+// interior cells only, so the probe's pass over the ghost cells makes the
+// copies itself: three launches (2-D 128^2: 32 us a pass where the copies
+// and a probe, apply and repair per slab, 15 launches, took 92).
+int iz_fill_ghost_newton(izem_ctx *c, double *T, double *W_i, double *cp, double *ha, double *v,
+                         const double *dtp, double scale) {
+  if (c->d.wall || c->d.nscbc) {
+    int r = iz_comm_cons(c, v, IZ_NV, 1, T, W_i, cp, dtp, scale);
+    if (r) return r;
+    return iz_ghost_newton(c, T, W_i, cp, ha, v);
+  }
+  return newton_domains(c, ghost_faces, 2 * c->d.ndim, c->o.forcesum, v, W_i, T, cp, ha, 0, 1);
 }
 
 extern "C" int izem_upd_prim_var_ghost(izem_ctx *c, double *T, double *W_i, double *cp,
@@ -2465,7 +2597,7 @@ extern "C" int izem_rhs(izem_ctx *c, const double *dx_i, const double *dy_i, con
   hipLaunchKernelGGL(rhs_update_kernel(d), dim3(iz_blocks(n_interior(d), 256)), dim3(256), 0,
                      c->stream, d, 0, c->F[0], c->F[1], c->F[2], seams_of(c), c->o.vis, c->sf,
                      c->fd, dx_i, dy_i, dz_i,
-                     (const double *)nullptr, 0.0, 0.0, (const double *)nullptr,
+                     (const double *)nullptr, 0.0, 0.0, (double *)nullptr,
                      (double *)nullptr, f, 0, T, 0.0, (unsigned long long *)nullptr);
   IZ_CHECK(hipGetLastError());
   return IZEM_OK;
@@ -2479,33 +2611,23 @@ extern "C" int izem_rk3(izem_ctx *c, const double *dt, const double *dx_i, const
   static const double bk3[3] = {0.00, 0.75, 1.00 / 3.00};
   static const double ck3[3] = {1.00, 0.25, 2.00 / 3.00};
   const IzDims &d = c->d;
-  long ntot = (long)IZ_NV * d.nc;
-  int pc = iz_prof_begin(c, IZP_OTHER);
-  hipLaunchKernelGGL(k_copy, dim3(iz_blocks(ntot, 256)), dim3(256), 0, c->stream, v, c->v0, ntot);
-  iz_prof_end(c, pc);
   for (int ik = 0; ik < 3; ik++) {
     int r = stage_fluxes(c, dx_i, dy_i, dz_i, T, W_i, cp, ha, sensor, v);
     if (r) return r;
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, c->masks, 2 * IZ_NEG_MASKS);
     int pk = iz_prof_begin(c, IZP_RHS);
+    // the first stage keeps the state it starts from in v0
     hipLaunchKernelGGL(rhs_update_kernel(d), dim3(iz_blocks(n_interior(d), 256)), dim3(256), 0,
-                       c->stream, d, 1, c->F[0], c->F[1], c->F[2], seams_of(c), c->o.vis, c->sf,
-                       c->fd, dx_i, dy_i, dz_i, dt,
+                       c->stream, d, ik == 0 ? 2 : 1, c->F[0], c->F[1], c->F[2], seams_of(c),
+                       c->o.vis, c->sf, c->fd, dx_i, dy_i, dz_i, dt,
                        bk3[ik], ck3[ik], c->v0, v, (double *)nullptr, c->o.forcesum, T, 1.0e-5,
                        c->masks + 3);
     iz_prof_end(c, pk);
-    IzBox b0 = domain_box(d, 0);
+    static const int interior = 0;
     pk = iz_prof_begin(c, IZP_NEWTON);
-    hipLaunchKernelGGL(k_newton_apply, dim3(iz_blocks(box_count(b0), 256)), dim3(256), 0,
-                       c->stream, d, b0, v, T, W_i, cp, ha, c->masks + 3, 200, 1, c->status,
-                       c->iters + 3);
-    hipLaunchKernelGGL(k_newton_repair, dim3(1), dim3(1024), 0, c->stream, d, b0, v, T, W_i, cp,
-                       ha, c->masks + 3, 200, 1.0e-5, c->negT_rec, c->status, c->iters + 3);
+    newton_finish(c, &interior, 1, v, W_i, T, cp, ha, 0);
     iz_prof_end(c, pk);
     IZ_CHECK(hipGetLastError());
-    r = iz_comm_cons(c, v, IZ_NV, 1, T, W_i, cp, dt, 1.0);
-    if (r) return r;
-    r = iz_ghost_newton(c, T, W_i, cp, ha, v);
+    r = iz_fill_ghost_newton(c, T, W_i, cp, ha, v, dt, 1.0);
     if (r) return r;
   }
   return IZEM_OK;
@@ -2516,18 +2638,16 @@ extern "C" int izem_timestep(izem_ctx *c, const double *dx_i, const double *dy_i
                              const double *T, const double *v) {
   if (!c || !dx_i || !dy_i || !dz_i || !cp || !W_i || !T || !v) return IZEM_E_ARG;
   const IzDims &d = c->d;
-  unsigned nb = iz_blocks_capped(c, n_interior(d), 256, 16);
   int pk = iz_prof_begin(c, IZP_OTHER);
-  hipLaunchKernelGGL(k_dt_init, dim3(1), dim3(64), 0, c->stream, c->red);
-  hipLaunchKernelGGL(k_dt_conv, dim3(nb), dim3(256), 0, c->stream, d, v, T, W_i, cp, dx_i, dy_i,
-                     dz_i, c->red);
-  int visdt = c->o.vis && c->o.vis_dt;
-  if (visdt) {
+  const int visdt = c->o.vis && c->o.vis_dt;
+  if (visdt)
     hipLaunchKernelGGL(k_dt_visc, dim3(iz_blocks_capped(c, n_interior(d), 128, 32)), dim3(128),
                        0, c->stream, d, v, T, W_i, cp, dx_i, dy_i, dz_i, c->red);
-  }
+  else
+    hipLaunchKernelGGL(k_dt_conv, dim3(iz_blocks_capped(c, n_interior(d), 256, 16)), dim3(256), 0,
+                       c->stream, d, v, T, W_i, cp, dx_i, dy_i, dz_i, c->red);
   double rvd0_i = c->o.Sc / c->o.sqgmr, rlamcp0_i = c->o.Pr / c->o.sqgmr;
-  hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(1), 0, c->stream, c->red, c->o.CFL, c->o.CFLmin,
+  hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(64), 0, c->stream, c->red, c->o.CFL, c->o.CFLmin,
                      c->o.Fo, c->o.CPR, visdt, c->o.reaction, rvd0_i, rlamcp0_i, c->ts);
   iz_prof_end(c, pk);
   IZ_CHECK(hipGetLastError());

@@ -71,7 +71,7 @@ struct izem_ctx {
   // device words: Newton probe masks (blocking iterations [0..6] and
   // negative temperatures [8..14] per domain), status, iteration counts
   unsigned long long *masks;
-  int *negT_rec;  // cells recorded by the negative-temperature repair
+  int *negT_rec;  // cells recorded by the negative-temperature repair, per mask slot
   int *status;
   int *iters;
   double *red;  // timestep reductions [24]
@@ -107,6 +107,10 @@ static inline unsigned iz_blocks_capped(const izem_ctx *c, long n, int bs, int p
 
 // internal entry points across translation units
 int iz_ghost_newton(izem_ctx *ctx, double *T, double *W_i, double *cp, double *ha, double *v);
+// the faces' conditions and the ghost cells' primitives (iz_comm_cons with
+// bcs = 1, then iz_ghost_newton)
+int iz_fill_ghost_newton(izem_ctx *ctx, double *T, double *W_i, double *cp, double *ha, double *v,
+                         const double *dtp, double scale);
 // bcs = 1: the periodic exchange and the non-periodic faces' conditions
 // (comm_cons + upd_boundaries); 0: the exchange alone.  The characteristic
 // outflow needs the primitives T, W_i, cp and the step dt (scale x *dtp);

@@ -156,3 +156,21 @@ def test_set_bc_refuses(adi, thd):
             s.set_bc(bc)
     s.set_bc((0, 0, 1, 1, 0, 0))
     s.close()
+
+
+@pytest.mark.parametrize("kind,n,bc", CASES + [("2d", 7, (0,) * 6), ("3d", 9, (0,) * 6)])
+def test_stage_ghost_cells_are_the_fills(oracle, adi, thd, kind, n, bc):
+    """The ghost cells that an RK step leaves (filled by the pass that probes
+    them) are bit for bit those of the separate copies and force_sumY on the
+    same interior, on every face."""
+    import torch
+    box, run, s = _setup(oracle, adi, thd, kind, n, bc)
+    s.rk3(torch.tensor([0.05], dtype=torch.float64, device="cuda:0"))
+    s.sync()
+    assert s.status() == 0
+    w = s.v.clone()
+    assert s.lib.izem_comm_cons(s.ctx, C.c_void_p(w.data_ptr())) == 0
+    for dom in [q * e for q in range(1, box.ndim + 1) for e in (-1, 1)]:
+        assert s.lib.izem_force_sumY(s.ctx, dom, C.c_void_p(w.data_ptr())) == 0
+    s.sync()
+    assert torch.equal(w, s.v)
