@@ -7,12 +7,14 @@
 // tolerance).  Reference: saras13015/Phd devel-izem/src (file:line cited
 // per kernel).
 #include "flow_device.h"
+#include "iz_math.h"
 #include "izem_ctx.h"
 
 #include <stdlib.h>
 #include <string.h>
 
 __constant__ IzThd c_thd;
+__constant__ IzThx c_thx;
 
 // ===================================================================
 // Euler fluxes (euler_LLF_x/_y/_z: module_weno.f90:537-1044, 1055-1584,
@@ -1304,6 +1306,52 @@ __global__ void k_sensor_ducros(IzDims d, double treduc, const double *__restric
   if (ducloc > treduc) sensor[c] = 1;
 }
 
+// Block order of the kernels that take 7-point stencils along y and z of
+// tens of fields (k_visc_fused, k_rhs_update).  In storage order the seven
+// planes of a z stencil are tens of MB apart and every XCD's L2 (4 MB) sees
+// all of them, so each plane comes from beyond the L2 seven times.  Here the
+// interior is cut into bands of rows that are walked along z, and each
+// XCD (hardware blocks b, b + 8, ... share one) takes a contiguous part of
+// that walk: the planes that its blocks in flight need are a few rows wide
+// and mostly stay in its L2 (256^3: 24 GB fetched per k_rhs_update launch
+// against 38 in storage order).  Launches at 256^3 with bands of 8 / 16 / 32
+// rows, and one band: k_visc_fused 4.71 / 4.75 / 4.77 / 5.32 ms,
+// k_rhs_update 6.44 / 6.43 / 6.38 / 7.22 (6.57 in storage order); at 193 x
+// 129 x 97 0.81 / 0.79 / 0.79 / 0.82 and 1.05 / 0.99 / 0.98 / 1.08.
+struct IzBand {
+  int n;     // bands of about IZ_BAND_ROWS rows, one row more or less
+  int bpk;   // blocks per band and plane
+  long nb;   // blocks in all (bands x planes x bpk)
+};
+#ifndef IZ_BAND_ROWS
+#define IZ_BAND_ROWS 32
+#endif
+static IzBand band_of(const IzDims &d, int bs) {
+  IzBand b;
+  b.n = (d.ny + IZ_BAND_ROWS / 2) / IZ_BAND_ROWS;
+  if (b.n < 1) b.n = 1;
+  b.bpk = (int)iz_blocks((long)((d.ny + b.n - 1) / b.n) * d.nx, bs);
+  b.nb = (long)b.n * d.nz * b.bpk;
+  return b;
+}
+static unsigned band_grid(const IzBand &b) { return (unsigned)(((b.nb + 7) / 8) * 8); }
+// the cell of thread t of block blk (bs threads); false: none
+__device__ inline bool band_cell(const IzDims &d, const IzBand &b, unsigned blk, int bs, int t,
+                                 int &i, int &j, int &k) {
+  const long per = (b.nb + 7) / 8, L = (long)(blk % 8) * per + blk / 8;
+  if (L >= b.nb) return false;
+  const long bp = (long)b.bpk * d.nz;
+  const int band = (int)(L / bp), r = (int)(L - band * bp);
+  k = r / b.bpk;
+  const int idx = (r - k * b.bpk) * bs + t;
+  const int j0 = (int)((long)band * d.ny / b.n), rows = (int)((long)(band + 1) * d.ny / b.n) - j0;
+  if (idx >= rows * d.nx) return false;
+  const int q = idx / d.nx;
+  j = j0 + q;
+  i = idx - q * d.nx;
+  return true;
+}
+
 // ===================================================================
 // Viscous and species-diffusion fluxes: viscflux_xy / viscflux_xyz
 // (module_viscflux.f90:721-1135, 1660-2189), periodic faces.
@@ -1324,8 +1372,12 @@ __global__ void k_visc_prim(IzDims d, IzDomSet ds, const double *__restrict__ v,
 }
 
 // mixture-averaged transport of one cell (prim_vis_vars :989-1230)
+#if IZ_NG == 4
+// WENO7 keeps the reference's expressions: its weights lift differences in
+// the last bit of the transport to 2e-10 of the state over 66 iterations of a
+// shock tube, and its time is in the faces.
 __device__ inline void d_transport(double rho, double T, double W_i, const double *Xa, double *dm,
-                                   double &mu, double &ct, bool want_mu) {
+                                   double &mu, double &ct, bool want_mu, int sym) {
   const double eps = 1.0e-12;
   double Kl = 0.5 * 1.0e-5 / c_thd.laminf;
   double Ku = 1.0e-1 / c_thd.muinf;
@@ -1391,6 +1443,84 @@ __device__ inline void d_transport(double rho, double T, double W_i, const doubl
   }
   mu = mus;
 }
+#else
+// The exponentials are most of the work: D_kl is symmetric where the fits are
+// (sym, checked when the context is made), so 36 serve the 72 pairs, 1 / D_kl
+// is the exponential of the negated fit, and the ratios sqrt(eta_m / eta_l) of
+// Wilke's rule are products of exp(+-s / 2).  54 exponentials and 36
+// reciprocals per cell where the reference's expressions take 90, 162
+// divisions and 81 square roots (k_visc_fused at 160^3 1.53 -> 1.31 ms, of
+// which the rest is memory).
+__device__ inline void d_transport(double rho, double T, double W_i, const double *Xa, double *dm,
+                                   double &mu, double &ct, bool want_mu, int sym) {
+#pragma clang fp contract(on)
+  const double eps = 1.0e-12;
+  const double lt1 = d_log(T * c_thd.Tinf);
+  const double lt2 = lt1 * lt1;
+  const double lt3 = lt2 * lt1;
+  auto fit = [&](const double *cf) { return cf[0] + cf[1] * lt1 + cf[2] * lt2 + cf[3] * lt3; };
+  {
+    const double P = rho * T * W_i;
+    const double Kd = 1.0e-4 * c_thd.p0 / (c_thd.pinf * c_thd.Dinf);
+    double s[IZ_NRV], xe[IZ_NRV];
+#pragma unroll
+    for (int m = 0; m < IZ_NRV; m++) {
+      s[m] = 0.0;
+      xe[m] = Xa[m] + eps;
+    }
+#pragma unroll
+    for (int m = 0; m < IZ_NRV; m++)
+#pragma unroll
+      for (int l = m + 1; l < IZ_NRV; l++) {
+        const double e = d_exp(-fit(c_thd.CofD[m][l]));
+        double f = e;
+        if (!sym) f = d_exp(-fit(c_thd.CofD[l][m]));
+        s[m] += xe[l] * e;
+        s[l] += xe[m] * f;
+      }
+    // sum over the other species of xe W, from both ends (a difference
+    // from the total would cancel where one species is nearly all)
+    double up[IZ_NRV], dn = 0.0;
+    up[0] = 0.0;
+#pragma unroll
+    for (int m = 1; m < IZ_NRV; m++) up[m] = up[m - 1] + xe[m - 1] * c_thd.Wc[m - 1];
+    const double kp = Kd * W_i / P;
+#pragma unroll
+    for (int m = IZ_NRV - 1; m >= 0; m--) {
+      dm[m] = (up[m] + dn) * kp * d_rcp(s[m]);
+      dn += xe[m] * c_thd.Wc[m];
+    }
+  }
+  double w1 = 0.0, cc = 0.0;
+#pragma unroll
+  for (int l = 0; l < IZ_NRV; l++) {
+    const double c1 = d_exp(fit(c_thd.CofLam[l]));
+    cc += Xa[l] * d_rcp(c1);
+    w1 += Xa[l] * c1;
+  }
+  ct = (0.5 * 1.0e-5 / c_thd.laminf) * (1.0 / cc + w1);
+  mu = 0.0;
+  if (!want_mu) return;
+  double h[IZ_NRV], g[IZ_NRV];  // sqrt(eta) and its reciprocal
+#pragma unroll
+  for (int l = 0; l < IZ_NRV; l++) {
+    h[l] = d_exp(0.5 * fit(c_thd.CofEta[l]));
+    g[l] = d_rcp(h[l]);
+  }
+  double mus = 0.0;
+#pragma unroll
+  for (int m = 0; m < IZ_NRV; m++) {
+    double c4 = 0.0;
+#pragma unroll
+    for (int l = 0; l < IZ_NRV; l++) {
+      const double c3 = 1.0 + c_thd.wilke_c1[m][l] * (h[m] * g[l]);
+      c4 += c3 * c3 * c_thd.wilke_c2[m][l] * Xa[l];
+    }
+    mus += h[m] * h[m] * Xa[m] / c4;
+  }
+  mu = (1.0e-1 / c_thd.muinf) * mus;
+}
+#endif
 
 // Gradients and viscous fluxes in one pass (d?_fixed1 + the flux part of
 // viscflux_xy/_xyz, module_viscflux.f90:721-1135, 1660-2189).  The
@@ -1405,15 +1535,21 @@ __device__ inline void d_transport(double rho, double T, double W_i, const doubl
 // stored; the derivative slots of fd are not written.
 template <bool PHYS>
 __global__ void __attribute__((amdgpu_flat_work_group_size(128, 128), amdgpu_waves_per_eu(2)))
-k_visc_fused(IzDims d, IzDomSet ds, double sqgmr, double rvd0, double rlam0,
+k_visc_fused(IzDims d, IzBand bd, IzDomSet ds, int sym, double sqgmr, double rvd0, double rlam0,
              const double *__restrict__ v, const double *__restrict__ T,
              const double *__restrict__ W_i, const double *__restrict__ ha,
              const double *__restrict__ prim, const double *__restrict__ dx_i,
              const double *__restrict__ dy_i, const double *__restrict__ dz_i,
              double *__restrict__ fd, double *__restrict__ sf) {
-  long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  int i, j, k, dom;
-  if (!domset_cell(ds, tid, dom, i, j, k)) return;
+  // the interior in band order, then the ghost slabs
+  int i, j, k, dom = 0;
+  const unsigned nbi = (unsigned)(((bd.nb + 7) / 8) * 8);
+  if (blockIdx.x < nbi) {
+    if (!band_cell(d, bd, blockIdx.x, 128, threadIdx.x, i, j, k)) return;
+  } else {
+    const long tid = (long)(blockIdx.x - nbi) * 128 + threadIdx.x;
+    if (!domset_cell(ds, tid, dom, i, j, k)) return;
+  }
   const long nc = d.nc;
   const long c = iz_cidx(d, i, j, k);
   // derivative location: the periodic image of a ghost-slab cell
@@ -1429,7 +1565,7 @@ k_visc_fused(IzDims d, IzDomSet ds, double sqgmr, double rvd0, double rlam0,
 #pragma unroll
   for (int l = 0; l < IZ_NRV; l++) X[l] = prim[(3 + l) * nc + c];
   const double r0 = v[c], Wi = W_i[c];
-  d_transport(r0, T[c], Wi, X, dm, mu, ct, true);
+  d_transport(r0, T[c], Wi, X, dm, mu, ct, true, sym);
   double rho_i = 1.0 / r0;
   double uxs = v[nc + c] * rho_i, vys = v[2 * nc + c] * rho_i, wzs = v[3 * nc + c] * rho_i;
   double rmu = -sqgmr * mu;
@@ -1614,7 +1750,7 @@ __global__ void k_visc_apply(IzDims d, const double *__restrict__ sf,
 template <bool PHYS, bool SEAMS>
 __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256),
                                amdgpu_waves_per_eu(IZ_RHS_WAVES, IZ_RHS_WAVES)))
-k_rhs_update(IzDims d, int mode, const double *__restrict__ Fx, const double *__restrict__ Fy,
+k_rhs_update(IzDims d, IzBand bd, int mode, const double *__restrict__ Fx, const double *__restrict__ Fy,
              const double *__restrict__ Fz, IzSeams sm, int vis, const double *__restrict__ sf,
              const double *__restrict__ fd, const double *__restrict__ dx_i,
              const double *__restrict__ dy_i, const double *__restrict__ dz_i,
@@ -1624,13 +1760,9 @@ k_rhs_update(IzDims d, int mode, const double *__restrict__ Fx, const double *__
              unsigned long long *__restrict__ mask) {
   // one cell per thread (a grid-stride loop here was 2.7x slower: the
   // y/z face and viscous stencil neighbours lose their L2 reuse)
-  const long ncin = (long)d.nx * d.ny * d.nz;
   unsigned long long msk = 0ull, neg = 0ull;
-  const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (tid < ncin) {
-    int i = (int)(tid % d.nx);
-    long r = tid / d.nx;
-    int j = (int)(r % d.ny), k = (int)(r / d.ny);
+  int i, j, k;
+  if (band_cell(d, bd, blockIdx.x, 256, threadIdx.x, i, j, k)) {
     long c = iz_cidx(d, i, j, k);
     const long nfx = (long)(d.nx + 1) * d.ny * d.nz, nfy = (long)d.nx * (d.ny + 1) * d.nz,
                nfz = (long)d.nx * d.ny * (d.nz + 1);
@@ -1757,7 +1889,7 @@ __device__ inline double d_filter_delta2(const IzDims &d, const double *dx_i, co
 // minimum for every species lets k_dt_final pick that species' value, which
 // is the minimum the reference takes over that one species.
 __global__ void __attribute__((amdgpu_flat_work_group_size(128, 128), amdgpu_waves_per_eu(2, 2)))
-k_dt_visc(IzDims d, const double *__restrict__ v, const double *__restrict__ T,
+k_dt_visc(IzDims d, int sym, const double *__restrict__ v, const double *__restrict__ T,
                           const double *__restrict__ W_i, const double *__restrict__ cp,
                           const double *__restrict__ dx_i, const double *__restrict__ dy_i,
                           const double *__restrict__ dz_i, double *__restrict__ red) {
@@ -1777,7 +1909,7 @@ k_dt_visc(IzDims d, const double *__restrict__ v, const double *__restrict__ T,
 #pragma unroll
     for (int l = 0; l < IZ_NRV; l++)
       X[l] = v[(IZ_NIV + l) * d.nc + c] / (v[c] * W_i[c] * c_thd.Wc[l]);
-    d_transport(v[c], T[c], W_i[c], X, dm, mu, ct, false);
+    d_transport(v[c], T[c], W_i[c], X, dm, mu, ct, false, sym);
     const double d2 = d_filter_delta2(d, dx_i, dy_i, dz_i, i, j, k);
 #pragma unroll
     for (int l = 0; l < IZ_NRV; l++) {
@@ -1888,17 +2020,17 @@ static long box_count(const IzBox &b) {
   return (long)(b.i1 - b.i0 + 1) * (b.j1 - b.j0 + 1) * (b.k1 - b.k0 + 1);
 }
 static long n_interior(const IzDims &d) { return (long)d.nx * d.ny * d.nz; }
-// the interior and the 2 * ndim ghost slabs, in domain_select's order; the
+// the interior (where asked for) and the 2 * ndim ghost slabs, in domain_select's order; the
 // slabs of a direction with physical faces are left out (the viscous fluxes
 // there are never read: the derivative closures next to a physical face use
 // interior points only)
-static IzDomSet domain_set(const IzDims &d) {
+static IzDomSet domain_set(const IzDims &d, bool interior) {
   IzDomSet s{};
   s.n = 0;
   s.first[0] = 0;
   for (int dom = -d.ndim; dom <= d.ndim; dom++) {
     const int dir = (dom < 0 ? -dom : dom) - 1;
-    if (dom != 0 && ((d.phys >> (2 * dir)) & 3)) continue;
+    if (dom == 0 ? !interior : ((d.phys >> (2 * dir)) & 3)) continue;
     s.box[s.n] = domain_box(d, dom);
     s.dom[s.n] = dom;
     s.first[s.n + 1] = s.first[s.n] + box_count(s.box[s.n]);
@@ -1957,6 +2089,39 @@ extern "C" int izem_create(izem_ctx **out, const izem_grid *g, const double *thd
   if (hipMemcpyToSymbol(HIP_SYMBOL(c_thd), thd, sizeof(IzThd)) != hipSuccess) {
     izem_destroy(c);
     return IZEM_E_HIP;
+  }
+  {
+    const IzThd *t = (const IzThd *)thd;
+    c->dsym = 1;
+    for (int m = 0; m < IZ_NRV; m++)
+      for (int l = 0; l < m; l++)
+        if (memcmp(t->CofD[m][l], t->CofD[l][m], sizeof t->CofD[m][l])) c->dsym = 0;
+  }
+  {
+    // see IzThx
+    const IzThd *t = (const IzThd *)thd;
+    IzThx x;
+    x.tlo = t->Tpolymin[0];
+    x.thi = t->Tpolymax[0];
+    x.tlim = t->Tpolylim[0];
+    for (int l = 0; l < IZ_NRV; l++) {
+      if (t->Tpolymin[l] > x.tlo) x.tlo = t->Tpolymin[l];
+      if (t->Tpolymax[l] < x.thi) x.thi = t->Tpolymax[l];
+      if (t->Tpolylim[l] != x.tlim) x.thi = -1.0;  // no common range: never taken
+      for (int r = 0; r < 2; r++) {
+        const double *a = t->HeatCap[l][r];
+        const double f = t->Wc_i[l] / t->Tinf, g = t->gam2 * t->Wc_i[l];
+        for (int q = 0; q < 5; q++) {
+          x.h[r][l][q] = f * a[q] / (q + 1);
+          x.c[r][l][q] = g * a[q];
+        }
+        x.h[r][l][5] = f * a[5];
+      }
+    }
+    if (hipMemcpyToSymbol(HIP_SYMBOL(c_thx), &x, sizeof x) != hipSuccess) {
+      izem_destroy(c);
+      return IZEM_E_HIP;
+    }
   }
   c->nfaces[0] = (long)(d.nx + 1) * d.ny * d.nz;
   c->nfaces[1] = (long)d.nx * (d.ny + 1) * d.nz;
@@ -2211,7 +2376,7 @@ extern "C" int izem_wenorec(izem_ctx *c, int n, int js, const double *vp, const 
 }
 
 // k_rhs_update for the context's faces and decomposition
-typedef void (*IzRhsKernel)(IzDims, int, const double *, const double *, const double *, IzSeams,
+typedef void (*IzRhsKernel)(IzDims, IzBand, int, const double *, const double *, const double *, IzSeams,
                             int, const double *, const double *, const double *, const double *,
                             const double *, const double *, double, double, double *,
                             double *, double *, int, const double *, double,
@@ -2383,19 +2548,22 @@ static int visc_fluxes(izem_ctx *c, const double *dx_i, const double *dy_i, cons
   int pk = iz_prof_begin(c, IZP_VISC);
   // every domain's primitives are written before any domain's fluxes read
   // them (a slab cell's derivatives come from its interior image)
-  const IzDomSet ds = domain_set(d);
+  const IzDomSet ds = domain_set(d, true);
   const long ncell = ds.first[ds.n];
   hipLaunchKernelGGL(k_visc_prim, dim3(iz_blocks(ncell, 256)), dim3(256), 0, c->stream, d, ds, v,
                      W_i, c->prim);
   const double rvd0 = c->o.sqgmr / c->o.Sc, rlam0 = c->o.sqgmr * c->o.ggmopr;
+  const IzBand bd = band_of(d, 128);
+  const IzDomSet slabs = domain_set(d, false);
+  const dim3 grid(band_grid(bd) + iz_blocks(slabs.first[slabs.n], 128));
   if (d.phys)
-    hipLaunchKernelGGL(k_visc_fused<true>, dim3(iz_blocks(ncell, 128)), dim3(128), 0, c->stream,
-                       d, ds, c->o.sqgmr, rvd0, rlam0, v, T, W_i, ha, c->prim, dx_i, dy_i, dz_i,
-                       c->fd, c->sf);
+    hipLaunchKernelGGL(k_visc_fused<true>, grid, dim3(128), 0, c->stream, d, bd, slabs, c->dsym,
+                       c->o.sqgmr, rvd0, rlam0, v, T, W_i, ha, c->prim, dx_i, dy_i, dz_i, c->fd,
+                       c->sf);
   else
-    hipLaunchKernelGGL(k_visc_fused<false>, dim3(iz_blocks(ncell, 128)), dim3(128), 0, c->stream,
-                       d, ds, c->o.sqgmr, rvd0, rlam0, v, T, W_i, ha, c->prim, dx_i, dy_i, dz_i,
-                       c->fd, c->sf);
+    hipLaunchKernelGGL(k_visc_fused<false>, grid, dim3(128), 0, c->stream, d, bd, slabs, c->dsym,
+                       c->o.sqgmr, rvd0, rlam0, v, T, W_i, ha, c->prim, dx_i, dy_i, dz_i, c->fd,
+                       c->sf);
   iz_prof_end(c, pk);
   IZ_CHECK(hipGetLastError());
   return IZEM_OK;
@@ -2594,8 +2762,9 @@ extern "C" int izem_rhs(izem_ctx *c, const double *dx_i, const double *dy_i, con
   int r = stage_fluxes(c, dx_i, dy_i, dz_i, T, W_i, cp, ha, sensor, v);
   if (r) return r;
   const IzDims &d = c->d;
-  hipLaunchKernelGGL(rhs_update_kernel(d), dim3(iz_blocks(n_interior(d), 256)), dim3(256), 0,
-                     c->stream, d, 0, c->F[0], c->F[1], c->F[2], seams_of(c), c->o.vis, c->sf,
+  const IzBand bd = band_of(d, 256);
+  hipLaunchKernelGGL(rhs_update_kernel(d), dim3(band_grid(bd)), dim3(256), 0,
+                     c->stream, d, bd, 0, c->F[0], c->F[1], c->F[2], seams_of(c), c->o.vis, c->sf,
                      c->fd, dx_i, dy_i, dz_i,
                      (const double *)nullptr, 0.0, 0.0, (double *)nullptr,
                      (double *)nullptr, f, 0, T, 0.0, (unsigned long long *)nullptr);
@@ -2616,8 +2785,9 @@ extern "C" int izem_rk3(izem_ctx *c, const double *dt, const double *dx_i, const
     if (r) return r;
     int pk = iz_prof_begin(c, IZP_RHS);
     // the first stage keeps the state it starts from in v0
-    hipLaunchKernelGGL(rhs_update_kernel(d), dim3(iz_blocks(n_interior(d), 256)), dim3(256), 0,
-                       c->stream, d, ik == 0 ? 2 : 1, c->F[0], c->F[1], c->F[2], seams_of(c),
+    const IzBand bd = band_of(d, 256);
+    hipLaunchKernelGGL(rhs_update_kernel(d), dim3(band_grid(bd)), dim3(256), 0,
+                       c->stream, d, bd, ik == 0 ? 2 : 1, c->F[0], c->F[1], c->F[2], seams_of(c),
                        c->o.vis, c->sf, c->fd, dx_i, dy_i, dz_i, dt,
                        bk3[ik], ck3[ik], c->v0, v, (double *)nullptr, c->o.forcesum, T, 1.0e-5,
                        c->masks + 3);
@@ -2642,7 +2812,7 @@ extern "C" int izem_timestep(izem_ctx *c, const double *dx_i, const double *dy_i
   const int visdt = c->o.vis && c->o.vis_dt;
   if (visdt)
     hipLaunchKernelGGL(k_dt_visc, dim3(iz_blocks_capped(c, n_interior(d), 128, 32)), dim3(128),
-                       0, c->stream, d, v, T, W_i, cp, dx_i, dy_i, dz_i, c->red);
+                       0, c->stream, d, c->dsym, v, T, W_i, cp, dx_i, dy_i, dz_i, c->red);
   else
     hipLaunchKernelGGL(k_dt_conv, dim3(iz_blocks_capped(c, n_interior(d), 256, 16)), dim3(256), 0,
                        c->stream, d, v, T, W_i, cp, dx_i, dy_i, dz_i, c->red);

@@ -5,9 +5,11 @@
 // are the reference's own roundings, not a re-associated variant.
 #pragma once
 
+#include "iz_math.h"
 #include "izem_common.h"
 
 extern __constant__ IzThd c_thd;
+extern __constant__ IzThx c_thx;
 
 // Wmix_i_scalar: devel-izem/src/module_thermodynamics.f90:739-756
 __device__ inline double d_wmix_scalar(const double *Y) {
@@ -98,7 +100,7 @@ __device__ inline void d_ha_scalar(double temp, double *ha) {
 
 // newton (one cell): module_thermodynamics.f90:271-508.  Returns DF and the
 // cp / ha of this evaluation.
-__device__ inline double d_newton_cell(const double *vc, double T, double &cp_out,
+__device__ inline double d_newton_cell_ref(const double *vc, double T, double &cp_out,
                                        double *ha_out) {
   const double gam2_i = 1.0 / c_thd.gam2;
   double rho_i = 1.0 / vc[0];
@@ -122,6 +124,61 @@ __device__ inline double d_newton_cell(const double *vc, double T, double &cp_ou
   for (int is = 0; is < IZ_NRV; is++) wrk = wrk + Ya[is] * c_thd.Wc_i[is];
   cp_out = cp;
   return F / (wrk - cp * gam2_i);
+}
+
+#if IZ_NG == 3
+// species enthalpies and heat capacity of the mixture Y (cp of unit density)
+// at T where every species is inside its polynomials' range: Horner's form
+// with the factors folded in, 15 operations per species where the general
+// evaluation (four ranges per species, its own powers and factors) takes
+// about 150
+template <int RANGE>
+__device__ inline void d_thermo_range(double t, const double *Y, double &cp, double *h) {
+#pragma clang fp contract(on)
+  cp = 0.0;
+#pragma unroll
+  for (int l = 0; l < IZ_NRV; l++) {
+    const double *a = c_thx.h[RANGE][l], *b = c_thx.c[RANGE][l];
+    h[l] = ((((a[4] * t + a[3]) * t + a[2]) * t + a[1]) * t + a[0]) * t + a[5];
+    cp += Y[l] * ((((b[4] * t + b[3]) * t + b[2]) * t + b[1]) * t + b[0]);
+  }
+}
+// whether T is in that range, and the evaluation there
+__device__ inline bool d_thermo_in_range(double T) {
+  const double t = T * c_thd.Tinf;
+  return t >= c_thx.tlo && t < c_thx.thi;
+}
+__device__ inline void d_thermo(double T, const double *Y, double &cp, double *h) {
+  const double t = T * c_thd.Tinf;
+  if (t < c_thx.tlim) d_thermo_range<0>(t, Y, cp, h);
+  else d_thermo_range<1>(t, Y, cp, h);
+}
+#endif
+
+// the increment by the folded polynomials where they hold, else (and for
+// WENO7, whose runs follow the reference's roundings through shocks) in the
+// reference's expressions
+__device__ inline double d_newton_cell(const double *vc, double T, double &cp_out,
+                                       double *ha_out) {
+#if IZ_NG == 3
+  if (d_thermo_in_range(T)) {
+#pragma clang fp contract(on)
+    const double rho_i = 1.0 / vc[0];
+    double F = 0.5 * (vc[1] * vc[1] + vc[2] * vc[2] + vc[3] * vc[3]) * (rho_i * rho_i) -
+               vc[4] * rho_i;
+    double Ya[IZ_NRV], w = 0.0;
+#pragma unroll
+    for (int l = 0; l < IZ_NRV; l++) Ya[l] = vc[IZ_NIV + l] * rho_i;
+    d_thermo(T, Ya, cp_out, ha_out);
+#pragma unroll
+    for (int l = 0; l < IZ_NRV; l++) {
+      F += Ya[l] * (ha_out[l] - T * c_thd.Wc_i[l]);
+      w += Ya[l] * c_thd.Wc_i[l];
+    }
+    return F / (w - cp_out * (1.0 / c_thd.gam2));
+  }
+#endif
+  return d_newton_cell_ref(vc, T, cp_out, ha_out);
 }
 
 // ------------------------------------------------------------------ WENO

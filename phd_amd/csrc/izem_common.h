@@ -38,6 +38,17 @@ struct IzThd {
   double gam2, Tinf, p0, pinf, Dinf, laminf, muinf;
 };
 
+// The same enthalpy and heat-capacity polynomials with their factors folded
+// in, h[range][species] = Wc_i / Tinf (a0, a1/2, a2/3, a3/4, a4/5, a5) and
+// c[range][species] = gam2 Wc_i (a0..a4), and the temperatures (kelvin) at
+// which every species is inside its polynomials' range with a common middle
+// temperature (tlo <= t < thi; empty where there is none).
+struct IzThx {
+  double h[2][IZ_NRV][6];
+  double c[2][IZ_NRV][5];
+  double tlo, thi, tlim;
+};
+
 // phys: bit f set when face f (W, E, S, N, B, F) is a physical boundary
 // with extrapolated ghosts (bc_extrapolation) instead of a periodic one
 // np: ranks of the decomposed run whose shock-sensor views are reproduced,

@@ -67,6 +67,7 @@ struct izem_ctx {
   // fluxes, stresses + heat flux
   double *prim, *fd, *sf;
   int nderiv, nsf;
+  int dsym;  // the binary diffusion fits are symmetric (D_kl = D_lk bit for bit)
   double *v0;
   // device words: Newton probe masks (blocking iterations [0..6] and
   // negative temperatures [8..14] per domain), status, iteration counts

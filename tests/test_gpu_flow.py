@@ -341,3 +341,38 @@ def test_viscflux_with_fits_from_tranfit(oracle, adi, mech):
     s.sync()
     err = _relerr(f_gpu.cpu().numpy(), f_ref, box)
     assert err.max() <= TOL, err
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(11, 47, 9), (11, 48, 8), (13, 81, 9), (70, 97, 1)])
+def test_rhs_shifts_with_the_state(adi, thd, nx, ny, nz):
+    """The right-hand side of a periodic state rolled along y is the rolled
+    right-hand side, bit for bit (every cell's arithmetic is the same wherever
+    it lies): the blocks of the viscous and update kernels take the rows in
+    bands, whose edges fall elsewhere in the rolled state."""
+    import torch
+    from phd_amd.ics import Box, P_ATM, conserved_from_primitive, periodic_fill
+    ndim = 3 if nz > 1 else 2
+    box = Box(nx, ny, nz, 3, ndim, (nx * 4e-5, ny * 4e-5, nz * 4e-5))
+    rng = np.random.default_rng(8)
+    T = 900.0 + 300.0 * rng.random((nz, ny, nx))
+    Y = rng.random((9, nz, ny, nx))
+    Y /= Y.sum(axis=0)
+    u = 20.0 * rng.standard_normal((3, nz, ny, nx))
+    v0, T0 = conserved_from_primitive(box, adi, thd, T, P_ATM, Y, u)
+    out = []
+    for shift in (0, 17):
+        # the conserved state is rolled, not its recipe: the host's sums
+        # round by position
+        v, Tn = v0.copy(), T0.copy()
+        I = box.interior()
+        v[(slice(None),) + I] = np.roll(v0[(slice(None),) + I], shift, axis=-2)
+        Tn[I] = np.roll(T0[I], shift, axis=-2)
+        periodic_fill(box, Tn)
+        s = _gpu_solver(box)
+        s.load_state(v, Tn)
+        f = torch.zeros_like(s.v)
+        s.rhs(f)
+        s.sync()
+        out.append(f.cpu().numpy()[(slice(None),) + box.interior()])
+    assert np.all(np.isfinite(out[0])) and np.abs(out[0]).max() > 0.0
+    assert np.array_equal(np.roll(out[0], 17, axis=-2), out[1])
