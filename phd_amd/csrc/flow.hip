@@ -43,6 +43,9 @@ __constant__ IzThx c_thx;
 #ifndef IZ_EULER_WAVES
 #define IZ_EULER_WAVES 2
 #endif
+#ifndef IZ_EULER_FAST_WAVES
+#define IZ_EULER_FAST_WAVES 2
+#endif
 
 // per-cell part of the stencil presolve (module_weno.f90:634-650), with the
 // expressions of the per-stencil loop evaluated once per cell
@@ -69,19 +72,11 @@ __device__ inline void eu_stage_cell(const double *__restrict__ v, const double 
 // F^ of one face from its IZ_S staged stencil cells: Q(q, st) is staged
 // quantity q of stencil point st (st = ng - 1 is i_l, st = ng is i_r); cL, cR are
 // the HBM indices of i_l, i_r (for h_k); F^ goes to F[m * nfaces + fidx].
-// FAST = false keeps the reference's dense projections (w = el . U, g =
-// el . F over all 14 columns, in its summation order: bit parity with the
-// oracle).  FAST = true uses the structure of el: with
-//   S = -b1 U_0 + b2 (u . m) - b2 E - b2 sum_l psi_l U_l   (and the same of F)
-// every row but the tangential ones is S-plus-few-terms: row 1 is U_0 + S,
-// rows 0 and 2 are -S/2 -+ (u_n U_0 - U_n) / (2 c), row 5 is
-// -(1 + xi) / b2 S - sum_l psi_l U_l, and species row 6 + s is U_{5+s} + Y_s S.
-// The characteristic projections then cost about a tenth of the dense ones;
-// results differ from the dense order by rounding only.
-// SITE gives every calling kernel an instantiation of its own: with a single
+// The reference's dense projections (w = el . U, g = el . F over all 14
+// columns, in its summation order: bit parity with the oracle).  SITE gives every calling kernel an instantiation of its own: with a single
 // caller each is inlined as before, where a shared one is left out of line.
-template <int DIR, int QS, int SS, bool FAST, int SITE>
-__device__ inline void eu_face(const double *tile, int off, bool js,
+template <int DIR, int QS, int SS, int SITE>
+__device__ inline void eu_face_ref(const double *tile, int off, bool js,
                                const double *__restrict__ ha, long nc, long cL, long cR,
                                double *__restrict__ F, long nfaces, long fidx) {
   // staged quantity q of stencil point st
@@ -150,33 +145,6 @@ __device__ inline void eu_face(const double *tile, int off, bool js,
   const double un_c = uc[cn - 1];
   const double hb2 = 0.5 * b2;
 
-  // FAST: per stencil point, S of U and of F, sum_l psi_l U_l and its F
-  // counterpart, and u_n U_0 - U_n with its F counterpart
-  double sw[IZ_S], sg[IZ_S], pw[IZ_S], pg[IZ_S], dw[IZ_S], dg[IZ_S];
-  if constexpr (FAST) {
-#pragma unroll
-    for (int st = 0; st < IZ_S; st++) {
-      const double u = Q(IZ_QU, st), p = Q(IZ_QP, st);
-      const double u0 = Q(0, st), un = Q(cn, st), u4 = Q(4, st);
-      double aw = -b1 * u0 - b2 * u4, ag = -b1 * un - b2 * (u * (u4 + p));
-#pragma unroll
-      for (int c = 1; c <= 3; c++) {
-        const double vc = Q(c, st);
-        aw = aw + b2 * uc[c - 1] * vc;
-        ag = ag + b2 * uc[c - 1] * ((c == cn) ? vc * u + p : vc * u);
-      }
-      double ps = 0.0;
-#pragma unroll
-      for (int l = 0; l < IZ_NRV; l++) ps = ps + psi[l] * Q(IZ_NIV + l, st);
-      pw[st] = ps;
-      pg[st] = ps * u;
-      sw[st] = aw - b2 * ps;
-      sg[st] = ag - b2 * pg[st];
-      dw[st] = un_c * u0 - un;
-      dg[st] = un_c * un - (un * u + p);
-    }
-  }
-
   double ghat[IZ_NV];
 #pragma unroll 1
   for (int m = 0; m < IZ_NV; m++) {
@@ -189,9 +157,7 @@ __device__ inline void eu_face(const double *tile, int off, bool js,
     // row m of the left eigenvector matrix (module_weno.f90:775-874)
     double e[IZ_NV];
     double lam;
-    if (FAST) {
-      lam = (m == 0) ? lmax0 : (m == 2 ? lmax2 : lmax1);
-    } else if (m == 0) {
+    if (m == 0) {
       e[0] = 0.5 * (b1 + un_c * cs_c_i);
 #pragma unroll
       for (int c = 1; c <= 3; c++)
@@ -245,27 +211,7 @@ __device__ inline void eu_face(const double *tile, int off, bool js,
     for (int st = 0; st < IZ_S; st++) {
       const double u = Qm(IZ_QU, st), p = Qm(IZ_QP, st);
       double wc, gc;
-      if (FAST && m != 3 && m != 4) {
-        const double hc = 0.5 * cs_c_i;
-        if (m == 0) {
-          wc = -0.5 * sw[st] + hc * dw[st];
-          gc = -0.5 * sg[st] + hc * dg[st];
-        } else if (m == 1) {
-          wc = Qm(0, st) + sw[st];
-          gc = Qm(cn, st) + sg[st];
-        } else if (m == 2) {
-          wc = -0.5 * sw[st] - hc * dw[st];
-          gc = -0.5 * sg[st] - hc * dg[st];
-        } else if (m == 5) {
-          const double k = (1.0 + xi) / b2;
-          wc = -k * sw[st] - pw[st];
-          gc = -k * sg[st] - pg[st];
-        } else {
-          const double y = Yc[m - 6], vs = Qm(IZ_NIV + m - 6, st);
-          wc = vs + y * sw[st];
-          gc = vs * u + y * sg[st];
-        }
-      } else if (m == 3 || m == 4) {
+      if (m == 3 || m == 4) {
         const int tc = (m == 3) ? t1 : t2;
         const double et0 = -uc[tc - 1];
         const double v0 = Qm(0, st), vt = Qm(tc, st);
@@ -339,6 +285,204 @@ __device__ inline void eu_face(const double *tile, int off, bool js,
   }
 }
 
+// The same face through the structure of el (izem_flux_mode 1): with
+//   S = -b1 U_0 + b2 (u . m) - b2 E - b2 sum_l psi_l U_l   (and the same of F)
+// every row but the tangential ones is S-plus-few-terms: row 1 is U_0 + S,
+// rows 0 and 2 are -S/2 -+ (u_n U_0 - U_n) / (2 c), row 5 is
+// -(1 + xi) / b2 S - sum_l psi_l U_l, and species row 6 + s is U_{5+s} + Y_s S.
+// The characteristic projections then cost about a tenth of the dense ones.
+// FMA contraction, the folded thermodynamic polynomials and one reciprocal
+// per reconstructed field; fields are taken one after the other and enter F^
+// as they come, so that few of them are live at a time: 204 VGPRs, two waves
+// per SIMD (three or four spill: 3.6 and 4.3 ms).  The kernel is bound by FP64
+// issue: 4.5 -> 2.0 (x), 2.2 (y, z) ms per launch at 256^3.  Results differ from the dense order by rounding only.
+template <int DIR, int QS, int SS, int SITE>
+__device__ inline void eu_face_fast(const double *tile, int off, bool js,
+                                    const double *__restrict__ ha, long nc, long cL, long cR,
+                                    double *__restrict__ F, long nfaces, long fidx) {
+#pragma clang fp contract(on)
+  // The stencil is read from LDS again by every field: an opaque copy of the
+  // offset, taken anew by fresh(), keeps the compiler from holding the values
+  // of an earlier reading in registers (which spills), and the scheduling
+  // barrier from moving a field's reads ahead of the fields before it.
+  int offm = off;
+  auto fresh = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+v"(offm));
+  };
+  auto Q = [&](int q, int st) { return tile[offm + q * QS + st * SS]; };
+  constexpr int cn = 1 + DIR;             // normal momentum column
+  constexpr int t1 = (DIR == 0) ? 2 : 1;  // tangential columns (el rows 4, 5)
+  constexpr int t2 = (DIR == 2) ? 2 : 3;
+  // Roe average of i_l and i_r (module_weno.f90:654-667, 726-735)
+  double uc[3], Yc[IZ_NRV], ht_c, et_c;
+  {
+    constexpr int SL = IZ_NG - 1, SR = IZ_NG;  // stencil points of i_l, i_r
+    const double riL = 1.0 / Q(0, SL), riR = 1.0 / Q(0, SR);
+    const double r = sqrt(Q(0, SR) * riL);
+    const double r1 = 1.0 / (r + 1.0), r2 = r * r1;
+    double htL = 0.0, htR = 0.0, kL = 0.0, kR = 0.0;
+#pragma unroll
+    for (int l = 0; l < IZ_NRV; l++) {
+      const double yL = Q(IZ_NIV + l, SL) * riL, yR = Q(IZ_NIV + l, SR) * riR;
+      htL += ha[l * nc + cL] * yL;
+      htR += ha[l * nc + cR] * yR;
+      Yc[l] = r2 * yR + r1 * yL;
+    }
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      const double uL = Q(1 + q, SL) * riL, uR = Q(1 + q, SR) * riR;
+      kL += uL * uL;
+      kR += uR * uR;
+      uc[q] = r2 * uR + r1 * uL;
+    }
+    ht_c = r2 * (htR + 0.5 * kR) + r1 * (htL + 0.5 * kL);
+    et_c = r2 * (Q(4, SR) * riR) + r1 * (Q(4, SL) * riL);
+  }
+  // EOS-compatible average state (module_weno.f90:750-761)
+  double W_i_c = 0.0;
+#pragma unroll
+  for (int l = 0; l < IZ_NRV; l++) W_i_c += Yc[l] * c_thd.Wc_i[l];
+  const double T_c = (ht_c - et_c) / W_i_c;
+  double cp_c, psi[IZ_NRV];
+#if IZ_NG == 3
+  if (d_thermo_in_range(T_c)) {
+    d_thermo(T_c, Yc, cp_c, psi);
+  } else
+#endif
+  {
+    cp_c = d_cp_scalar(T_c, Yc);
+    d_ha_scalar(T_c, psi);
+  }
+  const double gam_c = 1.0 / (1.0 - c_thd.gam2 * W_i_c / cp_c);
+  const double cs_c_2 = gam_c * T_c * W_i_c;
+  const double cs_c = sqrt(cs_c_2);
+  {
+    const double wrk = (gam_c / (gam_c - 1.0)) * T_c;
+#pragma unroll
+    for (int l = 0; l < IZ_NRV; l++) psi[l] = wrk * c_thd.Wc_i[l] - psi[l];
+  }
+  const double hc = 0.5 / cs_c;
+  const double q = 0.5 * (uc[0] * uc[0] + uc[1] * uc[1] + uc[2] * uc[2]);
+  const double b2 = (gam_c - 1.0) / cs_c_2;
+  const double b1 = b2 * q;
+  const double un_c = uc[cn - 1];
+  fresh();
+  double lmax0 = 0.0, lmax1 = 0.0, lmax2 = 0.0;
+  double u[IZ_S], sw[IZ_S], sg[IZ_S];
+  double gp[IZ_S], gm[IZ_S], g0, g1, g2, g5;
+  {
+    // per stencil point, S and sum_l psi_l U_l of U and of F, and u_n U_0 -
+    // U_n with its F counterpart
+    double pw[IZ_S], dw[IZ_S], dg[IZ_S];
+#pragma unroll
+    for (int st = 0; st < IZ_S; st++) {
+      u[st] = Q(IZ_QU, st);
+      const double cs = Q(IZ_QC, st), p = Q(IZ_QP, st);
+      lmax0 = fmax(fabs(u[st] - cs), lmax0);
+      lmax1 = fmax(fabs(u[st]), lmax1);
+      lmax2 = fmax(fabs(u[st] + cs), lmax2);
+      const double u0 = Q(0, st), un = Q(cn, st), u4 = Q(4, st);
+      double m = uc[0] * Q(1, st) + uc[1] * Q(2, st) + uc[2] * Q(3, st) - u4;
+      double ps = 0.0;
+#pragma unroll
+      for (int l = 0; l < IZ_NRV; l++) ps += psi[l] * Q(IZ_NIV + l, st);
+      pw[st] = ps;
+      // F = u U + p (e_n + u e_4), and U_n = u U_0
+      const double s0 = b2 * (m - ps);
+      sw[st] = s0 - b1 * u0;
+      sg[st] = u[st] * s0 + (b2 * (p * (un_c - u[st])) - b1 * un);
+      dw[st] = un_c * u0 - un;
+      dg[st] = un_c * un - (un * u[st] + p);
+    }
+    // rows 0 and 2
+#pragma unroll
+    for (int st = 0; st < IZ_S; st++) {
+      const double w = hc * dw[st] - 0.5 * sw[st], g = hc * dg[st] - 0.5 * sg[st];
+      gp[st] = g + lmax0 * w;
+      gm[st] = g - lmax0 * w;
+    }
+    g0 = d_weno_face_fused(js, gp, gm);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int st = 0; st < IZ_S; st++) {
+      const double w = -hc * dw[st] - 0.5 * sw[st], g = -hc * dg[st] - 0.5 * sg[st];
+      gp[st] = g + lmax2 * w;
+      gm[st] = g - lmax2 * w;
+    }
+    g2 = d_weno_face_fused(js, gp, gm);
+    __builtin_amdgcn_sched_barrier(0);
+    // row 5: -(1 + xi) / b2 with xi = b1 - b2 ht
+    const double k = (1.0 + (b1 - b2 * ht_c)) / b2;
+#pragma unroll
+    for (int st = 0; st < IZ_S; st++) {
+      const double w = -k * sw[st] - pw[st], g = -k * sg[st] - pw[st] * u[st];
+      gp[st] = g + lmax1 * w;
+      gm[st] = g - lmax1 * w;
+    }
+    g5 = d_weno_face_fused(js, gp, gm);
+  }
+  // row 1
+  fresh();
+#pragma unroll
+  for (int st = 0; st < IZ_S; st++) {
+    const double w = Q(0, st) + sw[st], g = Q(cn, st) + sg[st];
+    gp[st] = g + lmax1 * w;
+    gm[st] = g - lmax1 * w;
+  }
+  g1 = d_weno_face_fused(js, gp, gm);
+  const double g02 = g0 + g2, gs = g02 + g1, gd = cs_c * (g2 - g0);
+  F[fidx] = gs;
+  F[(long)cn * nfaces + fidx] = un_c * gs + gd;
+  double f4 = ht_c * g02 + un_c * gd + q * g1 + g5;
+  // the tangential rows: U_t - u_t U_0, carried by u
+#pragma unroll
+  for (int tt = 0; tt < 2; tt++) {
+    const int tc = tt == 0 ? t1 : t2;
+    const double ut = uc[tc - 1];
+    fresh();
+#pragma unroll
+    for (int st = 0; st < IZ_S; st++) {
+      const double w = Q(tc, st) - ut * Q(0, st), g = u[st] * w;
+      gp[st] = g + lmax1 * w;
+      gm[st] = g - lmax1 * w;
+    }
+    const double gt = d_weno_face_fused(js, gp, gm);
+    F[(long)tc * nfaces + fidx] = ut * gs + gt;
+    f4 += ut * gt;
+  }
+  F[4 * nfaces + fidx] = f4;
+  // species rows; the last species from row 5 and the others
+  const double wrk = -1.0 / psi[IZ_NRV - 1];
+  double last = g5;
+#pragma unroll
+  for (int l = 0; l < IZ_NRV - 1; l++) {
+    const double y = Yc[l];
+    fresh();
+#pragma unroll
+    for (int st = 0; st < IZ_S; st++) {
+      const double vs = Q(IZ_NIV + l, st);
+      const double w = vs + y * sw[st], g = vs * u[st] + y * sg[st];
+      gp[st] = g + lmax1 * w;
+      gm[st] = g - lmax1 * w;
+    }
+    const double gl = d_weno_face_fused(js, gp, gm);
+    F[(long)(IZ_NIV + l) * nfaces + fidx] = y * g02 + gl;
+    last += psi[l] * gl;
+  }
+  F[(long)(IZ_NV - 1) * nfaces + fidx] = Yc[IZ_NRV - 1] * g02 + wrk * last;
+}
+
+template <int DIR, int QS, int SS, bool FAST, int SITE>
+__device__ inline void eu_face(const double *tile, int off, bool js,
+                               const double *__restrict__ ha, long nc, long cL, long cR,
+                               double *__restrict__ F, long nfaces, long fidx) {
+  if constexpr (FAST)
+    eu_face_fast<DIR, QS, SS, SITE>(tile, off, js, ha, nc, cL, cR, F, nfaces, fidx);
+  else
+    eu_face_ref<DIR, QS, SS, SITE>(tile, off, js, ha, nc, cL, cR, F, nfaces, fidx);
+}
+
 // LDS bytes of one block of k_euler_faces<DIR>; tile0 = cells staged per
 // wave for x (64 + IZ_S - 1, and IZ_S - 1 more per row boundary that 64
 // consecutive faces can cross)
@@ -378,7 +522,7 @@ __device__ inline int eu_flags_view(const uint8_t *tsn, int stride, int il, int 
 // the flag view of the rank of its right cell
 template <int DIR, bool FAST, bool RANKS>
 __global__ void __attribute__((amdgpu_flat_work_group_size(IZ_EU_BLOCK, IZ_EU_BLOCK),
-                               amdgpu_waves_per_eu(IZ_EULER_WAVES, IZ_EULER_WAVES)))
+                               amdgpu_waves_per_eu(FAST ? IZ_EULER_FAST_WAVES : IZ_EULER_WAVES)))
 k_euler_faces(IzDims d, const double *__restrict__ v, const double *__restrict__ T,
               const double *__restrict__ W_i, const double *__restrict__ cp,
               const double *__restrict__ ha, const uint8_t *__restrict__ sensor, int weno_avg,
