@@ -225,3 +225,40 @@ def test_surrogate_trains_conserves_and_gains(mech, thd, adi):
     assert res["max_abs_dT_K"] <= 2.0
     assert res["fallback_rate"] < 1.0
     assert res["surrogate_cells_per_s"] > res["vode_cells_per_s"]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K,pad", [(1, 1, 1, 0), (127, 63, 31, 1), (128, 64, 64, 0),
+                                       (129, 65, 65, 3), (257, 131, 96, 4), (64, 6, 200, 8)])
+def test_gemm_tile_edges(mech, ta, tb, M, N, K, pad):
+    # tile edges, rows the wide loads and stores may not be used on (pad), and
+    # that nothing beyond the N columns is written
+    import torch
+    from oracle.mlp_oracle import gelu
+    s = _solver(mech)
+    rng = np.random.default_rng(M + N + K)
+    A = rng.normal(size=(M, K)); B = rng.normal(size=(K, N))
+    Ab, Af = _bf16_bits(A); Bb, Bf = _bf16_bits(B)
+
+    def dev(x):
+        st = np.zeros((x.shape[0], x.shape[1] + pad), x.dtype)
+        st[:, :x.shape[1]] = x
+        return torch.tensor(st, device="cuda"), st.shape[1]
+    dA, lda = dev(Ab if ta == 0 else np.ascontiguousarray(Ab.T))
+    dB, ldb = dev(np.ascontiguousarray(Bb.T) if tb == 0 else Bb)
+    bias = rng.normal(size=N).astype(np.float32)
+    dbias = torch.tensor(bias, device="cuda")
+    ldc = N + pad
+    Cf = torch.full((M, ldc), 7.0, dtype=torch.float32, device="cuda")
+    Cb = torch.full((M, ldc), 7, dtype=torch.int16, device="cuda")
+    assert s.lib.izem_mlp_gemm(s.ctx, ta, tb, 1, M, N, K, _p(dA), lda, _p(dB), ldb, _p(dbias),
+                               None, 0, _p(Cf), ldc, _p(Cb), ldc) == 0
+    s.sync()
+    z = Af @ Bf + bias
+    cf, cb = Cf.cpu().numpy(), Cb.cpu().numpy()
+    # FP32 sums of K products and a bias: K + 1 roundings of the largest partial sum
+    tol = (K + 2) * 2.0 ** -24 * (np.abs(Af) @ np.abs(Bf) + np.abs(bias))
+    assert np.all(np.abs(cf[:, :N] - z) <= tol)
+    act = (np.ascontiguousarray(cb[:, :N]).view(np.uint16).astype(np.uint32) << 16).view(np.float32)
+    assert np.all(np.abs(act - gelu(z)) <= 2 ** -8 * np.abs(gelu(z)) + 1.2 * tol + 7e-7)
+    assert np.all(cf[:, N:] == 7.0) and np.all(cb[:, N:] == 7)
