@@ -12,6 +12,8 @@
 
 #include <stdlib.h>
 #include <string.h>
+#include <type_traits>
+#include <utility>
 
 __constant__ IzThd c_thd;
 __constant__ IzThx c_thx;
@@ -69,12 +71,33 @@ __device__ inline void eu_stage_cell(const double *__restrict__ v, const double 
   dst[IZ_QC * fs] = cs;
 }
 
+// rows of the left eigenvector matrix projected together (eu_face_ref):
+// the sums of four fit the registers of two waves per SIMD with six stencil
+// points (244 VGPRs), those of two with eight
+#define IZ_EU_GROUP (IZ_NG == 3 ? 4 : 2)
+template <int M>
+using EuRow = std::integral_constant<int, M>;
+template <int M0, class F, int... I>
+__device__ inline void eu_row_group(F &f, std::integer_sequence<int, I...>) {
+  f(EuRow<M0 + I>{}...);
+}
+// f on the rows M0 .. IZ_NV - 1, a group at a time
+template <int M0, class F>
+__device__ inline void eu_species_rows(F &f) {
+  if constexpr (M0 < IZ_NV) {
+    constexpr int G = IZ_NV - M0 < IZ_EU_GROUP ? IZ_NV - M0 : IZ_EU_GROUP;
+    eu_row_group<M0>(f, std::make_integer_sequence<int, G>{});
+    eu_species_rows<M0 + G>(f);
+  }
+}
+
 // F^ of one face from its IZ_S staged stencil cells: Q(q, st) is staged
 // quantity q of stencil point st (st = ng - 1 is i_l, st = ng is i_r); cL, cR are
 // the HBM indices of i_l, i_r (for h_k); F^ goes to F[m * nfaces + fidx].
 // The reference's dense projections (w = el . U, g = el . F over all 14
-// columns, in its summation order: bit parity with the oracle).  SITE gives every calling kernel an instantiation of its own: with a single
-// caller each is inlined as before, where a shared one is left out of line.
+// columns, in its summation order: bit parity with the oracle).  SITE gives every calling
+// kernel an instantiation of its own: with a single caller each is inlined
+// as before, where a shared one is left out of line.
 template <int DIR, int QS, int SS, int SITE>
 __device__ inline void eu_face_ref(const double *tile, int off, bool js,
                                const double *__restrict__ ha, long nc, long cL, long cR,
@@ -145,101 +168,121 @@ __device__ inline void eu_face_ref(const double *tile, int off, bool js,
   const double un_c = uc[cn - 1];
   const double hb2 = 0.5 * b2;
 
+  // entry (m, c) of the left eigenvector matrix (module_weno.f90:775-874),
+  // rows 3 and 4 excepted (two nonzeros, below)
+  auto el = [&](auto mc, int c) -> double {
+    constexpr int m = decltype(mc)::value;
+    if constexpr (m == 0 || m == 2) {
+      if (c == 0) return m == 0 ? 0.5 * (b1 + un_c * cs_c_i) : 0.5 * (b1 - un_c * cs_c_i);
+      if (c == cn)
+        return m == 0 ? -0.5 * (b2 * uc[c - 1] + cs_c_i) : -0.5 * (b2 * uc[c - 1] - cs_c_i);
+      if (c <= 3) return -0.5 * (b2 * uc[c - 1]);
+      if (c == 4) return 0.5 * b2;
+      return hb2 * psi[c - IZ_NIV];
+    } else if constexpr (m == 1) {
+      if (c == 0) return 1.0 - b1;
+      if (c <= 3) return b2 * uc[c - 1];
+      if (c == 4) return -b2;
+      const double a = hb2 * psi[c - IZ_NIV];
+      return -a - a;
+    } else if constexpr (m == 5) {
+      const double opx = (1 + xi);
+      if (c == 0) return opx * q;
+      if (c <= 3) return -opx * uc[c - 1];
+      if (c == 4) return opx;
+      return xi * psi[c - IZ_NIV];
+    } else {
+      const double y = Yc[m - 6];
+      if (c == 0) return -b1 * y;
+      if (c <= 3) return b2 * uc[c - 1] * y;
+      if (c == 4) return -b2 * y;
+      const double x = -((b2 * y) * psi[c - IZ_NIV]);
+      return c - IZ_NIV == m - 6 ? x + 1.0 : x;
+    }
+  };
   double ghat[IZ_NV];
-#pragma unroll 1
-  for (int m = 0; m < IZ_NV; m++) {
-    // the stencil is re-read from LDS for every characteristic field: an
-    // opaque copy of the offset keeps the compiler from hoisting the 96
-    // loop-invariant reads into registers (which spills at two waves/SIMD)
+  // Characteristic fields M of one group: w = el . U and g = el . F of every
+  // stencil point, summed column by column (each sum in the reference's
+  // order).  A staged value and its flux are read and formed once for the
+  // group, so the LDS, which held this kernel up with one row at a time, is
+  // read a group's size less often: 1.68 -> 1.35 (x), 1.82 -> 1.40 (y, z) ms
+  // per launch at 160^3; groups of two 1.47 and 1.54.  The opaque offset keeps
+  // the compiler from carrying a group's reads to the next one in registers.
+  auto project = [&](auto... M) {
+    constexpr int G = sizeof...(M);
     int offm = off;
     asm volatile("" : "+v"(offm));
     auto Qm = [&](int q, int st) { return tile[offm + q * QS + st * SS]; };
-    // row m of the left eigenvector matrix (module_weno.f90:775-874)
-    double e[IZ_NV];
-    double lam;
-    if (m == 0) {
-      e[0] = 0.5 * (b1 + un_c * cs_c_i);
+    double w[G][IZ_S], g[G][IZ_S], u[IZ_S], p[IZ_S];
 #pragma unroll
-      for (int c = 1; c <= 3; c++)
-        e[c] = (c == cn) ? -0.5 * (b2 * uc[c - 1] + cs_c_i) : -0.5 * (b2 * uc[c - 1]);
-      e[4] = 0.5 * b2;
-#pragma unroll
-      for (int l = 0; l < IZ_NRV; l++) e[5 + l] = hb2 * psi[l];
-      lam = lmax0;
-    } else if (m == 1) {
-      e[0] = 1.0 - b1;
-      e[1] = b2 * ux_c; e[2] = b2 * vy_c; e[3] = b2 * wz_c;
-      e[4] = -b2;
-#pragma unroll
-      for (int l = 0; l < IZ_NRV; l++) { const double a = hb2 * psi[l]; e[5 + l] = -a - a; }
-      lam = lmax1;
-    } else if (m == 2) {
-      e[0] = 0.5 * (b1 - un_c * cs_c_i);
-#pragma unroll
-      for (int c = 1; c <= 3; c++)
-        e[c] = (c == cn) ? -0.5 * (b2 * uc[c - 1] - cs_c_i) : -0.5 * (b2 * uc[c - 1]);
-      e[4] = 0.5 * b2;
-#pragma unroll
-      for (int l = 0; l < IZ_NRV; l++) e[5 + l] = hb2 * psi[l];
-      lam = lmax2;
-    } else if (m == 5) {
-      const double opx = (1 + xi);
-      e[0] = opx * q;
-      e[1] = -opx * ux_c; e[2] = -opx * vy_c; e[3] = -opx * wz_c;
-      e[4] = opx;
-#pragma unroll
-      for (int l = 0; l < IZ_NRV; l++) e[5 + l] = xi * psi[l];
-      lam = lmax1;
-    } else if (m >= 6) {
-      const int s1 = m - 6;
-      const double y = Yc[s1];
-      e[0] = -b1 * y;
-      e[1] = b2 * ux_c * y; e[2] = b2 * vy_c * y; e[3] = b2 * wz_c * y;
-      e[4] = -b2 * y;
-      const double by = b2 * y;
-#pragma unroll
-      for (int l = 0; l < IZ_NRV; l++) {
-        const double x = -(by * psi[l]);
-        e[5 + l] = (l == s1) ? x + 1.0 : x;
-      }
-      lam = lmax1;
-    } else {
-      lam = lmax1;  // m = 3, 4: two nonzeros, handled below
+    for (int st = 0; st < IZ_S; st++) {
+      u[st] = Qm(IZ_QU, st);
+      p[st] = Qm(IZ_QP, st);
     }
+#pragma unroll
+    for (int c = 0; c < IZ_NV; c++) {
+      const double e[G] = {el(M, c)...};
+#pragma unroll
+      for (int st = 0; st < IZ_S; st++) {
+        const double v = Qm(c, st);
+        double f;
+        if (c == 0) f = Qm(cn, st);
+        else if (c == cn) f = v * u[st] + p[st];
+        else if (c == 4) f = u[st] * (v + p[st]);
+        else f = v * u[st];
+#pragma unroll
+        for (int k = 0; k < G; k++) {
+          w[k][st] = c == 0 ? e[k] * v : w[k][st] + e[k] * v;
+          g[k][st] = c == 0 ? e[k] * f : g[k][st] + e[k] * f;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the sums are complete here: left to itself the compiler moves a row's
+    // additions past the reconstruction of the rows before and spills the terms
+#pragma unroll
+    for (int k = 0; k < G; k++)
+#pragma unroll
+      for (int st = 0; st < IZ_S; st++) asm volatile("" : "+v"(w[k][st]), "+v"(g[k][st]));
+    constexpr int rows[G] = {decltype(M)::value...};
+#pragma unroll
+    for (int k = 0; k < G; k++) {
+      const double lam = rows[k] == 0 ? lmax0 : rows[k] == 2 ? lmax2 : lmax1;
+      double gp[IZ_S], gm[IZ_S];
+#pragma unroll
+      for (int st = 0; st < IZ_S; st++) {
+        gp[st] = 0.5 * (g[k][st] + lam * w[k][st]);
+        gm[st] = g[k][st] - gp[st];
+      }
+      double gl, gr;
+      d_weno_face(js, gp, gm, gl, gr);
+      ghat[rows[k]] = gl + gr;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if constexpr (IZ_EU_GROUP == 4) {
+    project(EuRow<0>{}, EuRow<1>{}, EuRow<2>{}, EuRow<5>{});
+  } else {
+    project(EuRow<0>{}, EuRow<2>{});
+    project(EuRow<1>{}, EuRow<5>{});
+  }
+  eu_species_rows<6>(project);
+  // rows 3 and 4: a tangential momentum and the mass
+#pragma unroll
+  for (int m = 3; m <= 4; m++) {
+    int offm = off;
+    asm volatile("" : "+v"(offm));
+    auto Qm = [&](int q, int st) { return tile[offm + q * QS + st * SS]; };
+    const int tc = (m == 3) ? t1 : t2;
+    const double et0 = -uc[tc - 1];
     double gp[IZ_S], gm[IZ_S];
 #pragma unroll
     for (int st = 0; st < IZ_S; st++) {
-      const double u = Qm(IZ_QU, st), p = Qm(IZ_QP, st);
-      double wc, gc;
-      if (m == 3 || m == 4) {
-        const int tc = (m == 3) ? t1 : t2;
-        const double et0 = -uc[tc - 1];
-        const double v0 = Qm(0, st), vt = Qm(tc, st);
-        const double f0 = Qm(cn, st);
-        const double ft = (tc == cn) ? vt * u + p : vt * u;
-        wc = et0 * v0 + vt;
-        gc = et0 * f0 + ft;
-      } else {
-        const double v0 = Qm(0, st);
-        wc = e[0] * v0;
-        gc = e[0] * Qm(cn, st);
-#pragma unroll
-        for (int cc = 1; cc <= 3; cc++) {
-          const double vc = Qm(cc, st);
-          wc = wc + e[cc] * vc;
-          gc = gc + e[cc] * ((cc == cn) ? vc * u + p : vc * u);
-        }
-        const double v4 = Qm(4, st);
-        wc = wc + e[4] * v4;
-        gc = gc + e[4] * (u * (v4 + p));
-#pragma unroll
-        for (int l = IZ_NIV; l < IZ_NV; l++) {
-          const double vl = Qm(l, st);
-          wc = wc + e[l] * vl;
-          gc = gc + e[l] * (vl * u);
-        }
-      }
-      gp[st] = 0.5 * (gc + lam * wc);
+      const double u = Qm(IZ_QU, st);
+      const double v0 = Qm(0, st), vt = Qm(tc, st);
+      const double f0 = Qm(cn, st), ft = vt * u;
+      const double wc = et0 * v0 + vt, gc = et0 * f0 + ft;
+      gp[st] = 0.5 * (gc + lmax1 * wc);
       gm[st] = gc - gp[st];
     }
     double gl, gr;
@@ -295,7 +338,8 @@ __device__ inline void eu_face_ref(const double *tile, int off, bool js,
 // per reconstructed field; fields are taken one after the other and enter F^
 // as they come, so that few of them are live at a time: 204 VGPRs, two waves
 // per SIMD (three or four spill: 3.6 and 4.3 ms).  The kernel is bound by FP64
-// issue: 4.5 -> 2.0 (x), 2.2 (y, z) ms per launch at 256^3.  Results differ from the dense order by rounding only.
+// issue: 4.5 -> 2.0 (x), 2.2 (y, z) ms per launch at 256^3.  Results
+// differ from the dense order by rounding only.
 template <int DIR, int QS, int SS, int SITE>
 __device__ inline void eu_face_fast(const double *tile, int off, bool js,
                                     const double *__restrict__ ha, long nc, long cL, long cR,
