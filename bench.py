@@ -25,6 +25,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 METRIC = "cell-steps/s 256^3 reacting H2 (FP64); chem cells/s surrogate vs VODE @|dT|<=2K"
+# the reference's compiled chemistry, which the CPU baseline integrates with
+REF_CHEM = os.path.join(ROOT, "oracle", "_ref", "libpsrref.so")
 PEAK_FP64_TFLOPS = 78.6
 PEAK_BF16_TFLOPS = 2500.0  # dense MFMA
 PEAK_HBM_GBS = 8000.0
@@ -414,7 +416,9 @@ def main():
     from phd_amd.solver import Options, Solver, profile_read, profile_start
 
     cpu = None
-    if not args.no_cpu_baseline:
+    if not args.no_cpu_baseline and not os.path.exists(REF_CHEM):
+        log(f"no CPU baseline: the reference's DVODE is not built ({REF_CHEM})")
+    elif not args.no_cpu_baseline:
         # before anything touches the GPU: the workers are forked
         log("CPU baseline (oracle flow + reference DVODE, one process per core)")
         cpu = cpu_baseline()

@@ -2,12 +2,16 @@
 tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg, never by
 the product package.
 
-Two independent checkers live here:
+The checkers that live here:
   * ``Oracle``  -- liboracle.so, the C restatement of the reference flow path
                    and kinetics (izem_oracle.c);
   * ``RefChem`` -- oracle/_ref/libpsrref.so, the reference's own CHEMKIN-II +
                    DVODE Fortran compiled from its sources, driven through the
-                   harness in oracle/ref/psr_driver.f.
+                   harness in oracle/ref/psr_driver.f;
+  * ``VodeChem`` -- the same DVODE from the netlib as scipy ships it, on the
+                   kinetics of liboracle.so: it stands in for RefChem where
+                   the reference's sources are not there to build from
+                   (``refchem`` picks one).
 """
 from __future__ import annotations
 
@@ -253,3 +257,74 @@ class RefChem:
                               C.byref(C.c_double(atol)), C.byref(ist), C.byref(nst),
                               C.byref(nfe), C.byref(nje))
         return Tc.value, Yc, ist.value, nst.value, nfe.value, nje.value
+
+
+class VodeChem:
+    """RefChem's calls without the reference's build: CHEMKIN's functions by
+    the C restatement in liboracle.so (which is held against RefChem where
+    both are there), and the reactor substep by DVODE itself as scipy ships it
+    (BDF, full Jacobian by differences: METH 2, MITER 2, ITASK 1), the
+    integrator of the reference's REACTION_V (chemkin/reaction_v.f)."""
+
+    def __init__(self, mech=None):
+        from phd_amd import chemdata as cd
+        mech = mech or cd.read_mechanism()
+        self._o = Oracle()
+        self._m = make_mech(mech)
+        self._rhs = self._o.lib["ora_reactor_rhs"]
+        self._rhs.argtypes = [C.c_void_p, C.c_double, C.c_void_p, C.c_void_p]
+        self._rhs.restype = None
+        self.kk = mech.kk
+
+    def wdot(self, rho, T, Y):
+        Y = np.ascontiguousarray(Y, dtype=np.float64)
+        w = np.zeros(self.kk)
+        self._o.lib.ora_ckwyr(C.byref(self._m), float(rho), float(T), _p(Y), _p(w))
+        return w
+
+    def hms(self, T):
+        h = np.zeros(self.kk)
+        self._o.lib.ora_ckhms(C.byref(self._m), C.c_double(T), _p(h))
+        return h
+
+    def cvbs(self, T, Y):
+        Y = np.ascontiguousarray(Y, dtype=np.float64)
+        return self._o.lib.ora_ckcvbs(C.byref(self._m), float(T), _p(Y))
+
+    def rhs(self, rho, z):
+        z = np.ascontiguousarray(z, dtype=np.float64)
+        zp = np.zeros(self.kk + 1)
+        self._o.lib.ora_reactor_rhs(C.byref(self._m), float(rho), _p(z), _p(zp))
+        return zp
+
+    def psr(self, T, rho, Y, dt, rtol=None, atol=None):
+        """As RefChem.psr; with rtol/atol None the tolerances that the
+        reference PSR_CHEMKIN is compiled with."""
+        from scipy.integrate import ode
+        if rtol is None:
+            rtol, atol = 1.0e-6, 1.0e-10
+        # plain addresses: the callback is most of this call's time
+        f, m, rho = self._rhs, C.addressof(self._m), float(rho)
+        z, zp = np.zeros(self.kk + 1), np.zeros(self.kk + 1)
+        pz, pzp = z.ctypes.data, zp.ctypes.data
+
+        def rhs(t, y):
+            z[:] = y
+            f(m, rho, pz, pzp)
+            return zp
+
+        r = ode(rhs).set_integrator("vode", method="bdf", with_jacobian=True, rtol=rtol,
+                                    atol=atol, nsteps=100000)
+        r.set_initial_value(np.concatenate([[T], Y]), 0.0)
+        y = r.integrate(dt)
+        nst, nfe, nje = r._integrator.iwork[10:13]
+        return float(y[0]), y[1:].copy(), r.get_return_code(), int(nst), int(nfe), int(nje)
+
+
+def refchem(mech=None, ref_dir: str | None = None):
+    """The DVODE to compare with: the reference's own build where it is
+    there, else VodeChem on the given (default: the bundled) mechanism."""
+    try:
+        return RefChem(ref_dir)
+    except FileNotFoundError:
+        return VodeChem(mech)

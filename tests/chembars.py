@@ -1,7 +1,7 @@
 """Accuracy bars of the chemistry substep referenced to DVODE itself.
 
-The reference's DVODE (oracle/_ref, compiled from its sources) is run twice
-per cell: at the tolerances under test, and at rtol 1e-11 / atol 1e-17 as the
+The reference's DVODE (oracle/_ref, compiled from its sources; without that
+build the same DVODE as scipy ships it, oracle.VodeChem) is run twice per cell: at the tolerances under test, and at rtol 1e-11 / atol 1e-17 as the
 exact solution.  Errors are measured in DVODE's own norm: each component z_i
 of a cell's state (T, Y_1..Y_K) scaled by rtol |z_i| + atol (DVEWSET, ITOL =
 1), and per cell the root mean square over the components (DVNORM).  Bars:

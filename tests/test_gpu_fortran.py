@@ -152,7 +152,10 @@ def test_fortran_host_reacting_iteration(oracle, adi, thd, mech):
     from phd_amd.solver import Options, Solver
     from tests import chembars
     F = _flib()
-    rc = RefChem()
+    try:
+        rc = RefChem()  # its COMMON blocks are the mechanism the Fortran host hands over
+    except FileNotFoundError as e:
+        pytest.skip(str(e))
     box, v, T = ics.config1_state(adi, thd, n=16, seed=7, T_peak=1800.0)
     run0 = OracleRun(oracle, adi, thd, box, v, T)
     run0.prim_all()

@@ -1,23 +1,16 @@
 """The chemistry integrator's source (phd_amd/csrc/chem_device.h), built for
-the host with g++, against the reference's own compiled DVODE
-(oracle/_ref): both kinetics forms, the C3 cell recipe, the reactor
+the host with g++, against the reference's own compiled DVODE (oracle/_ref;
+without that build DVODE as scipy ships it, oracle.VodeChem): both kinetics forms, the C3 cell recipe, the reactor
 substep of izem_psr_batch.  Bars as in the GPU test: |dT| <= 2e-4 T and
 |dY_k| <= 2e-4 |Y_k| + 1e-8 per cell, every cell integrated (ok)."""
-import os
-
 import numpy as np
 import pytest
 
-REF = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle", "_ref",
-                   "libpsrref.so")
-
-
-@pytest.mark.skipif(not os.path.exists(REF), reason="oracle/_ref not built")
 @pytest.mark.parametrize("kinetics", [0, 1])
 def test_host_integrator_vs_reference_dvode(host_bdf, thd, kinetics):
-    from oracle.oracle import RefChem
+    from oracle.oracle import refchem
     from phd_amd import ics
-    rc = RefChem()
+    rc = refchem()
     n = 48
     T, p, Y = ics.config3_cells(thd, n, seed=11)
     Wmix = 1.0 / (Y / (np.array(thd.W) * 1000.0)).sum(axis=1)
@@ -42,17 +35,16 @@ def test_host_integrator_vs_reference_dvode(host_bdf, thd, kinetics):
     assert np.all(np.abs(Yh.sum(axis=1) - 1.0) <= 1e-12)
 
 
-@pytest.mark.skipif(not os.path.exists(REF), reason="oracle/_ref not built")
 def test_host_integrator_global_error_like_dvode(host_bdf, thd):
     """At the same rtol/atol the integrator's global error is like DVODE's:
     both measured against DVODE run at rtol 1e-11, atol 1e-17, in DVODE's
     error norm (tests/chembars.py), on C3 cells at two substeps and on the
     cells of a 3-D decaying-HIT state over an igniting 2e-4 s substep."""
-    from oracle.oracle import Oracle, RefChem
+    from oracle.oracle import Oracle, refchem
     from phd_amd import chemdata as cd, ics
     from tests import chembars
     from tests.flowcase import OracleRun, small_state
-    rc = RefChem()
+    rc = refchem()
     cases = []
     for seed, n, dt in ((11, 64, 1e-6), (7, 48, 1e-7), (5, 48, 1e-5)):
         T, p, Y = ics.config3_cells(thd, n, seed=seed)
@@ -113,14 +105,13 @@ def test_closed_form_jacobian_columns(host_bdf, thd):
     assert worst <= 1e-5
 
 
-@pytest.mark.skipif(not os.path.exists(REF), reason="oracle/_ref not built")
 def test_closed_form_jacobian_integrator_like_dvode(host_bdf, thd):
     """The integrator with the closed-form mass-fraction columns keeps
     DVODE's accuracy (tests/chembars.py) on C3 cells at 1e-6 s."""
-    from oracle.oracle import RefChem
+    from oracle.oracle import refchem
     from phd_amd import ics
     from tests import chembars
-    rc = RefChem()
+    rc = refchem()
     T, p, Y = ics.config3_cells(thd, 64, seed=11)
     Wmix = 1.0 / (Y / (np.array(thd.W) * 1000.0)).sum(axis=1)
     rho = (p * 10.0) * Wmix / (8.314510e7 * T)

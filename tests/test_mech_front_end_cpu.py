@@ -3,9 +3,10 @@ falloff (5 values), 4-value Troe, a named falloff collider (+N2), explicit
 reverse parameters (REV) and an irreversible reaction
 (tests/golden/h2_air_sri_rev.inp), parsed by phd_amd.chemdata, turned into
 straight-line code by phd_amd.codegen_mech and into device tables by
-izem_chem_setup's flat image.  Both kinetics forms are compiled for the host
+izem_chem_setup's flat image.  The kinetics forms are compiled for the host
 from the kernels' own headers and checked against the reference's
-interpreter + CKWYR/FUN/DVODE built from its sources (oracle/_ref/sri)."""
+interpreter + CKWYR/FUN/DVODE built from its sources (oracle/_ref/sri;
+without that build oracle.VodeChem on the same mechanism)."""
 import ctypes as C
 import os
 import shutil
@@ -18,8 +19,6 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 SRI_MECH = os.path.join(HERE, "golden", "h2_air_sri_rev.inp")
 SRI_DIR = os.path.join(ROOT, "oracle", "_ref", "sri")
-needs_ref = pytest.mark.skipif(not os.path.exists(os.path.join(SRI_DIR, "chem.bin")),
-                               reason="oracle/_ref/sri not built")
 
 
 @pytest.mark.parametrize("line,aux", [
@@ -67,13 +66,13 @@ def sri_host(tmp_path_factory):
     return L
 
 
-@needs_ref
 @pytest.mark.parametrize("kinetics", [0, 1])
 def test_front_end_rhs_vs_reference_fun(sri_host, kinetics):
     """Reactor RHS (T and Y rates) of the table-driven (0) and straight-line
     (1) kinetics against the reference FUN at 300 random states."""
-    from oracle.oracle import RefChem
-    rc = RefChem(SRI_DIR)
+    from oracle.oracle import refchem
+    from phd_amd import chemdata as cd
+    rc = refchem(cd.read_mechanism(SRI_MECH), SRI_DIR)
     rng = np.random.default_rng(5)
     worst = 0.0
     for _ in range(300):
@@ -88,15 +87,14 @@ def test_front_end_rhs_vs_reference_fun(sri_host, kinetics):
     assert worst <= 1e-10
 
 
-@needs_ref
-@pytest.mark.parametrize("kinetics", [0, 1])
+@pytest.mark.parametrize("kinetics", [0, 1, 2])
 def test_front_end_integration_vs_reference_dvode(sri_host, thd, kinetics):
     """48 ignition cells (the C3 recipe) over 1e-6 s with the test mechanism:
-    the integrator with either kinetics form against the reference DVODE,
+    the integrator with each kinetics form against the reference DVODE,
     with the bars of the bundled mechanism's test."""
-    from oracle.oracle import RefChem
-    from phd_amd import ics
-    rc = RefChem(SRI_DIR)
+    from oracle.oracle import refchem
+    from phd_amd import chemdata as cd, ics
+    rc = refchem(cd.read_mechanism(SRI_MECH), SRI_DIR)
     n = 48
     T, p, Y = ics.config3_cells(thd, n, seed=12)
     Wmix = 1.0 / (Y / (np.array(thd.W) * 1000.0)).sum(axis=1)
