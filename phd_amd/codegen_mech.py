@@ -42,6 +42,7 @@ from __future__ import annotations
 import hashlib
 import math
 import os
+from fractions import Fraction
 
 import numpy as np
 
@@ -70,7 +71,8 @@ def mechanism_hash(mech: cd.Mechanism) -> str:
 def _basis(mech: cd.Mechanism):
     """Basis species of the element space, those nearest to zero enthalpy at
     298 K first, and B[k][j]: species k has the elements of sum_j B_kj
-    basis_j."""
+    basis_j (solved in fractions, so that any composition is exact to one
+    rounding)."""
     ncf = np.asarray(mech.ncf, dtype=np.float64)
     T = 298.15
 
@@ -82,8 +84,19 @@ def _basis(mech: cd.Mechanism):
     for k in sorted(range(mech.kk), key=h298):
         if np.linalg.matrix_rank(ncf[basis + [k]]) > len(basis):
             basis.append(k)
-    B, *_ = np.linalg.lstsq(ncf[basis].T, ncf.T, rcond=None)
-    B = np.round(B.T * 12) / 12.0
+    # Gauss-Jordan on [basis compositions as columns | all compositions]
+    rows = [[Fraction(x).limit_denominator(10 ** 6) for x in list(ncf[basis, e]) + list(ncf[:, e])]
+            for e in range(ncf.shape[1])]
+    nb, used = len(basis), 0
+    for j in range(nb):
+        p = next(i for i in range(used, len(rows)) if rows[i][j] != 0)
+        rows[used], rows[p] = rows[p], rows[used]
+        rows[used] = [x / rows[used][j] for x in rows[used]]
+        for i in range(len(rows)):
+            if i != used and rows[i][j] != 0:
+                rows[i] = [x - rows[i][j] * y for x, y in zip(rows[i], rows[used])]
+        used += 1
+    B = np.array([[float(rows[j][nb + k]) for j in range(nb)] for k in range(mech.kk)])
     assert np.allclose(B @ ncf[basis], ncf)
     return basis, B
 
@@ -127,7 +140,7 @@ def generate(mech: cd.Mechanism) -> str:
     R = mech.reactions
     # species up to the last one that any reaction changes
     live = [k for k in range(kk) if any(_net(r).get(k) for r in R)]
-    w(f"#define GEN_NLIVE {max(live) + 1}")
+    w(f"#define GEN_NLIVE {max(live, default=-1) + 1}")
 
     # reactions that are one rate: the same sides, no falloff, the same third
     # bodies, reverse from the equilibrium constant
@@ -216,29 +229,38 @@ def generate(mech: cd.Mechanism) -> str:
              "  const double rtp = ruT * (1.0 / 1.01325e6), pfac = 1.01325e6 / ru * it;"]
         used = sorted({k for g in groups if R[g[0]]["rev"] and not R[g[0]].get("rpar")
                        for k, n in _net(R[g[0]]).items() if n and k not in basis})
-        for k in used:
-            o.append(f"  double w{k};")
+        tms = sorted(set(float(t) for t in mech.tmid))
 
-        def g100(k):
-            """w_k at 100 K"""
-            c = np.asarray(mech.a[k][0]) - sum(B[k][j] * np.asarray(mech.a[b][0])
-                                               for j, b in enumerate(basis))
-            return float(c[0] * (math.log(100.0) - 1.0) + c[1] / 2 * 1e2 + c[2] / 6 * 1e4 +
-                         c[3] / 12 * 1e6 + c[4] / 20 * 1e8 + c[6] - c[5] / 100.0)
+        def gibbs(k, T):
+            """(S/R - H/RT of species k relative to the basis at T)"""
+            def smh(q):
+                a = mech.a[q][1 if T > mech.tmid[q] else 0]
+                return (a[0] * (math.log(T) - 1.0) + a[1] / 2 * T + a[2] / 6 * T ** 2 +
+                        a[3] / 12 * T ** 3 + a[4] / 20 * T ** 4 + a[6] - a[5] / T)
+            return float(smh(k) - sum(B[k][j] * smh(b) for j, b in enumerate(basis)))
 
         def poly(c, names=("", " * T", " * T2", " * T3", " * T4")):
             return " + ".join(f"{_lit(x)}{n}" for x, n in zip(c, names)).replace("+ -", "- ")
 
-        def thermo(rng):
+        def smh_poly(c):
+            return (f"{_lit(c[0])} * (lt - 1.0) + {_lit(c[1] / 2)} * T + {_lit(c[2] / 6)} * T2 + "
+                    f"{_lit(c[3] / 12)} * T3 + {_lit(c[4] / 20)} * T4"
+                    f" + {_lit(c[6])} - {_lit(c[5])} * it;".replace("+ -", "- "))
+
+        def relative(k, rng):
+            a = [np.asarray(mech.a[k][rng])] + [np.asarray(mech.a[b][rng]) for b in basis]
+            return a[0] - sum(B[k][j] * a[1 + j] for j in range(len(basis)))
+
+        def thermo(rng, ks):
             q = []
-            # S/R - H/RT of the species relative to the basis
-            for k in used:
-                a = [np.asarray(mech.a[k][rng])] + [np.asarray(mech.a[b][rng]) for b in basis]
-                c = a[0] - sum(B[k][j] * a[1 + j] for j in range(len(basis)))
-                q.append(f"    w{k} = {_lit(c[0])} * (lt - 1.0) + {_lit(c[1] / 2)} * T + "
-                         f"{_lit(c[2] / 6)} * T2 + {_lit(c[3] / 12)} * T3 + {_lit(c[4] / 20)} * T4"
-                         f" + {_lit(c[6])} - {_lit(c[5])} * it;".replace("+ -", "- "))
-            for k in range(kk):
+            # S/R - H/RT of the species relative to the basis; where ranges
+            # differ, of each species by itself (combined below)
+            if len(tms) == 1:
+                q += [f"    w{k} = {smh_poly(relative(k, rng))}" for k in used]
+            else:
+                q += [f"    g{k} = {smh_poly(mech.a[k][rng])}" for k in ks
+                      if k in used or k in basis]
+            for k in ks:
                 a, wt = mech.a[k][rng], mech.wt[k]
                 cv = [a[0] - 1.0] + list(a[1:5])
                 q.append("  " + store(f"cvk{k}", f"{_lit(8.314510e7 / wt)} * ({poly(cv)})"))
@@ -247,13 +269,22 @@ def generate(mech: cd.Mechanism) -> str:
                                       .replace("+ -", "- ")))
             return q
 
-        tm = sorted(set(float(t) for t in mech.tmid))
-        assert len(tm) == 1, "one common mid temperature expected"
-        o.append(f"  if (T > {_lit(tm[0])}) {{")
-        o += thermo(1)
-        o.append("  } else {")
-        o += thermo(0)
-        o.append("  }")
+        if len(tms) == 1:
+            o += [f"  double w{k};" for k in used]
+        else:
+            o += [f"  double g{k};" for k in range(kk) if k in used or k in basis]
+        for tm in tms:
+            ks = [k for k in range(kk) if mech.tmid[k] == tm]
+            o.append(f"  if (T > {_lit(tm)}) {{")
+            o += thermo(1, ks)
+            o.append("  } else {")
+            o += thermo(0, ks)
+            o.append("  }")
+        if len(tms) > 1:
+            for k in used:
+                t = "".join(f" + {_lit(-B[k][j])} * g{b}" for j, b in enumerate(basis)
+                            if B[k][j] != 0).replace("+ -", "- ")
+                o.append(f"  const double w{k} = g{k}{t};")
         need_inv = {k for g in groups if R[g[0]]["rev"] and not R[g[0]].get("rpar")
                     for k, n in _net(R[g[0]]).items() if n > 0}
         for k in used:
@@ -292,7 +323,7 @@ def generate(mech: cd.Mechanism) -> str:
                 # products, the next one always that which keeps the partial
                 # product nearest to 1 at 100 K, so that none
                 # leaves the range of a double where the product does not
-                left = [(f"r{k}", -g100(k)) if n > 0 else (f"e{k}", g100(k))
+                left = [(f"r{k}", -gibbs(k, 100.0)) if n > 0 else (f"e{k}", gibbs(k, 100.0))
                         for k, n in nu.items() if k not in basis for _ in range(abs(n))]
                 fac, at100 = [kf], -max(R[m]["EoR"] for m in g) / 100.0
                 while left:
@@ -417,8 +448,7 @@ def generate(mech: cd.Mechanism) -> str:
         o.append("  const double rho_i = d_rcp(rho);")
         for k in range(kk):
             o.append(f"  zp[{1 + k}] = wd{k} * ({_lit(mech.wt[k])} * rho_i);")
-        o.append("  const double sum = " + " + ".join(f"{load(f'uk{k}')} * wd{k}" for k in live) +
-                 ";")
+        o.append("  const double sum = " + _sum([f"{load(f'uk{k}')} * wd{k}" for k in live]) + ";")
         o.append("  zp[0] = -sum * d_rcp(rho * cvb);")
         return o
 
@@ -506,7 +536,7 @@ def generate(mech: cd.Mechanism) -> str:
             for k in range(kk):
                 v = f"y{k} * {_lit(mech.wt[k] / mech.wt[m])}" if k in live else "0.0"
                 o.append(f"    J[{1 + k}][{1 + m}] = {v};")
-            ds = " + ".join(f"{load(f'uk{k}')} * y{k}" for k in live)
+            ds = _sum([f"{load(f'uk{k}')} * y{k}" for k in live])
             o.append(f"    J[0][{1 + m}] = -(({ds}) * {_lit(1.0 / mech.wt[m])} + f0T * "
                      f"{load(f'cvk{m}')}) * cvi;")
             o.append("  }")
@@ -551,18 +581,23 @@ def generate(mech: cd.Mechanism) -> str:
         for k in range(kk):
             v = f"y{k} * ({_lit(mech.wt[k])} * rho_i)" if k in live else "0.0"
             o.append(f"  J[{1 + k}][0] = {v};")
-        o.append("  const double ut = (" + " + ".join(f"{load(f'uk{k}')} * y{k}" for k in live) +
+        o.append("  const double ut = (" + _sum([f"{load(f'uk{k}')} * y{k}" for k in live]) +
                  ") * rho_i;")
-        o.append("  const double cf = " + " + ".join(f"{load(f'cvk{k}')} * f0[{1 + k}]"
-                                                      for k in live) + ";")
+        o.append("  const double cf = " + _sum([f"{load(f'cvk{k}')} * f0[{1 + k}]"
+                                                for k in live]) + ";")
         # d cvb / dT from the mixture's polynomial
-        o.append("  double p1, p2, p3, p4;")
-        for cond, rng in ((f"if (T > {_lit(mech.tmid[0])})", 1), ("else", 0)):
-            o.append(f"  {cond} {{")
-            for q in range(1, 5):
-                o.append(f"    p{q} = " + _sum([f"{_lit(mech.a[k][rng][q] * q)} * c{k}"
-                                                for k in range(kk)]) + ";")
-            o.append("  }")
+        tms = sorted(set(float(t) for t in mech.tmid))
+        op = "=" if len(tms) == 1 else "+="
+        o.append("  double p1, p2, p3, p4;" if len(tms) == 1 else
+                 "  double p1 = 0.0, p2 = 0.0, p3 = 0.0, p4 = 0.0;")
+        for tm in tms:
+            for cond, rng in ((f"if (T > {_lit(tm)})", 1), ("else", 0)):
+                o.append(f"  {cond} {{")
+                for q in range(1, 5):
+                    o.append(f"    p{q} {op} " + _sum([f"{_lit(mech.a[k][rng][q] * q)} * c{k}"
+                                                       for k in range(kk) if mech.tmid[k] == tm]) +
+                             ";")
+                o.append("  }")
         o.append("  const double dcv = (p1 + T * (p2 + T * (p3 + T * p4))) * (ru * rho_i);")
         o.append("  J[0][0] = -(ut + cf + f0[0] * dcv) * cvi;")
         return o
