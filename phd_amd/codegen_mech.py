@@ -341,15 +341,17 @@ def generate(mech: cd.Mechanism) -> str:
                 if r["fal"] == 2:
                     # SRI: the T-only factors of F = d (a e^(-b/T) + e^(-T/c))^X T^e
                     a_, b_, c_, d_, e_ = fp[3:8]
-                    o.append(store(f"srib{i}", f"{_lit(a_)} * d_exp({_lit(-b_)} * it) + "
-                                               f"d_exp(-T / {_lit(c_)})"))
+                    # (the centring temperatures may be 1e-30 or 1e30: beyond
+                    # d_exp's arguments)
+                    o.append(store(f"srib{i}", f"{_lit(a_)} * exp({_lit(-b_)} * it) + "
+                                               f"exp(-T / {_lit(c_)})"))
                     o.append(store(f"srid{i}", f"{_lit(d_)} * pow(T, {_lit(e_)})"))
                 elif r["fal"] >= 3 and troe_const(r) is None:
                     al, t3, t1 = fp[3], fp[4], fp[5]
-                    fc = (f"(1.0 - {_lit(al)}) * d_exp(-T / {_lit(t3)}) + {_lit(al)} * "
-                          f"d_exp(-T / {_lit(t1)})")
+                    fc = (f"(1.0 - {_lit(al)}) * exp(-T / {_lit(t3)}) + {_lit(al)} * "
+                          f"exp(-T / {_lit(t1)})")
                     if r["fal"] == 4:
-                        fc += f" + d_exp(-{_lit(fp[6])} * it)"
+                        fc += f" + exp({_lit(-fp[6])} * it)"
                     o.append(store(f"fclog{i}", f"log10(fmax({fc}, 1e-300))"))
         return o
 
