@@ -557,7 +557,12 @@ def generate(mech: cd.Mechanism) -> str:
             nu = _net(r)
             slope = lambda b_, E_: f"({_lit(b_)} + {_lit(E_)} * it) * it"
             if len(g) > 1:
-                o.append(f"  const double af{i} = {load(f'dkf{i}')} / {load(f'kf{i}')};")
+                # (a sum that underflows or cancels has no slope)
+                safe = all(R[m]["A"] > 0 for m in g) and any(R[m]["EoR"] <= 0 for m in g)
+                q = f"{load(f'dkf{i}')} / {load(f'kf{i}')}"
+                if not safe:
+                    q = f"{load(f'kf{i}')} != 0.0 ? {q} : 0.0"
+                o.append(f"  const double af{i} = {q};")
             else:
                 o.append(f"  const double af{i} = {slope(r['b'], r['EoR'])};")
             f, b = sides(i)
