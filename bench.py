@@ -46,6 +46,13 @@ def read_traffic(kernel: str, n: int):
     return float(m.group(1)) if m else None
 
 
+def closed_form(tune) -> bool:
+    """Whether the chemistry ran with the closed-form Jacobian under these
+    settings (waves, blocks per CU, Jacobian age, kinetics, ...): asked for,
+    or what kinetics -1 takes at one wave for the bundled mechanism."""
+    return tune[3] == 2 or (tune[3] == -1 and tune[0] == 1)
+
+
 def _cpu_step_worker(arg):
     """One full reacting step (timestep, chemistry(dt/2), SSP-RK3,
     chemistry(dt/2)) on an n^3 box of the workload recipe: the oracle's C
@@ -505,7 +512,7 @@ def main():
     if c_cnt:
         from phd_amd.flops import chem_flops
         c_avg_s = c_ms / c_cnt / 1e3
-        c_flop = chem_flops(chem_stats, closed_form=tuned[3] == 2) / c_cnt
+        c_flop = chem_flops(chem_stats, closed_form=closed_form(tuned or tune)) / c_cnt
         c_ach = c_flop / c_avg_s / 1e12
         chem_roof = {"kernel": "k_reaction_queue", "bound": "fp64-valu", "achieved": c_ach,
                      "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
