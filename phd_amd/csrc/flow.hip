@@ -340,8 +340,8 @@ __device__ inline void eu_face_ref(const double *tile, int off, bool js,
 // per SIMD (three or four spill: 3.6 and 4.3 ms).  The kernel is bound by FP64
 // issue: 4.5 -> 2.0 (x), 2.2 (y, z) ms per launch at 256^3.  Results
 // differ from the dense order by rounding only.
-template <int DIR, int QS, int SS, int SITE>
-__device__ inline void eu_face_fast(const double *tile, int off, bool js,
+template <int DIR, int QS, int SS, int SITE, bool WIDE = false>
+__device__ __forceinline__ void eu_face_fast(const double *tile, int off, bool js,
                                     const double *__restrict__ ha, long nc, long cL, long cR,
                                     double *__restrict__ F, long nfaces, long fidx) {
 #pragma clang fp contract(on)
@@ -446,7 +446,7 @@ __device__ inline void eu_face_fast(const double *tile, int off, bool js,
       gp[st] = g + lmax0 * w;
       gm[st] = g - lmax0 * w;
     }
-    g0 = d_weno_face_fused(js, gp, gm);
+    g0 = d_weno_face_fused<WIDE>(js, gp, gm);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int st = 0; st < IZ_S; st++) {
@@ -454,7 +454,7 @@ __device__ inline void eu_face_fast(const double *tile, int off, bool js,
       gp[st] = g + lmax2 * w;
       gm[st] = g - lmax2 * w;
     }
-    g2 = d_weno_face_fused(js, gp, gm);
+    g2 = d_weno_face_fused<WIDE>(js, gp, gm);
     __builtin_amdgcn_sched_barrier(0);
     // row 5: -(1 + xi) / b2 with xi = b1 - b2 ht
     const double k = (1.0 + (b1 - b2 * ht_c)) / b2;
@@ -464,7 +464,7 @@ __device__ inline void eu_face_fast(const double *tile, int off, bool js,
       gp[st] = g + lmax1 * w;
       gm[st] = g - lmax1 * w;
     }
-    g5 = d_weno_face_fused(js, gp, gm);
+    g5 = d_weno_face_fused<WIDE>(js, gp, gm);
   }
   // row 1
   fresh();
@@ -474,7 +474,7 @@ __device__ inline void eu_face_fast(const double *tile, int off, bool js,
     gp[st] = g + lmax1 * w;
     gm[st] = g - lmax1 * w;
   }
-  g1 = d_weno_face_fused(js, gp, gm);
+  g1 = d_weno_face_fused<WIDE>(js, gp, gm);
   const double g02 = g0 + g2, gs = g02 + g1, gd = cs_c * (g2 - g0);
   F[fidx] = gs;
   F[(long)cn * nfaces + fidx] = un_c * gs + gd;
@@ -491,7 +491,7 @@ __device__ inline void eu_face_fast(const double *tile, int off, bool js,
       gp[st] = g + lmax1 * w;
       gm[st] = g - lmax1 * w;
     }
-    const double gt = d_weno_face_fused(js, gp, gm);
+    const double gt = d_weno_face_fused<WIDE>(js, gp, gm);
     F[(long)tc * nfaces + fidx] = ut * gs + gt;
     f4 += ut * gt;
   }
@@ -510,11 +510,19 @@ __device__ inline void eu_face_fast(const double *tile, int off, bool js,
       gp[st] = g + lmax1 * w;
       gm[st] = g - lmax1 * w;
     }
-    const double gl = d_weno_face_fused(js, gp, gm);
+    const double gl = d_weno_face_fused<WIDE>(js, gp, gm);
     F[(long)(IZ_NIV + l) * nfaces + fidx] = y * g02 + gl;
     last += psi[l] * gl;
   }
   F[(long)(IZ_NV - 1) * nfaces + fidx] = Yc[IZ_NRV - 1] * g02 + wrk * last;
+  // f4 and last hold every reconstructed field: the face is formed again where
+  // the short reconstruction left its range (iz_weno.h).  Of an inert step at
+  // 193 x 129 x 97 this test of a face takes nothing measurable, one of every
+  // field 0.6 %, the wide form throughout 2 %.
+  if constexpr (IZ_NG == 3 && !WIDE) {
+    if (__builtin_expect(!(fabs(f4 + last) < INFINITY), 0))
+      eu_face_fast<DIR, QS, SS, SITE, true>(tile, off, js, ha, nc, cL, cR, F, nfaces, fidx);
+  }
 }
 
 template <int DIR, int QS, int SS, bool FAST, int SITE>

@@ -6,6 +6,7 @@
 #pragma once
 
 #include "iz_math.h"
+#include "iz_weno.h"
 #include "izem_common.h"
 
 extern __constant__ IzThd c_thd;
@@ -183,9 +184,6 @@ __device__ inline double d_newton_cell(const double *vc, double T, double &cp_ou
 
 // ------------------------------------------------------------------ WENO
 // wenopar / wenorec / wenorec_nw, ng = 3: module_weno.f90:114-190, 236-527
-#define IZ_Z1 (13.0 / 12.0)
-#define IZ_Z2 (1.0 / 4.0)
-#define IZ_EPS_WENO 1.0e-10
 
 __device__ inline void d_betas(const double *q, int i, double *beta) {
   // q is 1-based
@@ -332,49 +330,14 @@ __device__ inline void d_weno_face(bool js, const double *gp, const double *gm, 
 }
 
 // ------------------------------------------------ fused reconstruction
-// gl + gr of a face from the split fluxes scaled by two, gp2 = g + lam w and
-// gm2 = g - lam w: what wenorec (js) or wenorec_nw gives for gp2 / 2 and
-// gm2 / 2, added.  The smoothness indicators scale with the square, so eps
-// does too.  WENO5 brings the weights to a common denominator, which leaves
-// one reciprocal of the eight divisions; its terms are products of four
-// indicator squares, finite for fluxes up to 1e19 times the unit scale.
+// (see iz_weno.h; WENO7 keeps the reference's form)
 #if IZ_NG == 3
-// one side: q[0..4] in its upwind order, numerator and denominator of the
-// weighted candidates (times 6)
-__device__ inline void d_weno5_side(double q0, double q1, double q2, double q3, double q4,
-                                    double &num, double &den) {
-#pragma clang fp contract(on)
-  const double e4 = 4.0 * IZ_EPS_WENO;
-  // candidate 0: q2 q3 q4, 1: q1 q2 q3, 2: q0 q1 q2
-  const double a0 = (q2 + q4) - 2.0 * q3, b0 = 3.0 * q2 - 4.0 * q3 + q4;
-  const double a1 = (q1 + q3) - 2.0 * q2, b1 = q1 - q3;
-  const double a2 = (q0 + q2) - 2.0 * q1, b2 = q0 - 4.0 * q1 + 3.0 * q2;
-  double t0 = IZ_Z1 * (a0 * a0) + (IZ_Z2 * (b0 * b0) + e4);
-  double t1 = IZ_Z1 * (a1 * a1) + (IZ_Z2 * (b1 * b1) + e4);
-  double t2 = IZ_Z1 * (a2 * a2) + (IZ_Z2 * (b2 * b2) + e4);
-  t0 = t0 * t0;
-  t1 = t1 * t1;
-  t2 = t2 * t2;
-  const double w0 = 3.0 * (t1 * t2), w1 = 6.0 * (t0 * t2), w2 = t0 * t1;
-  const double v0 = 2.0 * q2 + (5.0 * q3 - q4);
-  const double v1 = 5.0 * q2 + (2.0 * q3 - q1);
-  const double v2 = 11.0 * q2 + (2.0 * q0 - 7.0 * q1);
-  den = w0 + w1 + w2;
-  num = w0 * v0 + w1 * v1 + w2 * v2;
-}
+template <bool WIDE>
 __device__ inline double d_weno_face_fused(bool js, const double *gp, const double *gm) {
-#pragma clang fp contract(on)
-  if (js) {
-    double n1, d1, n2, d2;
-    d_weno5_side(gp[0], gp[1], gp[2], gp[3], gp[4], n1, d1);
-    d_weno5_side(gm[5], gm[4], gm[3], gm[2], gm[1], n2, d2);
-    return (n1 * d2 + n2 * d1) * (d_rcp(d1 * d2) * (1.0 / 12.0));
-  }
-  const double a = 2.0 * (gp[4] + gm[1]) - 13.0 * (gp[3] + gm[2]) + 47.0 * (gp[2] + gm[3]) +
-                   27.0 * (gp[1] + gm[4]) - 3.0 * (gp[0] + gm[5]);
-  return a * (1.0 / 120.0);
+  return d_weno5_face_fused<WIDE>(js, gp, gm);
 }
 #else
+template <bool WIDE>
 __device__ inline double d_weno_face_fused(bool js, const double *gp, const double *gm) {
   double hp[IZ_S], hm[IZ_S], gl, gr;
 #pragma unroll

@@ -34,6 +34,17 @@ IZ_HD inline double d_rcp(double x) {
 #endif
 }
 
+// e with |x| = m 2^e, 1/2 <= m < 1, for finite nonzero x
+IZ_HD inline int d_exponent(double x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_frexp_exp(x);
+#else
+  int e;
+  (void)frexp(x, &e);
+  return e;
+#endif
+}
+
 IZ_HD inline double d_exp(double x) {
   const double t = rint(x * 1.4426950408889634);
   const double a = fma(t, -0.6931471803691238, x);

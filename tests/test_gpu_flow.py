@@ -109,6 +109,32 @@ def test_euler_flux_parity(oracle, adi, thd, kind, n, mode):
     assert s.status() == 0
 
 
+@pytest.mark.parametrize("scale", [1e14, 1e18, 1e25, 1e60])
+def test_euler_fluxes_of_large_states(oracle, adi, thd, scale):
+    """Mode 1 against mode 0 with all conserved variables scaled alike (so
+    temperature, velocity and composition stay and the fluxes scale): the
+    products of the weights' common denominator leave the range of a double
+    from about 1e17 on, the reference's form does not."""
+    import torch
+    box, v, T = small_state(adi, thd, "3d", 12)
+    run = OracleRun(oracle, adi, thd, box, v, T)
+    run.prim_all()
+    run.sensor[box.interior()] = 1
+    run.v *= scale
+    f = []
+    for mode in (0, 1):
+        s = _gpu_solver(box, mode=mode)
+        _upload(s, run)
+        out = torch.zeros((14,) + box.shape, dtype=torch.float64, device="cuda:0")
+        for d in range(box.ndim):
+            s.euler_llf(d, out)
+        s.sync()
+        f.append(out.cpu().numpy())
+    assert np.all(np.isfinite(f[0]))
+    err = _relerr(f[1], f[0], box)
+    assert err.max() <= TOL, err
+
+
 @pytest.mark.parametrize("mode", [0, 1])
 @pytest.mark.parametrize("kind,n", CASES)
 def test_euler_flux_linear_path(oracle, adi, thd, kind, n, mode):
