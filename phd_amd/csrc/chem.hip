@@ -39,7 +39,9 @@ struct IzChem {
   // autotuned: register budget (waves per SIMD the kernel is compiled
   // for: 1, 2 or 4), resident 64-lane blocks per CU, Jacobian reuse age
   int waves, blocks_per_cu, jac_age;
-  int generated;  // the loaded mechanism is the compiled-in one (mech_gen.h)
+  // the straight-line forms (mech_gen.h) that may run: bit f - 1 set where
+  // the loaded mechanism is the compiled-in one and form f passed the check
+  int generated;
   // work counters of the integrations since the last izem_chem_stats:
   // BDF steps, RHS evaluations, Jacobians, LU solves
   unsigned long long *stats;
@@ -362,9 +364,10 @@ void iz_chem_destroy(izem_ctx *ctx) {
 // iteration matrix only, so end
 // temperatures agree to 1e-6 relative and the step totals to 3 %; a build
 // of the straight-line kernel that departs from its source (as some builds
-// of its heavily spilling variants did) fails this and the context keeps
-// to the tables.  The work counters and the status word are not touched.
-static int gen_bdf_check(izem_ctx *ctx, const IzMech &m, bool &agree) {
+// of its heavily spilling variants did) fails this and the context does
+// without that form.  ok: bit f - 1 set where form f agrees.  The work
+// counters and the status word are not touched.
+static int gen_bdf_check(izem_ctx *ctx, const IzMech &m, int &ok) {
   constexpr int n = 64, nsp = CK_NEQ - 1;
   const double dt = 1.0e-6;
   double T[3][n], rho[n], Y[3][n * nsp];
@@ -426,16 +429,9 @@ static int gen_bdf_check(izem_ctx *ctx, const IzMech &m, bool &agree) {
   if (dn) (void)hipFree(dn);
   if (dst) (void)hipFree(dst);
   if (rc != IZEM_OK) return rc;
-  agree = true;
-  for (int v = 1; v < 3; v++) {
-    long s0 = 0, s1 = 0;
-    for (int c = 0; c < n; c++) {
-      s0 += nst[0][c];
-      s1 += nst[v][c];
-      if (!(fabs(T[v][c] - T[0][c]) <= 1.0e-6 * T[0][c])) agree = false;
-    }
-    if (!(labs(s1 - s0) <= 0.03 * s0)) agree = false;
-  }
+  ok = 0;
+  for (int v = 1; v < 3; v++)
+    if (iz_forms_agree(n, T[0], nst[0], T[v], nst[v])) ok |= 1 << (v - 1);
   return IZEM_OK;
 }
 
@@ -482,17 +478,15 @@ extern "C" int izem_chem_setup(izem_ctx *ctx, const double *mf, long nmech, doub
   ctx->chem->rtol = rtol;
   ctx->chem->atol = atol;
   ctx->chem->trim = trim;
+  ctx->chem->generated = 0;
   if (same) {
-    bool agree = false;
-    int rc = gen_bdf_check(ctx, m, agree);
+    int rc = gen_bdf_check(ctx, m, ctx->chem->generated);
     if (rc != IZEM_OK) return rc;
-    if (!agree) same = 0;
   }
-  ctx->chem->generated = same;
   // the closed-form Jacobian is the faster straight-line form on short and
   // long substeps alike (2^20 flow half steps: 1.07 against 1.38 ms; 2^18
   // ignition cells: 28 against 34 ms)
-  ctx->chem->use_gen = same ? 2 : 0;
+  ctx->chem->use_gen = iz_chem_form(ctx->chem->generated, 1, -1);
   return IZEM_OK;
 }
 
@@ -510,9 +504,9 @@ extern "C" int izem_chem_tune(izem_ctx *ctx, int waves, int blocks_per_cu, int j
   if (!ctx || !ctx->chem || !(waves == 1 || waves == 2 || waves == 4) || blocks_per_cu < 1 ||
       blocks_per_cu > 64 || jac_age < 1 || kinetics < -1 || kinetics > 2)
     return IZEM_E_ARG;
-  if (kinetics >= 1 && (!ctx->chem->generated || waves != 1)) return IZEM_E_ARG;
-  ctx->chem->use_gen = (kinetics == 0 || waves != 1) ? 0
-                       : kinetics > 0 ? kinetics : (ctx->chem->generated ? 2 : 0);
+  const int form = iz_chem_form(ctx->chem->generated, waves, kinetics);
+  if (form < 0) return IZEM_E_ARG;
+  ctx->chem->use_gen = form;
   ctx->chem->waves = waves;
   ctx->chem->blocks_per_cu = blocks_per_cu;
   ctx->chem->jac_age = jac_age;

@@ -4,9 +4,34 @@
 // builds of the integrator.
 #pragma once
 
+#include <math.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include "chem_tables.h"
+
+// The setup check's verdict on one straight-line form of the kinetics: its n
+// cells' end temperatures T and steps n1 against the table-driven form's T0
+// and n0
+static inline bool iz_forms_agree(int n, const double *T0, const int *n0, const double *T,
+                                  const int *n1) {
+  long s0 = 0, s1 = 0;
+  for (int c = 0; c < n; c++) {
+    s0 += n0[c];
+    s1 += n1[c];
+    if (!(fabs(T[c] - T0[c]) <= 1.0e-6 * T0[c])) return false;
+  }
+  return labs(s1 - s0) <= 0.03 * s0;
+}
+
+// The kinetics form that runs for a requested one (0 tables, 1 straight-line,
+// 2 with the closed-form Jacobian, -1 the fastest there is) at a register
+// budget; ok: bit f - 1 set where form f passed the setup check.  -1: refused.
+static inline int iz_chem_form(int ok, int waves, int kinetics) {
+  if (kinetics >= 1) return waves == 1 && (ok >> (kinetics - 1) & 1) ? kinetics : -1;
+  if (kinetics == 0 || waves != 1) return 0;
+  return ok & 2 ? 2 : ok & 1;
+}
 
 // The flat image holds, in order: kk, ii; wt[KMAX]; a[KMAX][2][7];
 // tmid[KMAX]; A, b, EoR [IMAX each]; nu[IMAX][6]; nunk[IMAX][6];
