@@ -175,6 +175,7 @@ struct PsrQueue {
   int *nsteps, *status;
   int cell;
   ChemCount w;
+  __device__ inline bool sorted() const { return order != nullptr; }
   __device__ inline bool next(double &r, double *y) {
     if ((int)threadIdx.x >= lanes) return false;
     const int q = atomicAdd(counter, 1);
@@ -229,6 +230,7 @@ struct FlowQueue {
   long c;
   double dtmax;
   ChemCount w;
+  __device__ inline bool sorted() const { return order != nullptr; }
   __device__ inline bool next(double &r, double *y) {
     if ((int)threadIdx.x >= lanes) return false;
     const long q = atomicAdd(counter, 1);

@@ -317,6 +317,10 @@ IZ_HD inline void d_nordsieck_rescale(Z &z, int q, double rh) {
   }
 }
 
+// Turns after which the lanes of a wave with table-driven kinetics stop taking
+// cells together (see d_bdf_run).
+#define IZ_EACH_AFTER 192
+
 struct BdfResult {
   int nst, nfe, nje, ok;
   int nsol;  // LU back-substitutions (one per corrector iteration)
@@ -344,12 +348,16 @@ IZ_HD inline double d_fd_increment(int j, double yj, double wj, double r0) {
 // Kinetics policies: rhs(rho, y, f) evaluates the reactor right-hand side;
 // rhs_c(rho, y, f, c) does the same and keeps in c what the Jacobian at the
 // same y can reuse; jac_c(rho, y, f0, c, hl0, w, r0, P), given f0 = f(y) and
-// the c of that evaluation, writes P = -hl0 * J with a finite-difference
-// Jacobian (DVJAC with MF = 22, vode.f:3728-3770).  None of them writes y.
+// the c of that evaluation, writes P = -hl0 * J with a Jacobian by finite
+// differences (DVJAC with MF = 22, vode.f:3728-3770) or in closed form
+// (KinGenAJ).  None of them writes y.
 // NACT: the leading equations that react; the ones after them are zero
 // rates (an inert last species), whose corrections stay exactly zero.
+// EACH: a lane always takes its next cell as soon as its own is finished
+// (see d_bdf_run).
 struct KinTables {
   static constexpr int NACT = N_;
+  static constexpr bool EACH = false;
   struct Cache {};
   IZ_MHD inline void rhs(double rho, const double *y, double *f) const {
     d_reactor_rhs(rho, y, f);
@@ -391,6 +399,19 @@ struct KinTables {
 // initial-step search, made by the same code as the step's predictor
 // evaluation, so the right-hand side is compiled in twice only: at this
 // place and in the corrector).
+// A new cell's Jacobian is evaluated while the other lanes of its wave wait.  In
+// the straight-line forms that costs a turn or less.  The table-driven
+// one takes ten right-hand sides for it: lanes that take cells one by one then
+// make the wave pay for a Jacobian in almost every turn, and a substep of a few
+// steps per cell takes longer than with all lanes in step.  There the lanes
+// take cells together, when the whole wave is done, until one cell has kept the
+// wave for IZ_EACH_AFTER turns: beyond that what waiting lanes lose
+// is more.  262144 to 300007 cells at one wave per SIMD, one by one / together /
+// this rule: 61.5 / 25.9 / 26.2 ms at 1.2e-8 s (3 steps a cell), 115 / 67.3 /
+// 68.0 at 1e-7, 171 / 114 / 115 at 3e-7, 421 / 536 / 411 at 1e-6.  After 128
+// turns 140 ms at 3e-7, after 320 430 ms at 1e-6.  Cells in the stiffness order
+// (io.sorted()) have neighbours of like step counts: together throughout, 330
+// / 289 ms at 1e-6.
 // J is the caller's storage for the saved Jacobian.  The first step of
 // every integration evaluates a new one before any read, so the caller
 // initialises J once (the kernels once per lane, not once per cell).
@@ -409,6 +430,7 @@ IZ_HD IZ_FORCEINLINE void d_bdf_run(const Kin &kin, Z &z, double (&J)[N_][N_], I
   enum { STEP = -1, FIRST = 0, RESTART = 5 };
   BdfResult res{0, 0, 0, 1, 0};
   bool alive = false, more = true;
+  int turn = 0;         // since the wave's lanes last took cells together
   int ev = FIRST;
   double rho = 1.0, h = 0.0, t = 0.0, hub = 0.0, hg = 0.0;
   int q = 1, nqwait = 2, ncf = 0, kflag = 0;
@@ -419,7 +441,13 @@ IZ_HD IZ_FORCEINLINE void d_bdf_run(const Kin &kin, Z &z, double (&J)[N_][N_], I
   int nslp = 0, nslj = 0;
   int icf = 0;          // 1: corrector failed with a saved J, 2: with a current J
   for (;;) {
-    if (!alive && more) {
+    bool take = !alive && more;
+    if constexpr (!Kin::EACH) {
+      const bool busy = IZ_ANY(alive);
+      turn = busy ? turn + 1 : 0;
+      take = take && (!busy || (turn > IZ_EACH_AFTER && !io.sorted()));
+    }
+    if (take) {
       double y[N_];
       more = io.next(rho, y);
       if (more) {
@@ -747,6 +775,7 @@ struct BdfOneCell {
   double rho, *y;
   bool taken;
   BdfResult res;
+  IZ_MHD inline bool sorted() const { return false; }
   IZ_MHD inline bool next(double &r, double *yc) {
     if (taken) return false;
     taken = true;
@@ -774,6 +803,7 @@ IZ_HD inline BdfResult d_bdf_integrate(const Kin &kin, Z &z, double (&J)[N_][N_]
 // shared by the Jacobian columns that perturb mass fractions
 struct KinGen {
   static constexpr int NACT = 1 + GEN_NLIVE;
+  static constexpr bool EACH = true;
   struct Cache { double kt[GEN_NKT]; };  // rate constants at the evaluated T
   IZ_MHD inline void rhs(double rho, const double *y, double *f) const {
     double kt[GEN_NKT];
