@@ -265,6 +265,55 @@ def test_reaction_dvode_vs_reference(oracle, adi, thd, mech):
     assert abs(DTmax_gpu - DTt) <= 2.0 * abs(DTd - DTt) + 10.0 * rtol * Tend
 
 
+@pytest.mark.parametrize("kind,dts", [("2d", (1e-8, 1e-6, 1e-5)), ("3d", (1e-8, 2e-5))])
+@pytest.mark.parametrize("kinetics,waves", [(0, 1), (0, 2), (0, 4), (1, 1), (2, 1)])
+def test_flow_kernel_does_what_the_batch_kernel_does(adi, thd, mech, kind, dts, kinetics, waves):
+    """izem_reaction_dvode and izem_psr_batch are two instantiations of one
+    integrator: on the same cells, with the same conversions, the work counters
+    and the end temperatures are equal bit for bit (3-D: more cells than
+    resident lanes, so lanes take several).  A build of one of them that departs
+    from its source (the spilling straight-line kernels have been seen to) shows
+    here even where its results stay within the tolerance; the forms' step
+    counts agree to 3 %."""
+    import torch
+    from phd_amd import ics
+    from phd_amd.solver import Options, Solver
+    box, v, T = (ics.config1_state(adi, thd, n=96, T_peak=2200.0) if kind == "2d"
+                 else ics.config2_state(adi, thd, n=48, L=0.01))
+    s = Solver(box, Options(), adi=adi, thd=thd, mech=mech)
+    s.load_state(v, T)
+    v0, T0 = s.v.clone(), s.T.clone()
+    g = box.ng
+    sl = (slice(g, g + 1) if box.ndim == 2 else slice(2 * g, box.nz - 1),
+          slice(2 * g, box.ny - 1), slice(2 * g, box.nx - 1))
+    rho = v0[0][sl].reshape(-1)
+    for dt_s in dts:
+        dt = torch.tensor([dt_s / adi.time_ref], dtype=torch.float64, device="cuda:0")
+        steps = {}
+        for kin, w in {(kinetics, waves), (0, 1)}:
+            assert s.lib.izem_chem_tune(s.ctx, w, 4 * w, 50, kin) == 0
+            flow, batch = np.zeros(4, np.uint64), np.zeros(4, np.uint64)
+            s.v.copy_(v0); s.T.copy_(T0)
+            s.lib.izem_chem_stats(s.ctx, flow.ctypes.data)
+            s.reaction_selec(dt.data_ptr(), 1.0)
+            s.sync()
+            s.lib.izem_chem_stats(s.ctx, flow.ctypes.data)
+            Tk = (T0[sl].reshape(-1) * adi.T_ref).contiguous()
+            Y = torch.stack([v0[5 + l][sl].reshape(-1) * (1.0 / rho) for l in range(9)],
+                            dim=1).contiguous()
+            r = (rho * (adi.rho_ref * 1.0e-3)).contiguous()
+            assert s.lib.izem_psr_batch(s.ctx, Tk.numel(), C.c_void_p(Tk.data_ptr()),
+                                        C.c_void_p(r.data_ptr()), C.c_void_p(Y.data_ptr()),
+                                        float(dt.item()) * adi.time_ref, None) == 0
+            s.sync()
+            s.lib.izem_chem_stats(s.ctx, batch.ctypes.data)
+            assert s.status() == 0
+            assert np.array_equal(flow, batch), (kin, w, dt_s, flow, batch)
+            assert torch.equal(s.T[sl].reshape(-1), Tk * (1.0 / adi.T_ref)), (kin, w, dt_s)
+            steps[kin] = int(flow[0])
+        assert abs(steps[kinetics] - steps[0]) <= 0.03 * steps[0]
+
+
 def test_straight_line_kinetics_one_wave_only(mech):
     """The straight-line kinetics exist at one wave per SIMD only: asking for
     them at two or four is refused, and 'straight-line when available' at
