@@ -100,6 +100,30 @@ def test_splitk_and_colsum(mech):
     assert np.max(np.abs(cs.cpu().numpy() - Bf.sum(axis=0))) <= 1e-4 * np.abs(Bf).sum(axis=0).max()
 
 
+@pytest.mark.parametrize("M,N,K,ns", [(256, 256, 3000, 2), (257, 130, 5000, 11),
+                                      (32, 256, 2049, 9), (129, 65, 65, 3), (300, 64, 31, 8)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
+def test_splitk_blocks(mech, M, N, K, ns, ta, tb):
+    """Several tiles with several slices: slice counts that are no multiple of
+    8 (the last group of blocks is short), slices that end inside a 64-deep
+    tile (odd multiples of 32, and the remainder of K), more slices than K has
+    32-deep parts; the bar of test_splitk_and_colsum."""
+    import torch
+    s = _solver(mech)
+    rng = np.random.default_rng(M + K)
+    Ab, Af = _bf16_bits(rng.normal(size=(M, K)))
+    Bb, Bf = _bf16_bits(rng.normal(size=(K, N)))
+    dA = torch.tensor(np.ascontiguousarray(Ab.T) if ta else Ab, device="cuda")
+    dB = torch.tensor(Bb if tb else np.ascontiguousarray(Bb.T), device="cuda")
+    out = torch.full((M, N), np.nan, dtype=torch.float32, device="cuda")
+    work = torch.full((ns * M * N,), np.nan, dtype=torch.float32, device="cuda")
+    assert s.lib.izem_mlp_gemm_splitk(s.ctx, ta, tb, M, N, K, _p(dA), M if ta else K, _p(dB),
+                                      N if tb else K, ns, _p(work), _p(out)) == 0
+    s.sync()
+    ref = Af @ Bf
+    assert np.max(np.abs(out.cpu().numpy() - ref)) <= 1e-5 * np.abs(ref).max() * 4
+
+
 def test_forward_and_gradients_vs_fp64_oracle(mech):
     import torch
     from oracle import mlp_oracle as mo

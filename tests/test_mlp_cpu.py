@@ -70,3 +70,31 @@ def test_element_projector(thd):
     assert np.max(np.abs(P @ P - P)) <= 1e-14
     # the oracle's restatement agrees
     assert np.max(np.abs(mo.element_projector(thd.kncf, thd.awt) - P)) <= 1e-15
+
+
+def test_gelu_polynomial():
+    """mlp.hip's gelu in FP32, emulated from the coefficients in its source
+    (fused multiply-adds by way of FP64): the tail term |z| q(|z|) within 4e-8
+    and z Phi(z) within that and half an ulp, on a fine grid, far beyond the
+    fitted range and for tiny arguments."""
+    import os
+    import re
+    from scipy.special import ndtr
+    src = open(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "phd_amd", "csrc",
+                            "mlp.hip")).read()
+    body = src[src.index("inline float gelu(float z)"):src.index("inline float gelu_d")]
+    co = [float(x) for x in re.findall(r"(?:float p = |fmaf\(p, x, )(-?[0-9.e-]+)f", body)]
+    assert len(co) == 9 and co[0] < 0.0
+    far = np.geomspace(1e-30, 1e4, 100001)
+    z = np.concatenate([np.linspace(-14, 14, 1000001), far, -far]).astype(np.float32)
+    x = np.abs(z)
+    p = np.full_like(x, np.float32(co[0]))
+    for c in co[1:]:
+        p = (p.astype(np.float64) * x + np.float64(np.float32(c))).astype(np.float32)
+    tail = x.astype(np.float64) * np.exp2(p.astype(np.float64)).astype(np.float32)
+    exact = np.abs(z.astype(np.float64)) * ndtr(-np.abs(z.astype(np.float64)))
+    assert np.max(np.abs(tail - exact)) <= 4e-8
+    g = (np.maximum(z, 0).astype(np.float64) - tail).astype(np.float32)
+    ref = z.astype(np.float64) * ndtr(z.astype(np.float64))
+    half = 0.5 * np.spacing(np.abs(ref).astype(np.float32)).astype(np.float64)
+    assert np.max(np.abs(g - ref) - half) <= 4e-8
