@@ -159,6 +159,9 @@ int izem_profile_read(izem_ctx *ctx, double *ms, int *count);
  * stencils of 6 values; out = (vminus, vplus) pairs */
 int izem_wenorec(izem_ctx *ctx, int n, int js, const double *vp, const double *vm,
                  double *out);
+/* the kernels' own exp (f = 0), log (1) and reciprocal (2) on n device values,
+ * for tests of the functions themselves.  No counterpart in the reference. */
+int izem_math(izem_ctx *ctx, int f, int n, const double *x, double *y);
 /* euler_LLF_x / _y / _z (module_weno.f90:537, 1055, 1595): x assigns fl,
  * y and z add to it; sensor: one byte per cell (logical shock_sensor) */
 int izem_euler_llf_x(izem_ctx *ctx, const double *dx_i, const double *T, const double *W_i,

@@ -15,7 +15,7 @@ EXPORTS = [
     "izem_create", "izem_destroy", "izem_synchronize", "izem_set_stream", "izem_status",
     "izem_time_state", "izem_get_time_state", "izem_set_time_state", "izem_profile",
     "izem_profile_read",
-    "izem_wenorec", "izem_euler_llf_x", "izem_euler_llf_y", "izem_euler_llf_z",
+    "izem_wenorec", "izem_math", "izem_euler_llf_x", "izem_euler_llf_y", "izem_euler_llf_z",
     "izem_viscflux", "izem_force_sumY", "izem_prim_inv_var", "izem_upd_prim_var_woT",
     "izem_comm_cons", "izem_upd_prim_var_ghost", "izem_prim_inv_var_mach", "izem_shock_sensor", "izem_shock_sensor_ducros", "izem_rk3", "izem_rhs",
     "izem_timestep", "izem_chem_setup", "izem_chem_tune", "izem_chem_stats", "izem_ckwyr", "izem_psr_batch", "izem_psr_batch_noalloc", "izem_chem_order", "izem_chem_order_read", "izem_reaction_dvode", "izem_step", "izem_flux_mode",
@@ -127,6 +127,7 @@ def _declare(lib):
     lib.izem_profile.argtypes = [vp, C.c_int]
     lib.izem_profile_read.argtypes = [vp, vp, vp]
     lib.izem_wenorec.argtypes = [vp, C.c_int, C.c_int, vp, vp, vp]
+    lib.izem_math.argtypes = [vp, C.c_int, C.c_int, vp, vp]
     for n in ("x", "y", "z"):
         getattr(lib, f"izem_euler_llf_{n}").argtypes = [vp] * 9
     lib.izem_viscflux.argtypes = [vp] * 9

@@ -2163,6 +2163,13 @@ __global__ void k_dt_final(double *__restrict__ red, double CFL, double CFLmin, 
 }
 
 
+// the functions of iz_math.h for their unit tests
+__global__ void k_math_batch(int f, int n, const double *__restrict__ x, double *__restrict__ y) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  y[t] = f == 0 ? d_exp(x[t]) : f == 1 ? d_log(x[t]) : d_rcp(x[t]);
+}
+
 // batched wenorec for unit tests of the reconstruction itself
 __global__ void k_wenorec_batch(int n, int js, const double *__restrict__ vp,
                                 const double *__restrict__ vm, double *__restrict__ out) {
@@ -2567,6 +2574,14 @@ extern "C" int izem_wenorec(izem_ctx *c, int n, int js, const double *vp, const 
   if (n == 0) return IZEM_OK;
   hipLaunchKernelGGL(k_wenorec_batch, dim3(iz_blocks(n, 256)), dim3(256), 0, c->stream, n, js,
                      vp, vm, out);
+  IZ_CHECK(hipGetLastError());
+  return IZEM_OK;
+}
+
+extern "C" int izem_math(izem_ctx *c, int f, int n, const double *x, double *y) {
+  if (!c || f < 0 || f > 2 || n < 0 || !x || !y) return IZEM_E_ARG;
+  if (n == 0) return IZEM_OK;
+  hipLaunchKernelGGL(k_math_batch, dim3(iz_blocks(n, 256)), dim3(256), 0, c->stream, f, n, x, y);
   IZ_CHECK(hipGetLastError());
   return IZEM_OK;
 }

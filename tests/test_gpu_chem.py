@@ -265,6 +265,49 @@ def test_reaction_dvode_vs_reference(oracle, adi, thd, mech):
     assert abs(DTmax_gpu - DTt) <= 2.0 * abs(DTd - DTt) + 10.0 * rtol * Tend
 
 
+def test_device_math(mech):
+    """d_exp, d_log and d_rcp as the GPU computes them (the hardware's
+    reciprocal refined, its ldexp and frexp) against extended precision: 0.8,
+    1.1 and 1 ulp over the arguments that iz_math.h states, and its corner
+    cases."""
+    import torch
+    s = _solver(mech)
+
+    def dev(f, x):
+        d = torch.tensor(np.ascontiguousarray(x), dtype=torch.float64, device="cuda:0")
+        y = torch.empty_like(d)
+        assert s.lib.izem_math(s.ctx, f, d.numel(), C.c_void_p(d.data_ptr()),
+                               C.c_void_p(y.data_ptr())) == 0
+        s.sync()
+        return y.cpu().numpy()
+
+    def ulps(y, ref):
+        return np.max(np.abs(y - ref) / np.spacing(np.abs(ref).astype(np.float64)))
+
+    rng = np.random.default_rng(7)
+    L = np.longdouble
+    half = np.log(2.0) * (np.arange(-1000, 1000) + 0.5)
+    x = np.concatenate([rng.uniform(-708, 709, 200000), rng.uniform(-2, 2, 200000), half,
+                        np.nextafter(half, 1e9), [0.0, -0.0, 1e-300]])
+    x = x[(x > -708) & (x < 709)]
+    assert ulps(dev(0, x), np.exp(x.astype(L))) <= 0.8
+    y = dev(0, np.array([710.0, 1e6, 1e9, -746.0, -1e6, -1e9, np.nan, -740.0]))
+    assert np.all(np.isinf(y[:3])) and np.all(y[3:6] == 0.0) and np.isnan(y[6])
+    assert abs(y[7] - np.exp(-740.0)) <= 5e-324
+    r = np.sqrt(0.5)
+    x = np.concatenate([np.exp(rng.uniform(-708, 709, 200000)),
+                        1.0 + rng.uniform(-0.3, 0.5, 200000),
+                        1.0 + rng.uniform(-1e-8, 1e-8, 1000), 2.0 ** np.arange(-1020, 1020),
+                        [r, np.nextafter(r, 0), np.nextafter(r, 1), 1e-310]])
+    x = x[x != 1.0]
+    assert ulps(dev(1, x), np.log(x.astype(L))) <= 1.1
+    y = dev(1, np.array([1.0, -1.0, np.nan, 0.0]))
+    assert y[0] == 0.0 and np.all(np.isnan(y[1:]))
+    x = np.exp(rng.uniform(-706, 706, 400000)) * rng.choice([-1.0, 1.0], 400000)
+    x = np.concatenate([x, rng.uniform(1, 2, 200000), 2.0 ** np.arange(-1020, 1020)])
+    assert ulps(dev(2, x), 1.0 / x.astype(L)) <= 1.0
+
+
 @pytest.mark.parametrize("kind,dts", [("2d", (1e-8, 1e-6, 1e-5)), ("3d", (1e-8, 2e-5))])
 @pytest.mark.parametrize("kinetics,waves", [(0, 1), (0, 2), (0, 4), (1, 1), (2, 1)])
 def test_flow_kernel_does_what_the_batch_kernel_does(adi, thd, mech, kind, dts, kinetics, waves):
