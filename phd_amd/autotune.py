@@ -2,11 +2,10 @@
 
 The persistent work-queue kernels (izem_psr_batch, izem_reaction_dvode) are
 compiled in several variants: table-driven kinetics at a register budget of
-1, 2 or 4 waves per SIMD, straight-line kinetics at 1 wave per SIMD with a
-finite-difference Jacobian or with its mass-fraction columns in closed form,
-and
-launched with a chosen number of resident 64-lane blocks per CU.  Which combination is fastest depends on
-the cells' stiffness (steps per cell), the device and the mechanism.  The
+1, 2 or 4 waves per SIMD, straight-line kinetics at 1 wave per SIMD with the
+Jacobian by finite differences or in closed form (the default), and launched
+with a chosen number of resident 64-lane blocks per CU.  Which combination is
+fastest depends on the cells' stiffness (steps per cell), the device and the mechanism.  The
 tuner times each candidate with izem_psr_batch on a sample of the cells the
 caller will integrate, keeps the fastest and applies it with
 izem_chem_tune; with that variant it then times izem_psr_batch's stiffness

@@ -1,7 +1,8 @@
 """Build the IZEM HIP library for gfx950 in-tree (phd_amd/libizem_hip.so).
 
 The flow and chemistry kernels are compiled with -ffp-contract=off.  The
-flow kernels reproduce the reference's rounding operation by operation.  The
+flow kernels that keep the reference's operation order (flow.hip says which)
+so reproduce its rounding; the others turn contraction on by a pragma.  The
 chemistry integrator and its straight-line kinetics turn contraction on
 expression by expression (a pragma), which rounds every inlined copy alike;
 left to the optimiser it was decided per copy, and one build took twice

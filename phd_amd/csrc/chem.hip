@@ -8,8 +8,8 @@
 // DVODE (chemkin/vode.f:4286) -> FUN (reaction_v.f:69-114) -> CKWYR
 // (vode.f:1797).  The integrator is this project's own implementation of
 // the Nordsieck-form BDF method (orders 1-5, fixed-leading-coefficient
-// rescaling on step changes, chord Newton with a finite-difference
-// Jacobian, weighted RMS error control); it agrees with DVODE to within the
+// rescaling on step changes, chord Newton with a Jacobian in closed form or
+// by finite differences, weighted RMS error control); it agrees with DVODE to within the
 // integration tolerance, not bit for bit.
 #include "izem_ctx.h"
 
@@ -163,8 +163,8 @@ struct ChemCount {
 
 // The work queue: a lane takes the next position from a device counter as
 // soon as its cell is finished, so lanes stay busy whatever the cells' step
-// counts.  Lanes from `lanes` on take none: a batch of fewer cells than
-// lanes is spread over every SIMD's wave (see chem_grid).
+// counts.  Lanes from `lanes` on take none: a small batch is spread over one
+// wave per CU (see persistent_grid).
 struct PsrQueue {
   int n, lanes;
   double *T;
@@ -702,7 +702,8 @@ extern "C" int izem_chem_order_read(izem_ctx *ctx, long cap, long *n, int *perm,
 }
 
 // blocks of a persistent launch over n cells, and the lanes of each that take
-// cells.  Up to one full wave per CU the cells are spread over all the CUs:
+// cells.  Up to one full wave per CU (64 cells per CU, whatever the tuned
+// blocks per CU) the cells are spread over all the CUs, one wave on each:
 // a wave of few cells seldom runs the branches (Jacobian, pivoting, third
 // corrector iteration) that only some cells need, and the launch lasts as
 // long as its slowest cell's chain of steps (1000 ignition cells: 10.9 ms

@@ -1,11 +1,14 @@
 // flow.hip -- FP64 HIP kernels of the IZEM reacting-flow right-hand side and
 // SSP-RK3 time step for CDNA4 (gfx950).
 //
-// Compiled with -ffp-contract=off: every kernel evaluates the reference's
-// expressions in the reference's order, so its results are the reference
-// algorithm's own roundings (flux parity is a bit-level property, not a
-// tolerance).  Reference: saras13015/Phd devel-izem/src (file:line cited
-// per kernel).
+// Compiled with -ffp-contract=off.  The Euler faces of izem_flux_mode 0, the
+// WENO7 build's other kernels, the stencils and the stage update evaluate the
+// reference's expressions in the reference's order, so their results are the
+// reference algorithm's own roundings.  With ng = 3 the Newton inversion and
+// the transport properties (in either flux mode) and the Euler faces of mode
+// 1 are re-associated and contracted where a pragma says so: they agree with
+// the reference to rounding.  Reference: saras13015/Phd devel-izem/src
+// (file:line cited per kernel).
 #include "flow_device.h"
 #include "iz_math.h"
 #include "izem_ctx.h"

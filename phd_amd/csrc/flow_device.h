@@ -1,8 +1,9 @@
 // flow_device.h -- per-cell FP64 device functions of the flow solver.
 //
-// Every function keeps the operation order of the reference Fortran (cited
-// per function) and is compiled with -ffp-contract=off, so that the results
-// are the reference's own roundings, not a re-associated variant.
+// Compiled with -ffp-contract=off; the functions keep the operation order of
+// the reference Fortran (cited per function), so that the results are the
+// reference's own roundings, but for d_newton_cell and d_thermo of the ng = 3
+// build, which are re-associated and contracted and agree to rounding.
 #pragma once
 
 #include "iz_math.h"

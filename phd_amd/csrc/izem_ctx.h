@@ -70,12 +70,17 @@ struct izem_ctx {
   int dsym;  // the binary diffusion fits are symmetric (D_kl = D_lk bit for bit)
   double *v0;
   // device words: Newton probe masks (blocking iterations [0..6] and
-  // negative temperatures [8..14] per domain), status, iteration counts
+  // negative temperatures [8..14] per domain), status, iteration counts.  The
+  // masks are zero between Newton passes: whatever probes into them must be
+  // followed by k_newton_repair on the same domains (newton_finish), which
+  // clears what it has read.
   unsigned long long *masks;
   int *negT_rec;  // cells recorded by the negative-temperature repair, per mask slot
   int *status;
   int *iters;
-  double *red;  // timestep reductions [24]
+  // timestep reductions [24], at their starting values between izem_timestep
+  // calls: k_dt_final puts them back after it has read them
+  double *red;
   double *ts;   // dt_4[4], dtmin, DTmax
   IzChem *chem;
   IzProf prof;
