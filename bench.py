@@ -187,8 +187,7 @@ def chem_vode_rate(s, thd, ncell: int):
     drho = d(rho)
     nst = torch.zeros(ncell, dtype=torch.int32, device="cuda:0")
     el, rc = {}, 0
-    # index order, then stiffest first (izem_chem_order): same end states,
-    # the waves of the second hold cells of like step counts
+    # index order, then stiffest first (izem_chem_order): same end states
     for order in (0, 1):
         dT, dY = d(T), d(Y)
         rc |= s.lib.izem_chem_order(s.ctx, order)
@@ -403,7 +402,7 @@ def main():
                     help="cells per side of the coupled learned-chemistry shear layer (0: skip)")
     ap.add_argument("--shear-steps", type=int, default=5)
     ap.add_argument("--flux-mode", type=int, default=1,
-                    help="Euler face kernels: 0 reference operation order (bit parity), "
+                    help="Euler face kernels: 0 reference operation order (bit parity of the faces), "
                          "1 structured projections (within 1e-12 of the reference)")
     ap.add_argument("--chem-tune", type=str, default=None,
                     help="waves,blocks_per_cu,jac_age,kinetics for the chemistry kernels "

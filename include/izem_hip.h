@@ -355,7 +355,9 @@ int izem_reaction_selec(izem_ctx *ctx, const double *dt, double scale, double *T
  * reference's dense characteristic projections in its summation order (bit
  * parity with it); 1 the projections through the structure of the left
  * eigenvectors (a shared scalar per stencil point; a tenth of the work,
- * results within rounding of mode 0).  No counterpart in the reference. */
+ * results within rounding of mode 0).  With ng = 3 the Newton inversion and
+ * the transport properties agree with the reference to rounding in either
+ * mode.  No counterpart in the reference. */
 int izem_flux_mode(izem_ctx *ctx, int mode);
 /* one iteration of the main loop (izem.f90:242-389): timestep, then with
  * chemistry reaction_selec(dt/2) -> rk3(dt) -> reaction_selec(dt/2)

@@ -45,7 +45,8 @@ class Options:
     rtol: float = 1.0e-6
     atol: float = 1.0e-12
     trim_box: int = 1   # reaction_dvode skips ng+1 planes at global faces
-    # Euler face kernels: 0 the reference's operation order (bit parity),
+    # Euler face kernels: 0 the reference's operation order (bit parity of the
+    # faces; with ng = 3 Newton and transport agree to rounding in either mode),
     # 1 projections through the eigenvectors' structure (izem_flux_mode)
     flux_mode: int = 0
     # WENO%SHOCK_SENSOR_TYPE (0 ADAMSSHARIFF, 1 DUCROS) and WENO%DUCROS_TREDUC
