@@ -357,6 +357,40 @@ def test_flow_kernel_does_what_the_batch_kernel_does(adi, thd, mech, kind, dts, 
         assert abs(steps[kinetics] - steps[0]) <= 0.03 * steps[0]
 
 
+@pytest.mark.parametrize("waves", [1, 2])
+def test_table_kinetics_keep_a_waves_lanes_in_step(mech, thd, waves):
+    """Table-driven reactors over a substep of a few steps: five times as many
+    cells as resident lanes take about five times as long as one cell per lane
+    (4.7 and 4.8 times).  Lanes that take cells one by one make a wave pay a
+    ten-evaluation Jacobian in almost every turn: 11.7 times at one wave per
+    SIMD, 9.9 at two.  Bar: 6."""
+    import time
+    import torch
+    s = _solver(mech)
+    assert s.lib.izem_chem_tune(s.ctx, waves, 4 * waves, 50, 0) == 0
+    lanes = 64 * 4 * waves * torch.cuda.get_device_properties(0).multi_processor_count
+    T, rho, Y = _cells(thd, 4096, seed=9)
+    d = lambda a: torch.tensor(np.ascontiguousarray(a), dtype=torch.float64, device="cuda:0")
+    T, rho, Y = d(T), d(rho), d(Y)
+    best = {}
+    for n in (lanes, 5 * lanes):
+        rep = -(-n // 4096)
+        r = rho.repeat(rep)[:n].contiguous()
+        for _ in range(4):
+            t, y = T.repeat(rep)[:n].contiguous(), Y.repeat(rep, 1)[:n].contiguous()
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            assert s.lib.izem_psr_batch(s.ctx, n, C.c_void_p(t.data_ptr()),
+                                        C.c_void_p(r.data_ptr()), C.c_void_p(y.data_ptr()),
+                                        1.2e-8, None) == 0
+            s.sync()
+            best[n] = min(best.get(n, 1e9), time.perf_counter() - t0)
+    print(f"tables, {waves} waves: {lanes} cells {1e3 * best[lanes]:.2f} ms, five times as many "
+          f"{1e3 * best[5 * lanes]:.2f}")
+    assert s.status() == 0
+    assert best[5 * lanes] <= 6.0 * best[lanes]
+
+
 def test_straight_line_kinetics_one_wave_only(mech):
     """The straight-line kinetics exist at one wave per SIMD only: asking for
     them at two or four is refused, and 'straight-line when available' at
