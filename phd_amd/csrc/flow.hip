@@ -865,12 +865,13 @@ __device__ inline void d_force_sumY(double *vc) {
 // T is negative after iteration it (the repair branch, :120-139).  Cells
 // stop once their increment has fallen far below eps: Newton's quadratic
 // contraction keeps all later increments below it.
+template <bool FRESH>
 __device__ inline unsigned long long d_newton_probe(const double *vc, double T, double eps,
                                                     unsigned long long &neg) {
   unsigned long long mask = 0ull;
   for (int it = 1; it <= 64; it++) {
     double cpv, h[IZ_NRV];
-    double DF = d_newton_cell(vc, T, cpv, h);
+    double DF = d_newton_cell<FRESH>(vc, T, cpv, h);
     T = T + DF;
     if (T < 0.0) neg |= 1ull << (it - 1);
     double e = sqrt(DF * DF);
@@ -993,7 +994,7 @@ k_force_probe(IzDims d, IzNewtonSet s, int fill, int forcesum, double *__restric
 #pragma unroll
       for (int l = IZ_NIV; l < IZ_NV; l++) v[l * d.nc + c] = vc[l];
     }
-    if (eps > 0.0) m |= d_newton_probe(vc, T[c], eps, neg);
+    if (eps > 0.0) m |= d_newton_probe<true>(vc, T[c], eps, neg);
   }
   block_or_probe(m, neg, masks + nset_slot(s, q));
 }
@@ -1042,7 +1043,7 @@ k_newton_apply(IzDims d, IzNewtonSet s, const double *__restrict__ v,
   W_i[c] = w;
   double Tc = T[c], cpv = 0.0, h[IZ_NRV];
   for (int it = 0; it < N; it++) {
-    double DF = d_newton_cell(vc, Tc, cpv, h);
+    double DF = d_newton_cell<true>(vc, Tc, cpv, h);
     Tc = Tc + DF;
   }
   T[c] = Tc;
@@ -1141,7 +1142,7 @@ k_newton_repair(IzDims d, IzNewtonSet set, int repair, double *__restrict__ v,
 #pragma unroll
       for (int l = 0; l < IZ_NV; l++) vc[l] = v[l * d.nc + c];
       double cpv, h[IZ_NRV];
-      const double DF = d_newton_cell(vc, T[c], cpv, h);
+      const double DF = d_newton_cell<true>(vc, T[c], cpv, h);
       cp[c] = cpv;
 #pragma unroll
       for (int l = 0; l < IZ_NRV; l++) ha[l * d.nc + c] = h[l];
@@ -1238,7 +1239,7 @@ __global__ void k_upd_prim_woT(IzDims d, IzBox b, const double *__restrict__ v,
   for (int l = 0; l < IZ_NRV; l++) w = w + (vc[IZ_NIV + l] / vc[0]) * c_thd.Wc_i[l];
   W_i[c] = w;
   double cpv, h[IZ_NRV];
-  (void)d_newton_cell(vc, T[c], cpv, h);
+  (void)d_newton_cell<false>(vc, T[c], cpv, h);
   cp[c] = cpv;
 #pragma unroll
   for (int l = 0; l < IZ_NRV; l++) ha[l * d.nc + c] = h[l];
@@ -1575,8 +1576,11 @@ __global__ void k_visc_prim(IzDims d, IzDomSet ds, const double *__restrict__ v,
 // WENO7 keeps the reference's expressions: its weights lift differences in
 // the last bit of the transport to 2e-10 of the state over 66 iterations of a
 // shock tube, and its time is in the faces.
+// FRESH: the tables at an index offset by z, see d_newton_cell
+template <bool FRESH = false>
 __device__ inline void d_transport(double rho, double T, double W_i, const double *Xa, double *dm,
-                                   double &mu, double &ct, bool want_mu, int sym) {
+                                   double &mu, double &ct, bool want_mu, int sym,
+                                   int z = 0) {
   const double eps = 1.0e-12;
   double Kl = 0.5 * 1.0e-5 / c_thd.laminf;
   double Ku = 1.0e-1 / c_thd.muinf;
@@ -1650,8 +1654,11 @@ __device__ inline void d_transport(double rho, double T, double W_i, const doubl
 // reciprocals per cell where the reference's expressions take 90, 162
 // divisions and 81 square roots (k_visc_fused at 160^3 1.53 -> 1.31 ms, of
 // which the rest is memory).
+// FRESH: the tables at an index offset by z, see d_newton_cell
+template <bool FRESH = false>
 __device__ inline void d_transport(double rho, double T, double W_i, const double *Xa, double *dm,
-                                   double &mu, double &ct, bool want_mu, int sym) {
+                                   double &mu, double &ct, bool want_mu, int sym,
+                                   int z = 0) {
 #pragma clang fp contract(on)
   const double eps = 1.0e-12;
   const double lt1 = d_log(T * c_thd.Tinf);
@@ -1671,9 +1678,9 @@ __device__ inline void d_transport(double rho, double T, double W_i, const doubl
     for (int m = 0; m < IZ_NRV; m++)
 #pragma unroll
       for (int l = m + 1; l < IZ_NRV; l++) {
-        const double e = d_exp(-fit(c_thd.CofD[m][l]));
+        const double e = d_exp(-fit(c_thd.CofD[FRESH ? m + z : m][l]));
         double f = e;
-        if (!sym) f = d_exp(-fit(c_thd.CofD[l][m]));
+        if (!sym) f = d_exp(-fit(c_thd.CofD[FRESH ? l + z : l][m]));
         s[m] += xe[l] * e;
         s[l] += xe[m] * f;
       }
@@ -1693,7 +1700,7 @@ __device__ inline void d_transport(double rho, double T, double W_i, const doubl
   double w1 = 0.0, cc = 0.0;
 #pragma unroll
   for (int l = 0; l < IZ_NRV; l++) {
-    const double c1 = d_exp(fit(c_thd.CofLam[l]));
+    const double c1 = d_exp(fit(c_thd.CofLam[FRESH ? l + z : l]));
     cc += Xa[l] * d_rcp(c1);
     w1 += Xa[l] * c1;
   }
@@ -1703,7 +1710,7 @@ __device__ inline void d_transport(double rho, double T, double W_i, const doubl
   double h[IZ_NRV], g[IZ_NRV];  // sqrt(eta) and its reciprocal
 #pragma unroll
   for (int l = 0; l < IZ_NRV; l++) {
-    h[l] = d_exp(0.5 * fit(c_thd.CofEta[l]));
+    h[l] = d_exp(0.5 * fit(c_thd.CofEta[FRESH ? l + z : l]));
     g[l] = d_rcp(h[l]);
   }
   double mus = 0.0;
@@ -1712,8 +1719,8 @@ __device__ inline void d_transport(double rho, double T, double W_i, const doubl
     double c4 = 0.0;
 #pragma unroll
     for (int l = 0; l < IZ_NRV; l++) {
-      const double c3 = 1.0 + c_thd.wilke_c1[m][l] * (h[m] * g[l]);
-      c4 += c3 * c3 * c_thd.wilke_c2[m][l] * Xa[l];
+      const double c3 = 1.0 + c_thd.wilke_c1[FRESH ? m + z : m][l] * (h[m] * g[l]);
+      c4 += c3 * c3 * c_thd.wilke_c2[FRESH ? m + z : m][l] * Xa[l];
     }
     mus += h[m] * h[m] * Xa[m] / c4;
   }
@@ -2030,7 +2037,7 @@ k_rhs_update(IzDims d, IzBand bd, int mode, const double *__restrict__ Fx, const
       if (forcesum) d_force_sumY(vc);
 #pragma unroll
       for (int m = 0; m < IZ_NV; m++) v[m * d.nc + c] = vc[m];
-      msk = d_newton_probe(vc, T[c], eps, neg);
+      msk = d_newton_probe<false>(vc, T[c], eps, neg);
     }
   }
   if (mode != 0) block_or_probe(msk, neg, mask);
@@ -2108,7 +2115,9 @@ k_dt_visc(IzDims d, int sym, const double *__restrict__ v, const double *__restr
 #pragma unroll
     for (int l = 0; l < IZ_NRV; l++)
       X[l] = v[(IZ_NIV + l) * d.nc + c] / (v[c] * W_i[c] * c_thd.Wc[l]);
-    d_transport(v[c], T[c], W_i[c], X, dm, mu, ct, false, sym);
+    int z = 0;
+    asm volatile("" : "+s"(z));
+    d_transport<true>(v[c], T[c], W_i[c], X, dm, mu, ct, false, sym, z);
     const double d2 = d_filter_delta2(d, dx_i, dy_i, dz_i, i, j, k);
 #pragma unroll
     for (int l = 0; l < IZ_NRV; l++) {

@@ -59,33 +59,37 @@ __device__ inline double d_dhpoly(const double *h, double t1, double t2, double 
 // Per-species enthalpy and cp contribution at nondimensional T, with the
 // four-branch NASA-7 evaluation of newton / upd_prim_var_woT / ha_scalar
 // (module_thermodynamics.f90:327-498, 522-689, 873-978).
-__device__ inline void d_species_h_cp(int is, double T, double Ya, double &h, double &cpc) {
+// FRESH: species is's tables at the index is + z (d_newton_cell)
+template <bool FRESH = false>
+__device__ inline void d_species_h_cp(int is, double T, double Ya, double &h, double &cpc,
+                                      int z = 0) {
+  const int q = FRESH ? is + z : is;
   const double Tinf_i = 1.0 / c_thd.Tinf, onethird = 1.0 / 3.0;
   double t1 = T * c_thd.Tinf, t2 = t1 * t1, t3 = t2 * t1, t4 = t3 * t1, t5 = t4 * t1;
-  const double *hl = c_thd.HeatCap[is][0], *hh = c_thd.HeatCap[is][1];
+  const double *hl = c_thd.HeatCap[q][0], *hh = c_thd.HeatCap[q][1];
   double fh = c_thd.Wc_i[is] * Tinf_i;
   double fc = Ya * c_thd.gam2 * c_thd.Wc_i[is];
   double hv = 0.0;
-  if (t1 < c_thd.Tpolymin[is]) {
-    t1 = c_thd.Tpolymin[is]; t2 = t1 * t1; t3 = t2 * t1; t4 = t3 * t1; t5 = t4 * t1;
+  if (t1 < c_thd.Tpolymin[q]) {
+    t1 = c_thd.Tpolymin[q]; t2 = t1 * t1; t3 = t2 * t1; t4 = t3 * t1; t5 = t4 * t1;
     double ha0 = d_hpoly(hl, t1, t2, t3, t4, t5, onethird);
     double dha0 = d_dhpoly(hl, t1, t2, t3, t4);
-    hv = hv + fh * (dha0 * (T * c_thd.Tinf - c_thd.Tpolymin[is]) + ha0);
+    hv = hv + fh * (dha0 * (T * c_thd.Tinf - c_thd.Tpolymin[q]) + ha0);
     double dcp0 = hl[1] + hl[2] * t1 * 2.0 + hl[3] * t2 * 3.0 + hl[4] * t3 * 4.0;
-    cpc = fc * (dcp0 * (T * c_thd.Tinf - c_thd.Tpolymin[is]) + dha0);
-  } else if (t1 < c_thd.Tpolylim[is]) {
+    cpc = fc * (dcp0 * (T * c_thd.Tinf - c_thd.Tpolymin[q]) + dha0);
+  } else if (t1 < c_thd.Tpolylim[q]) {
     hv = hv + fh * d_hpoly(hl, t1, t2, t3, t4, t5, onethird);
     cpc = fc * d_dhpoly(hl, t1, t2, t3, t4);
-  } else if (t1 < c_thd.Tpolymax[is]) {
+  } else if (t1 < c_thd.Tpolymax[q]) {
     hv = hv + fh * d_hpoly(hh, t1, t2, t3, t4, t5, onethird);
     cpc = fc * d_dhpoly(hh, t1, t2, t3, t4);
   } else {
-    t1 = c_thd.Tpolymax[is]; t2 = t1 * t1; t3 = t2 * t1; t4 = t3 * t1; t5 = t4 * t1;
+    t1 = c_thd.Tpolymax[q]; t2 = t1 * t1; t3 = t2 * t1; t4 = t3 * t1; t5 = t4 * t1;
     double ha0 = d_hpoly(hh, t1, t2, t3, t4, t5, onethird);
     double dha0 = d_dhpoly(hh, t1, t2, t3, t4);
-    hv = hv + fh * (dha0 * (T * c_thd.Tinf - c_thd.Tpolymax[is]) + ha0);
+    hv = hv + fh * (dha0 * (T * c_thd.Tinf - c_thd.Tpolymax[q]) + ha0);
     double dcp0 = hh[1] + hh[2] * t1 * 2.0 + hh[3] * t2 * 3.0 + hh[4] * t3 * 4.0;
-    cpc = fc * (dcp0 * (T * c_thd.Tinf - c_thd.Tpolymax[is]) + dha0);
+    cpc = fc * (dcp0 * (T * c_thd.Tinf - c_thd.Tpolymax[q]) + dha0);
   }
   h = hv;
 }
@@ -102,8 +106,9 @@ __device__ inline void d_ha_scalar(double temp, double *ha) {
 
 // newton (one cell): module_thermodynamics.f90:271-508.  Returns DF and the
 // cp / ha of this evaluation.
+template <bool FRESH>
 __device__ inline double d_newton_cell_ref(const double *vc, double T, double &cp_out,
-                                       double *ha_out) {
+                                       double *ha_out, int z) {
   const double gam2_i = 1.0 / c_thd.gam2;
   double rho_i = 1.0 / vc[0];
   double F = -vc[4] * rho_i + 0.5 * (vc[1] * vc[1] + vc[2] * vc[2] + vc[3] * vc[3]) *
@@ -116,7 +121,7 @@ __device__ inline double d_newton_cell_ref(const double *vc, double T, double &c
   for (int is = 0; is < IZ_NRV; is++) {
     double wrk1 = -T;
     double h, cpc;
-    d_species_h_cp(is, T, Ya[is], h, cpc);
+    d_species_h_cp<FRESH>(is, T, Ya[is], h, cpc, z);
     cp = cp + cpc;
     ha_out[is] = h;
     F = F + Ya[is] * (h + wrk1 * c_thd.Wc_i[is]);
@@ -134,13 +139,15 @@ __device__ inline double d_newton_cell_ref(const double *vc, double T, double &c
 // with the factors folded in, 15 operations per species where the general
 // evaluation (four ranges per species, its own powers and factors) takes
 // about 150
-template <int RANGE>
-__device__ inline void d_thermo_range(double t, const double *Y, double &cp, double *h) {
+// FRESH: the tables at the index l + z (d_newton_cell)
+template <int RANGE, bool FRESH>
+__device__ inline void d_thermo_range(double t, const double *Y, double &cp, double *h, int z) {
 #pragma clang fp contract(on)
   cp = 0.0;
 #pragma unroll
   for (int l = 0; l < IZ_NRV; l++) {
-    const double *a = c_thx.h[RANGE][l], *b = c_thx.c[RANGE][l];
+    const int q = FRESH ? l + z : l;
+    const double *a = c_thx.h[RANGE][q], *b = c_thx.c[RANGE][q];
     h[l] = ((((a[4] * t + a[3]) * t + a[2]) * t + a[1]) * t + a[0]) * t + a[5];
     cp += Y[l] * ((((b[4] * t + b[3]) * t + b[2]) * t + b[1]) * t + b[0]);
   }
@@ -150,18 +157,32 @@ __device__ inline bool d_thermo_in_range(double T) {
   const double t = T * c_thd.Tinf;
   return t >= c_thx.tlo && t < c_thx.thi;
 }
-__device__ inline void d_thermo(double T, const double *Y, double &cp, double *h) {
+template <bool FRESH = false>
+__device__ inline void d_thermo(double T, const double *Y, double &cp, double *h, int z = 0) {
   const double t = T * c_thd.Tinf;
-  if (t < c_thx.tlim) d_thermo_range<0>(t, Y, cp, h);
-  else d_thermo_range<1>(t, Y, cp, h);
+  if (t < c_thx.tlim) d_thermo_range<0, FRESH>(t, Y, cp, h, z);
+  else d_thermo_range<1, FRESH>(t, Y, cp, h, z);
 }
 #endif
 
 // the increment by the folded polynomials where they hold, else (and for
 // WENO7, whose runs follow the reference's roundings through shocks) in the
-// reference's expressions
+// reference's expressions.
+// FRESH: the species' tables are read at an index the compiler does not know
+// to be 0.  Left to itself it takes their few hundred loads out of the Newton
+// iteration and the loop over cells, where they fill the scalar registers and
+// spill (760 of them in k_force_probe, 250 VGPRs): a launch over one small domain
+// spent most of its time on that.  k_force_probe / k_newton_apply on the
+// interior of a 192^2 box 14.3 / 12.2 -> 6.9 / 6.1 us (153 and 138 VGPRs, 75 and
+// no spills), the interior's apply at 256^3 1.55 -> 1.25 ms; k_dt_visc, whose
+// transport tables are read so too, 30.5 -> 24.6 us and 3.26 -> 2.81 ms.  Not
+// in k_rhs_update, which waits for memory and loses with it (6.70 -> 7.03 ms
+// at 256^3).
+template <bool FRESH>
 __device__ inline double d_newton_cell(const double *vc, double T, double &cp_out,
                                        double *ha_out) {
+  int z = 0;
+  if constexpr (FRESH) asm volatile("" : "+s"(z));
 #if IZ_NG == 3
   if (d_thermo_in_range(T)) {
 #pragma clang fp contract(on)
@@ -171,7 +192,7 @@ __device__ inline double d_newton_cell(const double *vc, double T, double &cp_ou
     double Ya[IZ_NRV], w = 0.0;
 #pragma unroll
     for (int l = 0; l < IZ_NRV; l++) Ya[l] = vc[IZ_NIV + l] * rho_i;
-    d_thermo(T, Ya, cp_out, ha_out);
+    d_thermo<FRESH>(T, Ya, cp_out, ha_out, z);
 #pragma unroll
     for (int l = 0; l < IZ_NRV; l++) {
       F += Ya[l] * (ha_out[l] - T * c_thd.Wc_i[l]);
@@ -180,7 +201,7 @@ __device__ inline double d_newton_cell(const double *vc, double T, double &cp_ou
     return F / (w - cp_out * (1.0 / c_thd.gam2));
   }
 #endif
-  return d_newton_cell_ref(vc, T, cp_out, ha_out);
+  return d_newton_cell_ref<FRESH>(vc, T, cp_out, ha_out, z);
 }
 
 // ------------------------------------------------------------------ WENO
